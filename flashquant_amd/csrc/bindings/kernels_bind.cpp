@@ -169,6 +169,39 @@ at::Tensor tq4_decompress_rotated(const at::Tensor& packed, const at::Tensor& no
     return result;
 }
 
+// Keys and values of a paged cache (num_blocks, block_size, H * (D + 8)) as (num_blocks * block_size, H, D) tensors
+// (_decompress_cache, src/flashquant/vllm/impl.py:265-318), in rotated space when `rotation` is None.
+std::tuple<at::Tensor, at::Tensor> tq4_decompress_cache(const at::Tensor& kv_cache, int64_t num_kv_heads, int64_t head_dim,
+                                                        const at::Tensor& centroids, const std::optional<at::Tensor>& rotation,
+                                                        at::ScalarType dtype, const std::optional<at::Tensor>& out_k,
+                                                        const std::optional<at::Tensor>& out_v) {
+    fqbind::require_gpu(kv_cache, "kv_cache");
+    const int64_t H = num_kv_heads, D = head_dim;
+    require(kv_cache.dim() == 3 && kv_cache.scalar_type() == at::kByte && H > 0 && D > 0 && kv_cache.size(2) == H * (D + 8),
+            "kv_cache must be uint8 of shape (num_blocks, block_size, num_kv_heads * (head_dim + 8))");
+    require(centroids.scalar_type() == at::kFloat && centroids.numel() == 16, "centroids must be 16 float32 values");
+    require(dtype == at::kHalf || dtype == at::kBFloat16 || (dtype == at::kFloat && !rotation.has_value()),
+            "decompress_cache: dtype must be float16 or bfloat16 (or float32 in rotated space)");
+    c10::DeviceGuard guard(kv_cache.device());
+    const at::Tensor cache = kv_cache.contiguous();
+    const at::Tensor cc = centroids.to(kv_cache.device()).contiguous();
+    const int64_t slots = cache.size(0) * cache.size(1);
+    RotationArg rot;
+    if (rotation.has_value()) rot = rotation_arg(*rotation, kv_cache.device(), D);
+    auto result = [&](const std::optional<at::Tensor>& out) {
+        if (!out.has_value()) return at::empty({slots, H, D}, cache.options().dtype(dtype));
+        require(out->is_cuda() && out->is_contiguous() && out->scalar_type() == dtype && out->numel() >= slots * H * D,
+                "out must be a contiguous GPU tensor of the requested dtype with room for (slots, H, D)");
+        return out->flatten().narrow(0, 0, slots * H * D).view({slots, H, D});
+    };
+    at::Tensor k = result(out_k), v = result(out_v);
+    const int st = fq_tq4_decompress_cache(cache.data_ptr<uint8_t>(), cc.data_ptr<float>(), rot.ptr, rot.col_major,
+                                           k.data_ptr(), v.data_ptr(), fqbind::dtype_code(dtype, "tq4_decompress_cache"),
+                                           slots, int(H), int(D), fqbind::current_stream(kv_cache));
+    fqbind::raise_on_error(st, "tq4_decompress_cache");
+    return {k, v};
+}
+
 at::Tensor tq4_decompress(const at::Tensor& packed, const at::Tensor& norms, const at::Tensor& centroids,
                           at::ScalarType dtype, const std::optional<at::Tensor>& out) {
     fqbind::require_gpu(packed, "packed");
@@ -806,6 +839,10 @@ void bind_kernels(py::module_& m) {
     m.def("tq4_compress_store", &tq4_compress_store, py::arg("key"), py::arg("value"), py::arg("rotation_T_even"),
           py::arg("rotation_T_odd"), py::arg("boundaries"), py::arg("kv_cache"), py::arg("slot_mapping"),
           "Compress key and value (N, H, D) and write them into the packed paged cache at slot_mapping");
+    m.def("tq4_decompress_cache", &tq4_decompress_cache, py::arg("kv_cache"), py::arg("num_kv_heads"), py::arg("head_dim"),
+          py::arg("centroids"), py::arg("rotation"), py::arg("dtype"), py::arg("out_k") = py::none(),
+          py::arg("out_v") = py::none(),
+          "Keys and values of a paged TQ4 cache as (slots, H, D) tensors in dtype; rotated space when rotation is None.");
     m.def("tq4_decompress", &tq4_decompress, py::arg("packed"), py::arg("norms"), py::arg("centroids"),
           py::arg("dtype"), py::arg("out") = py::none(),
           "TQ4 decompress to (N, H, D) in dtype, rotated space.");

@@ -52,10 +52,23 @@ __device__ __forceinline__ float two_roundings(float c, float n) {
 // register i of lane half h holds coordinate 16 h + i.
 __device__ __forceinline__ int row_to_coord(int r) { return 16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3); }
 
-template <int D, int DT>
+// The packed rows of a launch.  Contiguous: `packed` (M, D/2) and `norms` (M,).  CACHE: rows 0 .. M-1 are the keys
+// and M .. 2M-1 (tiles from `num_tiles / 2` on) the values of a paged cache's token rows
+// [K idx H*D/2 | K norm H*4 | V idx H*D/2 | V norm H*4], read where they are; row (t, h) of either lies
+// t * row_bytes + h * D/2 (norm: + 4 h) behind its section's start.  Bound by the launch's start and end (about 8 tiles
+// a workgroup) and then by HBM: 24,016 tokens x 8 heads of 128 in bf16 took 89 us as four strided copies of the
+// sections and a launch each for keys and values, 38 us this way (124 MB: 25 us at the rate of a plain copy).
+struct DecRotSource {
+    const uint8_t* packed;
+    const float* norms;
+    int H;                    // CACHE: KV heads, and
+    float inv_H;              // 1 / H
+};
+
+template <int D, int DT, bool CACHE>
 __global__ __launch_bounds__(DecRotCfg<D>::THREADS) void tq4_decompress_rotate_kernel(
-    const uint32_t* __restrict__ packed, const float* __restrict__ norms, const float* __restrict__ centroids,
-    const float* __restrict__ rotation, int col_major, uint16_t* __restrict__ out, int64_t M, int64_t num_tiles) {
+    const DecRotSource src, const float* __restrict__ centroids, const float* __restrict__ rotation, int col_major,
+    uint16_t* __restrict__ out, uint16_t* __restrict__ out_v, int64_t M, int64_t num_tiles) {
     using C = DecRotCfg<D>;
     __shared__ __attribute__((aligned(16))) uint8_t xs[2][C::TT * C::STRIDE];   // dequantised rows, 16-bit
     __shared__ __attribute__((aligned(16))) uint8_t os[C::TT * C::STRIDE];      // rotated rows, 16-bit
@@ -75,11 +88,23 @@ __global__ __launch_bounds__(DecRotCfg<D>::THREADS) void tq4_decompress_rotate_k
     {
         const int j = 32 * cb + row_to_coord(n32);
 #pragma unroll
-        for (int ks = 0; ks < C::NK; ++ks)
+        for (int ks = 0; ks < C::NK; ++ks) {
+            // a lane's eight elements of a k-step are contiguous in a column-major matrix (what a QR factor is);
+            // asked for one by one they were 64 requests of 64 lines each in front of the first tile
+            float rk[8];
+            const int k0 = 16 * ks + 8 * kg;
+            if (col_major) {
+                const float4v lo = *reinterpret_cast<const float4v*>(rotation + int64_t(j) * D + k0);
+                const float4v hi = *reinterpret_cast<const float4v*>(rotation + int64_t(j) * D + k0 + 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { rk[e] = lo[e]; rk[4 + e] = hi[e]; }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) rk[e] = rotation[int64_t(k0 + e) * D + j];
+            }
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const int k = 16 * ks + 8 * kg + e;
-                const float r = col_major ? rotation[k + int64_t(j) * D] : rotation[int64_t(k) * D + j];
+                const float r = rk[e];
                 if constexpr (kBf16) {
                     const uint16_t t0 = float_to_bf16(r);
                     const uint16_t t1 = float_to_bf16(r - bf16_to_float(t0));
@@ -91,20 +116,45 @@ __global__ __launch_bounds__(DecRotCfg<D>::THREADS) void tq4_decompress_rotate_k
                     a_lo[ks][e] = _Float16((r - float(hi)) * 4096.0f);
                 }
             }
+        }
     }
     __syncthreads();
 
     // ---- staging: unit u of a tile = packed dword u % UPR of tile row u / UPR ------------------
     uint32_t word[C::UPT];
     float nrm[C::UPT];
+    const int64_t half_tiles = CACHE ? num_tiles / 2 : num_tiles;
     auto issue_loads = [&](int64_t tile) {
+        if constexpr (CACHE) {
+            // (t0, h0) of the tile's first row once, wave-uniform; a row's own from there with one float32
+            // multiply (its numerator stays below 64 + H: exact)
+            const bool is_v = tile >= half_tiles;
+            const uint32_t row0 = uint32_t(is_v ? tile - half_tiles : tile) * uint32_t(C::TT);
+            const uint32_t t0 = row0 / uint32_t(src.H), h0 = row0 - t0 * uint32_t(src.H);
+            const int row_bytes = src.H * (D + 8);
+            const uint8_t* base = src.packed + int64_t(t0) * row_bytes + (is_v ? src.H * (D / 2 + 4) : 0);
+#pragma unroll
+            for (int i = 0; i < C::UPT; ++i) {
+                const int u = tid + i * C::THREADS;
+                const int r = u / C::UPR;
+                const bool live = int64_t(row0) + r < M;
+                const int local = live ? int(h0) + r : int(h0);
+                const int dt = int((float(local) + 0.5f) * src.inv_H), h = local - dt * src.H;
+                const uint8_t* row = base + dt * row_bytes;
+                word[i] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(row + h * (D / 2)) + u % C::UPR);
+                nrm[i] = *reinterpret_cast<const float*>(row + src.H * (D / 2) + 4 * h);
+            }
+            return;
+        }
+        const uint32_t* packed = reinterpret_cast<const uint32_t*>(src.packed);
+        const float* norms = src.norms;
         if ((tile + 1) * C::TT <= M) {          // uniform: a whole tile needs no per-row conditions
-            const uint32_t* src = packed + tile * C::TT * C::UPR;
+            const uint32_t* first = packed + tile * C::TT * C::UPR;
             const float* nsrc = norms + tile * C::TT;
 #pragma unroll
             for (int i = 0; i < C::UPT; ++i) {
                 const int u = tid + i * C::THREADS;
-                word[i] = __builtin_nontemporal_load(src + u);
+                word[i] = __builtin_nontemporal_load(first + u);
                 nrm[i] = nsrc[u / C::UPR];
             }
             return;
@@ -131,14 +181,17 @@ __global__ __launch_bounds__(DecRotCfg<D>::THREADS) void tq4_decompress_rotate_k
             *reinterpret_cast<uint4v*>(&xs[buf][(u / C::UPR) * C::STRIDE + (u % C::UPR) * 16]) = uint4v{h[0], h[1], h[2], h[3]};
         }
     };
-    auto store_tile = [&](int64_t tile) {
+    auto store_tile = [&](int64_t any_tile) {
         constexpr int OC = D / 8;            // 16-byte chunks per output row
+        const bool is_v = CACHE && any_tile >= half_tiles;
+        const int64_t tile = is_v ? any_tile - half_tiles : any_tile;
+        uint16_t* dst = is_v ? out_v : out;
         for (int c = tid; c < C::TT * OC; c += C::THREADS) {
             const int r = c / OC, q = c % OC;
             const int64_t row = tile * C::TT + r;
             if (row < M) {
                 const uint4v v = *reinterpret_cast<const uint4v*>(&os[r * C::STRIDE + q * 16]);
-                __builtin_nontemporal_store(v, reinterpret_cast<uint4v*>(out + row * D) + q);
+                __builtin_nontemporal_store(v, reinterpret_cast<uint4v*>(dst + row * D) + q);
             }
         }
     };
@@ -195,19 +248,35 @@ __global__ __launch_bounds__(DecRotCfg<D>::THREADS) void tq4_decompress_rotate_k
     }
 }
 
-template <int D, int DT>
-int launch_decompress_rotate(const uint8_t* packed, const float* norms, const float* centroids, const float* rotation,
-                             int col_major, void* out, int64_t M, hipStream_t s) {
+template <int D, int DT, bool CACHE>
+int launch_decompress_rotate(const DecRotSource& src, const float* centroids, const float* rotation, int col_major,
+                             void* out, void* out_v, int64_t M, hipStream_t s) {
     using C = DecRotCfg<D>;
-    const int64_t tiles = (M + C::TT - 1) / C::TT;
+    const int64_t tiles = (M + C::TT - 1) / C::TT * (CACHE ? 2 : 1);
     // workgroups per CU: three fit the LDS at head_dim <= 128; the fp16 route holds two
     // accumulators per wavefront and runs faster with two
     const int64_t cap = int64_t(fq_host::device_cu_count()) * ((D == 256 || DT == FQ_F16) ? 2 : 3);
     const unsigned grid = unsigned(tiles < cap ? tiles : cap);
-    hipLaunchKernelGGL((tq4_decompress_rotate_kernel<D, DT>), dim3(grid), dim3(C::THREADS), 0, s,
-                       reinterpret_cast<const uint32_t*>(packed), norms, centroids, rotation, col_major,
-                       static_cast<uint16_t*>(out), M, tiles);
+    hipLaunchKernelGGL((tq4_decompress_rotate_kernel<D, DT, CACHE>), dim3(grid), dim3(C::THREADS), 0, s, src, centroids,
+                       rotation, col_major, static_cast<uint16_t*>(out), static_cast<uint16_t*>(out_v), M, tiles);
     return fq_host::check_launch();
+}
+
+template <bool CACHE>
+int decompress_rotate_any(const DecRotSource& src, const float* centroids, const float* rotation, int col_major, void* out,
+                          void* out_v, int dtype, int64_t M, int D, hipStream_t s) {
+#define FQ_DECROT_CASE(DD)                                                                                              \
+    case DD:                                                                                                            \
+        return dtype == FQ_F16                                                                                          \
+                   ? launch_decompress_rotate<DD, FQ_F16, CACHE>(src, centroids, rotation, col_major, out, out_v, M, s) \
+                   : launch_decompress_rotate<DD, FQ_BF16, CACHE>(src, centroids, rotation, col_major, out, out_v, M, s);
+    switch (D) {
+        FQ_DECROT_CASE(64)
+        FQ_DECROT_CASE(128)
+        FQ_DECROT_CASE(256)
+        default: return FQ_ERR_UNSUPPORTED_DIM;
+    }
+#undef FQ_DECROT_CASE
 }
 
 }  // namespace
@@ -225,17 +294,17 @@ extern "C" int fq_tq4_decompress_rotated(const uint8_t* packed, const float* nor
     if (!fq_host::aligned(packed, 4) || !fq_host::aligned(norms, 4) || !fq_host::aligned(rotation, 4) ||
         !fq_host::aligned(out, 16))
         return FQ_ERR_MISALIGNED;
-    hipStream_t s = static_cast<hipStream_t>(stream);
-#define FQ_DECROT_CASE(DD)                                                                                          \
-    case DD:                                                                                                        \
-        return out_dtype == FQ_F16                                                                                  \
-                   ? launch_decompress_rotate<DD, FQ_F16>(packed, norms, centroids, rotation, rotation_col_major, out, M, s) \
-                   : launch_decompress_rotate<DD, FQ_BF16>(packed, norms, centroids, rotation, rotation_col_major, out, M, s);
-    switch (D) {
-        FQ_DECROT_CASE(64)
-        FQ_DECROT_CASE(128)
-        FQ_DECROT_CASE(256)
-        default: return FQ_ERR_UNSUPPORTED_DIM;
-    }
-#undef FQ_DECROT_CASE
+    const DecRotSource src{packed, norms, 1, 1.0f};
+    return decompress_rotate_any<false>(src, centroids, rotation, rotation_col_major, out, nullptr, out_dtype, M, D,
+                                        static_cast<hipStream_t>(stream));
 }
+
+namespace fq_host {
+// The keys and values of `tokens` cache rows, rotated back (fq_tq4_decompress_cache has checked the arguments).
+int decompress_cache_rotated(const uint8_t* cache, int64_t tokens, int H, int D, const float* centroids,
+                             const float* rotation, int col_major, void* out_k, void* out_v, int dtype, void* stream) {
+    const fq::DecRotSource src{cache, nullptr, H, 1.0f / float(H)};
+    return fq::decompress_rotate_any<true>(src, centroids, rotation, col_major, out_k, out_v, dtype, tokens * H, D,
+                                           static_cast<hipStream_t>(stream));
+}
+}  // namespace fq_host

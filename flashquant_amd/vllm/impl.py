@@ -84,22 +84,13 @@ class TQ4AttentionKernels:
                          out_k: Optional[torch.Tensor] = None,
                          out_v: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
         """(key_cache, value_cache) of shape (NB, BS, H, D) in ``compute_dtype``: rotated space, or
-        the original space with ``apply_rotation`` (then one launch per tensor does both steps)."""
+        the original space with ``apply_rotation``; one launch for both tensors, straight from the cache rows."""
         require_gpu(kv_cache, "kv_cache")
-        C = native()
         nb, bs, _ = kv_cache.shape
         h, d = self.num_kv_heads, self.head_size
-        flat = kv_cache.reshape(nb * bs, self.total_bytes)
-        k_packed = flat[:, :self.k_idx_end].contiguous().reshape(-1, h, d // 2)
-        k_norms = flat[:, self.k_idx_end:self.k_norm_end].contiguous().view(torch.float32).reshape(-1, h, 1)
-        v_packed = flat[:, self.k_norm_end:self.v_idx_end].contiguous().reshape(-1, h, d // 2)
-        v_norms = flat[:, self.v_idx_end:].contiguous().view(torch.float32).reshape(-1, h, 1)
-        if apply_rotation:
-            key_out = C.tq4_decompress_rotated(k_packed, k_norms, self.centroids, self.rotation, compute_dtype, out_k)
-            value_out = C.tq4_decompress_rotated(v_packed, v_norms, self.centroids, self.rotation, compute_dtype, out_v)
-        else:
-            key_out = C.tq4_decompress(k_packed, k_norms, self.centroids, compute_dtype, out_k)
-            value_out = C.tq4_decompress(v_packed, v_norms, self.centroids, compute_dtype, out_v)
+        key_out, value_out = native().tq4_decompress_cache(kv_cache, h, d, self.centroids,
+                                                           self.rotation if apply_rotation else None, compute_dtype,
+                                                           out_k, out_v)
         return key_out.reshape(nb, bs, h, d), value_out.reshape(nb, bs, h, d)
 
 

@@ -234,6 +234,17 @@ int fq_tq4_decompress_rotated(const uint8_t* packed, const float* norms, const f
                               void* out, int out_dtype, int64_t M, int D, void* stream);
 
 /*
+ * The keys and values of a whole paged cache in the compute dtype, one launch for both: _decompress_cache,
+ * src/flashquant/vllm/impl.py:265-318 (the four section slices, tq4_decompress, and with apply_rotation the
+ * product with the rotation).
+ *   kv_cache   (num_slots, H*(D+8)) u8 token rows; num_slots = num_blocks * block_size
+ *   rotation   (D, D) f32, or NULL: the output stays in rotated space
+ *   out_k/v    (num_slots, H, D) out_dtype (FQ_F32 only without rotation), 16-byte aligned
+ */
+int fq_tq4_decompress_cache(const uint8_t* kv_cache, const float* centroids, const float* rotation, int rotation_col_major,
+                            void* out_k, void* out_v, int out_dtype, int64_t num_slots, int H, int D, void* stream);
+
+/*
  * Fused TQ4 attention (prefill): un-rotated query, packed keys and values,
  * original-space output.  Takes the role of the reference's fused launcher
  * (csrc/cuda/fused_tq_attention.cu:468-479); operator defined by

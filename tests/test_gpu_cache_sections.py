@@ -1,0 +1,60 @@
+"""Operators that read or write the sections of paged token rows in place, against the same operators on
+contiguous copies of those sections (bit for bit)."""
+import math
+
+import pytest
+import torch
+
+from flashquant_amd import kernels as K
+from flashquant_amd.vllm.impl import TQ4AttentionKernels
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def random_cache(pages, page, h, d, seed):
+    g = torch.Generator().manual_seed(seed)
+    row = h * (d + 8)
+    cache = torch.randint(0, 256, (pages, page, row), dtype=torch.uint8, generator=g)
+    flat = cache.view(-1, row)
+    n = flat.shape[0]
+    sections = []
+    for first in (0, h * (d // 2 + 4)):
+        norms = torch.rand(n, h, generator=g) * 30 + 0.01
+        flat[:, first + h * d // 2: first + h * (d // 2 + 4)] = norms.view(torch.uint8)
+        sections += [flat[:, first: first + h * d // 2].reshape(n, h, d // 2).contiguous(), norms.view(n, h, 1)]
+    return cache.to(DEV), [t.to(DEV) for t in sections]
+
+
+# one token, a tile that ends inside a token, several tiles of a workgroup, heads that do not divide a tile
+@pytest.mark.parametrize("pages,page,h", [(1, 1, 1), (3, 16, 1), (1, 8, 3), (5, 16, 8), (200, 32, 8), (7, 16, 40), (40, 16, 5)])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_decompress_cache_equals_decompress_of_its_sections(pages, page, h, d):
+    layer = TQ4AttentionKernels(h, d, 1.0 / math.sqrt(d), torch.device(DEV))
+    cache, (kp, kn, vp, vn) = random_cache(pages, page, h, d, 7 * pages + h + d)
+    for dtype in (torch.bfloat16, torch.float16):
+        for rotate in (True, False):
+            k, v = layer.decompress_cache(cache, dtype, apply_rotation=rotate)
+            assert k.shape == v.shape == (pages, page, h, d) and k.dtype == dtype
+            for got, p, n in ((k, kp, kn), (v, vp, vn)):
+                want = (K.tq4_decompress_rotated(p, n, layer.centroids, layer.rotation, dtype) if rotate
+                        else K.tq4_decompress(p, n, layer.centroids, dtype))
+                assert torch.equal(got.view(-1, h, d), want)
+    k, v = layer.decompress_cache(cache, torch.float32, apply_rotation=False)
+    assert torch.equal(v.view(-1, h, d), K.tq4_decompress(vp, vn, layer.centroids, torch.float32))
+    # given outputs are written in place, a little beyond them stays as it is
+    n = pages * page * h * d
+    big = torch.full((2, n + 64), 7.0, dtype=torch.bfloat16, device=DEV)
+    k, v = layer.decompress_cache(cache, torch.bfloat16, out_k=big[0], out_v=big[1])
+    assert k.data_ptr() == big.data_ptr() and (big[:, n:] == 7).all()
+    assert torch.equal(v.view(-1, h, d), K.tq4_decompress_rotated(vp, vn, layer.centroids, layer.rotation, torch.bfloat16))
+
+
+def test_decompress_cache_of_no_pages_and_argument_errors():
+    layer = TQ4AttentionKernels(8, 128, 1.0, torch.device(DEV))
+    k, v = layer.decompress_cache(torch.empty(0, 16, 8 * 136, dtype=torch.uint8, device=DEV), torch.bfloat16)
+    assert k.shape == v.shape == (0, 16, 8, 128)
+    with pytest.raises(ValueError):
+        layer.decompress_cache(torch.zeros(1, 16, 8 * 136, dtype=torch.uint8, device=DEV), torch.float32)
+    with pytest.raises(ValueError):
+        layer.decompress_cache(torch.zeros(1, 16, 7 * 136, dtype=torch.uint8, device=DEV), torch.bfloat16)
