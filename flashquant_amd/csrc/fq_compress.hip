@@ -86,6 +86,7 @@ constexpr int kBucketCells = 128;
 constexpr int kBucketCopies = 32;
 struct BucketTable {
     uint2v cell[kBucketCells * kBucketCopies];   // x = threshold bits, y = base count
+    uint2v plain[kBucketCells];                  // one of each, what the copies are made from
     float bnd[16];
     float inv_w;
     float offset;
@@ -129,11 +130,18 @@ __device__ __forceinline__ void build_bucket_table(BucketTable& t, const float* 
             }
         }
         if (inside > 1 || !(span > 0.0f)) t.slow = 1;
-        for (int k = 0; k < kBucketCopies; ++k) t.cell[c * kBucketCopies + k] = uint2v{float_to_bits(thr), uint32_t(base)};
+        t.plain[c] = uint2v{float_to_bits(thr), uint32_t(base)};
     }
     if (tid == 0) {
         t.inv_w = inv_w;
         t.offset = offset;
+    }
+    __syncthreads();
+    // the copies, 16 bytes a lane and consecutive lanes side by side (each thread writing the 32 copies of its own
+    // cell, 256 bytes from its neighbour's, put all lanes of a store into the same two banks)
+    for (int i = tid; i < kBucketCells * kBucketCopies / 2; i += nthreads) {
+        const uint2v v = t.plain[i / (kBucketCopies / 2)];
+        reinterpret_cast<uint4v*>(&t.cell[0])[i] = uint4v{v.x, v.y, v.x, v.y};
     }
     __syncthreads();
 }
