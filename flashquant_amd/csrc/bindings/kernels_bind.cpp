@@ -607,6 +607,30 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> prod_compress(const at::Tensor& x
     return {packed, norms, gam};
 }
 
+void prod_store_rows(const at::Tensor& kv_cache, const at::Tensor& slot_mapping, const at::Tensor& k_packed,
+                     const at::Tensor& k_norms, const at::Tensor& k_gamma, const at::Tensor& v_packed,
+                     const at::Tensor& v_norms) {
+    fqbind::require_gpu(kv_cache, "kv_cache");
+    require(k_packed.dim() == 3 && k_packed.scalar_type() == at::kByte && k_packed.size(2) % 4 == 0 && k_packed.size(1) > 0,
+            "k_packed must be uint8 of shape (N, H, D/2), D a multiple of 8");
+    const int64_t N = k_packed.size(0), H = k_packed.size(1), half = k_packed.size(2), row_bytes = H * (2 * half + 12);
+    require(v_packed.scalar_type() == at::kByte && v_packed.numel() == k_packed.numel(), "v_packed must be uint8 with the size of k_packed");
+    for (const at::Tensor* t : {&k_norms, &k_gamma, &v_norms})
+        require(t->scalar_type() == at::kFloat && t->numel() == N * H, "norms must be float32 with one value per (token, head)");
+    require(kv_cache.scalar_type() == at::kByte && kv_cache.is_contiguous() && kv_cache.numel() % row_bytes == 0,
+            "kv_cache must be a contiguous uint8 tensor of token rows of H * (D + 12) bytes");
+    require(slot_mapping.numel() == N, "slot_mapping must hold one slot per token");
+    c10::DeviceGuard guard(kv_cache.device());
+    const auto dev = kv_cache.device();
+    const at::Tensor sm = slot_mapping.to(dev, at::kLong).contiguous();
+    const at::Tensor kp = k_packed.to(dev).contiguous(), vp = v_packed.to(dev).contiguous();
+    const at::Tensor kn = k_norms.to(dev).contiguous(), kg = k_gamma.to(dev).contiguous(), vn = v_norms.to(dev).contiguous();
+    const int st = fq_prod_store_rows(kv_cache.data_ptr<uint8_t>(), sm.data_ptr<int64_t>(), kp.data_ptr<uint8_t>(),
+                                      kn.data_ptr<float>(), kg.data_ptr<float>(), vp.data_ptr<uint8_t>(), vn.data_ptr<float>(),
+                                      N, kv_cache.numel() / row_bytes, int(H), int(2 * half), fqbind::current_stream(kv_cache));
+    fqbind::raise_on_error(st, "prod_store_rows");
+}
+
 at::Tensor prod_paged_decode(const at::Tensor& q, const at::Tensor& kv_cache, const at::Tensor& block_table,
                              const at::Tensor& seq_lens, const at::Tensor& centroids_k3, const at::Tensor& centroids_v,
                              const at::Tensor& rotation, const at::Tensor& sketch, int64_t num_kv_heads,
@@ -885,6 +909,9 @@ void bind_kernels(py::module_& m) {
           py::arg("block_size"), py::arg("sm_scale") = py::none(), py::arg("causal") = true,
           py::arg("out") = py::none(),
           "Variable-length prefill over the packed paged TQ4 cache: un-rotated q (tokens, H_Q, D), original-space output");
+    m.def("prod_store_rows", &prod_store_rows, py::arg("kv_cache"), py::arg("slot_mapping"), py::arg("k_packed"),
+          py::arg("k_norms"), py::arg("k_gamma"), py::arg("v_packed"), py::arg("v_norms"),
+          "Write TurboQuantProd token rows into the paged cache at the flat slots of slot_mapping.");
     m.def("prod_compress", &prod_compress, py::arg("x"), py::arg("rotation"), py::arg("sketch_rot"),
           py::arg("boundaries"), py::arg("centroids"),
           "TurboQuantProd key compress: (packed nibbles sign<<3|idx (N,H,D/2), norms (N,H,1), residual norms (N,H,1))");

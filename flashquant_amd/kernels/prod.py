@@ -56,18 +56,10 @@ def prod_store_rows(
     v_packed: torch.Tensor,
     v_norms: torch.Tensor,
 ) -> None:
-    """Assemble token rows and scatter them into the paged cache (num_blocks,
-    block_size, H*(D+12)) at the flat slots of ``slot_mapping`` (device tensors)."""
+    """Write the tokens' rows into the paged cache (num_blocks, block_size,
+    H*(D+12)) at the flat slots of ``slot_mapping`` (device tensors), one launch."""
     require_gpu(kv_cache, "kv_cache")
-    n, h, half = k_packed.shape
-    k_norm, k_gamma_off, v_idx, v_norm, row_bytes = prod_page_layout(h, 2 * half)
-    row = torch.empty(n, row_bytes, dtype=torch.uint8, device=kv_cache.device)
-    row[:, :k_norm] = k_packed.reshape(n, -1)
-    row[:, k_norm:k_gamma_off] = k_norms.reshape(n, h).contiguous().view(torch.uint8)
-    row[:, k_gamma_off:v_idx] = k_gamma.reshape(n, h).contiguous().view(torch.uint8)
-    row[:, v_idx:v_norm] = v_packed.reshape(n, -1)
-    row[:, v_norm:] = v_norms.reshape(n, h).contiguous().view(torch.uint8)
-    kv_cache.view(-1, row_bytes)[slot_mapping.long()] = row
+    native().prod_store_rows(kv_cache, slot_mapping, k_packed, k_norms, k_gamma, v_packed, v_norms)
 
 
 def prod_paged_decode(

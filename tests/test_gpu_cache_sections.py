@@ -58,3 +58,25 @@ def test_decompress_cache_of_no_pages_and_argument_errors():
         layer.decompress_cache(torch.zeros(1, 16, 8 * 136, dtype=torch.uint8, device=DEV), torch.float32)
     with pytest.raises(ValueError):
         layer.decompress_cache(torch.zeros(1, 16, 7 * 136, dtype=torch.uint8, device=DEV), torch.bfloat16)
+
+
+@pytest.mark.parametrize("n,h", [(1, 8), (3, 1), (130, 8), (9, 24)])
+@pytest.mark.parametrize("d", [64, 128])
+def test_prod_store_rows_writes_the_rows_and_nothing_else(n, h, d):
+    g = torch.Generator().manual_seed(n + h)
+    pages, page = n // 16 + 2, 16
+    kn, kg, vi, vn, row = K.prod_page_layout(h, d)
+    cache = torch.randint(0, 256, (pages, page, row), dtype=torch.uint8, generator=g)
+    slots = torch.randperm(pages * page, generator=g)[:n]
+    slots[0] = slots[0] - pages * page                      # counted from the end, as an indexed store does
+    packed = [torch.randint(0, 256, (n, h, d // 2), dtype=torch.uint8, generator=g) for _ in range(2)]
+    norms = [torch.rand(n, h, 1, generator=g) for _ in range(3)]
+    want = cache.clone().view(-1, row)
+    want[slots, :kn] = packed[0].view(n, -1)
+    for at, t in ((kn, norms[0]), (kg, norms[1]), (vn, norms[2])):
+        want[slots, at: at + 4 * h] = t.view(n, h).view(torch.uint8)
+    want[slots, vi:vn] = packed[1].view(n, -1)
+    got = cache.to(DEV)
+    dev = [t.to(DEV) for t in (slots, packed[0], norms[0], norms[1], packed[1], norms[2])]
+    K.prod_store_rows(got, *dev)
+    assert torch.equal(got.cpu().view(-1, row), want)
