@@ -46,15 +46,13 @@ struct PrefillCfg {
     static constexpr int KBYTES = 64 * KSTRIDE;           // 17408 at D = 128
     static constexpr int VBYTES = D * 128;                // V^T tile: D coordinate rows x 64 tokens fp16
     static constexpr int BUF = KBYTES + VBYTES;           // 33792 at D = 128
-    static constexpr int STAGE = 64 * D;                  // per-wavefront staging area for the rotations
     static constexpr int NKS = D / 16;                    // k-steps of the score product
     static constexpr int NOB = D / 32;                    // 32-coordinate blocks of the output
-    static constexpr int NJ = D / 32;                     // 32-wide k-steps of the head rotations
     static constexpr int PB = D / 2;                      // packed bytes per token and head
     // The rotation matrix as MFMA operands (two fp16 terms), shared by the wavefronts of a workgroup:
-    // block (column block cb, k-step j) holds one 16-byte operand per lane and term.  They lie where
-    // the lookup tables are between the query stage and the end of the tile loop (64 KB).
-    static constexpr int RTERM = NKS * NJ * 64 * 16;      // bytes per term: 32768 at D = 128
+    // a block of 32 x 16 holds one 16-byte operand per lane and term.  They lie where the lookup
+    // tables are between the query stage and the end of the tile loop (64 KB).
+    static constexpr int RTERM = NKS * NOB * 64 * 16;     // bytes per term: 32768 at D = 128
 };
 
 struct PrefillParams {
@@ -79,6 +77,7 @@ struct PrefillParams {
     const uint8_t* cache;          // (num_blocks, block_size, H_KV * 136)
     int max_blocks, num_blocks, bs_log2;
     int round_slots;               // workgroups running at a time (one per CU)
+    bool out_wide;                 // `out` is 16-byte aligned (its rows are multiples of 128 bytes apart)
 };
 
 __device__ __forceinline__ uint32_t scale_pair(uint32_t pair, half2v n2) {
@@ -98,8 +97,8 @@ __device__ __forceinline__ uint32_t pack_rtz(float a, float b) {
 template <int D, int DT, bool PAGED>
 __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillParams p) {
     using Cfg = PrefillCfg<D>;
-    constexpr int kPfKStride = Cfg::KSTRIDE, kPfKBytes = Cfg::KBYTES, kPfBufBytes = Cfg::BUF, kPfStageBytes = Cfg::STAGE;
-    constexpr int NKS = Cfg::NKS, NOB = Cfg::NOB, NJ = Cfg::NJ, PB = Cfg::PB;
+    constexpr int kPfKStride = Cfg::KSTRIDE, kPfKBytes = Cfg::KBYTES, kPfBufBytes = Cfg::BUF;
+    constexpr int NKS = Cfg::NKS, NOB = Cfg::NOB, PB = Cfg::PB;
     __shared__ __attribute__((aligned(256))) uint32_t lut[256 * 64];
     extern __shared__ __attribute__((aligned(16))) uint8_t bufs[];   // 2 x (K tile | V^T tile)
     // Rows whose norm times a centroid would not fit fp16 are stored divided by a power of two.
@@ -113,7 +112,6 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     const int lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int m32 = lane & 31, hf = lane >> 5;     // 32x32 MFMA: column (query row) and lane half
-    const int n16 = lane & 15, g4 = lane >> 4;     // 16x16 MFMA of the rotations
     // Workgroups reach the CUs in the order of their linear index, round after round, and under a
     // causal mask their durations grow with the query position.  Position fastest, (batch, head)
     // slow, and the position order reversed in every other round over the chip: whichever way the
@@ -312,88 +310,113 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
 
     issue_loads(0);
 
-    // ---- the rotation matrix, split once per workgroup ------------------------------------------------
-    // Wavefront cb fetches column block cb of R^T (or of R), splits it into two fp16 terms and
-    // leaves the operands in LDS; every wavefront then reads the blocks it multiplies with from
-    // there (each wavefront fetching and splitting the whole matrix for itself, three times per
-    // workgroup, was an eighth of the kernel's time).
+    // ---- the rotation matrix as the A operand of v_mfma_f32_32x32x16_f16, split once per workgroup ------
+    // Both rotations are transposed products, matrix block x row block: a lane then owns one query row in
+    // the operand (its own 16-byte pieces of the query, or its registers of O) and in the result, and no row
+    // passes through LDS.  Block (32 result coordinates, 16 contraction coordinates): lane (m32, hf) holds
+    // eight contraction coordinates of result coordinate m32, as two fp16 terms.  Wavefront w fetches and
+    // splits blocks BPW * w .., every wavefront reads all of them.
+    //
+    // What it replaced staged the rows through LDS for the 16x16x32 MFMA (16 to 32 lanes on a bank) and stored the
+    // results 2 bytes a lane: a workgroup per CU on 64 tokens of 32 heads over 64 keys took 33 us and 27 us with one
+    // query row, 24 and 15.5 us this way (the tile itself: 2 us); 4 x 32 heads x 8192 tokens 2.94 -> 2.77 ms.
+    constexpr int BPW = NOB * NKS / 8;
     uint8_t* rshare = reinterpret_cast<uint8_t*>(lut);
-    auto share_rotation = [&](bool transposed) {
-        if (w < NKS) {
-            float rbv[NJ][8];
-            load_rotation_any<D>(p.rotation, p.rot_col_major != 0, transposed, 16 * w, n16, g4, rbv);
-            half8 rhi[NJ], rlo[NJ];
-            split_rotation_block<D>(rbv, rhi, rlo);
+    float rbv[BPW][8];
+    // `back`: x @ R with the contraction index in the order of the accumulator registers (element 4 a + c of half
+    // hf = coordinate 8 a + 4 hf + c of the k-step), else x @ R^T in the natural order
+    auto fetch_rotation = [&](bool back) {
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                *reinterpret_cast<half8*>(rshare + ((w * NJ + j) * 64 + lane) * 16) = rhi[j];
-                *reinterpret_cast<half8*>(rshare + Cfg::RTERM + ((w * NJ + j) * 64 + lane) * 16) = rlo[j];
+        for (int i = 0; i < BPW; ++i) {
+            const int blk = BPW * w + i, j = 32 * (blk / NKS) + m32, k0 = 16 * (blk % NKS);
+            const int k1 = back ? k0 + 4 * hf : k0 + 8 * hf, step = back ? 8 : 4;    // coordinates k1 + 0..3, k1 + step + 0..3
+            if (back == (p.rot_col_major != 0)) {          // a lane's coordinates are neighbours in memory
+                const float4v lo = *reinterpret_cast<const float4v*>(p.rotation + j * D + k1);
+                const float4v hi = *reinterpret_cast<const float4v*>(p.rotation + j * D + k1 + step);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { rbv[i][e] = lo[e]; rbv[i][4 + e] = hi[e]; }
+            } else {                                       // the lanes' are
+#pragma unroll
+                for (int e = 0; e < 8; ++e) rbv[i][e] = p.rotation[(k1 + (e >> 2) * step + (e & 3)) * D + j];
             }
         }
     };
-    auto shared_rotation_block = [&](int cb, half8 (&rhi)[NJ], half8 (&rlo)[NJ]) {
+    auto share_rotation = [&]() {
+        half8 rhi[BPW], rlo[BPW];
+        split_rotation_block<32 * BPW>(rbv, rhi, rlo);
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            rhi[j] = *reinterpret_cast<const half8*>(rshare + ((cb * NJ + j) * 64 + lane) * 16);
-            rlo[j] = *reinterpret_cast<const half8*>(rshare + Cfg::RTERM + ((cb * NJ + j) * 64 + lane) * 16);
+        for (int i = 0; i < BPW; ++i) {
+            *reinterpret_cast<half8*>(rshare + ((BPW * w + i) * 64 + lane) * 16) = rhi[i];
+            *reinterpret_cast<half8*>(rshare + Cfg::RTERM + ((BPW * w + i) * 64 + lane) * 16) = rlo[i];
         }
     };
+    auto rotation_term = [&](int term, int jb, int ks) {
+        return *reinterpret_cast<const half8*>(rshare + term * Cfg::RTERM + ((jb * NKS + ks) * 64 + lane) * 16);
+    };
+    // the power of two that brings a row's largest magnitude (over both lane halves) into [1, 2)
+    auto row_exponent = [&](float mx) {
+        mx = max_xor32(mx);
+        const int ex = int((float_to_bits(mx) >> 23) & 0xffu) - 127;
+        return (ex < -100 || ex > 100) ? 0 : ex;
+    };
+    auto pow2 = [](int e) { return bits_to_float(uint32_t(127 + e) << 23); };
 
     // ---- query: rotate this wavefront's 32 rows, round to the query dtype, scale to fp16 ----------
     half8 qb[NKS];
-    float krow;
+    float krow = 0.0f;
     {
         const uint16_t* qbase = PAGED ? p.q + (q_row0 + hq) * D : p.q + (q_row0 + int64_t(hq) * NQ) * D;
-        uint16_t* st = reinterpret_cast<uint16_t*>(bufs + w * kPfStageBytes);   // (32 rows, D) raw 16-bit
-        // the rows are exact in fp16 up to a power of two: fp16-split MFMA, two terms
-        half8 a[2][NJ];
-        float up[2];
+        const int pos = pos0 + m32 < NQ ? pos0 + m32 : NQ - 1;
+        uint4v raw[NKS];
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb) {
-            int pos = pos0 + 16 * rb + n16;
-            pos = pos < NQ ? pos : NQ - 1;
-            uint4v raw[NJ];
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) raw[j] = *reinterpret_cast<const uint4v*>(qbase + int64_t(pos) * q_stride + 32 * j + 8 * g4);
-            rows_as_f16<D, DT>(raw, a[rb], up[rb]);
-        }
-        share_rotation(true);
-        __syncthreads();
-        for (int cb = 0; cb < NKS; ++cb) {
-            half8 rhi[NJ], rlo[NJ];
-            shared_rotation_block(cb, rhi, rlo);
-#pragma unroll
-            for (int rb = 0; rb < 2; ++rb) {
-                const float4v acc = rotate_block_f16<D>(a[rb], rhi, rlo);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) st[(16 * rb + 4 * g4 + i) * D + 16 * cb + n16] = store_elem<DT>(acc[i] * up[rb]);
-            }
-        }
-        __syncthreads();
-        float qf[NKS][8];
+        for (int ks = 0; ks < NKS; ++ks)
+            raw[ks] = *reinterpret_cast<const uint4v*>(qbase + int64_t(pos) * q_stride + 16 * ks + 8 * hf);
+        fetch_rotation(false);
+        // the rows are exact in fp16 up to a power of two
+        half8 qa[NKS];
         float mx = 0.0f;
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) {
-            const uint2v lo = *reinterpret_cast<const uint2v*>(st + m32 * D + 16 * ks + 4 * hf);
-            const uint2v hi = *reinterpret_cast<const uint2v*>(st + m32 * D + 16 * ks + 8 + 4 * hf);
-            const uint32_t wds[4] = {lo.x, lo.y, hi.x, hi.y};
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                qf[ks][2 * i] = load_elem<DT>(uint16_t(wds[i] & 0xffffu));
-                qf[ks][2 * i + 1] = load_elem<DT>(uint16_t(wds[i] >> 16));
-                mx = __builtin_fmaxf(mx, __builtin_fmaxf(__builtin_fabsf(qf[ks][2 * i]), __builtin_fabsf(qf[ks][2 * i + 1])));
-            }
-        }
-        mx = __builtin_fmaxf(mx, xor_shuffle(mx, 32));
-        int ex = int((float_to_bits(mx) >> 23) & 0xffu) - 127;
-        if (ex < -100 || ex > 100) ex = 0;
-        const float down = bits_to_float(uint32_t(127 - ex) << 23);
-        krow = p.scale_log2e * bits_to_float(uint32_t(127 + ex) << 23);
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) qb[ks][e] = _Float16(qf[ks][e] * down);
-        __syncthreads();   // the staging area becomes tile buffers, the rotation operands lookup tables
+            for (int i = 0; i < 4; ++i)
+                mx = __builtin_fmaxf(mx, __builtin_fmaxf(__builtin_fabsf(load_elem<DT>(uint16_t(raw[ks][i] & 0xffffu))),
+                                                         __builtin_fabsf(load_elem<DT>(uint16_t(raw[ks][i] >> 16)))));
+        const int ex = row_exponent(mx);
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                qa[ks][2 * i] = _Float16(load_elem<DT>(uint16_t(raw[ks][i] & 0xffffu)) * pow2(-ex));
+                qa[ks][2 * i + 1] = _Float16(load_elem<DT>(uint16_t(raw[ks][i] >> 16)) * pow2(-ex));
+            }
+        share_rotation();
+        __syncthreads();
+        float16v rot[NOB];
+        float mr = 0.0f;
+#pragma unroll
+        for (int jb = 0; jb < NOB; ++jb) {
+            float16v hi, lo;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) { hi[r] = 0.0f; lo[r] = 0.0f; }
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) {
+                hi = __builtin_amdgcn_mfma_f32_32x32x16_f16(rotation_term(0, jb, ks), qa[ks], hi, 0, 0, 0);
+                lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(rotation_term(1, jb, ks), qa[ks], lo, 0, 0, 0);
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                rot[jb][r] = load_elem<DT>(store_elem<DT>((hi[r] + lo[r] * (1.0f / 4096.0f)) * pow2(ex)));
+                mr = __builtin_fmaxf(mr, __builtin_fabsf(rot[jb][r]));
+            }
+        }
+        const int er = row_exponent(mr);
+        krow = p.scale_log2e * pow2(er);
+        // the result registers 8 u .. 8 u + 7 of a block are the operand of k-step u (the order of the K tile)
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) qb[ks][e] = _Float16(rot[ks >> 1][8 * (ks & 1) + e] * pow2(-er));
+        __syncthreads();   // the rotation operands become lookup tables
     }
     fill_pair_tables<8>(lut, p.centroids_k[lane & 15], p.centroids_v[lane & 15], 15, w, lane);
     __syncthreads();
@@ -585,46 +608,78 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     // ---- normalise, rotate back, store -------------------------------------------------------------------
     const float l_tot = l_run + xor_shuffle(l_run, 32);
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-    float* stf = reinterpret_cast<float*>(bufs + w * kPfStageBytes);   // (16 rows, D) float32
-    uint16_t* obase = PAGED ? p.out + (q_row0 + hq) * D : p.out + (q_row0 + int64_t(hq) * NQ) * D;
+    fetch_rotation(true);
     __syncthreads();                // every wavefront is done with the lookup tables
-    share_rotation(false);          // (the barrier below orders it before its readers)
-    for (int half_rows = 0; half_rows < 2; ++half_rows) {
-        __syncthreads();
-        if ((m32 >> 4) == half_rows) {
+    share_rotation();
+    __syncthreads();
+    if (!unit_live) return;
+    // float32 rows: both operands as two fp16 terms, three MFMA terms; rows already rounded to 16 bits (the
+    // paged form) are exact in one
+    float mo = 0.0f;
 #pragma unroll
-            for (int ob = 0; ob < NOB; ++ob)
+    for (int ob = 0; ob < NOB; ++ob)
 #pragma unroll
-                for (int rq = 0; rq < 4; ++rq) {
-                    float4v v = {O[ob][4 * rq] * inv, O[ob][4 * rq + 1] * inv, O[ob][4 * rq + 2] * inv, O[ob][4 * rq + 3] * inv};
-                    if (PAGED) {
+        for (int r = 0; r < 16; ++r) {
+            const float v = O[ob][r] * inv;
+            O[ob][r] = PAGED ? load_elem<DT>(store_elem<DT>(v)) : v;
+            mo = __builtin_fmaxf(mo, __builtin_fabsf(O[ob][r]));
+        }
+    const int eo = row_exponent(mo);
+    half8 ohi[NKS], olo[NKS];
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) v[e] = load_elem<DT>(store_elem<DT>(v[e]));
+    for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+            const float a0 = O[ks >> 1][8 * (ks & 1) + e] * pow2(-eo), a1 = O[ks >> 1][8 * (ks & 1) + e + 1] * pow2(-eo);
+            if (PAGED) {
+                ohi[ks][e] = _Float16(a0); ohi[ks][e + 1] = _Float16(a1);
+            } else {
+                const auto h2 = __builtin_amdgcn_cvt_pkrtz(a0, a1);
+                const auto l2 = __builtin_amdgcn_cvt_pkrtz((a0 - float(h2[0])) * 4096.0f, (a1 - float(h2[1])) * 4096.0f);
+                ohi[ks][e] = h2[0]; ohi[ks][e + 1] = h2[1];
+                olo[ks][e] = l2[0]; olo[ks][e + 1] = l2[1];
+            }
+        }
+    const int opos = pos0 + m32;
+    uint16_t* obase = PAGED ? p.out + (q_row0 + hq) * D : p.out + (q_row0 + int64_t(hq) * NQ) * D;
+    uint16_t* orow = obase + int64_t(opos) * q_stride;
+#pragma unroll
+    for (int cb = 0; cb < NOB; ++cb) {
+        float16v hi, lo;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { hi[r] = 0.0f; lo[r] = 0.0f; }
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) {
+            const half8 rh = rotation_term(0, cb, ks);
+            hi = __builtin_amdgcn_mfma_f32_32x32x16_f16(rh, ohi[ks], hi, 0, 0, 0);
+            lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(rotation_term(1, cb, ks), ohi[ks], lo, 0, 0, 0);
+            if (!PAGED) lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(rh, olo[ks], lo, 0, 0, 0);
+        }
+        // registers 4 q + c of half hf = coordinate 32 cb + 8 q + 4 hf + c; the halves exchange a quad of every two,
+        // so that a lane stores eight neighbours at a time
+        uint32_t wd[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float v0 = (hi[2 * i] + lo[2 * i] * (1.0f / 4096.0f)) * pow2(eo);
+            const float v1 = (hi[2 * i + 1] + lo[2 * i + 1] * (1.0f / 4096.0f)) * pow2(eo);
+            wd[i] = uint32_t(store_elem<DT>(v0)) | uint32_t(store_elem<DT>(v1)) << 16;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q += 2) {
+            const auto x = __builtin_amdgcn_permlane32_swap(wd[2 * q], wd[2 * q + 2], false, false);
+            const auto y = __builtin_amdgcn_permlane32_swap(wd[2 * q + 1], wd[2 * q + 3], false, false);
+            const uint4v v = {x[0], y[0], x[1], y[1]};
+            uint16_t* dst = orow + 32 * cb + 8 * q + 8 * hf;
+            if (opos < NQ) {
+                if (p.out_wide) {
+                    *reinterpret_cast<uint4v*>(dst) = v;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        dst[2 * e] = uint16_t(v[e] & 0xffffu);
+                        dst[2 * e + 1] = uint16_t(v[e] >> 16);
                     }
-                    *reinterpret_cast<float4v*>(stf + (m32 & 15) * D + 32 * ob + 8 * rq + 4 * hf) = v;
                 }
-        }
-        __syncthreads();
-        float a[NJ][8];
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const float4v lo = *reinterpret_cast<const float4v*>(stf + n16 * D + 32 * j + 8 * g4);
-            const float4v hi = *reinterpret_cast<const float4v*>(stf + n16 * D + 32 * j + 8 * g4 + 4);
-            a[j][0] = lo.x; a[j][1] = lo.y; a[j][2] = lo.z; a[j][3] = lo.w;
-            a[j][4] = hi.x; a[j][5] = hi.y; a[j][6] = hi.z; a[j][7] = hi.w;
-        }
-        // float32 rows: both operands as two fp16 terms, three MFMA terms
-        half8 ahi[NJ], alo[NJ];
-        float up;
-        rows_split_f16<D>(a, ahi, alo, up);
-        for (int cb = 0; cb < NKS; ++cb) {
-            half8 rhi[NJ], rlo[NJ];
-            shared_rotation_block(cb, rhi, rlo);
-            const float4v acc = rotate_block_f16x3<D>(ahi, alo, rhi, rlo);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int pos = pos0 + 16 * half_rows + 4 * g4 + i;
-                if (unit_live && pos < NQ) obase[int64_t(pos) * q_stride + 16 * cb + n16] = store_elem<DT>(acc[i] * up);
             }
         }
     }
@@ -714,6 +769,7 @@ extern "C" int fq_fused_tq_attention_strided(const void* q, const uint8_t* k_pac
     p.cu_seqlens_q = nullptr; p.seq_lens = nullptr; p.block_table = nullptr; p.cache = nullptr;
     p.max_blocks = 0; p.num_blocks = 0; p.bs_log2 = 0;
     p.round_slots = fq_host::device_cu_count();
+    p.out_wide = fq_host::aligned(out, 16);
     return D == 64 ? launch_prefill<64, false>(p, grid, dtype, s) : launch_prefill<128, false>(p, grid, dtype, s);
 }
 
@@ -768,6 +824,7 @@ extern "C" int fq_paged_tq4_prefill(const void* q, const int32_t* cu_seqlens_q, 
     p.max_blocks = max_blocks_per_seq; p.num_blocks = int(num_blocks);
     p.bs_log2 = block_size == 8 ? 3 : (block_size == 16 ? 4 : 5);
     p.round_slots = fq_host::device_cu_count();
+    p.out_wide = fq_host::aligned(out, 16);
 
     const int64_t units = int64_t((max_q_len + 31) / 32) * p.G;
     const int64_t wgs = (units + 7) / 8;
