@@ -473,6 +473,12 @@ void tq4_compress_append(const at::Tensor& x, const at::Tensor& rot_T_even, cons
     fqbind::raise_on_error(st, "tq4_compress_append");
 }
 
+// Room for the partial results of attention over split contexts; undefined where these sizes are never split.
+at::Tensor attention_workspace(const at::Tensor& q, int64_t seqs, int64_t max_q, int64_t max_kv, int64_t HQ, int64_t HKV, int64_t D) {
+    const size_t bytes = fq_attention_workspace_bytes(int(seqs), int(max_q), max_kv, int(HQ), int(HKV), int(D));
+    return bytes == 0 ? at::Tensor() : at::empty({int64_t(bytes)}, q.options().dtype(at::kByte));
+}
+
 at::Tensor fused_tq_attention(const at::Tensor& q, const at::Tensor& k_packed, const at::Tensor& k_norms,
                               const at::Tensor& v_packed, const at::Tensor& v_norms, const at::Tensor& centroids_k,
                               const at::Tensor& centroids_v, const at::Tensor& rotation,
@@ -518,11 +524,13 @@ at::Tensor fused_tq_attention(const at::Tensor& q, const at::Tensor& k_packed, c
     const at::Tensor ck = centroids_k.to(q.device()).contiguous(), cv = centroids_v.to(q.device()).contiguous();
     const RotationArg rot = rotation_arg(rotation, q.device(), D);
     at::Tensor result = at::empty_like(qc);
-    const int st = fq_fused_tq_attention_strided(
+    const at::Tensor ws = attention_workspace(q, B, NQ, NKV, HQ, HKV, D);
+    const int st = fq_fused_tq_attention_split(
         qc.data_ptr(), kp.data_ptr<uint8_t>(), kn.data_ptr<float>(), vp.data_ptr<uint8_t>(), vn.data_ptr<float>(),
         ck.data_ptr<float>(), cv.data_ptr<float>(), rot.ptr, rot.col_major, result.data_ptr(),
         int(B), int(HQ), int(HKV), int(NQ), int(NKV), k_cap, v_cap, int(D), float(scale), is_causal ? 1 : 0,
-        fqbind::dtype_code(q.scalar_type(), "fused_tq_attention"), fqbind::current_stream(q));
+        fqbind::dtype_code(q.scalar_type(), "fused_tq_attention"), ws.defined() ? ws.data_ptr() : nullptr,
+        ws.defined() ? size_t(ws.numel()) : 0, fqbind::current_stream(q));
     fqbind::raise_on_error(st, "fused_tq_attention");
     return result;
 }
@@ -568,12 +576,13 @@ at::Tensor paged_tq4_prefill(const at::Tensor& q, const at::Tensor& cu_seqlens_q
     } else {
         result = at::zeros_like(qc);
     }
-    const int st = fq_paged_tq4_prefill(
+    const at::Tensor ws = attention_workspace(q, S, max_seqlen_q, bt.size(1) * block_size, HQ, num_kv_heads, head_dim);
+    const int st = fq_paged_tq4_prefill_split(
         qc.data_ptr(), cu.data_ptr<int32_t>(), kv_cache.data_ptr<uint8_t>(), bt.data_ptr<int32_t>(),
         sl.data_ptr<int32_t>(), ck.data_ptr<float>(), cv.data_ptr<float>(), rot.ptr, rot.col_major, result.data_ptr(),
         int(S), int(max_seqlen_q), int(HQ), int(num_kv_heads), int(head_dim), int(block_size), int(bt.size(1)),
-        kv_cache.size(0), float(scale), causal ? 1 : 0, fqbind::dtype_code(q.scalar_type(), "paged_tq4_prefill"),
-        fqbind::current_stream(q));
+        kv_cache.size(0), float(scale), causal ? 1 : 0, fqbind::dtype_code(q.scalar_type(), "paged_tq4_prefill"), T,
+        ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? size_t(ws.numel()) : 0, fqbind::current_stream(q));
     fqbind::raise_on_error(st, "paged_tq4_prefill");
     return result;
 }

@@ -1,0 +1,120 @@
+// Order and split of the workgroups of the fused attention kernel.
+//
+// A workgroup's time is a fixed part (the two rotations, about kSplitMinTiles tiles' worth) plus its key tiles, and
+// under a causal mask or in a batch of prompts, later chunks and single queries the tiles differ by two orders of
+// magnitude.  Nothing on the host knows the lengths, so every workgroup works out from them which piece of the work is
+// its own:
+//   * work is handed out longest first (the workgroups of a KV-head group in the order of their linear index), so that
+//     the short ones fill the end of the launch;
+//   * where a sequence's keys are long for its few queries (`split_w`, `max_pieces`, set by the host from what it
+//     knows), they are cut into pieces of about the share of a CU; the pieces leave partial results, combined by a
+//     launch of their own.
+// Measured (MI355X, bf16, 32 query heads over 8 KV heads of 128): a batch of 12 with six prompts, three later chunks and
+// three single queries, 10,556 new tokens, 467 us in grid order and 385 us longest first; one query over 4 x 2500 tokens of a
+// ring buffer 67 us in one workgroup per KV head and 34 us in 5 pieces, over 1 x 16,384 tokens 390 and 39 us (32 pieces).
+// Everything here is arithmetic on the lengths alone: the same in every workgroup and in the combine launch.
+#pragma once
+
+#include <cstdint>
+
+#if defined(__HIPCC__)
+#define FQ_HD __host__ __device__ __forceinline__
+#else
+#define FQ_HD inline
+#endif
+
+namespace fq {
+
+constexpr int kSplitMinTiles = 8;        // tiles of 64 keys: a piece shorter than this is mostly prologue
+
+// One sequence as the kernel sees it.
+struct SeqShape {
+    int NQ, NKV, qoff;       // queries, keys, position of the first query among the keys
+    int units, W;            // (32 positions x one query head) units, workgroups of 8 units
+    int all_tiles;
+};
+
+FQ_HD SeqShape make_seq_shape(int NQ, int NKV, int qoff, int G, int max_w) {
+    SeqShape s;
+    s.NQ = NQ > 0 ? NQ : 0;
+    s.NKV = NKV;
+    s.qoff = qoff;
+    s.units = ((s.NQ + 31) >> 5) * G;
+    s.W = (s.units + 7) >> 3;
+    s.W = s.W < max_w ? s.W : max_w;
+    s.all_tiles = (NKV + 63) >> 6;
+    return s;
+}
+
+// Key tiles that the furthest row of workgroup x sees; does not decrease with x.
+FQ_HD int tiles_of(const SeqShape& s, int x, int G, bool causal) {
+    if (!causal) return s.all_tiles;
+    const int last_unit = 8 * x + 7 < s.units - 1 ? 8 * x + 7 : s.units - 1;
+    int pos = 32 * (last_unit / G) + 31;
+    pos = pos < s.NQ - 1 ? pos : s.NQ - 1;
+    const int t = ((s.qoff + pos) >> 6) + 1;
+    return t < s.all_tiles ? t : s.all_tiles;
+}
+
+// First workgroup of the sequence with at least T tiles (W when there is none).
+FQ_HD int first_with(const SeqShape& s, int T, int G, bool causal) {
+    if (T <= 0) return 0;
+    if (T > s.all_tiles) return s.W;
+    if (!causal) return 0;
+    const int64_t P = 64 * int64_t(T - 1) - s.qoff;      // the position whose row sees T tiles
+    if (P <= 0) return 0;
+    if (P > s.NQ - 1) return s.W;
+    const int64_t b = P > 31 ? P / 32 : 0;               // its block of 32 positions: ceil((P - 31) / 32)
+    const int64_t x = b * G / 8;                         // first x whose last unit 8 x + 7 reaches unit b G
+    return x < s.W ? int(x) : s.W;
+}
+
+// Pieces that every workgroup's keys of this sequence are cut into.
+FQ_HD int pieces_of(const SeqShape& s, int share, int split_w, int max_pieces, int G, bool causal) {
+    if (max_pieces < 2 || s.W == 0 || s.W > split_w) return 1;
+    const int n = (tiles_of(s, s.W - 1, G, causal) + share / 2) / share;
+    return n < 1 ? 1 : (n > max_pieces ? max_pieces : n);
+}
+
+// Tiles of the share that one of `slots` CUs would have of the whole batch.
+FQ_HD int share_of(uint32_t tile_sum, int slots) {
+    const int s = int((tile_sum + uint32_t(slots) - 1) / uint32_t(slots));
+    return s > kSplitMinTiles ? s : kSplitMinTiles;
+}
+
+// Workgroups x of the sequence whose pieces have at least T tiles: x >= this.
+FQ_HD int first_piece_with(const SeqShape& s, int T, int pieces, int G, bool causal) {
+    if (T <= 0) return 0;
+    const int64_t whole = int64_t(T - 1) * pieces + 1;
+    return whole > s.all_tiles ? s.W : first_with(s, int(whole), G, causal);
+}
+
+// What the host allows: workgroups per sequence that may be split and pieces per workgroup.  The first kind of batch
+// leaves more than half of the CUs without work (few prompts, or the chunks of a few): every workgroup may be split as
+// far as a round of workgroups goes, if the tiles saved (2.1 us each) outweigh the combine launch (6 us) and its traffic (132 KB
+// a workgroup and piece, written and read).  Else only sequences of one workgroup (single queries of a mixed batch) are.
+struct SplitPlan {
+    int split_w, max_pieces;
+};
+inline SplitPlan plan_split(int num_seqs, int H_KV, int max_w, int64_t max_tiles, int cus) {
+    SplitPlan none{0, 1};
+    if (max_tiles < 2 * kSplitMinTiles) return none;
+    auto pieces = [&](int64_t items) {
+        int64_t n = cus / (items > 0 ? items : 1);
+        n = n < max_tiles / kSplitMinTiles ? n : max_tiles / kSplitMinTiles;
+        return int(n < 32 ? n : 32);
+    };
+    const int64_t items = int64_t(num_seqs) * H_KV * max_w;
+    const int n = pieces(items);
+    if (n >= 2) {
+        const double saved = 2.1 * double(max_tiles) * (1.0 - 1.0 / n), cost = 6.0 + 0.066 * double(items) * n;
+        if (saved > 1.3 * cost) return {max_w, n};
+    }
+    if (max_w > 1) {
+        const int n1 = pieces(int64_t(num_seqs) * H_KV);
+        if (n1 >= 2) return {1, n1};
+    }
+    return none;
+}
+
+}  // namespace fq

@@ -36,6 +36,7 @@
 #include "fq_common.hpp"
 #include "fq_device.hpp"
 #include "fq_attention_any_dim.hpp"
+#include "fq_attention_schedule.hpp"
 
 namespace fq {
 
@@ -52,6 +53,7 @@ struct PrefillCfg {
     // The rotation matrix as MFMA operands (two fp16 terms), shared by the wavefronts of a workgroup:
     // a block of 32 x 16 holds one 16-byte operand per lane and term.  They lie where the lookup
     // tables are between the query stage and the end of the tile loop (64 KB).
+    static constexpr int SLOT = 8 * (32 * D + 64);        // floats: per unit 32 rows un-normalised, 32 maxima, 32 sums
     static constexpr int RTERM = NKS * NOB * 64 * 16;     // bytes per term: 32768 at D = 128
 };
 
@@ -77,6 +79,9 @@ struct PrefillParams {
     const uint8_t* cache;          // (num_blocks, block_size, H_KV * 136)
     int max_blocks, num_blocks, bs_log2;
     int round_slots;               // workgroups running at a time (one per CU)
+    // order and split of the work (fq_attention_schedule.hpp); workgroups in split pieces leave their rows in `part`
+    int num_seqs, max_w, split_w, max_pieces;
+    float* part;                   // slot of a workgroup's piece: PrefillCfg<D>::SLOT floats
     bool out_wide;                 // `out` is 16-byte aligned (its rows are multiples of 128 bytes apart)
 };
 
@@ -89,12 +94,114 @@ __device__ __forceinline__ uint32_t pack_rtz(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
 }
 
+template <bool PAGED>
+__device__ __forceinline__ SeqShape seq_shape(const PrefillParams& p, int s) {
+    int NQ = p.N_Q, NKV = p.N_KV, qoff = 0;
+    if (PAGED) {
+        NQ = p.cu_seqlens_q[s + 1] - p.cu_seqlens_q[s];
+        NKV = p.seq_lens[s];
+        const int room = p.max_blocks << p.bs_log2;
+        NKV = NKV < 0 ? 0 : (NKV > room ? room : NKV);
+        qoff = NKV - NQ > 0 ? NKV - NQ : 0;
+    }
+    return make_seq_shape(NQ, NKV, qoff, p.G, p.max_w);
+}
+
+__device__ __forceinline__ uint32_t wave_add(uint32_t v) {
+    int i = int(v);
+    i += __builtin_amdgcn_update_dpp(0, i, 0x121, 0xf, 0xf, false);   // row_ror:1, 2, 4, 8
+    i += __builtin_amdgcn_update_dpp(0, i, 0x122, 0xf, 0xf, false);
+    i += __builtin_amdgcn_update_dpp(0, i, 0x124, 0xf, 0xf, false);
+    i += __builtin_amdgcn_update_dpp(0, i, 0x128, 0xf, 0xf, false);
+    const auto a = __builtin_amdgcn_permlane16_swap(uint32_t(i), uint32_t(i), false, false);
+    const uint32_t b = a[0] + a[1];
+    const auto c = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    return uint32_t(__builtin_amdgcn_readfirstlane(int(c[0] + c[1])));
+}
+
+// The share of a CU of the whole batch (all KV heads), in tiles.  The sum may wrap on batches beyond any memory: the
+// share is then merely a poor one, and still the same everywhere.
+template <bool PAGED>
+__device__ __forceinline__ int batch_share(const PrefillParams& p, int lane) {
+    uint32_t sum = 0;
+    for (int s0 = 0; s0 < p.num_seqs; s0 += kWave) {
+        if (s0 + lane < p.num_seqs) {
+            const SeqShape sh = seq_shape<PAGED>(p, s0 + lane);
+            if (sh.W > 0)
+                sum += uint32_t(sh.W) * uint32_t(tiles_of(sh, 0, p.G, p.causal) + tiles_of(sh, sh.W - 1, p.G, p.causal) + 1) / 2;
+        }
+    }
+    return share_of(wave_add(sum) * uint32_t(p.H_KV), p.round_slots);
+}
+
+struct WorkItem {
+    int seq, x, piece, pieces;      // seq < 0: none
+};
+
+// The item of place `place` (of one KV head) in the order longest piece first: the largest tile count T that more than
+// `place` pieces reach, by bisection with a lane per sequence; then the place among the pieces of exactly T.
+template <bool PAGED>
+__device__ __forceinline__ WorkItem find_item(const PrefillParams& p, int place, int lane) {
+    const int G = p.G;
+    const bool causal = p.causal != 0;
+    const int share = p.max_pieces > 1 ? batch_share<PAGED>(p, lane) : 1;
+    const SeqShape none = make_seq_shape(0, 0, 0, G, 0);
+    const SeqShape first = lane < p.num_seqs ? seq_shape<PAGED>(p, lane) : none;
+    auto shape = [&](int s0) {
+        return s0 == 0 ? first : (s0 + lane < p.num_seqs ? seq_shape<PAGED>(p, s0 + lane) : none);
+    };
+    auto pieces = [&](const SeqShape& sh) { return pieces_of(sh, share, p.split_w, p.max_pieces, G, causal); };
+    auto count = [&](int T) {
+        uint32_t c = 0;
+        for (int s0 = 0; s0 < p.num_seqs; s0 += kWave) {
+            const SeqShape sh = shape(s0);
+            const int n = pieces(sh);
+            c += uint32_t(n * (sh.W - first_piece_with(sh, T, n, G, causal)));
+        }
+        return int(wave_add(c));
+    };
+    WorkItem item{-1, 0, 0, 1};
+    if (place >= count(0)) return item;
+    int lo = 0, hi = 1;               // count(lo) > place >= count(hi)
+    while (count(hi) > place) { lo = hi; hi *= 2; }      // (no sequence has 2^30 tiles: ends)
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (count(mid) > place) lo = mid;
+        else hi = mid;
+    }
+    int rem = place - count(hi);
+    for (int s0 = 0; s0 < p.num_seqs; s0 += kWave) {
+        const SeqShape sh = shape(s0);
+        const int n = pieces(sh), x0 = first_piece_with(sh, lo, n, G, causal);
+        const int mine = n * (first_piece_with(sh, hi, n, G, causal) - x0);
+        int before = mine;            // pieces of the lanes up to this one
+#pragma unroll
+        for (int d = 1; d < kWave; d <<= 1) {
+            const int v = __shfl_up(before, d, kWave);
+            if (lane >= d) before += v;
+        }
+        const uint64_t hit = __ballot(rem < before);
+        if (hit != 0) {
+            const int l = __ffsll(static_cast<unsigned long long>(hit)) - 1;
+            const int at = rem - (__builtin_amdgcn_readlane(before, l) - __builtin_amdgcn_readlane(mine, l));
+            item.pieces = __builtin_amdgcn_readlane(n, l);
+            item.seq = s0 + l;
+            item.piece = at % item.pieces;
+            item.x = __builtin_amdgcn_readlane(x0, l) + at / item.pieces;
+            return item;
+        }
+        rem -= __builtin_amdgcn_readlane(before, kWave - 1);
+    }
+    return item;
+}
+
 // PAGED: the sequences' queries are packed along the token axis of q (tokens, H_Q, 128), the keys
 // and values come from the paged TQ4 cache through the block table, query j of a sequence with
 // n queries and L keys sits at position L - n + j (the new tokens are the last ones), and the
 // attention result is rounded to the query dtype before the rotation back, as the attention
 // library's output is in the path this replaces (src/flashquant/vllm/impl.py:265-336, 470-512).
-template <int D, int DT, bool PAGED>
+// SCHED: workgroups take their work from find_item; else one workgroup per grid position, in the order below.
+template <int D, int DT, bool PAGED, bool SCHED>
 __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillParams p) {
     using Cfg = PrefillCfg<D>;
     constexpr int kPfKStride = Cfg::KSTRIDE, kPfKBytes = Cfg::KBYTES, kPfBufBytes = Cfg::BUF;
@@ -116,13 +223,23 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     // causal mask their durations grow with the query position.  Position fastest, (batch, head)
     // slow, and the position order reversed in every other round over the chip: whichever way the
     // rounds land on the CUs, each CU sees long and short workgroups alternate.
-    const int lin = int(blockIdx.x) + int(gridDim.x) * (int(blockIdx.y) + int(gridDim.y) * int(blockIdx.z));
-    const int pair = lin / int(gridDim.x);
-    const int b = pair / int(gridDim.y), hkv = pair % int(gridDim.y);
-    const int x_in_pair = lin % int(gridDim.x);
-    // The direction is a function of the pair alone (the round its first workgroup falls in), so
-    // inside a pair x -> wg is a bijection whatever the grid and the CU count are.
-    const bool flip = (((int64_t(pair) * int64_t(gridDim.x)) / p.round_slots) & 1) != 0;
+    int b, hkv, wg, piece = 0, pieces = 1;
+    if constexpr (SCHED) {
+        // the KV heads of a place are neighbours: each XCD serves few of them
+        const int at = int(blockIdx.x + gridDim.x * blockIdx.y);
+        const WorkItem it = find_item<PAGED>(p, at / p.H_KV, lane);
+        if (it.seq < 0) return;                            // the grid is sized for the most work possible
+        b = it.seq; hkv = at % p.H_KV; wg = it.x; piece = it.piece; pieces = it.pieces;
+    } else {
+        const int lin = int(blockIdx.x) + int(gridDim.x) * (int(blockIdx.y) + int(gridDim.y) * int(blockIdx.z));
+        const int pair = lin / int(gridDim.x);
+        b = pair / int(gridDim.y); hkv = pair % int(gridDim.y);
+        const int x_in_pair = lin % int(gridDim.x);
+        // The direction is a function of the pair alone (the round its first workgroup falls in), so
+        // inside a pair x -> wg is a bijection whatever the grid and the CU count are.
+        const bool flip = (((int64_t(pair) * int64_t(gridDim.x)) / p.round_slots) & 1) != 0;
+        wg = flip ? x_in_pair : int(gridDim.x) - 1 - x_in_pair;
+    }
 
     // ---- this sequence -----------------------------------------------------------------------
     int NQ = p.N_Q, NKV = p.N_KV, qoff = 0;
@@ -142,8 +259,6 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     // ---- units --------------------------------------------------------------------------
     const int nblk = (NQ + 31) >> 5;
     const int units = nblk * p.G;
-    const int wg = flip ? x_in_pair : int(gridDim.x) - 1 - x_in_pair;
-    if (PAGED && 8 * wg >= units) return;                  // the grid is sized for the longest sequence
     const int unit_raw = 8 * wg + w;
     const bool unit_live = unit_raw < units;
     const int unit = unit_live ? unit_raw : units - 1;
@@ -158,6 +273,13 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     if (p.causal) {
         ntiles = ((qoff + wg_maxpos) >> 6) + 1 < all_tiles ? ((qoff + wg_maxpos) >> 6) + 1 : all_tiles;
         my_tiles = ((qoff + my_maxpos) >> 6) + 1 < all_tiles ? ((qoff + my_maxpos) >> 6) + 1 : all_tiles;
+    }
+    // this piece's tiles: first_tile .. ntiles - 1 (of this wavefront: .. my_tiles - 1)
+    int first_tile = 0;
+    if (SCHED && pieces > 1) {
+        first_tile = int(int64_t(ntiles) * piece / pieces);
+        ntiles = int(int64_t(ntiles) * (piece + 1) / pieces);
+        my_tiles = my_tiles < ntiles ? my_tiles : ntiles;
     }
     if (!unit_live) my_tiles = 0;
 
@@ -308,7 +430,7 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
         }
     };
 
-    issue_loads(0);
+    issue_loads(first_tile);
 
     // ---- the rotation matrix as the A operand of v_mfma_f32_32x32x16_f16, split once per workgroup ------
     // Both rotations are transposed products, matrix block x row block: a lane then owns one query row in
@@ -587,12 +709,12 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     };
 
     // ---- tiles ----------------------------------------------------------------------------------------
-    dequant(0, 0);
-    issue_loads(1);
+    dequant(first_tile & 1, first_tile);
+    issue_loads(first_tile + 1);
     // The dequantisation of tile i + 1 and the products of tile i sit in one basic block (no
     // conditions between them), so that the lookups and LDS writes of the one interleave with
     // the MFMAs of the other.
-    int i = 0;
+    int i = first_tile;
     for (; i < my_tiles; ++i) {
         __syncthreads();                       // tile i is complete; the other buffer is free
         dequant((i + 1) & 1, i + 1);
@@ -603,6 +725,22 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
         __syncthreads();
         dequant((i + 1) & 1, i + 1);
         issue_loads(i + 2);
+    }
+
+    // ---- a piece of a workgroup's keys: the rows as they are, for the combine launch ------------------------
+    if (SCHED && pieces > 1) {
+        if (!unit_live) return;
+        const int64_t slot = ((int64_t(b) * p.H_KV + hkv) * p.split_w + wg) * p.max_pieces + piece;
+        float* dst = p.part + slot * Cfg::SLOT + w * (32 * D + 64);
+#pragma unroll
+        for (int ob = 0; ob < NOB; ++ob)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                *reinterpret_cast<float4v*>(dst + m32 * D + 32 * ob + 8 * q + 4 * hf) =
+                    float4v{O[ob][4 * q], O[ob][4 * q + 1], O[ob][4 * q + 2], O[ob][4 * q + 3]};
+        const float l_piece = l_run + xor_shuffle(l_run, 32);
+        dst[32 * D + lane] = hf == 0 ? m_run : l_piece;
+        return;
     }
 
     // ---- normalise, rotate back, store -------------------------------------------------------------------
@@ -685,20 +823,156 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     }
 }
 
-template <int D, bool PAGED>
-int launch_prefill(const PrefillParams& p, dim3 grid, int dtype, hipStream_t s) {
-    const size_t lds = 2 * size_t(PrefillCfg<D>::BUF);
-    const dim3 block(512);
-    if (dtype == FQ_F16) {
-        auto kern = fused_tq_attention_kernel<D, FQ_F16, PAGED>;
-        if (!fq_host::lds_limit_raised(reinterpret_cast<const void*>(kern), lds)) return FQ_ERR_LAUNCH;
-        hipLaunchKernelGGL(kern, grid, block, lds, s, p);
-    } else {
-        auto kern = fused_tq_attention_kernel<D, FQ_BF16, PAGED>;
-        if (!fq_host::lds_limit_raised(reinterpret_cast<const void*>(kern), lds)) return FQ_ERR_LAUNCH;
-        hipLaunchKernelGGL(kern, grid, block, lds, s, p);
+// Rows of the workgroups that ran in pieces: the pieces' rows weighted by 2^(m - max m), summed and normalised, rounded
+// as the kernel above rounds, rotated back.  A workgroup takes `rows` (4 or 16) rows of a unit, a wavefront a row at a
+// time; blockIdx.x numbers the (sequence, KV head, workgroup) triples that may have been split, blockIdx.y their row
+// groups.  Bound by the launch and two round trips (partials and matrix are asked for together): about 6 us.
+template <int D, int DT, bool PAGED>
+__global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillParams p, int rows) {
+    using Cfg = PrefillCfg<D>;
+    constexpr int NJ = D / 32, CBW = D / 64, CPL = D / 64;      // column blocks per wavefront, coordinates per lane
+    __shared__ __attribute__((aligned(16))) float os[16 * (D + 4)];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n16 = lane & 15, g4 = lane >> 4;
+    const int x = int(blockIdx.x) % p.split_w, pair = int(blockIdx.x) / p.split_w;
+    const int b = pair / p.H_KV, hkv = pair % p.H_KV;
+    const SeqShape sh = seq_shape<PAGED>(p, b);
+    const int groups = (int(gridDim.y) + 7) / 8, u = int(blockIdx.y) / groups, row0 = int(blockIdx.y) % groups * rows;
+    const int unit = 8 * x + u;
+    if (sh.W == 0 || sh.W > p.split_w || x >= sh.W || unit >= sh.units) return;
+    const int pos0 = 32 * (unit / p.G) + row0;
+    if (pos0 >= sh.NQ) return;
+    const int pieces = pieces_of(sh, batch_share<PAGED>(p, lane), p.split_w, p.max_pieces, p.G, p.causal != 0);
+    if (pieces < 2) return;
+
+    const float* src = p.part + (int64_t(blockIdx.x) * p.max_pieces) * Cfg::SLOT + u * (32 * D + 64);
+    float rbv[CBW][NJ][8];
+#pragma unroll
+    for (int i = 0; i < CBW; ++i)
+        load_rotation_any<D>(p.rotation, p.rot_col_major != 0, false, 16 * (wave + 4 * i), n16, g4, rbv[i]);
+    for (int r = wave; r < rows; r += 4) {
+        const float* head = src + 32 * D + row0 + r;
+        const bool have = lane < pieces;                        // (at most 32 pieces)
+        const float m = have ? head[int64_t(lane) * Cfg::SLOT] : -__builtin_inff();
+        const float l = have ? head[int64_t(lane) * Cfg::SLOT + 32] : 0.0f;
+        const float top = wave_max(m);
+        const float wgt = m == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(m - top);
+        float den = 0.0f, num[CPL];
+#pragma unroll
+        for (int e = 0; e < CPL; ++e) num[e] = 0.0f;
+        auto of_lane = [](float v, int k) { return bits_to_float(uint32_t(__builtin_amdgcn_readlane(int(float_to_bits(v)), k))); };
+        for (int k0 = 0; k0 < pieces; k0 += 8) {
+            float at[8][CPL];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {                       // eight pieces in flight (past the end: the last one again)
+                const int k = k0 + i < pieces ? k0 + i : pieces - 1;
+                const float* row = src + int64_t(k) * Cfg::SLOT + (row0 + r) * D + CPL * lane;
+#pragma unroll
+                for (int e = 0; e < CPL; ++e) at[i][e] = row[e];
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float wk = k0 + i < pieces ? of_lane(wgt, k0 + i) : 0.0f;
+                if (k0 + i < pieces) den = __builtin_fmaf(of_lane(l, k0 + i), wk, den);
+#pragma unroll
+                for (int e = 0; e < CPL; ++e) num[e] = wk > 0.0f ? __builtin_fmaf(at[i][e], wk, num[e]) : num[e];
+            }
+        }
+        const float inv = den > 0.0f ? 1.0f / den : 0.0f;
+#pragma unroll
+        for (int e = 0; e < CPL; ++e) {
+            const float v = num[e] * inv;
+            os[r * (D + 4) + CPL * lane + e] = PAGED ? load_elem<DT>(store_elem<DT>(v)) : v;
+        }
     }
-    return fq_host::check_launch();
+    __syncthreads();
+    float a[NJ][8];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const float4v v = *reinterpret_cast<const float4v*>(os + (n16 & (rows - 1)) * (D + 4) + 32 * j + 8 * g4 + 4 * h);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a[j][4 * h + e] = v[e];
+        }
+    half8 ahi[NJ], alo[NJ];
+    float up;
+    rows_split_f16<D>(a, ahi, alo, up);
+    const int hq = hkv * p.G + unit % p.G;
+    uint16_t* out = PAGED ? p.out + (int64_t(p.cu_seqlens_q[b]) * p.H_Q + hq) * D : p.out + (int64_t(b) * p.H_Q + hq) * sh.NQ * D;
+    const int stride = PAGED ? p.H_Q * D : D;
+#pragma unroll
+    for (int i = 0; i < CBW; ++i) {
+        half8 rhi[NJ], rlo[NJ];
+        split_rotation_block<D>(rbv[i], rhi, rlo);
+        const float4v acc = PAGED ? rotate_block_f16<D>(ahi, rhi, rlo) : rotate_block_f16x3<D>(ahi, alo, rhi, rlo);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int r = 4 * g4 + k;
+            if (r < rows && pos0 + r < sh.NQ)
+                out[int64_t(pos0 + r) * stride + 16 * (wave + 4 * i) + n16] = store_elem<DT>(acc[k] * up);
+        }
+    }
+}
+
+template <int D, int DT, bool PAGED, bool SCHED>
+int launch_prefill_as(const PrefillParams& p, dim3 grid, int max_q, hipStream_t s) {
+    const size_t lds = 2 * size_t(PrefillCfg<D>::BUF);
+    auto kern = fused_tq_attention_kernel<D, DT, PAGED, SCHED>;
+    if (!fq_host::lds_limit_raised(reinterpret_cast<const void*>(kern), lds)) return FQ_ERR_LAUNCH;
+    hipLaunchKernelGGL(kern, grid, dim3(512), lds, s, p);
+    const int st = fq_host::check_launch();
+    if constexpr (SCHED) {
+        if (st == FQ_OK && p.max_pieces > 1) {
+            const int rows = max_q <= 4 ? 4 : 16;
+            const int groups = max_q <= 16 ? 1 : 2;             // 32 rows a unit at most
+            hipLaunchKernelGGL((attention_combine_kernel<D, DT, PAGED>),
+                               dim3(unsigned(int64_t(p.num_seqs) * p.H_KV * p.split_w), 8 * groups), dim3(256), 0, s, p, rows);
+            return fq_host::check_launch();
+        }
+    }
+    return st;
+}
+
+template <bool PAGED, bool SCHED>
+int launch_prefill(const PrefillParams& p, int D, dim3 grid, int max_q, int dtype, hipStream_t s) {
+    if (D == 64)
+        return dtype == FQ_F16 ? launch_prefill_as<64, FQ_F16, PAGED, SCHED>(p, grid, max_q, s)
+                               : launch_prefill_as<64, FQ_BF16, PAGED, SCHED>(p, grid, max_q, s);
+    return dtype == FQ_F16 ? launch_prefill_as<128, FQ_F16, PAGED, SCHED>(p, grid, max_q, s)
+                           : launch_prefill_as<128, FQ_BF16, PAGED, SCHED>(p, grid, max_q, s);
+}
+
+// n workgroups in rows of at most 2^20 (a grid row holds fewer than 2^32 threads); the last row's surplus finds no work.
+inline dim3 folded_grid(int64_t n) {
+    const int64_t x = n < (1 << 20) ? n : (1 << 20);
+    return dim3(unsigned(x), unsigned((n + x - 1) / x));
+}
+
+inline int64_t workgroups_of(int64_t n_q, int G) { return ((n_q + 31) / 32 * G + 7) / 8; }
+
+// The split that a call of these sizes may use, and the bytes its partial rows take.
+inline SplitPlan plan_of(int num_seqs, int max_q, int64_t max_kv, int H_Q, int H_KV, int D) {
+    const int64_t max_w = workgroups_of(max_q, H_Q / H_KV);
+    if ((D != 64 && D != 128) || max_w < 1 || max_w > 0x7fffff || fq_host::force_any_dim_attention()) return SplitPlan{0, 1};
+    return plan_split(num_seqs, H_KV, int(max_w), (max_kv + 63) / 64, fq_host::device_cu_count());
+}
+inline size_t part_bytes(const SplitPlan& sp, int num_seqs, int H_KV, int D) {
+    if (sp.max_pieces < 2) return 0;
+    return size_t(num_seqs) * H_KV * sp.split_w * sp.max_pieces * (D == 64 ? PrefillCfg<64>::SLOT : PrefillCfg<128>::SLOT) * 4;
+}
+inline int use_plan(PrefillParams& p, const SplitPlan& sp, int D, void* workspace, size_t workspace_bytes) {
+    const size_t need = part_bytes(sp, p.num_seqs, p.H_KV, D);
+    p.split_w = 0;
+    p.max_pieces = 1;
+    p.part = nullptr;
+    if (need == 0 || workspace == nullptr) return FQ_OK;         // no workspace: nothing is split
+    if (workspace_bytes < need) return FQ_ERR_WORKSPACE;
+    if (!fq_host::aligned(workspace, 256)) return FQ_ERR_MISALIGNED;
+    p.split_w = sp.split_w;
+    p.max_pieces = sp.max_pieces;
+    p.part = static_cast<float*>(workspace);
+    return FQ_OK;
 }
 
 }  // namespace fq
@@ -714,6 +988,12 @@ extern "C" int fq_fused_tq_attention(const void* q, const uint8_t* k_packed, con
                                          is_causal, dtype, stream);
 }
 
+extern "C" size_t fq_attention_workspace_bytes(int num_seqs, int max_q_len, int64_t max_kv_len, int H_Q, int H_KV, int D) {
+    using namespace fq;
+    if (num_seqs <= 0 || max_q_len <= 0 || max_kv_len <= 0 || H_KV <= 0 || H_Q <= 0 || H_Q % H_KV != 0) return 0;
+    return part_bytes(plan_of(num_seqs, max_q_len, max_kv_len, H_Q, H_KV, D), num_seqs, H_KV, D);
+}
+
 extern "C" int fq_fused_tq_attention_strided(const void* q, const uint8_t* k_packed, const float* k_norms,
                                              const uint8_t* v_packed, const float* v_norms,
                                              const float* centroids_k, const float* centroids_v,
@@ -721,6 +1001,19 @@ extern "C" int fq_fused_tq_attention_strided(const void* q, const uint8_t* k_pac
                                              int B, int H_Q, int H_KV, int N_Q, int N_KV,
                                              int64_t k_capacity, int64_t v_capacity, int D,
                                              float sm_scale, int is_causal, int dtype, void* stream) {
+    return fq_fused_tq_attention_split(q, k_packed, k_norms, v_packed, v_norms, centroids_k, centroids_v, rotation,
+                                       rotation_col_major, out, B, H_Q, H_KV, N_Q, N_KV, k_capacity, v_capacity, D, sm_scale,
+                                       is_causal, dtype, nullptr, 0, stream);
+}
+
+extern "C" int fq_fused_tq_attention_split(const void* q, const uint8_t* k_packed, const float* k_norms,
+                                             const uint8_t* v_packed, const float* v_norms,
+                                             const float* centroids_k, const float* centroids_v,
+                                             const float* rotation, int rotation_col_major, void* out,
+                                             int B, int H_Q, int H_KV, int N_Q, int N_KV,
+                                             int64_t k_capacity, int64_t v_capacity, int D,
+                                             float sm_scale, int is_causal, int dtype, void* workspace,
+                                           size_t workspace_bytes, void* stream) {
     using namespace fq;
     if (B < 0 || H_Q <= 0 || H_KV <= 0 || N_Q < 0 || N_KV < 0 || H_Q % H_KV != 0) return FQ_ERR_BAD_SHAPE;
     if (k_capacity < N_KV || v_capacity < N_KV) return FQ_ERR_BAD_SHAPE;
@@ -770,7 +1063,21 @@ extern "C" int fq_fused_tq_attention_strided(const void* q, const uint8_t* k_pac
     p.max_blocks = 0; p.num_blocks = 0; p.bs_log2 = 0;
     p.round_slots = fq_host::device_cu_count();
     p.out_wide = fq_host::aligned(out, 16);
-    return D == 64 ? launch_prefill<64, false>(p, grid, dtype, s) : launch_prefill<128, false>(p, grid, dtype, s);
+    p.num_seqs = B;
+    p.max_w = int(wgs);
+    // A launch that fills the chip keeps the plain order, one that leaves CUs idle is split if the lengths allow (here
+    // they are known: a plan under which no workgroup would be split is dropped).
+    SplitPlan sp = plan_of(B, N_Q, N_KV, H_Q, H_KV, D);
+    if (sp.max_pieces > 1) {
+        const SeqShape sh = make_seq_shape(N_Q, N_KV, 0, p.G, p.max_w);
+        const uint32_t sum = uint32_t(B) * (uint32_t(sh.W) * uint32_t(tiles_of(sh, 0, p.G, p.causal) + tiles_of(sh, sh.W - 1, p.G, p.causal) + 1) / 2);
+        if (pieces_of(sh, share_of(sum * uint32_t(H_KV), p.round_slots), sp.split_w, sp.max_pieces, p.G, p.causal) < 2) sp = SplitPlan{0, 1};
+    }
+    const int st = use_plan(p, sp, D, workspace, workspace_bytes);
+    if (st != FQ_OK) return st;
+    if (p.max_pieces > 1)
+        return launch_prefill<false, true>(p, D, folded_grid(int64_t(B) * H_KV * wgs * p.max_pieces), N_Q, dtype, s);
+    return launch_prefill<false, false>(p, D, grid, N_Q, dtype, s);
 }
 
 extern "C" int fq_paged_tq4_prefill(const void* q, const int32_t* cu_seqlens_q, const uint8_t* kv_cache,
@@ -780,6 +1087,18 @@ extern "C" int fq_paged_tq4_prefill(const void* q, const int32_t* cu_seqlens_q, 
                                     int num_seqs, int max_q_len, int H_Q, int H_KV, int D, int block_size,
                                     int max_blocks_per_seq, int64_t num_blocks, float sm_scale, int is_causal,
                                     int dtype, void* stream) {
+    return fq_paged_tq4_prefill_split(q, cu_seqlens_q, kv_cache, block_table, seq_lens, centroids_k, centroids_v, rotation,
+                                      rotation_col_major, out, num_seqs, max_q_len, H_Q, H_KV, D, block_size,
+                                      max_blocks_per_seq, num_blocks, sm_scale, is_causal, dtype, 0, nullptr, 0, stream);
+}
+
+extern "C" int fq_paged_tq4_prefill_split(const void* q, const int32_t* cu_seqlens_q, const uint8_t* kv_cache,
+                                    const int32_t* block_table, const int32_t* seq_lens,
+                                    const float* centroids_k, const float* centroids_v,
+                                    const float* rotation, int rotation_col_major, void* out,
+                                    int num_seqs, int max_q_len, int H_Q, int H_KV, int D, int block_size,
+                                    int max_blocks_per_seq, int64_t num_blocks, float sm_scale, int is_causal,
+                                    int dtype, int64_t total_q, void* workspace, size_t workspace_bytes, void* stream) {
     using namespace fq;
     if (num_seqs < 0 || max_q_len < 0 || H_Q <= 0 || H_KV <= 0 || H_Q % H_KV != 0 || max_blocks_per_seq <= 0 ||
         num_blocks <= 0 || num_blocks > 0x7fffffffLL)
@@ -826,10 +1145,21 @@ extern "C" int fq_paged_tq4_prefill(const void* q, const int32_t* cu_seqlens_q, 
     p.round_slots = fq_host::device_cu_count();
     p.out_wide = fq_host::aligned(out, 16);
 
-    const int64_t units = int64_t((max_q_len + 31) / 32) * p.G;
-    const int64_t wgs = (units + 7) / 8;
+    const int64_t wgs = workgroups_of(max_q_len, p.G);
     if (wgs > 0x7fffffffLL) return FQ_ERR_BAD_SHAPE;
-    const dim3 grid(static_cast<unsigned>(wgs), H_KV, num_seqs);
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    return D == 64 ? launch_prefill<64, true>(p, grid, dtype, s) : launch_prefill<128, true>(p, grid, dtype, s);
+    p.num_seqs = num_seqs;
+    p.max_w = int(wgs);
+    const int st = use_plan(p, plan_of(num_seqs, max_q_len, int64_t(max_blocks_per_seq) * block_size, H_Q, H_KV, D), D,
+                            workspace, workspace_bytes);
+    if (st != FQ_OK) return st;
+    // places per KV head: every sequence of the longest kind, fewer when the tokens of the batch are known (a sequence
+    // takes at most (n / 32 + 1) G / 8 + 1 workgroups), and the pieces beyond the first of those that may be split
+    int64_t places = num_seqs * wgs;
+    if (total_q > 0) {
+        const int64_t most = (total_q / 32 + num_seqs) * p.G / 8 + num_seqs;
+        places = most < places ? most : places;
+    }
+    places += int64_t(num_seqs) * p.split_w * (p.max_pieces - 1);
+    if (places * H_KV > 0x7fffffffLL) return FQ_ERR_BAD_SHAPE;
+    return launch_prefill<true, true>(p, D, folded_grid(places * H_KV), max_q_len, dtype, static_cast<hipStream_t>(stream));
 }
