@@ -1,8 +1,8 @@
-// Fused TQ4 attention for head_dim 64 and 256 (and, as a cross-check, 128): the operator of
+// Fused TQ4 attention for any of the head dimensions 64, 128 and 256 in a plainer shape: the operator of
 // fq_fused_attention.hip (src/flashquant/kernels/cpu_reference.py:154-227, the launcher
-// csrc/cuda/fused_tq_attention.cu:468-511 takes all three dimensions) in a plainer shape.
-// The tuned kernel's tile layout is written for 128 coordinates; this one trades speed for
-// generality and shares nothing with it but the arithmetic rules:
+// csrc/cuda/fused_tq_attention.cu:468-511).  It is what the tuned kernel is checked against (the switch
+// FQ_OPT_ATTENTION_ANY_DIM) and takes paged batches of head_dim 256 beyond the tuned kernel's grid; it shares
+// nothing with the tuned kernel but the arithmetic rules:
 //   q_rot = (q @ R^T) rounded to the query dtype (float32 MFMA)
 //   K, V  = fp16(centroid[idx] * norm), scores and P.V on v_mfma_f32_16x16x32_f16
 //   out   = (softmax(...) V) @ R, rounded once (contiguous operands) or rounded before and after

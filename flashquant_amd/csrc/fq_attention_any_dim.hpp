@@ -34,6 +34,6 @@ int launch_attention_any_dim(const AnyDimParams& p, int D, bool paged, int max_q
 }  // namespace fq
 
 namespace fq_host {
-// FQ_ATTENTION_ANY_DIM=1 routes head_dim 128 to the general kernel too (both are kept tested).
+// FQ_ATTENTION_ANY_DIM=1 routes every head_dim to the general kernel (both are kept tested).
 bool force_any_dim_attention();
 }

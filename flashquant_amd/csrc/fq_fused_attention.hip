@@ -1,4 +1,4 @@
-// Fused TQ4 FlashAttention (prefill) for gfx950, head_dim 64 and 128: un-rotated query in,
+// Fused TQ4 FlashAttention (prefill) for gfx950, head_dim 64, 128 and 256: un-rotated query in,
 // packed TQ4 keys and values in, original-space output out.  (The figures in this comment are
 // those of head_dim 128.)
 //
@@ -31,6 +31,13 @@
 // 8 consecutive positions are exactly its 8 tokens.  The K tile uses the same
 // permutation on the coordinates, and the query operand is read to match.
 //
+// head_dim 256: tiles of 32 tokens (the accumulators of 32 rows, their query operand and the scores are 208 of a lane's
+// 256 registers), the second product in groups of two coordinate blocks, the rotation matrix in four rounds through LDS
+// (it is 256 KB in two terms).  Per flop the tile loop costs what it costs at 128: 2.6 us for 256 rows x 32 tokens, bound
+// like it by the chain K reads - scores - weights - V reads - output.  The general kernel (fq_attention_any_dim.hip), which
+// served this dimension with 16 rows a wavefront, read twice the LDS bytes per row: 16 heads x 3001 tokens fp16 516 -> 308 us,
+// 2 x 32 x 700 tokens bf16 260 -> 114 us, 16 x 65 tokens 93 -> 53 us; one query over 3 x 3500 tokens 369 -> 85 us (in pieces).
+//
 // The two head rotations run inside the kernel (prologue and epilogue) on the fp16 MFMA
 // with operands split into two fp16 terms, staged through the tile buffers.
 #include "fq_common.hpp"
@@ -40,21 +47,25 @@
 
 namespace fq {
 
-// Tile geometry for head_dim D (64 or 128).
+// Tile geometry for head_dim D (64, 128 or 256).
 template <int D>
 struct PrefillCfg {
+    static constexpr int TS = D == 256 ? 5 : 6;           // log2 of the tokens of a tile
+    static constexpr int TT = 1 << TS;
     static constexpr int KSTRIDE = 2 * D + 16;            // bytes per token row of the K tile (D fp16 + pad): 4 banks
-    static constexpr int KBYTES = 64 * KSTRIDE;           // 17408 at D = 128
-    static constexpr int VBYTES = D * 128;                // V^T tile: D coordinate rows x 64 tokens fp16
+    static constexpr int KBYTES = TT * KSTRIDE;           // 17408 at D = 128
+    static constexpr int VBYTES = 2 * D * TT;             // V^T tile: D coordinate rows x TT tokens fp16
     static constexpr int BUF = KBYTES + VBYTES;           // 33792 at D = 128
     static constexpr int NKS = D / 16;                    // k-steps of the score product
     static constexpr int NOB = D / 32;                    // 32-coordinate blocks of the output
     static constexpr int PB = D / 2;                      // packed bytes per token and head
     // The rotation matrix as MFMA operands (two fp16 terms), shared by the wavefronts of a workgroup:
     // a block of 32 x 16 holds one 16-byte operand per lane and term.  They lie where the lookup
-    // tables are between the query stage and the end of the tile loop (64 KB).
+    // tables are between the query stage and the end of the tile loop (64 KB), at D = 256 a quarter at a time.
     static constexpr int SLOT = 8 * (32 * D + 64);        // floats: per unit 32 rows un-normalised, 32 maxima, 32 sums
-    static constexpr int RTERM = NKS * NOB * 64 * 16;     // bytes per term: 32768 at D = 128
+    static constexpr int RROUNDS = D == 256 ? 4 : 1;
+    static constexpr int RBLK = NOB / RROUNDS;            // blocks of 32 result coordinates in a round
+    static constexpr int RTERM = NKS * RBLK * 64 * 16;    // bytes per term: 32768 at D = 128 and 256
 };
 
 struct PrefillParams {
@@ -90,8 +101,16 @@ __device__ __forceinline__ uint32_t scale_pair(uint32_t pair, half2v n2) {
     return __builtin_bit_cast(uint32_t, h);
 }
 
-__device__ __forceinline__ uint32_t pack_rtz(float a, float b) {
-    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
+// A pair of weights as fp16: towards zero in one instruction, at 256 coordinates to nearest.  Against 64 bits, fp16, 16 heads
+// x 3001 tokens: relative error 8.9e-4 on the general kernel that served this dimension, 9.1e-4 towards zero, 8.9e-4 to nearest.
+template <int D>
+__device__ __forceinline__ uint32_t pack_weights(float a, float b) {
+    if constexpr (D == 256) {
+        const half2v h = {_Float16(a), _Float16(b)};
+        return __builtin_bit_cast(uint32_t, h);
+    } else {
+        return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
+    }
 }
 
 template <bool PAGED>
@@ -205,12 +224,13 @@ template <int D, int DT, bool PAGED, bool SCHED>
 __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillParams p) {
     using Cfg = PrefillCfg<D>;
     constexpr int kPfKStride = Cfg::KSTRIDE, kPfKBytes = Cfg::KBYTES, kPfBufBytes = Cfg::BUF;
-    constexpr int NKS = Cfg::NKS, NOB = Cfg::NOB, PB = Cfg::PB;
+    constexpr int NKS = Cfg::NKS, NOB = Cfg::NOB, PB = Cfg::PB, TS = Cfg::TS, TT = Cfg::TT;
+    constexpr int NTB = TT / 32, NVS = TT / 16;    // 32-token blocks of the scores, k-steps of the second product
     __shared__ __attribute__((aligned(256))) uint32_t lut[256 * 64];
     extern __shared__ __attribute__((aligned(16))) uint8_t bufs[];   // 2 x (K tile | V^T tile)
     // Rows whose norm times a centroid would not fit fp16 are stored divided by a power of two.
     // big_tile[buf] = tile + 1 marks a tile that holds such rows; scale_exp[buf] holds the exponents,
-    // K rows 0..63 then V rows 0..63, each tagged with tile + 1 in its upper bits (an entry with
+    // K rows 0..TT-1 then V rows 0..TT-1, each tagged with tile + 1 in its upper bits (an entry with
     // another tag is left over from an earlier tile and reads as 0).
     __shared__ int big_tile[2];
     __shared__ __attribute__((aligned(16))) int scale_exp[2][128];
@@ -268,17 +288,21 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     int wg_maxpos = 32 * (last_unit / p.G) + 31;
     wg_maxpos = wg_maxpos < NQ - 1 ? wg_maxpos : NQ - 1;
     int my_maxpos = pos0 + 31 < NQ - 1 ? pos0 + 31 : NQ - 1;
-    const int all_tiles = (NKV + 63) >> 6;
+    const int all_tiles = (NKV + TT - 1) >> TS;
     int ntiles = all_tiles, my_tiles = all_tiles;
     if (p.causal) {
-        ntiles = ((qoff + wg_maxpos) >> 6) + 1 < all_tiles ? ((qoff + wg_maxpos) >> 6) + 1 : all_tiles;
-        my_tiles = ((qoff + my_maxpos) >> 6) + 1 < all_tiles ? ((qoff + my_maxpos) >> 6) + 1 : all_tiles;
+        ntiles = ((qoff + wg_maxpos) >> TS) + 1 < all_tiles ? ((qoff + wg_maxpos) >> TS) + 1 : all_tiles;
+        my_tiles = ((qoff + my_maxpos) >> TS) + 1 < all_tiles ? ((qoff + my_maxpos) >> TS) + 1 : all_tiles;
     }
-    // this piece's tiles: first_tile .. ntiles - 1 (of this wavefront: .. my_tiles - 1)
+    // this piece's tiles: first_tile .. ntiles - 1 (of this wavefront: .. my_tiles - 1).  Pieces are cut between the
+    // schedule's tiles of 64 keys.
     int first_tile = 0;
     if (SCHED && pieces > 1) {
-        first_tile = int(int64_t(ntiles) * piece / pieces);
-        ntiles = int(int64_t(ntiles) * (piece + 1) / pieces);
+        constexpr int SH = 6 - TS;
+        const int whole = (ntiles + (1 << SH) - 1) >> SH;
+        first_tile = int(int64_t(whole) * piece / pieces) << SH;
+        const int end = int(int64_t(whole) * (piece + 1) / pieces) << SH;
+        ntiles = ntiles < end ? ntiles : end;
         my_tiles = my_tiles < ntiles ? my_tiles : ntiles;
     }
     if (!unit_live) my_tiles = 0;
@@ -299,13 +323,19 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     const float* knp = p.k_norms + k_row0;
     const float* vnp = p.v_norms + v_row0;
     // Work items of the dequantisation.  K: (token of the tile, 16-coordinate group); V: (token pair, dword
-    // of the packed row).  head_dim 128: 512 of each, every thread takes one of both; head_dim 64: 256 of
-    // each, wavefronts 0..3 take the V items and wavefronts 4..7 the K items.
+    // of the packed row).  head_dim 128 and 256: 512 of each, every thread takes one of both; head_dim 64: 256
+    // of each, wavefronts 0..3 take the V items and wavefronts 4..7 the K items.
     constexpr bool kSplitRoles = D == 64;
     const bool does_k = !kSplitRoles || w >= 4;
     const bool does_v = !kSplitRoles || w < 4;
     int gqk, tk, jv, tp;
-    if constexpr (!kSplitRoles) {
+    if constexpr (D == 256) {
+        // as for 128, with 4 tokens x 16 groups and 4 pairs x 16 dwords a wavefront
+        gqk = (lane & 3) | ((lane >> 1) & 4) | ((lane >> 2) & 8);
+        tk = 4 * w + ((lane >> 2) & 1) + ((lane >> 3) & 2);
+        jv = (lane & 7) | ((lane >> 2) & 8) | ((w >> 2) << 4);
+        tp = 8 * ((w >> 1) & 1) + 2 * (w & 1) + ((lane >> 3) & 1) + 4 * ((lane >> 4) & 1);
+    } else if constexpr (!kSplitRoles) {
         // K lane bits (g0 g1 t0 g2 t1 t2): eight consecutive lanes hold four groups of two consecutive
         // tokens, so the 128 bytes they store with one 16-byte write each fall into 32 different banks
         // (token rows are 272 bytes apart: 4 banks).
@@ -327,24 +357,40 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
         tp = 8 * (w & 3) + 2 * (i8 >> 2) + (i8 & 1) + 4 * ((i8 >> 1) & 1);
     }
     const int k_wr = tk * kPfKStride + gqk * 32;
-    int v_wr[8];
+    // (256 coordinates: the registers are few, the variants of an offset are made where they are used)
+    int v_wr[TT == 64 ? 8 : 1];
     {
         const int tt = 2 * tp, t16 = tt & 15;
         const int posv = (tt & ~15) + 8 * ((t16 >> 2) & 1) + 4 * ((t16 >> 3) & 1) + (t16 & 3);
         const int giv = posv >> 3, within = posv & 7;
+        if constexpr (TT == 64) {
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int d = 8 * jv + k;
-            const int physg = giv ^ k ^ (jv & 7);
-            v_wr[k] = kPfKBytes + d * 128 + 16 * physg + 2 * within;
+            for (int k = 0; k < 8; ++k) {
+                const int d = 8 * jv + k;
+                const int physg = giv ^ k ^ (jv & 7);
+                v_wr[k] = kPfKBytes + d * 128 + 16 * physg + 2 * within;
+            }
+        } else {
+            v_wr[0] = kPfKBytes + jv * 512 + 16 * (giv ^ (jv & 7)) + 2 * within;
         }
     }
+    // Offset of coordinate 8 jv + k.  Tiles of 32 tokens: 128 bytes hold two coordinate rows of four groups, and the
+    // eight 16-byte places are permuted so that eight dwords of a store, or eight rows of an operand read, fall into eight.
+    auto v_write = [&](int k) {
+        if constexpr (TT == 64) {
+            return v_wr[k];
+        } else {
+            int base = v_wr[0];
+            asm volatile("" : "+v"(base));
+            return (base ^ (16 * (4 * (k & 1) + (k >> 1)))) + (k >> 1) * 128;
+        }
+    };
     uint2v kraw = {0u, 0u};
     uint32_t vra = 0u, vrb = 0u;
     float nk = 0.0f, nv0 = 0.0f, nv1 = 0.0f;
     auto issue_loads = [&](int tile_raw) {
         const int tile = tile_raw < ntiles ? tile_raw : ntiles - 1;   // past the end: the last tile again, never used
-        const int t0 = tile > 0 ? tile * 64 : 0;
+        const int t0 = tile > 0 ? tile * TT : 0;
         const int last = NKV > 0 ? NKV - 1 : 0;
         const int tkk = t0 + tk < last ? t0 + tk : last;
         const int ta = t0 + 2 * tp < last ? t0 + 2 * tp : last;
@@ -398,8 +444,8 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
             const int tag = (tile + 1) << 8;
             if (does_k && gqk == 0) scale_exp[buf][tk] = tag | ek;
             if (does_v && jv == 0) {
-                scale_exp[buf][64 + 2 * tp] = tag | ev0;
-                scale_exp[buf][64 + 2 * tp + 1] = tag | ev1;
+                scale_exp[buf][TT + 2 * tp] = tag | ev0;
+                scale_exp[buf][TT + 2 * tp + 1] = tag | ev1;
             }
             if ((ek | ev0 | ev1) != 0) big_tile[buf] = tile + 1;
         }
@@ -424,8 +470,8 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
             const uint32_t xs[4] = {xe.x, xe.y, xe.z, xe.w}, ys[4] = {yo.x, yo.y, yo.z, yo.w};
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                *reinterpret_cast<uint32_t*>(dst + v_wr[2 * c]) = scale_pair(xs[c], nv2);
-                *reinterpret_cast<uint32_t*>(dst + v_wr[2 * c + 1]) = scale_pair(ys[c], nv2);
+                *reinterpret_cast<uint32_t*>(dst + v_write(2 * c)) = scale_pair(xs[c], nv2);
+                *reinterpret_cast<uint32_t*>(dst + v_write(2 * c + 1)) = scale_pair(ys[c], nv2);
             }
         }
     };
@@ -442,15 +488,15 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     // What it replaced staged the rows through LDS for the 16x16x32 MFMA (16 to 32 lanes on a bank) and stored the
     // results 2 bytes a lane: a workgroup per CU on 64 tokens of 32 heads over 64 keys took 33 us and 27 us with one
     // query row, 24 and 15.5 us this way (the tile itself: 2 us); 4 x 32 heads x 8192 tokens 2.94 -> 2.77 ms.
-    constexpr int BPW = NOB * NKS / 8;
+    constexpr int RROUNDS = Cfg::RROUNDS, RBLK = Cfg::RBLK, BPW = RBLK * NKS / 8;
     uint8_t* rshare = reinterpret_cast<uint8_t*>(lut);
     float rbv[BPW][8];
     // `back`: x @ R with the contraction index in the order of the accumulator registers (element 4 a + c of half
     // hf = coordinate 8 a + 4 hf + c of the k-step), else x @ R^T in the natural order
-    auto fetch_rotation = [&](bool back) {
+    auto fetch_rotation = [&](bool back, int round) {
 #pragma unroll
         for (int i = 0; i < BPW; ++i) {
-            const int blk = BPW * w + i, j = 32 * (blk / NKS) + m32, k0 = 16 * (blk % NKS);
+            const int blk = BPW * w + i, j = 32 * (RBLK * round + blk / NKS) + m32, k0 = 16 * (blk % NKS);
             const int k1 = back ? k0 + 4 * hf : k0 + 8 * hf, step = back ? 8 : 4;    // coordinates k1 + 0..3, k1 + step + 0..3
             if (back == (p.rot_col_major != 0)) {          // a lane's coordinates are neighbours in memory
                 const float4v lo = *reinterpret_cast<const float4v*>(p.rotation + j * D + k1);
@@ -493,7 +539,7 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks)
             raw[ks] = *reinterpret_cast<const uint4v*>(qbase + int64_t(pos) * q_stride + 16 * ks + 8 * hf);
-        fetch_rotation(false);
+        fetch_rotation(false, 0);
         // the rows are exact in fp16 up to a power of two
         half8 qa[NKS];
         float mx = 0.0f;
@@ -511,24 +557,41 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
                 qa[ks][2 * i] = _Float16(load_elem<DT>(uint16_t(raw[ks][i] & 0xffffu)) * pow2(-ex));
                 qa[ks][2 * i + 1] = _Float16(load_elem<DT>(uint16_t(raw[ks][i] >> 16)) * pow2(-ex));
             }
-        share_rotation();
-        __syncthreads();
-        float16v rot[NOB];
+        float16v rot[D == 256 ? 1 : NOB];
+        uint32_t rot16[D == 256 ? NOB : 1][8];          // 256 coordinates: held as the 16-bit pairs they are rounded to
         float mr = 0.0f;
 #pragma unroll
-        for (int jb = 0; jb < NOB; ++jb) {
-            float16v hi, lo;
+        for (int round = 0; round < RROUNDS; ++round) {
+            if (round > 0) __syncthreads();             // every wavefront is done with the round before
+            share_rotation();
+            __syncthreads();
+            if (round + 1 < RROUNDS) fetch_rotation(false, round + 1);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) { hi[r] = 0.0f; lo[r] = 0.0f; }
+            for (int jr = 0; jr < RBLK; ++jr) {
+                const int jb = RBLK * round + jr;
+                float16v hi, lo;
 #pragma unroll
-            for (int ks = 0; ks < NKS; ++ks) {
-                hi = __builtin_amdgcn_mfma_f32_32x32x16_f16(rotation_term(0, jb, ks), qa[ks], hi, 0, 0, 0);
-                lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(rotation_term(1, jb, ks), qa[ks], lo, 0, 0, 0);
-            }
+                for (int r = 0; r < 16; ++r) { hi[r] = 0.0f; lo[r] = 0.0f; }
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                rot[jb][r] = load_elem<DT>(store_elem<DT>((hi[r] + lo[r] * (1.0f / 4096.0f)) * pow2(ex)));
-                mr = __builtin_fmaxf(mr, __builtin_fabsf(rot[jb][r]));
+                for (int ks = 0; ks < NKS; ++ks) {
+                    hi = __builtin_amdgcn_mfma_f32_32x32x16_f16(rotation_term(0, jr, ks), qa[ks], hi, 0, 0, 0);
+                    lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(rotation_term(1, jr, ks), qa[ks], lo, 0, 0, 0);
+                }
+                if constexpr (D == 256) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        const uint16_t x = store_elem<DT>((hi[2 * i] + lo[2 * i] * (1.0f / 4096.0f)) * pow2(ex));
+                        const uint16_t y = store_elem<DT>((hi[2 * i + 1] + lo[2 * i + 1] * (1.0f / 4096.0f)) * pow2(ex));
+                        mr = __builtin_fmaxf(mr, __builtin_fmaxf(__builtin_fabsf(load_elem<DT>(x)), __builtin_fabsf(load_elem<DT>(y))));
+                        rot16[jb][i] = uint32_t(x) | uint32_t(y) << 16;
+                    }
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        rot[jb][r] = load_elem<DT>(store_elem<DT>((hi[r] + lo[r] * (1.0f / 4096.0f)) * pow2(ex)));
+                        mr = __builtin_fmaxf(mr, __builtin_fabsf(rot[jb][r]));
+                    }
+                }
             }
         }
         const int er = row_exponent(mr);
@@ -537,7 +600,12 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) qb[ks][e] = _Float16(rot[ks >> 1][8 * (ks & 1) + e] * pow2(-er));
+            for (int e = 0; e < 8; ++e) {
+                float v;
+                if constexpr (D == 256) v = load_elem<DT>(uint16_t(rot16[ks >> 1][4 * (ks & 1) + (e >> 1)] >> (16 * (e & 1))));
+                else v = rot[ks >> 1][8 * (ks & 1) + e];
+                qb[ks][e] = _Float16(v * pow2(-er));
+            }
         __syncthreads();   // the rotation operands become lookup tables
     }
     fill_pair_tables<8>(lut, p.centroids_k[lane & 15], p.centroids_v[lane & 15], 15, w, lane);
@@ -545,11 +613,11 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
 
     // ---- lane-constant LDS read offsets ----------------------------------------------------------
     const int k_rd = m32 * kPfKStride + 16 * hf;
-    int v_rd[8];
+    int v_rd[TT == 64 ? 8 : 1];
     {
-        const int lanex = hf ^ (m32 & 7) ^ (m32 >> 3);
+        const int lanex = TT == 64 ? hf ^ (m32 & 7) ^ (m32 >> 3) : hf ^ (4 * (m32 & 1) + ((m32 >> 1) & 3)) ^ (m32 >> 3);
 #pragma unroll
-        for (int c = 0; c < 8; ++c) v_rd[c] = kPfKBytes + m32 * 128 + 16 * (lanex ^ c);
+        for (int c = 0; c < (TT == 64 ? 8 : 1); ++c) v_rd[c] = kPfKBytes + (TT == 64 ? m32 : m32 >> 1) * 128 + 16 * (lanex ^ c);
     }
 
     // ---- running state -----------------------------------------------------------------------------
@@ -564,9 +632,9 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
 
     auto compute = [&](int tile, int buf) {
         const uint8_t* kt = bufs + buf * kPfBufBytes;
-        float16v S[2];
+        float16v S[NTB];
 #pragma unroll
-        for (int tb = 0; tb < 2; ++tb) {
+        for (int tb = 0; tb < NTB; ++tb) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) S[tb][r] = 0.0f;
 #pragma unroll
@@ -575,7 +643,7 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
                 S[tb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qb[ks], S[tb], 0, 0, 0);
             }
         }
-        const int t0 = tile * 64;
+        const int t0 = tile * TT;
         // rows stored divided by a power of two (norms beyond fp16's range): wavefront-uniform, rare
         const bool big = __builtin_amdgcn_readfirstlane(big_tile[buf]) == tile + 1;
         auto exps_of = [&](int first) {        // the exponents of four consecutive rows of this tile
@@ -587,7 +655,7 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
         };
         if (big) {
 #pragma unroll
-            for (int tb = 0; tb < 2; ++tb)
+            for (int tb = 0; tb < NTB; ++tb)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const int4v e = exps_of(32 * tb + 8 * q + 4 * hf);
@@ -595,13 +663,13 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
                     for (int c = 0; c < 4; ++c) S[tb][4 * q + c] = __builtin_ldexpf(S[tb][4 * q + c], e[c]);
                 }
         }
-        const bool need_mask = (t0 + 63 >= NKV) || (p.causal && t0 + 63 > qoff + pos0);   // wavefront-uniform
+        const bool need_mask = (t0 + TT - 1 >= NKV) || (p.causal && t0 + TT - 1 > qoff + pos0);   // wavefront-uniform
         if (need_mask) {
             int lim = NKV - 1;
             if (p.causal && qpos < lim) lim = qpos;
             lim -= t0;                         // token offsets <= lim are visible
 #pragma unroll
-            for (int tb = 0; tb < 2; ++tb)
+            for (int tb = 0; tb < NTB; ++tb)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int off = 32 * tb + 8 * (r >> 2) + 4 * hf + (r & 3);
@@ -612,7 +680,7 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
         if (!big) {
             float mx = S[0][0];
 #pragma unroll
-            for (int tb = 0; tb < 2; ++tb)
+            for (int tb = 0; tb < NTB; ++tb)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) mx = __builtin_fmaxf(mx, S[tb][r]);
             cand = mx * krow;
@@ -621,10 +689,10 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
             // taken over score + e, so that these weights stay below 16 as well
             cand = -__builtin_inff();
 #pragma unroll
-            for (int tb = 0; tb < 2; ++tb)
+            for (int tb = 0; tb < NTB; ++tb)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const int4v e = exps_of(64 + 32 * tb + 8 * q + 4 * hf);
+                    const int4v e = exps_of(TT + 32 * tb + 8 * q + 4 * hf);
 #pragma unroll
                     for (int c = 0; c < 4; ++c)
                         cand = __builtin_fmaxf(cand, __builtin_fmaf(S[tb][4 * q + c], krow, float(e[c])));
@@ -632,24 +700,26 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
         }
         cand = max_xor32(cand);
         // the running maximum moves only when it would grow by more than 2^4: the weights stay
-        // below 16 and the rescale of the accumulator registers becomes rare
-        const float mnew = cand > m_run + 4.0f ? cand : m_run;
+        // below 16 and the rescale of the accumulator registers becomes rare.  At 256 coordinates it always moves, so
+        // that the largest weight is exactly 1, as on the general kernel: error against 64 bits 8.88e-4 (8.92e-4
+        // otherwise, 8.88e-4 there; fp16, 3001 tokens) for 5 % of the time.
+        const float mnew = cand > m_run + (D == 256 ? 0.0f : 4.0f) ? cand : m_run;
         const float ms = mnew == -__builtin_inff() ? 0.0f : mnew;
         const float alpha = __builtin_amdgcn_exp2f(m_run - ms);
         m_run = mnew;
-        uint4v pbv[4];
+        uint4v pbv[NVS];
         float ps = 0.0f;
         // two copies of the weight loop, so that the common one has no branch inside (the values of a
         // loop with a rare branch in it are copied where the paths meet)
         if (!big) {
             const half2v ones = {_Float16(1.0f), _Float16(1.0f)};
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
+            for (int s = 0; s < NVS; ++s) {
                 float pe[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
                     pe[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(S[s >> 1][8 * (s & 1) + e], krow, -ms));
-                const uint32_t pw[4] = {pack_rtz(pe[0], pe[1]), pack_rtz(pe[2], pe[3]), pack_rtz(pe[4], pe[5]), pack_rtz(pe[6], pe[7])};
+                const uint32_t pw[4] = {pack_weights<D>(pe[0], pe[1]), pack_weights<D>(pe[2], pe[3]), pack_weights<D>(pe[4], pe[5]), pack_weights<D>(pe[6], pe[7])};
                 // the denominator sums the weights as the second product sees them (fp16, one
                 // v_dot2_f32_f16 per pair)
 #pragma unroll
@@ -658,7 +728,7 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
             }
         } else {
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
+            for (int s = 0; s < NVS; ++s) {
                 float pe[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
@@ -667,11 +737,11 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
                 }
 #pragma unroll
                 for (int q = 0; q < 2; ++q) {
-                    const int4v ev = exps_of(64 + 32 * (s >> 1) + 8 * (2 * (s & 1) + q) + 4 * hf);
+                    const int4v ev = exps_of(TT + 32 * (s >> 1) + 8 * (2 * (s & 1) + q) + 4 * hf);
 #pragma unroll
                     for (int c = 0; c < 4; ++c) pe[4 * q + c] = __builtin_ldexpf(pe[4 * q + c], ev[c]);
                 }
-                pbv[s] = uint4v{pack_rtz(pe[0], pe[1]), pack_rtz(pe[2], pe[3]), pack_rtz(pe[4], pe[5]), pack_rtz(pe[6], pe[7])};
+                pbv[s] = uint4v{pack_weights<D>(pe[0], pe[1]), pack_weights<D>(pe[2], pe[3]), pack_weights<D>(pe[4], pe[5]), pack_weights<D>(pe[6], pe[7])};
             }
         }
         l_run = __builtin_fmaf(l_run, alpha, ps);
@@ -686,24 +756,35 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
         // not cover the LDS round trip): fences keep the groups in this order.
         auto v_operand = [&](int ob, int s) {
             const int c = (2 * s) ^ (4 * (ob & 1));
-            return *reinterpret_cast<const half8*>(kt + v_rd[c] + ob * 4096);
+            if constexpr (TT == 64) {
+                return *reinterpret_cast<const half8*>(kt + v_rd[c] + ob * (64 * TT));
+            } else {
+                int base = v_rd[0];
+                asm volatile("" : "+v"(base));
+                return *reinterpret_cast<const half8*>(kt + (base ^ (16 * c)) + ob * (64 * TT));
+            }
         };
-        half8 va[4][NOB];
+        // groups of VG blocks; at 256 coordinates the registers allow two blocks (of the eight) a group
+        constexpr int VG = D == 256 ? 2 : NOB, NG = NVS * NOB / VG;
+        half8 va[NG][VG];
+        auto read_group = [&](int g) {
 #pragma unroll
-        for (int s = 0; s < 2; ++s)
-#pragma unroll
-            for (int ob = 0; ob < NOB; ++ob) va[s][ob] = v_operand(ob, s);
+            for (int k = 0; k < VG; ++k) va[g][k] = v_operand((g * VG) % NOB + k, (g * VG) / NOB);
+        };
+        read_group(0);
+        read_group(1);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            if (s + 2 < 4) {
-#pragma unroll
-                for (int ob = 0; ob < NOB; ++ob) va[s + 2][ob] = v_operand(ob, s + 2);
+        for (int g = 0; g < NG; ++g) {
+            if (g + 2 < NG) {
+                read_group(g + 2);
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
-            for (int ob = 0; ob < NOB; ++ob)
-                O[ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[s][ob], __builtin_bit_cast(half8, pbv[s]), O[ob], 0, 0, 0);
+            for (int k = 0; k < VG; ++k) {
+                const int ob = (g * VG) % NOB + k;
+                O[ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[g][k], __builtin_bit_cast(half8, pbv[(g * VG) / NOB]), O[ob], 0, 0, 0);
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -746,11 +827,11 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     // ---- normalise, rotate back, store -------------------------------------------------------------------
     const float l_tot = l_run + xor_shuffle(l_run, 32);
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-    fetch_rotation(true);
+    fetch_rotation(true, 0);
     __syncthreads();                // every wavefront is done with the lookup tables
     share_rotation();
     __syncthreads();
-    if (!unit_live) return;
+    if (RROUNDS == 1 && !unit_live) return;
     // float32 rows: both operands as two fp16 terms, three MFMA terms; rows already rounded to 16 bits (the
     // paged form) are exact in one
     float mo = 0.0f;
@@ -783,14 +864,23 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     uint16_t* orow = obase + int64_t(opos) * q_stride;
 #pragma unroll
     for (int cb = 0; cb < NOB; ++cb) {
+        const int cr = cb % RBLK;                      // within the round
+        if (RROUNDS > 1 && cr == 0) {
+            if (cb > 0) {
+                __syncthreads();
+                share_rotation();
+                __syncthreads();
+            }
+            if (cb + RBLK < NOB) fetch_rotation(true, cb / RBLK + 1);
+        }
         float16v hi, lo;
 #pragma unroll
         for (int r = 0; r < 16; ++r) { hi[r] = 0.0f; lo[r] = 0.0f; }
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) {
-            const half8 rh = rotation_term(0, cb, ks);
+            const half8 rh = rotation_term(0, cr, ks);
             hi = __builtin_amdgcn_mfma_f32_32x32x16_f16(rh, ohi[ks], hi, 0, 0, 0);
-            lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(rotation_term(1, cb, ks), ohi[ks], lo, 0, 0, 0);
+            lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(rotation_term(1, cr, ks), ohi[ks], lo, 0, 0, 0);
             if (!PAGED) lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(rh, olo[ks], lo, 0, 0, 0);
         }
         // registers 4 q + c of half hf = coordinate 32 cb + 8 q + 4 hf + c; the halves exchange a quad of every two,
@@ -808,7 +898,7 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
             const auto y = __builtin_amdgcn_permlane32_swap(wd[2 * q + 1], wd[2 * q + 3], false, false);
             const uint4v v = {x[0], y[0], x[1], y[1]};
             uint16_t* dst = orow + 32 * cb + 8 * q + 8 * hf;
-            if (opos < NQ) {
+            if (opos < NQ && unit_live) {
                 if (p.out_wide) {
                     *reinterpret_cast<uint4v*>(dst) = v;
                 } else {
@@ -846,9 +936,10 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillPar
     if (pieces < 2) return;
 
     const float* src = p.part + (int64_t(blockIdx.x) * p.max_pieces) * Cfg::SLOT + u * (32 * D + 64);
-    float rbv[CBW][NJ][8];
+    constexpr bool kAhead = D <= 128;             // (256 coordinates: too many registers)
+    float rbv[kAhead ? CBW : 1][NJ][8];
 #pragma unroll
-    for (int i = 0; i < CBW; ++i)
+    for (int i = 0; i < (kAhead ? CBW : 0); ++i)
         load_rotation_any<D>(p.rotation, p.rot_col_major != 0, false, 16 * (wave + 4 * i), n16, g4, rbv[i]);
     for (int r = wave; r < rows; r += 4) {
         const float* head = src + 32 * D + row0 + r;
@@ -904,7 +995,8 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillPar
 #pragma unroll
     for (int i = 0; i < CBW; ++i) {
         half8 rhi[NJ], rlo[NJ];
-        split_rotation_block<D>(rbv[i], rhi, rlo);
+        if (!kAhead) load_rotation_any<D>(p.rotation, p.rot_col_major != 0, false, 16 * (wave + 4 * i), n16, g4, rbv[0]);
+        split_rotation_block<D>(rbv[kAhead ? i : 0], rhi, rlo);
         const float4v acc = PAGED ? rotate_block_f16<D>(ahi, rhi, rlo) : rotate_block_f16x3<D>(ahi, alo, rhi, rlo);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -939,6 +1031,9 @@ int launch_prefill(const PrefillParams& p, int D, dim3 grid, int max_q, int dtyp
     if (D == 64)
         return dtype == FQ_F16 ? launch_prefill_as<64, FQ_F16, PAGED, SCHED>(p, grid, max_q, s)
                                : launch_prefill_as<64, FQ_BF16, PAGED, SCHED>(p, grid, max_q, s);
+    if (D == 256)
+        return dtype == FQ_F16 ? launch_prefill_as<256, FQ_F16, PAGED, SCHED>(p, grid, max_q, s)
+                               : launch_prefill_as<256, FQ_BF16, PAGED, SCHED>(p, grid, max_q, s);
     return dtype == FQ_F16 ? launch_prefill_as<128, FQ_F16, PAGED, SCHED>(p, grid, max_q, s)
                            : launch_prefill_as<128, FQ_BF16, PAGED, SCHED>(p, grid, max_q, s);
 }
@@ -954,12 +1049,13 @@ inline int64_t workgroups_of(int64_t n_q, int G) { return ((n_q + 31) / 32 * G +
 // The split that a call of these sizes may use, and the bytes its partial rows take.
 inline SplitPlan plan_of(int num_seqs, int max_q, int64_t max_kv, int H_Q, int H_KV, int D) {
     const int64_t max_w = workgroups_of(max_q, H_Q / H_KV);
-    if ((D != 64 && D != 128) || max_w < 1 || max_w > 0x7fffff || fq_host::force_any_dim_attention()) return SplitPlan{0, 1};
+    if (max_w < 1 || max_w > 0x7fffff || fq_host::force_any_dim_attention()) return SplitPlan{0, 1};
     return plan_split(num_seqs, H_KV, int(max_w), (max_kv + 63) / 64, fq_host::device_cu_count());
 }
 inline size_t part_bytes(const SplitPlan& sp, int num_seqs, int H_KV, int D) {
     if (sp.max_pieces < 2) return 0;
-    return size_t(num_seqs) * H_KV * sp.split_w * sp.max_pieces * (D == 64 ? PrefillCfg<64>::SLOT : PrefillCfg<128>::SLOT) * 4;
+    const int slot = D == 64 ? PrefillCfg<64>::SLOT : (D == 128 ? PrefillCfg<128>::SLOT : PrefillCfg<256>::SLOT);
+    return size_t(num_seqs) * H_KV * sp.split_w * sp.max_pieces * slot * 4;
 }
 inline int use_plan(PrefillParams& p, const SplitPlan& sp, int D, void* workspace, size_t workspace_bytes) {
     const size_t need = part_bytes(sp, p.num_seqs, p.H_KV, D);
@@ -1027,9 +1123,9 @@ extern "C" int fq_fused_tq_attention_split(const void* q, const uint8_t* k_packe
     if (!fq_host::aligned(q, 16) || !fq_host::aligned(k_packed, 8) || !fq_host::aligned(v_packed, 4) ||
         !fq_host::aligned(rotation, 16) || !fq_host::aligned(out, 2))
         return FQ_ERR_MISALIGNED;
-    if (B > 65535 || H_KV > 65535) return FQ_ERR_BAD_SHAPE;
+    if (B > 65535 || H_KV > 65535 || (D == 256 && H_Q > 65535)) return FQ_ERR_BAD_SHAPE;
 
-    if (D == 256 || fq_host::force_any_dim_attention()) {   // the tuned tile layout serves 64 and 128 coordinates
+    if (fq_host::force_any_dim_attention()) {
         AnyDimParams a{};
         a.q = static_cast<const uint16_t*>(q);
         a.k_packed = k_packed; a.k_norms = k_norms; a.v_packed = v_packed; a.v_norms = v_norms;
@@ -1112,9 +1208,20 @@ extern "C" int fq_paged_tq4_prefill_split(const void* q, const int32_t* cu_seqle
     if (!fq_host::aligned(q, 16) || !fq_host::aligned(kv_cache, 16) || !fq_host::aligned(rotation, 16) ||
         !fq_host::aligned(out, 2))
         return FQ_ERR_MISALIGNED;
-    if (num_seqs > 65535 || H_KV > 65535) return FQ_ERR_BAD_SHAPE;
+    if (num_seqs > 65535 || H_KV > 65535 || (D == 256 && H_Q > 65535)) return FQ_ERR_BAD_SHAPE;
 
-    if (D == 256 || fq_host::force_any_dim_attention()) {
+    const int64_t wgs = workgroups_of(max_q_len, H_Q / H_KV);
+    const SplitPlan sp = plan_of(num_seqs, max_q_len, int64_t(max_blocks_per_seq) * block_size, H_Q, H_KV, D);
+    // places per KV head: every sequence of the longest kind, fewer when the tokens of the batch are known (a sequence
+    // takes at most (n / 32 + 1) G / 8 + 1 workgroups), and the pieces beyond the first of those that may be split
+    int64_t places = num_seqs * wgs;
+    if (total_q > 0) {
+        const int64_t most = (total_q / 32 + num_seqs) * (H_Q / H_KV) / 8 + num_seqs;
+        places = most < places ? most : places;
+    }
+    const bool fits = wgs <= 0x7fffffffLL && (places + int64_t(num_seqs) * sp.split_w * (sp.max_pieces - 1)) * H_KV <= 0x7fffffffLL;
+    // (the general kernel's grid has no such bound: head_dim 256 runs there beyond it)
+    if (fq_host::force_any_dim_attention() || (D == 256 && !fits)) {
         AnyDimParams a{};
         a.q = static_cast<const uint16_t*>(q);
         a.centroids_k = centroids_k; a.centroids_v = centroids_v;
@@ -1145,21 +1252,11 @@ extern "C" int fq_paged_tq4_prefill_split(const void* q, const int32_t* cu_seqle
     p.round_slots = fq_host::device_cu_count();
     p.out_wide = fq_host::aligned(out, 16);
 
-    const int64_t wgs = workgroups_of(max_q_len, p.G);
-    if (wgs > 0x7fffffffLL) return FQ_ERR_BAD_SHAPE;
+    if (!fits) return FQ_ERR_BAD_SHAPE;
     p.num_seqs = num_seqs;
     p.max_w = int(wgs);
-    const int st = use_plan(p, plan_of(num_seqs, max_q_len, int64_t(max_blocks_per_seq) * block_size, H_Q, H_KV, D), D,
-                            workspace, workspace_bytes);
+    const int st = use_plan(p, sp, D, workspace, workspace_bytes);
     if (st != FQ_OK) return st;
-    // places per KV head: every sequence of the longest kind, fewer when the tokens of the batch are known (a sequence
-    // takes at most (n / 32 + 1) G / 8 + 1 workgroups), and the pieces beyond the first of those that may be split
-    int64_t places = num_seqs * wgs;
-    if (total_q > 0) {
-        const int64_t most = (total_q / 32 + num_seqs) * p.G / 8 + num_seqs;
-        places = most < places ? most : places;
-    }
     places += int64_t(num_seqs) * p.split_w * (p.max_pieces - 1);
-    if (places * H_KV > 0x7fffffffLL) return FQ_ERR_BAD_SHAPE;
     return launch_prefill<true, true>(p, D, folded_grid(places * H_KV), max_q_len, dtype, static_cast<hipStream_t>(stream));
 }

@@ -56,8 +56,8 @@ typedef enum fq_option {
                                      wavefronts that only copy; 0: its computing wavefronts copy too     */
     FQ_OPT_DECODE_DIRECT = 1,     /* FQ_DECODE_DIRECT, default 0: 1 sends every shape to the direct
                                      decode kernel                                                      */
-    FQ_OPT_ATTENTION_ANY_DIM = 2, /* FQ_ATTENTION_ANY_DIM, default 0: 1 sends head_dim 128 to the general
-                                     attention kernel                                                   */
+    FQ_OPT_ATTENTION_ANY_DIM = 2, /* FQ_ATTENTION_ANY_DIM, default 0: 1 sends every head_dim to the
+                                     general attention kernel                                           */
     FQ_OPT_DECODE_TINY_SPIN = 3,  /* default 0: 1 makes the bounded waits between the wavefronts of the staged
                                      decode kernel give up after two polls, to exercise the failure path
                                      (NaN rows, fault counter) without hanging anything                */
@@ -259,8 +259,8 @@ int fq_tq4_decompress_cache(const uint8_t* kv_cache, const float* centroids, con
  *   out        (B, H_Q, N_Q, D) same dtype as q
  *   is_causal  key j > query i (counted from the top-left corner) is hidden;
  *              ignored when N_Q == 1, as in the reference
- * D in {64, 128, 256}: 128 runs the tuned kernel, 64 and 256 a general one
- * (the switch FQ_OPT_ATTENTION_ANY_DIM sends 128 there too).  H_Q a multiple
+ * D in {64, 128, 256} (the switch FQ_OPT_ATTENTION_ANY_DIM sends them to a
+ * general, slower kernel).  H_Q a multiple
  * of H_KV; 1 <= N_KV <= 2^24.  K and V are dequantised to fp16 with the norm folded in, so a
  * row norm times a centroid must stay below 65504.
  */

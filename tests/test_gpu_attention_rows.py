@@ -129,3 +129,31 @@ def test_split_attention_under_capture():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
+
+
+# (batch, query heads, KV heads, queries, keys, causal): one row, the edges of the 32-row blocks and of the 32-key tiles, fewer
+# and more rows than a workgroup has, an odd number of heads per KV head, contexts in pieces
+WIDE = [(1, 1, 1, 1, 1, False), (1, 4, 1, 31, 31, True), (2, 4, 2, 32, 33, True), (1, 8, 2, 33, 65, False), (1, 3, 1, 97, 97, True),
+        (1, 16, 4, 300, 300, True), (2, 8, 1, 1, 3001, False), (1, 8, 2, 5, 1055, False), (1, 4, 2, 130, 2049, False)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,hq,hkv,nq,nkv,causal", WIDE)
+def test_head_dim_256_rows(b, hq, hkv, nq, nkv, causal, dtype):
+    kv, c, r = _packed(b, hkv, nkv, 256, 71)
+    if nkv > 40:                                       # norms beyond fp16's range in some rows of one tile
+        kv[1][:, :, 35:38] *= 1e-3
+        kv[3][:, :, 36] *= 4000.0
+    q = torch.randn(b, hq, nq, 256, generator=torch.Generator().manual_seed(72)).to(dtype)
+    want = O.fused_tq_attention(q, *kv, c, c, r, is_causal=causal)
+    dev = [t.to(DEV) for t in (q, *kv, c, c, r)]
+    room = K.fused_tq_attention(*dev, is_causal=causal)
+    _close(room, want, dtype)
+    other = K.fused_tq_attention(*dev[:-1], r.t().contiguous().to(DEV).t(), is_causal=causal)      # the matrix in the other layout
+    assert torch.equal(other, room)
+
+
+@pytest.mark.parametrize("hq,hkv", [(8, 2), (5, 1)])
+@pytest.mark.parametrize("batch", range(len(BATCHES)))
+def test_paged_prefill_order_and_split_head_dim_256(batch, hq, hkv):
+    test_paged_prefill_order_and_split(batch, hq, hkv, 256)
