@@ -91,12 +91,17 @@ FQ_HD int first_piece_with(const SeqShape& s, int T, int pieces, int G, bool cau
 
 // What the host allows: workgroups per sequence that may be split and pieces per workgroup.  The first kind of batch
 // leaves more than half of the CUs without work (few prompts, or the chunks of a few): every workgroup may be split as
-// far as a round of workgroups goes, if the tiles saved (2.1 us each) outweigh the combine launch (6 us) and its traffic (132 KB
-// a workgroup and piece, written and read).  Else only sequences of one workgroup (single queries of a mixed batch) are.
+// far as a round of workgroups goes, if the tiles saved (2.1 us each, 5.2 at 256 coordinates) outweigh the combine launch
+// (6 us) and its traffic (132 KB a workgroup and piece, 264 at 256, written and read).  The second kind (`prompts`: sequences
+// of one known length under a causal mask) is about one round of workgroups, the longest with twice the average work: two
+// pieces, if half of the longest workgroup outweighs that traffic and the second prologues too.  (Whether the shares are
+// uneven enough pieces_of decides; more workgroups than 4/3 of a round never are.)  8 heads x 6000 tokens of 256 coordinates,
+// one KV head, 188 workgroups: 538 us in one piece, 416 us in two; 16 heads x 3001 tokens on 4 KV heads 307 and 299 us.  Else only sequences of one workgroup
+// (single queries of a mixed batch) are.
 struct SplitPlan {
     int split_w, max_pieces;
 };
-inline SplitPlan plan_split(int num_seqs, int H_KV, int max_w, int64_t max_tiles, int cus) {
+inline SplitPlan plan_split(int num_seqs, int H_KV, int max_w, int64_t max_tiles, int cus, int D, bool prompts) {
     SplitPlan none{0, 1};
     if (max_tiles < 2 * kSplitMinTiles) return none;
     auto pieces = [&](int64_t items) {
@@ -106,9 +111,13 @@ inline SplitPlan plan_split(int num_seqs, int H_KV, int max_w, int64_t max_tiles
     };
     const int64_t items = int64_t(num_seqs) * H_KV * max_w;
     const int n = pieces(items);
+    const double tile = D == 256 ? 5.2 : 2.1, slot = D == 256 ? 0.132 : 0.066, prologue = D == 256 ? 40.0 : 15.0;
     if (n >= 2) {
-        const double saved = 2.1 * double(max_tiles) * (1.0 - 1.0 / n), cost = 6.0 + 0.066 * double(items) * n;
+        const double saved = tile * double(max_tiles) * (1.0 - 1.0 / n), cost = 6.0 + slot * double(items) * n;
         if (saved > 1.3 * cost) return {max_w, n};
+    } else if (prompts && 3 * items <= 4 * int64_t(cus)) {
+        const double saved = tile * double(max_tiles) / 2, cost = 6.0 + slot * double(items) * 2 + prologue * double(items) / cus;
+        if (saved > 1.3 * cost) return {max_w, 2};
     }
     if (max_w > 1) {
         const int n1 = pieces(int64_t(num_seqs) * H_KV);

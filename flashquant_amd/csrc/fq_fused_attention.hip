@@ -1047,10 +1047,11 @@ inline dim3 folded_grid(int64_t n) {
 inline int64_t workgroups_of(int64_t n_q, int G) { return ((n_q + 31) / 32 * G + 7) / 8; }
 
 // The split that a call of these sizes may use, and the bytes its partial rows take.
-inline SplitPlan plan_of(int num_seqs, int max_q, int64_t max_kv, int H_Q, int H_KV, int D) {
+inline SplitPlan plan_of(int num_seqs, int max_q, int64_t max_kv, int H_Q, int H_KV, int D, bool prompts) {
     const int64_t max_w = workgroups_of(max_q, H_Q / H_KV);
     if (max_w < 1 || max_w > 0x7fffff || fq_host::force_any_dim_attention()) return SplitPlan{0, 1};
-    return plan_split(num_seqs, H_KV, int(max_w), (max_kv + 63) / 64, fq_host::device_cu_count());
+    if (prompts && max_kv > max_q) max_kv = max_q;               // the keys beyond the queries are hidden
+    return plan_split(num_seqs, H_KV, int(max_w), (max_kv + 63) / 64, fq_host::device_cu_count(), D, prompts);
 }
 inline size_t part_bytes(const SplitPlan& sp, int num_seqs, int H_KV, int D) {
     if (sp.max_pieces < 2) return 0;
@@ -1084,10 +1085,11 @@ extern "C" int fq_fused_tq_attention(const void* q, const uint8_t* k_packed, con
                                          is_causal, dtype, stream);
 }
 
-extern "C" size_t fq_attention_workspace_bytes(int num_seqs, int max_q_len, int64_t max_kv_len, int H_Q, int H_KV, int D) {
+extern "C" size_t fq_attention_workspace_bytes(int num_seqs, int max_q_len, int64_t max_kv_len, int H_Q, int H_KV, int D,
+                                               int prompts) {
     using namespace fq;
     if (num_seqs <= 0 || max_q_len <= 0 || max_kv_len <= 0 || H_KV <= 0 || H_Q <= 0 || H_Q % H_KV != 0) return 0;
-    return part_bytes(plan_of(num_seqs, max_q_len, max_kv_len, H_Q, H_KV, D), num_seqs, H_KV, D);
+    return part_bytes(plan_of(num_seqs, max_q_len, max_kv_len, H_Q, H_KV, D, prompts != 0 && max_q_len > 1), num_seqs, H_KV, D);
 }
 
 extern "C" int fq_fused_tq_attention_strided(const void* q, const uint8_t* k_packed, const float* k_norms,
@@ -1163,7 +1165,7 @@ extern "C" int fq_fused_tq_attention_split(const void* q, const uint8_t* k_packe
     p.max_w = int(wgs);
     // A launch that fills the chip keeps the plain order, one that leaves CUs idle is split if the lengths allow (here
     // they are known: a plan under which no workgroup would be split is dropped).
-    SplitPlan sp = plan_of(B, N_Q, N_KV, H_Q, H_KV, D);
+    SplitPlan sp = plan_of(B, N_Q, N_KV, H_Q, H_KV, D, p.causal != 0);
     if (sp.max_pieces > 1) {
         const SeqShape sh = make_seq_shape(N_Q, N_KV, 0, p.G, p.max_w);
         const uint32_t sum = uint32_t(B) * (uint32_t(sh.W) * uint32_t(tiles_of(sh, 0, p.G, p.causal) + tiles_of(sh, sh.W - 1, p.G, p.causal) + 1) / 2);
@@ -1211,7 +1213,7 @@ extern "C" int fq_paged_tq4_prefill_split(const void* q, const int32_t* cu_seqle
     if (num_seqs > 65535 || H_KV > 65535 || (D == 256 && H_Q > 65535)) return FQ_ERR_BAD_SHAPE;
 
     const int64_t wgs = workgroups_of(max_q_len, H_Q / H_KV);
-    const SplitPlan sp = plan_of(num_seqs, max_q_len, int64_t(max_blocks_per_seq) * block_size, H_Q, H_KV, D);
+    const SplitPlan sp = plan_of(num_seqs, max_q_len, int64_t(max_blocks_per_seq) * block_size, H_Q, H_KV, D, false);
     // places per KV head: every sequence of the longest kind, fewer when the tokens of the batch are known (a sequence
     // takes at most (n / 32 + 1) G / 8 + 1 workgroups), and the pieces beyond the first of those that may be split
     int64_t places = num_seqs * wgs;

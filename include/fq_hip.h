@@ -328,9 +328,11 @@ int fq_paged_tq4_prefill(const void* q, const int32_t* cu_seqlens_q, const uint8
  *   workspace        256-byte aligned, at least fq_attention_workspace_bytes bytes (0: these sizes are never split);
  *                    NULL: nothing is split
  *   max_kv_len       the longest context possible: N_KV, or max_blocks_per_seq * block_size
+ *   prompts          1: for fq_fused_tq_attention_split with is_causal (all sequences have these very lengths), else 0
  *   total_q          cu_seqlens_q[num_seqs] where the caller knows it (sizes the grid), else 0
  */
-size_t fq_attention_workspace_bytes(int num_seqs, int max_q_len, int64_t max_kv_len, int H_Q, int H_KV, int D);
+size_t fq_attention_workspace_bytes(int num_seqs, int max_q_len, int64_t max_kv_len, int H_Q, int H_KV, int D,
+                                    int prompts);
 
 int fq_fused_tq_attention_split(const void* q, const uint8_t* k_packed, const float* k_norms,
                                   const uint8_t* v_packed, const float* v_norms,
