@@ -96,7 +96,7 @@ FQ_HD int first_piece_with(const SeqShape& s, int T, int pieces, int G, bool cau
 // of one known length under a causal mask) is about one round of workgroups, the longest with twice the average work: two
 // pieces, if half of the longest workgroup outweighs that traffic and the second prologues too.  (Whether the shares are
 // uneven enough pieces_of decides; more workgroups than 4/3 of a round never are.)  8 heads x 6000 tokens of 256 coordinates,
-// one KV head, 188 workgroups: 538 us in one piece, 416 us in two; 16 heads x 3001 tokens on 4 KV heads 307 and 299 us.  Else only sequences of one workgroup
+// one KV head, 188 workgroups: 538 us in one piece, 347 us in two; 16 heads x 3001 tokens on 4 KV heads 307 and 240 us.  Else only sequences of one workgroup
 // (single queries of a mixed batch) are.
 struct SplitPlan {
     int split_w, max_pieces;

@@ -214,6 +214,155 @@ __device__ __forceinline__ WorkItem find_item(const PrefillParams& p, int place,
     return item;
 }
 
+// The rotation matrix as the A operand of v_mfma_f32_32x32x16_f16, split once per workgroup.
+// Both rotations are transposed products, matrix block x row block: a lane then owns one query row in
+// the operand (its own 16-byte pieces of the query, or its registers of O) and in the result, and no row
+// passes through LDS.  Block (32 result coordinates, 16 contraction coordinates): lane (m32, hf) holds
+// eight contraction coordinates of result coordinate m32, as two fp16 terms.  Wavefront w fetches and
+// splits blocks BPW * w .., every wavefront reads all of them.
+//
+// What it replaced staged the rows through LDS for the 16x16x32 MFMA (16 to 32 lanes on a bank) and stored the
+// results 2 bytes a lane: a workgroup per CU on 64 tokens of 32 heads over 64 keys took 33 us and 27 us with one
+// query row, 24 and 15.5 us this way (the tile itself: 2 us); 4 x 32 heads x 8192 tokens 2.94 -> 2.77 ms.
+template <int D>
+struct RotationBlocks {
+    using Cfg = PrefillCfg<D>;
+    static constexpr int NKS = Cfg::NKS, RBLK = Cfg::RBLK, BPW = RBLK * NKS / 8;
+    const float* rotation;
+    bool col_major;
+    uint8_t* share;               // 2 x RTERM bytes of LDS
+    int w, lane, m32, hf;
+    float rbv[BPW][8];
+    // `back`: x @ R with the contraction index in the order of the accumulator registers (element 4 a + c of half
+    // hf = coordinate 8 a + 4 hf + c of the k-step), else x @ R^T in the natural order
+    __device__ __forceinline__ void fetch(bool back, int round) {
+#pragma unroll
+        for (int i = 0; i < BPW; ++i) {
+            const int blk = BPW * w + i, j = 32 * (RBLK * round + blk / NKS) + m32, k0 = 16 * (blk % NKS);
+            const int k1 = back ? k0 + 4 * hf : k0 + 8 * hf, step = back ? 8 : 4;    // coordinates k1 + 0..3, k1 + step + 0..3
+            if (back == col_major) {                       // a lane's coordinates are neighbours in memory
+                const float4v lo = *reinterpret_cast<const float4v*>(rotation + j * D + k1);
+                const float4v hi = *reinterpret_cast<const float4v*>(rotation + j * D + k1 + step);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { rbv[i][e] = lo[e]; rbv[i][4 + e] = hi[e]; }
+            } else {                                       // the lanes' are
+#pragma unroll
+                for (int e = 0; e < 8; ++e) rbv[i][e] = rotation[(k1 + (e >> 2) * step + (e & 3)) * D + j];
+            }
+        }
+    }
+    __device__ __forceinline__ void put() {
+        half8 rhi[BPW], rlo[BPW];
+        split_rotation_block<32 * BPW>(rbv, rhi, rlo);
+#pragma unroll
+        for (int i = 0; i < BPW; ++i) {
+            *reinterpret_cast<half8*>(share + ((BPW * w + i) * 64 + lane) * 16) = rhi[i];
+            *reinterpret_cast<half8*>(share + Cfg::RTERM + ((BPW * w + i) * 64 + lane) * 16) = rlo[i];
+        }
+    }
+    __device__ __forceinline__ half8 term(int t, int jb, int ks) const {
+        return *reinterpret_cast<const half8*>(share + t * Cfg::RTERM + ((jb * NKS + ks) * 64 + lane) * 16);
+    }
+};
+
+// the power of two that brings a row's largest magnitude (over both lane halves) into [1, 2)
+__device__ __forceinline__ int row_exponent(float mx) {
+    mx = max_xor32(mx);
+    const int ex = int((float_to_bits(mx) >> 23) & 0xffu) - 127;
+    return (ex < -100 || ex > 100) ? 0 : ex;
+}
+__device__ __forceinline__ float pow2(int e) { return bits_to_float(uint32_t(127 + e) << 23); }
+
+// The end of a workgroup: the rows in the accumulators normalised, rotated back (the first round of the matrix already lies
+// in LDS) and stored.
+template <int D, int DT, bool PAGED>
+__device__ __forceinline__ void finish_rows(const PrefillParams& p, RotationBlocks<D>& rot, float16v (&O)[D / 32], float inv,
+                                            bool unit_live, int pos0, int hq, int NQ, int64_t q_row0, int q_stride) {
+    using Cfg = PrefillCfg<D>;
+    constexpr int NKS = Cfg::NKS, NOB = Cfg::NOB, RROUNDS = Cfg::RROUNDS, RBLK = Cfg::RBLK;
+    const int m32 = rot.m32, hf = rot.hf;
+    if (RROUNDS == 1 && !unit_live) return;
+    // float32 rows: both operands as two fp16 terms, three MFMA terms; rows already rounded to 16 bits (the
+    // paged form) are exact in one
+    float mo = 0.0f;
+#pragma unroll
+    for (int ob = 0; ob < NOB; ++ob)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float v = O[ob][r] * inv;
+            O[ob][r] = PAGED ? load_elem<DT>(store_elem<DT>(v)) : v;
+            mo = __builtin_fmaxf(mo, __builtin_fabsf(O[ob][r]));
+        }
+    const int eo = row_exponent(mo);
+    half8 ohi[NKS], olo[NKS];
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+            const float a0 = O[ks >> 1][8 * (ks & 1) + e] * pow2(-eo), a1 = O[ks >> 1][8 * (ks & 1) + e + 1] * pow2(-eo);
+            if (PAGED) {
+                ohi[ks][e] = _Float16(a0); ohi[ks][e + 1] = _Float16(a1);
+            } else {
+                const auto h2 = __builtin_amdgcn_cvt_pkrtz(a0, a1);
+                const auto l2 = __builtin_amdgcn_cvt_pkrtz((a0 - float(h2[0])) * 4096.0f, (a1 - float(h2[1])) * 4096.0f);
+                ohi[ks][e] = h2[0]; ohi[ks][e + 1] = h2[1];
+                olo[ks][e] = l2[0]; olo[ks][e + 1] = l2[1];
+            }
+        }
+    const int opos = pos0 + m32;
+    uint16_t* obase = PAGED ? p.out + (q_row0 + hq) * D : p.out + (q_row0 + int64_t(hq) * NQ) * D;
+    uint16_t* orow = obase + int64_t(opos) * q_stride;
+#pragma unroll
+    for (int cb = 0; cb < NOB; ++cb) {
+        const int cr = cb % RBLK;                      // within the round
+        if (RROUNDS > 1 && cr == 0) {
+            if (cb > 0) {
+                __syncthreads();
+                rot.put();
+                __syncthreads();
+            }
+            if (cb + RBLK < NOB) rot.fetch(true, cb / RBLK + 1);
+        }
+        float16v hi, lo;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { hi[r] = 0.0f; lo[r] = 0.0f; }
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) {
+            const half8 rh = rot.term(0, cr, ks);
+            hi = __builtin_amdgcn_mfma_f32_32x32x16_f16(rh, ohi[ks], hi, 0, 0, 0);
+            lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(rot.term(1, cr, ks), ohi[ks], lo, 0, 0, 0);
+            if (!PAGED) lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(rh, olo[ks], lo, 0, 0, 0);
+        }
+        // registers 4 q + c of half hf = coordinate 32 cb + 8 q + 4 hf + c; the halves exchange a quad of every two,
+        // so that a lane stores eight neighbours at a time
+        uint32_t wd[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float v0 = (hi[2 * i] + lo[2 * i] * (1.0f / 4096.0f)) * pow2(eo);
+            const float v1 = (hi[2 * i + 1] + lo[2 * i + 1] * (1.0f / 4096.0f)) * pow2(eo);
+            wd[i] = uint32_t(store_elem<DT>(v0)) | uint32_t(store_elem<DT>(v1)) << 16;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q += 2) {
+            const auto x = __builtin_amdgcn_permlane32_swap(wd[2 * q], wd[2 * q + 2], false, false);
+            const auto y = __builtin_amdgcn_permlane32_swap(wd[2 * q + 1], wd[2 * q + 3], false, false);
+            const uint4v v = {x[0], y[0], x[1], y[1]};
+            uint16_t* dst = orow + 32 * cb + 8 * q + 8 * hf;
+            if (opos < NQ && unit_live) {
+                if (p.out_wide) {
+                    *reinterpret_cast<uint4v*>(dst) = v;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        dst[2 * e] = uint16_t(v[e] & 0xffffu);
+                        dst[2 * e + 1] = uint16_t(v[e] >> 16);
+                    }
+                }
+            }
+        }
+    }
+}
+
 // PAGED: the sequences' queries are packed along the token axis of q (tokens, H_Q, 128), the keys
 // and values come from the paged TQ4 cache through the block table, query j of a sequence with
 // n queries and L keys sits at position L - n + j (the new tokens are the last ones), and the
@@ -478,56 +627,8 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
 
     issue_loads(first_tile);
 
-    // ---- the rotation matrix as the A operand of v_mfma_f32_32x32x16_f16, split once per workgroup ------
-    // Both rotations are transposed products, matrix block x row block: a lane then owns one query row in
-    // the operand (its own 16-byte pieces of the query, or its registers of O) and in the result, and no row
-    // passes through LDS.  Block (32 result coordinates, 16 contraction coordinates): lane (m32, hf) holds
-    // eight contraction coordinates of result coordinate m32, as two fp16 terms.  Wavefront w fetches and
-    // splits blocks BPW * w .., every wavefront reads all of them.
-    //
-    // What it replaced staged the rows through LDS for the 16x16x32 MFMA (16 to 32 lanes on a bank) and stored the
-    // results 2 bytes a lane: a workgroup per CU on 64 tokens of 32 heads over 64 keys took 33 us and 27 us with one
-    // query row, 24 and 15.5 us this way (the tile itself: 2 us); 4 x 32 heads x 8192 tokens 2.94 -> 2.77 ms.
-    constexpr int RROUNDS = Cfg::RROUNDS, RBLK = Cfg::RBLK, BPW = RBLK * NKS / 8;
-    uint8_t* rshare = reinterpret_cast<uint8_t*>(lut);
-    float rbv[BPW][8];
-    // `back`: x @ R with the contraction index in the order of the accumulator registers (element 4 a + c of half
-    // hf = coordinate 8 a + 4 hf + c of the k-step), else x @ R^T in the natural order
-    auto fetch_rotation = [&](bool back, int round) {
-#pragma unroll
-        for (int i = 0; i < BPW; ++i) {
-            const int blk = BPW * w + i, j = 32 * (RBLK * round + blk / NKS) + m32, k0 = 16 * (blk % NKS);
-            const int k1 = back ? k0 + 4 * hf : k0 + 8 * hf, step = back ? 8 : 4;    // coordinates k1 + 0..3, k1 + step + 0..3
-            if (back == (p.rot_col_major != 0)) {          // a lane's coordinates are neighbours in memory
-                const float4v lo = *reinterpret_cast<const float4v*>(p.rotation + j * D + k1);
-                const float4v hi = *reinterpret_cast<const float4v*>(p.rotation + j * D + k1 + step);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) { rbv[i][e] = lo[e]; rbv[i][4 + e] = hi[e]; }
-            } else {                                       // the lanes' are
-#pragma unroll
-                for (int e = 0; e < 8; ++e) rbv[i][e] = p.rotation[(k1 + (e >> 2) * step + (e & 3)) * D + j];
-            }
-        }
-    };
-    auto share_rotation = [&]() {
-        half8 rhi[BPW], rlo[BPW];
-        split_rotation_block<32 * BPW>(rbv, rhi, rlo);
-#pragma unroll
-        for (int i = 0; i < BPW; ++i) {
-            *reinterpret_cast<half8*>(rshare + ((BPW * w + i) * 64 + lane) * 16) = rhi[i];
-            *reinterpret_cast<half8*>(rshare + Cfg::RTERM + ((BPW * w + i) * 64 + lane) * 16) = rlo[i];
-        }
-    };
-    auto rotation_term = [&](int term, int jb, int ks) {
-        return *reinterpret_cast<const half8*>(rshare + term * Cfg::RTERM + ((jb * NKS + ks) * 64 + lane) * 16);
-    };
-    // the power of two that brings a row's largest magnitude (over both lane halves) into [1, 2)
-    auto row_exponent = [&](float mx) {
-        mx = max_xor32(mx);
-        const int ex = int((float_to_bits(mx) >> 23) & 0xffu) - 127;
-        return (ex < -100 || ex > 100) ? 0 : ex;
-    };
-    auto pow2 = [](int e) { return bits_to_float(uint32_t(127 + e) << 23); };
+    constexpr int RROUNDS = Cfg::RROUNDS, RBLK = Cfg::RBLK;
+    RotationBlocks<D> rot{p.rotation, p.rot_col_major != 0, reinterpret_cast<uint8_t*>(lut), w, lane, m32, hf, {}};
 
     // ---- query: rotate this wavefront's 32 rows, round to the query dtype, scale to fp16 ----------
     half8 qb[NKS];
@@ -539,7 +640,7 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks)
             raw[ks] = *reinterpret_cast<const uint4v*>(qbase + int64_t(pos) * q_stride + 16 * ks + 8 * hf);
-        fetch_rotation(false, 0);
+        rot.fetch(false, 0);
         // the rows are exact in fp16 up to a power of two
         half8 qa[NKS];
         float mx = 0.0f;
@@ -557,15 +658,15 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
                 qa[ks][2 * i] = _Float16(load_elem<DT>(uint16_t(raw[ks][i] & 0xffffu)) * pow2(-ex));
                 qa[ks][2 * i + 1] = _Float16(load_elem<DT>(uint16_t(raw[ks][i] >> 16)) * pow2(-ex));
             }
-        float16v rot[D == 256 ? 1 : NOB];
-        uint32_t rot16[D == 256 ? NOB : 1][8];          // 256 coordinates: held as the 16-bit pairs they are rounded to
+        float16v rows[D == 256 ? 1 : NOB];
+        uint32_t rows16[D == 256 ? NOB : 1][8];          // 256 coordinates: held as the 16-bit pairs they are rounded to
         float mr = 0.0f;
 #pragma unroll
         for (int round = 0; round < RROUNDS; ++round) {
             if (round > 0) __syncthreads();             // every wavefront is done with the round before
-            share_rotation();
+            rot.put();
             __syncthreads();
-            if (round + 1 < RROUNDS) fetch_rotation(false, round + 1);
+            if (round + 1 < RROUNDS) rot.fetch(false, round + 1);
 #pragma unroll
             for (int jr = 0; jr < RBLK; ++jr) {
                 const int jb = RBLK * round + jr;
@@ -574,8 +675,8 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
                 for (int r = 0; r < 16; ++r) { hi[r] = 0.0f; lo[r] = 0.0f; }
 #pragma unroll
                 for (int ks = 0; ks < NKS; ++ks) {
-                    hi = __builtin_amdgcn_mfma_f32_32x32x16_f16(rotation_term(0, jr, ks), qa[ks], hi, 0, 0, 0);
-                    lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(rotation_term(1, jr, ks), qa[ks], lo, 0, 0, 0);
+                    hi = __builtin_amdgcn_mfma_f32_32x32x16_f16(rot.term(0, jr, ks), qa[ks], hi, 0, 0, 0);
+                    lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(rot.term(1, jr, ks), qa[ks], lo, 0, 0, 0);
                 }
                 if constexpr (D == 256) {
 #pragma unroll
@@ -583,13 +684,13 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
                         const uint16_t x = store_elem<DT>((hi[2 * i] + lo[2 * i] * (1.0f / 4096.0f)) * pow2(ex));
                         const uint16_t y = store_elem<DT>((hi[2 * i + 1] + lo[2 * i + 1] * (1.0f / 4096.0f)) * pow2(ex));
                         mr = __builtin_fmaxf(mr, __builtin_fmaxf(__builtin_fabsf(load_elem<DT>(x)), __builtin_fabsf(load_elem<DT>(y))));
-                        rot16[jb][i] = uint32_t(x) | uint32_t(y) << 16;
+                        rows16[jb][i] = uint32_t(x) | uint32_t(y) << 16;
                     }
                 } else {
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
-                        rot[jb][r] = load_elem<DT>(store_elem<DT>((hi[r] + lo[r] * (1.0f / 4096.0f)) * pow2(ex)));
-                        mr = __builtin_fmaxf(mr, __builtin_fabsf(rot[jb][r]));
+                        rows[jb][r] = load_elem<DT>(store_elem<DT>((hi[r] + lo[r] * (1.0f / 4096.0f)) * pow2(ex)));
+                        mr = __builtin_fmaxf(mr, __builtin_fabsf(rows[jb][r]));
                     }
                 }
             }
@@ -602,8 +703,8 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 float v;
-                if constexpr (D == 256) v = load_elem<DT>(uint16_t(rot16[ks >> 1][4 * (ks & 1) + (e >> 1)] >> (16 * (e & 1))));
-                else v = rot[ks >> 1][8 * (ks & 1) + e];
+                if constexpr (D == 256) v = load_elem<DT>(uint16_t(rows16[ks >> 1][4 * (ks & 1) + (e >> 1)] >> (16 * (e & 1))));
+                else v = rows[ks >> 1][8 * (ks & 1) + e];
                 qb[ks][e] = _Float16(v * pow2(-er));
             }
         __syncthreads();   // the rotation operands become lookup tables
@@ -827,90 +928,11 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     // ---- normalise, rotate back, store -------------------------------------------------------------------
     const float l_tot = l_run + xor_shuffle(l_run, 32);
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-    fetch_rotation(true, 0);
+    rot.fetch(true, 0);
     __syncthreads();                // every wavefront is done with the lookup tables
-    share_rotation();
+    rot.put();
     __syncthreads();
-    if (RROUNDS == 1 && !unit_live) return;
-    // float32 rows: both operands as two fp16 terms, three MFMA terms; rows already rounded to 16 bits (the
-    // paged form) are exact in one
-    float mo = 0.0f;
-#pragma unroll
-    for (int ob = 0; ob < NOB; ++ob)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const float v = O[ob][r] * inv;
-            O[ob][r] = PAGED ? load_elem<DT>(store_elem<DT>(v)) : v;
-            mo = __builtin_fmaxf(mo, __builtin_fabsf(O[ob][r]));
-        }
-    const int eo = row_exponent(mo);
-    half8 ohi[NKS], olo[NKS];
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks)
-#pragma unroll
-        for (int e = 0; e < 8; e += 2) {
-            const float a0 = O[ks >> 1][8 * (ks & 1) + e] * pow2(-eo), a1 = O[ks >> 1][8 * (ks & 1) + e + 1] * pow2(-eo);
-            if (PAGED) {
-                ohi[ks][e] = _Float16(a0); ohi[ks][e + 1] = _Float16(a1);
-            } else {
-                const auto h2 = __builtin_amdgcn_cvt_pkrtz(a0, a1);
-                const auto l2 = __builtin_amdgcn_cvt_pkrtz((a0 - float(h2[0])) * 4096.0f, (a1 - float(h2[1])) * 4096.0f);
-                ohi[ks][e] = h2[0]; ohi[ks][e + 1] = h2[1];
-                olo[ks][e] = l2[0]; olo[ks][e + 1] = l2[1];
-            }
-        }
-    const int opos = pos0 + m32;
-    uint16_t* obase = PAGED ? p.out + (q_row0 + hq) * D : p.out + (q_row0 + int64_t(hq) * NQ) * D;
-    uint16_t* orow = obase + int64_t(opos) * q_stride;
-#pragma unroll
-    for (int cb = 0; cb < NOB; ++cb) {
-        const int cr = cb % RBLK;                      // within the round
-        if (RROUNDS > 1 && cr == 0) {
-            if (cb > 0) {
-                __syncthreads();
-                share_rotation();
-                __syncthreads();
-            }
-            if (cb + RBLK < NOB) fetch_rotation(true, cb / RBLK + 1);
-        }
-        float16v hi, lo;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) { hi[r] = 0.0f; lo[r] = 0.0f; }
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) {
-            const half8 rh = rotation_term(0, cr, ks);
-            hi = __builtin_amdgcn_mfma_f32_32x32x16_f16(rh, ohi[ks], hi, 0, 0, 0);
-            lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(rotation_term(1, cr, ks), ohi[ks], lo, 0, 0, 0);
-            if (!PAGED) lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(rh, olo[ks], lo, 0, 0, 0);
-        }
-        // registers 4 q + c of half hf = coordinate 32 cb + 8 q + 4 hf + c; the halves exchange a quad of every two,
-        // so that a lane stores eight neighbours at a time
-        uint32_t wd[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float v0 = (hi[2 * i] + lo[2 * i] * (1.0f / 4096.0f)) * pow2(eo);
-            const float v1 = (hi[2 * i + 1] + lo[2 * i + 1] * (1.0f / 4096.0f)) * pow2(eo);
-            wd[i] = uint32_t(store_elem<DT>(v0)) | uint32_t(store_elem<DT>(v1)) << 16;
-        }
-#pragma unroll
-        for (int q = 0; q < 4; q += 2) {
-            const auto x = __builtin_amdgcn_permlane32_swap(wd[2 * q], wd[2 * q + 2], false, false);
-            const auto y = __builtin_amdgcn_permlane32_swap(wd[2 * q + 1], wd[2 * q + 3], false, false);
-            const uint4v v = {x[0], y[0], x[1], y[1]};
-            uint16_t* dst = orow + 32 * cb + 8 * q + 8 * hf;
-            if (opos < NQ && unit_live) {
-                if (p.out_wide) {
-                    *reinterpret_cast<uint4v*>(dst) = v;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        dst[2 * e] = uint16_t(v[e] & 0xffffu);
-                        dst[2 * e + 1] = uint16_t(v[e] >> 16);
-                    }
-                }
-            }
-        }
-    }
+    finish_rows<D, DT, PAGED>(p, rot, O, inv, unit_live, pos0, hq, NQ, q_row0, q_stride);
 }
 
 // Rows of the workgroups that ran in pieces: the pieces' rows weighted by 2^(m - max m), summed and normalised, rounded
@@ -1007,6 +1029,64 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillPar
     }
 }
 
+// The same for whole prompts in pieces, where the rotation is the work: a workgroup as the one that left the pieces, its
+// wavefronts gather their 32 rows in the accumulators and end as that kernel does (the kernel above fetches and splits the
+// matrix for every 16 rows).  16 heads x 3001 tokens of 256 coordinates, 188 workgroups in two pieces: 298 us with the kernel
+// above, 240 with this one; 8 heads x 5000 tokens of 128, 157 workgroups: 140 and 121; 16 heads x 2000 tokens of 64, 128
+// workgroups: 54.6 and 48.3.  With 63 workgroups in four pieces the smaller workgroups above are faster (128 and 148 us at 256
+// coordinates, 55 and 68 at 128): this one runs from half a round of workgroups on.
+template <int D, int DT, bool PAGED>
+__global__ __launch_bounds__(512) void attention_combine_prompts_kernel(const PrefillParams p) {
+    using Cfg = PrefillCfg<D>;
+    constexpr int NOB = Cfg::NOB;
+    __shared__ __attribute__((aligned(16))) uint8_t share[2 * Cfg::RTERM];
+    const int tid = threadIdx.x, lane = tid & 63, m32 = lane & 31, hf = lane >> 5;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wg = int(blockIdx.x) % p.split_w, pair = int(blockIdx.x) / p.split_w;
+    const int b = pair / p.H_KV, hkv = pair % p.H_KV;
+    const SeqShape sh = seq_shape<PAGED>(p, b);
+    if (sh.W == 0 || sh.W > p.split_w || wg >= sh.W) return;
+    const int pieces = pieces_of(sh, batch_share<PAGED>(p, lane), p.split_w, p.max_pieces, p.G, p.causal != 0);
+    if (pieces < 2) return;
+    RotationBlocks<D> rot{p.rotation, p.rot_col_major != 0, share, w, lane, m32, hf, {}};
+    rot.fetch(true, 0);
+
+    const bool unit_live = 8 * wg + w < sh.units;              // a dead unit left no rows
+    const int unit = unit_live ? 8 * wg + w : sh.units - 1;
+    const int hq = hkv * p.G + unit % p.G, pos0 = 32 * (unit / p.G);
+    float16v O[NOB];
+#pragma unroll
+    for (int ob = 0; ob < NOB; ++ob)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) O[ob][r] = 0.0f;
+    float den = 0.0f;
+    if (unit_live) {
+        const float* src = p.part + int64_t(blockIdx.x) * p.max_pieces * Cfg::SLOT + w * (32 * D + 64);
+        float top = -__builtin_inff();
+        for (int k = 0; k < pieces; ++k) top = __builtin_fmaxf(top, src[int64_t(k) * Cfg::SLOT + 32 * D + m32]);
+        for (int k = 0; k < pieces; ++k) {
+            const float* slot = src + int64_t(k) * Cfg::SLOT;
+            const float m = slot[32 * D + m32], l = slot[32 * D + 32 + m32];
+            const float wk = m == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(m - top);
+            den = __builtin_fmaf(l, wk, den);
+#pragma unroll
+            for (int ob = 0; ob < NOB; ++ob)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float4v v = *reinterpret_cast<const float4v*>(slot + m32 * D + 32 * ob + 8 * q + 4 * hf);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        O[ob][4 * q + c] = wk > 0.0f ? __builtin_fmaf(v[c], wk, O[ob][4 * q + c]) : O[ob][4 * q + c];
+                }
+        }
+    }
+    rot.put();
+    __syncthreads();
+    const int64_t q_row0 = PAGED ? int64_t(p.cu_seqlens_q[b]) * p.H_Q : int64_t(b) * p.H_Q * p.N_Q;
+    finish_rows<D, DT, PAGED>(p, rot, O, den > 0.0f ? 1.0f / den : 0.0f, unit_live, pos0, hq, sh.NQ, q_row0,
+                              PAGED ? p.H_Q * D : D);
+}
+
 template <int D, int DT, bool PAGED, bool SCHED>
 int launch_prefill_as(const PrefillParams& p, dim3 grid, int max_q, hipStream_t s) {
     const size_t lds = 2 * size_t(PrefillCfg<D>::BUF);
@@ -1016,10 +1096,15 @@ int launch_prefill_as(const PrefillParams& p, dim3 grid, int max_q, hipStream_t 
     const int st = fq_host::check_launch();
     if constexpr (SCHED) {
         if (st == FQ_OK && p.max_pieces > 1) {
+            const int64_t slots = int64_t(p.num_seqs) * p.H_KV * p.split_w;
+            if (p.split_w > 1 && 2 * slots >= p.round_slots) {
+                hipLaunchKernelGGL((attention_combine_prompts_kernel<D, DT, PAGED>), dim3(unsigned(slots)), dim3(512), 0, s, p);
+                return fq_host::check_launch();
+            }
             const int rows = max_q <= 4 ? 4 : 16;
             const int groups = max_q <= 16 ? 1 : 2;             // 32 rows a unit at most
             hipLaunchKernelGGL((attention_combine_kernel<D, DT, PAGED>),
-                               dim3(unsigned(int64_t(p.num_seqs) * p.H_KV * p.split_w), 8 * groups), dim3(256), 0, s, p, rows);
+                               dim3(unsigned(slots), 8 * groups), dim3(256), 0, s, p, rows);
             return fq_host::check_launch();
         }
     }

@@ -157,3 +157,28 @@ def test_head_dim_256_rows(b, hq, hkv, nq, nkv, causal, dtype):
 @pytest.mark.parametrize("batch", range(len(BATCHES)))
 def test_paged_prefill_order_and_split_head_dim_256(batch, hq, hkv):
     test_paged_prefill_order_and_split(batch, hq, hkv, 256)
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("b,hq,hkv,nq,nkv,causal", [(4, 16, 8, 390, 2111, False), (1, 8, 1, 4201, 4201, True)])
+def test_prompts_in_pieces(b, hq, hkv, nq, nkv, causal, d):
+    """Enough workgroups of whole prompts in pieces for the combine launch that works like the attention workgroups; the last
+    workgroup of a sequence with fewer than eight units, the last unit with fewer than 32 rows."""
+    kv, c, r = _packed(b, hkv, nkv, d, 81)
+    q = torch.randn(b, hq, nq, d, generator=torch.Generator().manual_seed(82)).to(torch.float16)
+    want = O.fused_tq_attention(q, *kv, c, c, r, is_causal=causal)
+    got = K.fused_tq_attention(q.to(DEV), *[t.to(DEV) for t in kv], c.to(DEV), c.to(DEV), r.to(DEV), is_causal=causal)
+    _close(got, want, torch.float16)
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_paged_prompts_in_pieces(d):
+    ql, kv, hq, hkv, bs = [390, 7, 260, 300], [2100, 1500, 260, 1031], 16, 8, 16
+    c, _, r = book(d)
+    _, cache, table, sl = build_paged_case(kv, hq, hkv, d=d, bs=bs, seed=91, dtype=torch.bfloat16)
+    q = torch.randn(sum(ql), hq, d, generator=torch.Generator().manual_seed(92)).to(torch.bfloat16)
+    cu = torch.tensor([0] + list(torch.tensor(ql).cumsum(0)), dtype=torch.int32)
+    want = O.paged_prefill(q, cu, cache, table, sl, c, c, r, hkv, d, bs, causal=True)
+    got = K.paged_tq4_prefill(q.to(DEV), cu.to(DEV), max(ql), cache.to(DEV), table.to(DEV), sl.to(DEV), c.to(DEV), c.to(DEV),
+                              r.to(DEV), hkv, d, bs)
+    _close(got, want, torch.bfloat16)
