@@ -5,6 +5,7 @@
 // unwraps torch tensors and calls the C ABI of libfq_hip.so on torch's current
 // stream.  There is no CPU path: a tensor that is not on the GPU is an error.
 
+#include <algorithm>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
 
@@ -183,7 +184,8 @@ std::tuple<at::Tensor, at::Tensor> tq4_decompress_cache(const at::Tensor& kv_cac
     require(dtype == at::kHalf || dtype == at::kBFloat16 || (dtype == at::kFloat && !rotation.has_value()),
             "decompress_cache: dtype must be float16 or bfloat16 (or float32 in rotated space)");
     c10::DeviceGuard guard(kv_cache.device());
-    const at::Tensor cache = kv_cache.contiguous();
+    at::Tensor cache = kv_cache.contiguous();
+    if (reinterpret_cast<uintptr_t>(cache.data_ptr()) % 4 != 0) cache = cache.clone();    // the kernels read 4 bytes a lane
     const at::Tensor cc = centroids.to(kv_cache.device()).contiguous();
     const int64_t slots = cache.size(0) * cache.size(1);
     RotationArg rot;
@@ -621,23 +623,25 @@ void prod_store_rows(const at::Tensor& kv_cache, const at::Tensor& slot_mapping,
                      const at::Tensor& k_norms, const at::Tensor& k_gamma, const at::Tensor& v_packed,
                      const at::Tensor& v_norms) {
     fqbind::require_gpu(kv_cache, "kv_cache");
-    require(k_packed.dim() == 3 && k_packed.scalar_type() == at::kByte && k_packed.size(2) % 4 == 0 && k_packed.size(1) > 0,
-            "k_packed must be uint8 of shape (N, H, D/2), D a multiple of 8");
+    require(k_packed.dim() == 3 && k_packed.scalar_type() == at::kByte && k_packed.size(2) > 0 && k_packed.size(1) > 0,
+            "k_packed must be uint8 of shape (N, H, D/2)");
     const int64_t N = k_packed.size(0), H = k_packed.size(1), half = k_packed.size(2), row_bytes = H * (2 * half + 12);
     require(v_packed.scalar_type() == at::kByte && v_packed.numel() == k_packed.numel(), "v_packed must be uint8 with the size of k_packed");
     for (const at::Tensor* t : {&k_norms, &k_gamma, &v_norms})
         require(t->scalar_type() == at::kFloat && t->numel() == N * H, "norms must be float32 with one value per (token, head)");
-    require(kv_cache.scalar_type() == at::kByte && kv_cache.is_contiguous() && kv_cache.numel() % row_bytes == 0,
-            "kv_cache must be a contiguous uint8 tensor of token rows of H * (D + 12) bytes");
+    require(kv_cache.scalar_type() == at::kByte && kv_cache.numel() % row_bytes == 0,
+            "kv_cache must be a uint8 tensor of token rows of H * (D + 12) bytes");
+    const at::Tensor rows = kv_cache.view({kv_cache.numel() / row_bytes, row_bytes});     // the rows may lie apart, not their bytes
+    require(rows.stride(1) == 1 && (rows.size(0) <= 1 || rows.stride(0) >= row_bytes), "the bytes of a row of kv_cache must be contiguous");
     require(slot_mapping.numel() == N, "slot_mapping must hold one slot per token");
     c10::DeviceGuard guard(kv_cache.device());
     const auto dev = kv_cache.device();
     const at::Tensor sm = slot_mapping.to(dev, at::kLong).contiguous();
     const at::Tensor kp = k_packed.to(dev).contiguous(), vp = v_packed.to(dev).contiguous();
     const at::Tensor kn = k_norms.to(dev).contiguous(), kg = k_gamma.to(dev).contiguous(), vn = v_norms.to(dev).contiguous();
-    const int st = fq_prod_store_rows(kv_cache.data_ptr<uint8_t>(), sm.data_ptr<int64_t>(), kp.data_ptr<uint8_t>(),
+    const int st = fq_prod_store_rows(rows.data_ptr<uint8_t>(), std::max(rows.stride(0), row_bytes), sm.data_ptr<int64_t>(), kp.data_ptr<uint8_t>(),
                                       kn.data_ptr<float>(), kg.data_ptr<float>(), vp.data_ptr<uint8_t>(), vn.data_ptr<float>(),
-                                      N, kv_cache.numel() / row_bytes, int(H), int(2 * half), fqbind::current_stream(kv_cache));
+                                      N, rows.size(0), int(H), int(2 * half), fqbind::current_stream(kv_cache));
     fqbind::raise_on_error(st, "prod_store_rows");
 }
 

@@ -94,8 +94,9 @@ __global__ __launch_bounds__(DecRotCfg<D>::THREADS) void tq4_decompress_rotate_k
             float rk[8];
             const int k0 = 16 * ks + 8 * kg;
             if (col_major) {
-                const float4v lo = *reinterpret_cast<const float4v*>(rotation + int64_t(j) * D + k0);
-                const float4v hi = *reinterpret_cast<const float4v*>(rotation + int64_t(j) * D + k0 + 4);
+                typedef float4v float4a __attribute__((aligned(4)));       // the matrix need not be aligned to 16 bytes
+                const float4v lo = *reinterpret_cast<const float4a*>(rotation + int64_t(j) * D + k0);
+                const float4v hi = *reinterpret_cast<const float4a*>(rotation + int64_t(j) * D + k0 + 4);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) { rk[e] = lo[e]; rk[4 + e] = hi[e]; }
             } else {

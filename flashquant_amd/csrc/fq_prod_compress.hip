@@ -140,32 +140,44 @@ __global__ __launch_bounds__(256) void prod_compress_kernel(
 }
 
 // One wavefront per token: its row [K nibbles | K norm | K residual norm | V idx | V norm] assembled from the five
-// operands and written where its slot says, 4 bytes a lane.  Bound by the launch at a decode step's size and by HBM
-// beyond it.  As torch copies into a row buffer and an indexed store it was six launches and twice the bytes: 8 tokens
-// of 8 heads 30 us, one launch 4 us.
+// operands and written where its slot says, 4 bytes a lane (W = uint32_t; single bytes where the cache, its row stride
+// or an operand is not aligned to 4).  Bound by the launch at a decode step's size and by HBM beyond it.  As torch
+// copies into a row buffer and an indexed store it was six launches and twice the bytes: 8 tokens of 8 heads 30 us,
+// one launch 4 us.  `kw`, `nw`: units of one index section and of one section of norms.
+template <typename W>
 __global__ __launch_bounds__(256) void prod_store_rows_kernel(
-    uint32_t* __restrict__ cache, const int64_t* __restrict__ slots, const uint32_t* __restrict__ k_packed,
-    const uint32_t* __restrict__ k_norms, const uint32_t* __restrict__ k_gamma, const uint32_t* __restrict__ v_packed,
-    const uint32_t* __restrict__ v_norms, int64_t tokens, int64_t num_slots, int half_words, int H) {
+    W* __restrict__ cache, const int64_t* __restrict__ slots, const W* __restrict__ k_packed, const W* __restrict__ k_norms,
+    const W* __restrict__ k_gamma, const W* __restrict__ v_packed, const W* __restrict__ v_norms, int64_t tokens,
+    int64_t num_slots, int64_t row_stride, int kw, int nw) {
     const int lane = threadIdx.x & 63;
-    const int kw = H * half_words;                  // dwords of one index section
-    const int row_words = 2 * kw + 3 * H;
+    const int row_units = 2 * kw + 3 * nw;
     for (int64_t t = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6); t < tokens; t += int64_t(gridDim.x) * 4) {
         int64_t slot = slots[t];
         slot = slot < 0 ? slot + num_slots : slot;   // as an indexed store counts from the end
         if (slot < 0 || slot >= num_slots) continue;
-        uint32_t* row = cache + slot * row_words;
-        for (int i = lane; i < row_words; i += 64) {
-            const uint32_t* src;
+        W* row = cache + slot * row_stride;
+        for (int i = lane; i < row_units; i += 64) {
+            const W* src;
             int64_t at;
             if (i < kw) { src = k_packed; at = t * kw + i; }
-            else if (i < kw + H) { src = k_norms; at = t * H + (i - kw); }
-            else if (i < kw + 2 * H) { src = k_gamma; at = t * H + (i - kw - H); }
-            else if (i < 2 * kw + 2 * H) { src = v_packed; at = t * kw + (i - kw - 2 * H); }
-            else { src = v_norms; at = t * H + (i - 2 * kw - 2 * H); }
+            else if (i < kw + nw) { src = k_norms; at = t * nw + (i - kw); }
+            else if (i < kw + 2 * nw) { src = k_gamma; at = t * nw + (i - kw - nw); }
+            else if (i < 2 * kw + 2 * nw) { src = v_packed; at = t * kw + (i - kw - 2 * nw); }
+            else { src = v_norms; at = t * nw + (i - 2 * kw - 2 * nw); }
             row[i] = src[at];
         }
     }
+}
+
+template <typename W>
+int launch_prod_store_rows(uint8_t* cache, const int64_t* slots, const uint8_t* kp, const float* kn, const float* kg,
+                           const uint8_t* vp, const float* vn, int64_t tokens, int64_t num_slots, int64_t row_stride, int H,
+                           int D, unsigned grid, hipStream_t s) {
+    constexpr int B = int(sizeof(W));
+    auto in = [](const void* p) { return static_cast<const W*>(p); };
+    hipLaunchKernelGGL(prod_store_rows_kernel<W>, dim3(grid), dim3(256), 0, s, reinterpret_cast<W*>(cache), slots, in(kp), in(kn),
+                       in(kg), in(vp), in(vn), tokens, num_slots, row_stride / B, H * (D / 2) / B, H * 4 / B);
+    return fq_host::check_launch();
 }
 
 }  // namespace fq
@@ -174,22 +186,25 @@ namespace fq_host {
 int device_cu_count();
 }
 
-extern "C" int fq_prod_store_rows(uint8_t* kv_cache, const int64_t* slot_mapping, const uint8_t* k_packed,
-                                  const float* k_norms, const float* k_residual_norms, const uint8_t* v_packed,
-                                  const float* v_norms, int64_t num_tokens, int64_t num_slots, int H, int D, void* stream) {
+extern "C" int fq_prod_store_rows(uint8_t* kv_cache, int64_t row_stride, const int64_t* slot_mapping,
+                                  const uint8_t* k_packed, const float* k_norms, const float* k_residual_norms,
+                                  const uint8_t* v_packed, const float* v_norms, int64_t num_tokens, int64_t num_slots,
+                                  int H, int D, void* stream) {
     using namespace fq;
-    if (num_tokens < 0 || num_slots < 0 || H <= 0 || H > 65535 || D <= 0 || D % 8 != 0 || D > 4096) return FQ_ERR_BAD_SHAPE;
+    if (num_tokens < 0 || num_slots < 0 || H <= 0 || H > 65535 || D <= 0 || D % 2 != 0 || D > 4096) return FQ_ERR_BAD_SHAPE;
+    if (row_stride < int64_t(H) * (D + 12)) return FQ_ERR_BAD_SHAPE;
     if (num_tokens == 0) return FQ_OK;
     if (!kv_cache || !slot_mapping || !k_packed || !k_norms || !k_residual_norms || !v_packed || !v_norms)
         return FQ_ERR_NULL_POINTER;
-    if (!fq_host::aligned(kv_cache, 4) || !fq_host::aligned(k_packed, 4) || !fq_host::aligned(v_packed, 4)) return FQ_ERR_MISALIGNED;
     const int64_t wgs = (num_tokens + 3) / 4, cap = int64_t(fq_host::device_cu_count()) * 8;
-    hipLaunchKernelGGL(prod_store_rows_kernel, dim3(unsigned(wgs < cap ? wgs : cap)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), reinterpret_cast<uint32_t*>(kv_cache), slot_mapping,
-                       reinterpret_cast<const uint32_t*>(k_packed), reinterpret_cast<const uint32_t*>(k_norms),
-                       reinterpret_cast<const uint32_t*>(k_residual_norms), reinterpret_cast<const uint32_t*>(v_packed),
-                       reinterpret_cast<const uint32_t*>(v_norms), num_tokens, num_slots, D / 8, H);
-    return fq_host::check_launch();
+    const unsigned grid = unsigned(wgs < cap ? wgs : cap);
+    auto launch = [&](auto w) {
+        return launch_prod_store_rows<decltype(w)>(kv_cache, slot_mapping, k_packed, k_norms, k_residual_norms, v_packed, v_norms,
+                                                   num_tokens, num_slots, row_stride, H, D, grid, static_cast<hipStream_t>(stream));
+    };
+    const bool words = (H * (D / 2)) % 4 == 0 && row_stride % 4 == 0 && fq_host::aligned(kv_cache, 4) &&
+                       fq_host::aligned(k_packed, 4) && fq_host::aligned(v_packed, 4);
+    return words ? launch(uint32_t{}) : launch(uint8_t{});
 }
 
 extern "C" int fq_prod_compress(const void* x, int x_dtype, const float* rotation, int rotation_col_major,

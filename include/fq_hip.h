@@ -514,11 +514,12 @@ int fq_prod_compress(const void* x, int x_dtype, const float* rotation, int rota
 /*
  * Writes TurboQuantProd token rows [K nibbles | K norm | K residual norm | V idx | V norm] (H*(D+12) bytes) into the
  * paged cache: token i at flat slot slot_mapping[i] (negative: counted from the end; out of range: not stored).
+ *   row_stride         bytes from one token row of the cache to the next, at least H*(D+12)
  *   k_packed, v_packed (num_tokens, H, D/2) u8; the norms (num_tokens, H) f32
  */
-int fq_prod_store_rows(uint8_t* kv_cache, const int64_t* slot_mapping, const uint8_t* k_packed, const float* k_norms,
-                       const float* k_residual_norms, const uint8_t* v_packed, const float* v_norms, int64_t num_tokens,
-                       int64_t num_slots, int H, int D, void* stream);
+int fq_prod_store_rows(uint8_t* kv_cache, int64_t row_stride, const int64_t* slot_mapping, const uint8_t* k_packed,
+                       const float* k_norms, const float* k_residual_norms, const uint8_t* v_packed, const float* v_norms,
+                       int64_t num_tokens, int64_t num_slots, int H, int D, void* stream);
 
 int fq_prod_paged_decode(const void* q, const uint8_t* kv_cache, const int32_t* block_table,
                          const int32_t* seq_lens, const float* centroids_k3, const float* centroids_v,

@@ -80,3 +80,38 @@ def test_prod_store_rows_writes_the_rows_and_nothing_else(n, h, d):
     dev = [t.to(DEV) for t in (slots, packed[0], norms[0], norms[1], packed[1], norms[2])]
     K.prod_store_rows(got, *dev)
     assert torch.equal(got.cpu().view(-1, row), want)
+
+
+# rows further apart than their bytes, a cache that starts at an odd byte, rows whose sections are no whole words
+@pytest.mark.parametrize("h,d,gap,start", [(8, 128, 32, 0), (8, 128, 3, 0), (8, 128, 0, 1), (1, 66, 0, 0), (3, 10, 5, 2)])
+def test_prod_store_rows_of_any_alignment_and_row_stride(h, d, gap, start):
+    g = torch.Generator().manual_seed(h + d + gap)
+    n, pages, page = 37, 4, 16
+    kn, kg, vi, vn, row = K.prod_page_layout(h, d)
+    buf = torch.randint(0, 256, (start + pages * page * (row + gap),), dtype=torch.uint8, generator=g)
+    slots = torch.randperm(pages * page, generator=g)[:n]
+    packed = [torch.randint(0, 256, (n, h, d // 2), dtype=torch.uint8, generator=g) for _ in range(2)]
+    norms = [torch.rand(n, h, 1, generator=g) for _ in range(3)]
+
+    def cache_of(b):
+        return b[start:].view(pages, page, row + gap)[:, :, :row]
+
+    want = buf.clone()
+    flat = cache_of(want).view(-1, row)
+    flat[slots] = torch.cat([packed[0].view(n, -1), norms[0].view(n, h).view(torch.uint8), norms[1].view(n, h).view(torch.uint8),
+                             packed[1].view(n, -1), norms[2].view(n, h).view(torch.uint8)], dim=1)
+    got = buf.to(DEV)
+    dev = [t.to(DEV) for t in (slots, packed[0], norms[0], norms[1], packed[1], norms[2])]
+    K.prod_store_rows(cache_of(got), *dev)
+    assert torch.equal(got.cpu(), want)
+
+
+def test_decompress_cache_at_an_odd_byte():
+    layer = TQ4AttentionKernels(2, 64, 1.0, torch.device(DEV))
+    cache, _ = random_cache(3, 16, 2, 64, 5)
+    moved = torch.zeros(cache.numel() + 1, dtype=torch.uint8, device=DEV)[1:].view_as(cache)
+    moved.copy_(cache)
+    for rotate in (True, False):
+        for a, b in zip(layer.decompress_cache(moved, torch.bfloat16, apply_rotation=rotate),
+                        layer.decompress_cache(cache, torch.bfloat16, apply_rotation=rotate)):
+            assert torch.equal(a, b)
