@@ -1,6 +1,6 @@
 // Order and split of the workgroups of the fused attention kernel.
 //
-// A workgroup's time is a fixed part (the two rotations, about kSplitMinTiles tiles' worth) plus its key tiles, and
+// A workgroup's time is a fixed part (the two rotations, about eight tiles' worth) plus its key tiles, and
 // under a causal mask or in a batch of prompts, later chunks and single queries the tiles differ by two orders of
 // magnitude.  Nothing on the host knows the lengths, so every workgroup works out from them which piece of the work is
 // its own:
@@ -25,7 +25,11 @@
 
 namespace fq {
 
-constexpr int kSplitMinTiles = 8;        // tiles of 64 keys: a piece shorter than this is mostly prologue
+// The shortest piece, in tiles of 64 keys.  Pieces go to CUs that have nothing else to do, so a piece costs its rows in
+// the combine (2 KB a query head block of few queries) and not its prologue.  One query over a ring buffer of 4 x 2500 tokens,
+// 32 heads over 8: 30.2 us with at least 8 tiles a piece, 28.5 with 6, 26.0 with 5 and 25.9 with 4; 1 x 1300 tokens 34.5, 28.5,
+// 27.1 and 25.8; 8 heads over 1 of 256 coordinates, 1 x 2000 tokens, 2 queries 78.5, 72.0, 67.9 and 58.1.
+constexpr int kSplitMinTiles = 4;
 
 // One sequence as the kernel sees it.
 struct SeqShape {

@@ -55,7 +55,8 @@ def _packed(b, h, n, d, seed):
 
 # (batch, query heads, KV heads, queries, keys): one query, a few, more than one 32-row block, more than one workgroup of
 # queries, more pieces than one chunk of eight, key counts at and around multiples of a tile
-SPLIT = [(4, 32, 8, 1, 2500, 128), (1, 8, 2, 1, 1024, 128), (1, 8, 8, 1, 6001, 64), (2, 8, 1, 5, 4097, 128), (1, 16, 2, 33, 2111, 64),
+SPLIT = [(1, 8, 2, 1, 448, 128), (1, 8, 2, 1, 449, 128), (1, 4, 1, 3, 513, 64), (1, 8, 1, 2, 511, 256),   # the shortest that are split
+         (4, 32, 8, 1, 2500, 128), (1, 8, 2, 1, 1024, 128), (1, 8, 8, 1, 6001, 64), (2, 8, 1, 5, 4097, 128), (1, 16, 2, 33, 2111, 64),
          (1, 5, 1, 130, 4160, 128), (1, 8, 1, 17, 1023, 64), (1, 4, 4, 2, 16384, 128)]
 
 
