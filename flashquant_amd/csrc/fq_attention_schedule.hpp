@@ -95,8 +95,9 @@ FQ_HD int first_piece_with(const SeqShape& s, int T, int pieces, int G, bool cau
 
 // What the host allows: workgroups per sequence that may be split and pieces per workgroup.  The first kind of batch
 // leaves more than half of the CUs without work (few prompts, or the chunks of a few): every workgroup may be split as
-// far as a round of workgroups goes, if the tiles saved (2.1 us each, 5.2 at 256 coordinates) outweigh the combine launch
-// (6 us) and its traffic (132 KB a workgroup and piece, 264 at 256, written and read).  The second kind (`prompts`: sequences
+// far as a round of workgroups goes, if the tiles saved (1.4, 2.1 and 5.2 us each at 64, 128 and 256 coordinates) outweigh the
+// combine launch (6 us, 12 at 256) and its traffic (132 KB a workgroup and piece at 128, written and read): 16 heads over 4 of
+// 64 coordinates, 5 queries over 520 keys 16.6 us in one piece, 19.9 in two; a prompt of 520 tokens at 256 88.1 and 90.5.  The second kind (`prompts`: sequences
 // of one known length under a causal mask) is about one round of workgroups, the longest with twice the average work: two
 // pieces, if half of the longest workgroup outweighs that traffic and the second prologues too.  (Whether the shares are
 // uneven enough pieces_of decides; more workgroups than 4/3 of a round never are.)  8 heads x 6000 tokens of 256 coordinates,
@@ -115,9 +116,9 @@ inline SplitPlan plan_split(int num_seqs, int H_KV, int max_w, int64_t max_tiles
     };
     const int64_t items = int64_t(num_seqs) * H_KV * max_w;
     const int n = pieces(items);
-    const double tile = D == 256 ? 5.2 : 2.1, slot = D == 256 ? 0.132 : 0.066, prologue = D == 256 ? 40.0 : 15.0;
+    const double tile = D == 256 ? 5.2 : (D == 64 ? 1.4 : 2.1), slot = 0.033 * (D / 64), prologue = D == 256 ? 40.0 : 15.0;
     if (n >= 2) {
-        const double saved = tile * double(max_tiles) * (1.0 - 1.0 / n), cost = 6.0 + slot * double(items) * n;
+        const double saved = tile * double(max_tiles) * (1.0 - 1.0 / n), cost = (D == 256 ? 12.0 : 6.0) + slot * double(items) * n;
         if (saved > 1.3 * cost) return {max_w, n};
     } else if (prompts && 3 * items <= 4 * int64_t(cus)) {
         const double saved = tile * double(max_tiles) / 2, cost = 6.0 + slot * double(items) * 2 + prologue * double(items) / cus;
