@@ -937,6 +937,15 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     finish_rows<D, DT, PAGED>(p, rot, O, inv, unit_live, pos0, hq, NQ, q_row0, q_stride);
 }
 
+// The weight 2^(m - top) of a piece's row.  A piece without a visible key has m = -inf, a sum of 0 and rows of zeros; one whose
+// scores are all NaN has m = -inf and a sum of NaN, one with a score of +inf m = +inf: their weights multiply what they left,
+// also a weight of 0, so that a row which is no number in one piece is none in several.
+__device__ __forceinline__ float piece_weight(float m, float l, float top) {
+    return m == -__builtin_inff() && l == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(m - top);
+}
+// (0 only for rows that see no key: a sum that is NaN stays NaN)
+__device__ __forceinline__ float inverse_sum(float den) { return den == 0.0f ? 0.0f : 1.0f / den; }
+
 // Rows of the workgroups that ran in pieces: the pieces' rows weighted by 2^(m - max m), summed and normalised, rounded
 // as the kernel above rounds, rotated back.  A workgroup takes `rows` (4 or 16) rows of a unit, a wavefront a row at a
 // time; blockIdx.x numbers the (sequence, KV head, workgroup) triples that may have been split, blockIdx.y their row
@@ -976,7 +985,7 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillPar
         const float m = have ? head[int64_t(lane) * Cfg::SLOT] : -__builtin_inff();
         const float l = have ? head[int64_t(lane) * Cfg::SLOT + 32] : 0.0f;
         const float top = wave_max(m);
-        const float wgt = m == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(m - top);
+        const float wgt = piece_weight(m, l, top);
         float den = 0.0f, num[CPL];
 #pragma unroll
         for (int e = 0; e < CPL; ++e) num[e] = 0.0f;
@@ -992,13 +1001,15 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillPar
             }
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const float wk = k0 + i < pieces ? of_lane(wgt, k0 + i) : 0.0f;
-                if (k0 + i < pieces) den = __builtin_fmaf(of_lane(l, k0 + i), wk, den);
+                if (k0 + i < pieces) {
+                    const float wk = of_lane(wgt, k0 + i);
+                    den = __builtin_fmaf(of_lane(l, k0 + i), wk, den);
 #pragma unroll
-                for (int e = 0; e < CPL; ++e) num[e] = wk > 0.0f ? __builtin_fmaf(at[i][e], wk, num[e]) : num[e];
+                    for (int e = 0; e < CPL; ++e) num[e] = __builtin_fmaf(at[i][e], wk, num[e]);
+                }
             }
         }
-        const float inv = den > 0.0f ? 1.0f / den : 0.0f;
+        const float inv = inverse_sum(den);
 #pragma unroll
         for (int e = 0; e < CPL; ++e) {
             const float v = num[e] * inv;
@@ -1074,7 +1085,7 @@ __global__ __launch_bounds__(512) void attention_combine_prompts_kernel(const Pr
         for (int k = 0; k < pieces; ++k) {
             const float* slot = src + int64_t(k) * Cfg::SLOT;
             const float m = slot[32 * D + m32], l = slot[32 * D + 32 + m32];
-            const float wk = m == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(m - top);
+            const float wk = piece_weight(m, l, top);
             den = __builtin_fmaf(l, wk, den);
 #pragma unroll
             for (int ob = 0; ob < NOB; ++ob)
@@ -1082,15 +1093,14 @@ __global__ __launch_bounds__(512) void attention_combine_prompts_kernel(const Pr
                 for (int q = 0; q < 4; ++q) {
                     const float4v v = *reinterpret_cast<const float4v*>(slot + m32 * D + 32 * ob + 8 * q + 4 * hf);
 #pragma unroll
-                    for (int c = 0; c < 4; ++c)
-                        O[ob][4 * q + c] = wk > 0.0f ? __builtin_fmaf(v[c], wk, O[ob][4 * q + c]) : O[ob][4 * q + c];
+                    for (int c = 0; c < 4; ++c) O[ob][4 * q + c] = __builtin_fmaf(v[c], wk, O[ob][4 * q + c]);
                 }
         }
     }
     rot.put();
     __syncthreads();
     const int64_t q_row0 = PAGED ? int64_t(p.cu_seqlens_q[b]) * p.H_Q : int64_t(b) * p.H_Q * p.N_Q;
-    finish_rows<D, DT, PAGED>(p, rot, O, den > 0.0f ? 1.0f / den : 0.0f, unit_live, pos0, hq, sh.NQ, q_row0,
+    finish_rows<D, DT, PAGED>(p, rot, O, inverse_sum(den), unit_live, pos0, hq, sh.NQ, q_row0,
                               PAGED ? p.H_Q * D : D);
 }
 

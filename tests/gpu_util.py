@@ -1,9 +1,14 @@
 """Helpers for the GPU parity tests: seeded inputs, oracle-built paged caches."""
 from __future__ import annotations
 
+import ctypes
+import os
+
 import torch
 
 from oracle import tq_oracle as O
+
+LIB = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "flashquant_amd", "libfq_hip.so")
 
 _BOOKS = {}
 
@@ -43,3 +48,60 @@ def build_paged_case(lens, hq, hkv, d=128, bs=16, seed=3, dtype=torch.bfloat16, 
         O.store_rows(cache, slots, kp, kn, vp, vn)
     q = torch.randn(S, hq, d, generator=g).to(dtype)
     return q, cache, table, torch.tensor(lens, dtype=torch.int32)
+
+
+def _entry(name, restype=ctypes.c_int):
+    f = getattr(ctypes.CDLL(LIB), name)
+    f.restype = restype
+    return f
+
+
+def _args(*values):
+    """Tensors as their addresses, ints as 64-bit or 32-bit C integers (None: NULL, (n,): int64)."""
+    out = []
+    for v in values:
+        if v is None:
+            out.append(ctypes.c_void_p(0))
+        elif isinstance(v, torch.Tensor):
+            assert v.is_contiguous()
+            out.append(ctypes.c_void_p(v.data_ptr()))
+        elif isinstance(v, tuple):
+            out.append(ctypes.c_int64(v[0]))
+        elif isinstance(v, float):
+            out.append(ctypes.c_float(v))
+        else:
+            out.append(ctypes.c_int(v))
+    return out
+
+
+def _dtype(t):
+    return {torch.float16: 0, torch.bfloat16: 1}[t.dtype]
+
+
+def _stream():
+    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+
+def attention_workspace_bytes(seqs, max_q, max_kv, hq, hkv, d, prompts=False):
+    """Bytes that the attention wants in order to run contexts in pieces; 0: these sizes never do."""
+    f = _entry("fq_attention_workspace_bytes", ctypes.c_size_t)
+    return int(f(*_args(seqs, max_q, (max_kv,), hq, hkv, d, int(prompts))))
+
+
+def attention_in_one_piece(q, kp, kn, vp, vn, c, r, is_causal=False):
+    """fq_fused_tq_attention: the entry without a workspace, which never runs a context in pieces."""
+    b, hq, nq, d = q.shape
+    out, r = torch.empty_like(q), r.contiguous()
+    st = _entry("fq_fused_tq_attention")(*_args(q, kp, kn, vp, vn, c, c, r, 0, out, b, hq, kp.shape[1], nq, kp.shape[2], d,
+                                                d ** -0.5, int(is_causal), _dtype(q)), _stream())
+    assert st == 0, st
+    return out
+
+
+def prefill_in_one_piece(q, cu, max_q, cache, table, sl, c, r, hkv, d, bs, causal=True):
+    """fq_paged_tq4_prefill: the paged entry without a workspace."""
+    out, r = torch.zeros_like(q), r.contiguous()
+    st = _entry("fq_paged_tq4_prefill")(*_args(q, cu, cache, table, sl, c, c, r, 0, out, table.shape[0], max_q, q.shape[1], hkv,
+                                               d, bs, table.shape[1], (cache.shape[0],), d ** -0.5, int(causal), _dtype(q)), _stream())
+    assert st == 0, st
+    return out

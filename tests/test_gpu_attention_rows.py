@@ -7,7 +7,7 @@ import torch
 
 from flashquant_amd import kernels as K
 from oracle import tq_oracle as O
-from tests.gpu_util import book, build_paged_case
+from tests.gpu_util import attention_in_one_piece, attention_workspace_bytes, book, build_paged_case, prefill_in_one_piece
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -183,3 +183,112 @@ def test_paged_prompts_in_pieces(d):
     got = K.paged_tq4_prefill(q.to(DEV), cu.to(DEV), max(ql), cache.to(DEV), table.to(DEV), sl.to(DEV), c.to(DEV), c.to(DEV),
                               r.to(DEV), hkv, d, bs)
     _close(got, want, torch.bfloat16)
+
+
+# (batch, query heads, KV heads, queries, keys): rows for the combine launch by 4 and by 16 rows, and enough workgroups for
+# the one that works like the attention's workgroups
+IN_PIECES = [(1, 8, 2, 2, 2111), (1, 8, 2, 40, 2111), (4, 16, 8, 390, 2111)]
+# what is wrong with the inputs, and whether every row of the first KV head shows it
+POISON = {"query nan": False, "query inf": False, "key norm nan": True, "key norm inf": True, "all key norms nan": True,
+          "far key norm nan": True, "value norm nan": True, "value norm inf": True}
+
+
+def _poison(kind, kn, vn, row):
+    """NaN and infinities in the norms (tokens, any shape behind: views of the first KV head) or in the query row."""
+    nan, inf = float("nan"), float("inf")
+    if kind == "query nan":
+        row[5] = nan
+    elif kind == "query inf":
+        row[5] = inf
+    elif kind == "key norm nan":
+        kn[1500] = nan
+    elif kind == "key norm inf":
+        kn[700] = inf
+    elif kind == "all key norms nan":
+        kn[:] = nan
+    elif kind == "far key norm nan":            # in a piece whose weights are nothing beside the others'
+        kn[:] *= 40
+        kn[0:250] *= 1e-6
+        kn[3] = nan
+    elif kind == "value norm nan":
+        vn[10] = nan
+    elif kind == "value norm inf":
+        vn[2000] = inf
+
+
+def _check_poisoned(got, one_piece, clean, everywhere, row, heads):
+    """`got` has no number where the run in one piece has none; rows of other KV heads (and other rows than the poisoned
+    query) are the clean ones.  (rows of `heads`, D) tensors."""
+    got, one_piece, clean = (t.float() for t in (got, one_piece, clean))
+    assert torch.equal(got.isfinite(), one_piece.isfinite())
+    bad = ~got.isfinite()
+    if everywhere:
+        assert bad[:heads].all()
+    else:
+        assert bad[0, row].all()
+        bad = bad.clone()
+        bad[0, row] = False
+        assert not bad.any()
+        ok = got.isfinite()
+        assert torch.equal(got[ok], clean[ok])
+    assert torch.equal(got[heads:], clean[heads:])
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("kind", list(POISON))
+@pytest.mark.parametrize("b,hq,hkv,nq,nkv", IN_PIECES)
+def test_nan_and_inf_stay_visible_in_pieces(b, hq, hkv, nq, nkv, kind, d):
+    """A row whose scores, weights or values are no numbers is no number either, in pieces as in one."""
+    assert attention_workspace_bytes(b, nq, nkv, hq, hkv, d) > 0
+    kv, c, r = _packed(b, hkv, nkv, d, 95)
+    q = torch.randn(b, hq, nq, d, generator=torch.Generator().manual_seed(96)).to(torch.bfloat16).to(DEV)
+    kv, c, r = [t.to(DEV) for t in kv], c.to(DEV), r.to(DEV)
+    clean = K.fused_tq_attention(q, *kv, c, c, r)
+    _poison(kind, kv[1][0, 0], kv[3][0, 0], q[0, 0, 1])
+    got = K.fused_tq_attention(q, *kv, c, c, r)
+    want = attention_in_one_piece(q, *kv, c, r)
+    if "far" in kind:
+        clean[0, :hq // hkv] = got[0, :hq // hkv]
+    _check_poisoned(*(t.flatten(0, 1) for t in (got, want, clean)), POISON[kind], 1, hq // hkv)
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("kind", list(POISON))
+@pytest.mark.parametrize("ql,kv,hq,hkv", [([2, 1], [2111, 1800], 8, 2), ([390, 260, 300, 350], [2111, 2100, 2048, 2050], 16, 8)])
+def test_nan_and_inf_stay_visible_in_pieces_paged(ql, kv, hq, hkv, kind, d):
+    bs = 16
+    assert attention_workspace_bytes(len(ql), max(ql), max(kv), hq, hkv, d) > 0
+    c, _, r = book(d)
+    _, cache, table, sl = build_paged_case(kv, hq, hkv, d=d, bs=bs, seed=97, dtype=torch.bfloat16)
+    q = torch.randn(sum(ql), hq, d, generator=torch.Generator().manual_seed(98)).to(torch.bfloat16).to(DEV)
+    cu = torch.tensor([0] + list(torch.tensor(ql).cumsum(0)), dtype=torch.int32).to(DEV)
+    cache, table, sl, c, r = (t.to(DEV) for t in (cache, table, sl, c, r))
+    args = (cu, max(ql), cache, table, sl, c)
+    clean = K.paged_tq4_prefill(q, *args, c, r, hkv, d, bs, causal=False)
+    pos = torch.arange(kv[0])
+    slots = table[0].long().cpu()[pos // bs] * bs + pos % bs
+    norms = cache.view(-1, hkv * (d + 8)).view(torch.float32)
+    kn, vn = norms[slots, hkv * d // 8], norms[slots, hkv * (d + 4) // 4]
+    _poison(kind, kn, vn, q[1, 0])
+    norms[slots, hkv * d // 8], norms[slots, hkv * (d + 4) // 4] = kn, vn
+    got = K.paged_tq4_prefill(q, *args, c, r, hkv, d, bs, causal=False)
+    want = prefill_in_one_piece(q, *args, r, hkv, d, bs, causal=False)
+    first = lambda t: t[:ql[0]].transpose(0, 1)                     # noqa: E731  (heads, rows of the first sequence, D)
+    if "far" in kind:
+        clean[:ql[0], :hq // hkv] = got[:ql[0], :hq // hkv]
+    _check_poisoned(first(got), first(want), first(clean), POISON[kind], 1, hq // hkv)
+    assert torch.equal(got[ql[0]:], clean[ql[0]:])
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_nan_stays_where_it_is_seen_in_causal_prompts(d):
+    """Rows in front of a NaN key see nothing of it, the others are no numbers: in pieces as in one."""
+    n, key = 4201, 2500
+    assert attention_workspace_bytes(1, n, n, 8, 1, d, prompts=True) > 0
+    kv, c, r = _packed(1, 1, n, d, 99)
+    kv[1][..., key, :] = float("nan")
+    q = torch.randn(1, 8, n, d, generator=torch.Generator().manual_seed(100)).to(torch.bfloat16).to(DEV)
+    kv, c, r = [t.to(DEV) for t in kv], c.to(DEV), r.to(DEV)
+    got = K.fused_tq_attention(q, *kv, c, c, r, is_causal=True)
+    assert got[:, :, :key].isfinite().all() and not got[:, :, key:].isfinite().any()
+    assert torch.equal(got.isfinite(), attention_in_one_piece(q, *kv, c, r, is_causal=True).isfinite())
