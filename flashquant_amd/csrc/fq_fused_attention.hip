@@ -1026,9 +1026,27 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillPar
 #pragma unroll
             for (int e = 0; e < 4; ++e) a[j][4 * h + e] = v[e];
         }
+    // two fp16 terms, scaled row by row (the rows of a block may differ by any factor): lanes n16 + 16 g hold row n16
     half8 ahi[NJ], alo[NJ];
-    float up;
-    rows_split_f16<D>(a, ahi, alo, up);
+    float mx = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) mx = __builtin_fmaxf(mx, __builtin_fabsf(a[j][e]));
+    const int ex = row_exponent(max_xor16(mx));
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+            const float a0 = a[j][e] * pow2(-ex), a1 = a[j][e + 1] * pow2(-ex);
+            const auto h2 = __builtin_amdgcn_cvt_pkrtz(a0, a1);
+            const auto l2 = __builtin_amdgcn_cvt_pkrtz((a0 - float(h2[0])) * 4096.0f, (a1 - float(h2[1])) * 4096.0f);
+            ahi[j][e] = h2[0]; ahi[j][e + 1] = h2[1];
+            alo[j][e] = l2[0]; alo[j][e + 1] = l2[1];
+        }
+    float up[4];                       // of the result rows 4 g4 + k
+#pragma unroll
+    for (int k = 0; k < 4; ++k) up[k] = pow2(__shfl(ex, 4 * g4 + k, kWave));
     const int hq = hkv * p.G + unit % p.G;
     uint16_t* out = PAGED ? p.out + (int64_t(p.cu_seqlens_q[b]) * p.H_Q + hq) * D : p.out + (int64_t(b) * p.H_Q + hq) * sh.NQ * D;
     const int stride = PAGED ? p.H_Q * D : D;
@@ -1042,7 +1060,7 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillPar
         for (int k = 0; k < 4; ++k) {
             const int r = 4 * g4 + k;
             if (r < rows && pos0 + r < sh.NQ)
-                out[int64_t(pos0 + r) * stride + 16 * (wave + 4 * i) + n16] = store_elem<DT>(acc[k] * up);
+                out[int64_t(pos0 + r) * stride + 16 * (wave + 4 * i) + n16] = store_elem<DT>(acc[k] * up[k]);
         }
     }
 }

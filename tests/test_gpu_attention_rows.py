@@ -292,3 +292,49 @@ def test_nan_stays_where_it_is_seen_in_causal_prompts(d):
     got = K.fused_tq_attention(q, *kv, c, c, r, is_causal=True)
     assert got[:, :, :key].isfinite().all() and not got[:, :, key:].isfinite().any()
     assert torch.equal(got.isfinite(), attention_in_one_piece(q, *kv, c, r, is_causal=True).isfinite())
+
+
+def _rows_close(got, want, limit, what=""):
+    """The worst row's relative error (2-norms over the last dimension)."""
+    got, want = got.cpu().double().flatten(0, -2), want.cpu().double().flatten(0, -2)
+    rel = (got - want).norm(dim=1) / want.norm(dim=1)
+    assert rel.max() <= limit, f"{what} row {int(rel.argmax())}: relative error {rel.max():.2e}, limit {limit:.2e}"
+
+
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("nq", [3, 12])
+def test_rows_of_very_different_size_in_one_block(nq, d, paged):
+    """Every other row attends to one token whose value is some 2^32 times the others': the rows beside it keep their precision
+    (the combine launch rotates 4 or 16 rows at a time)."""
+    hq, hkv, n, bs, dtype = 4, 1, 2111, 16, torch.bfloat16
+    assert attention_workspace_bytes(1, nq, n, hq, hkv, d) > 0
+    kv, c, r = _packed(1, hkv, n, d, 101)
+    kv[3] *= 0.05
+    kv[3][..., 0, :] = 1e9
+    key = O.decompress(kv[0].reshape(1, n, d // 2), kv[1].reshape(1, n, 1), c)[0, 0] @ r          # the key of that token
+    q = torch.randn(1, hq, nq, d, generator=torch.Generator().manual_seed(102)) * 0.5
+    q += 60 * d ** 0.5 / 11.3 * (key / key.norm()) * torch.tensor([1.0, -1.0]).repeat(nq)[:nq, None]
+    q = q.to(dtype)
+    want = O.fused_tq_attention(q, *kv, c, c, r).float()          # (its rotated query is rounded as the kernel's is)
+    assert want[0, :, 0].norm() > 2e8 * want[0, :, 1].norm()
+    dev = [t.to(DEV) for t in (*kv, c, r)]
+    if paged:
+        pages = (n + bs - 1) // bs
+        cache = torch.zeros(pages, bs, hkv * (d + 8), dtype=torch.uint8)
+        O.store_rows(cache, torch.arange(n), kv[0][0].transpose(0, 1).contiguous(), kv[1][0].transpose(0, 1).contiguous(),
+                     kv[2][0].transpose(0, 1).contiguous(), kv[3][0].transpose(0, 1).contiguous())
+        args = (torch.tensor([0, nq], dtype=torch.int32, device=DEV), nq, cache.to(DEV),
+                torch.arange(pages, dtype=torch.int32, device=DEV)[None], torch.tensor([n], dtype=torch.int32, device=DEV), dev[4])
+        qd = q[0].transpose(0, 1).contiguous().to(DEV)
+        got = K.paged_tq4_prefill(qd, *args, dev[4], dev[5], hkv, d, bs, causal=False).transpose(0, 1)[None]
+        one = prefill_in_one_piece(qd, *args, dev[5], hkv, d, bs, causal=False).transpose(0, 1)[None]
+    else:
+        qd = q.to(DEV)
+        got = K.fused_tq_attention(qd, *dev[:5], dev[4], dev[5])
+        one = attention_in_one_piece(qd, *dev[:4], dev[4], dev[5])
+    # bf16 rounds by up to 2^-9 of a value: the result and the output here, the output there; weights and keys are held in
+    # fp16 (2^-10 of a weight, and a key's 2^-12 moves a score of up to 60 by less than 60 * 2^-12 / sqrt(d) < 2^-9)
+    limit = 3 * 2 ** -9 + 2 ** -10 + 2 ** -9
+    _rows_close(one, want, limit, "in one piece")
+    _rows_close(got, want, limit, "in pieces")
