@@ -282,8 +282,10 @@ __device__ __forceinline__ void finish_rows(const PrefillParams& p, RotationBloc
     constexpr int NKS = Cfg::NKS, NOB = Cfg::NOB, RROUNDS = Cfg::RROUNDS, RBLK = Cfg::RBLK;
     const int m32 = rot.m32, hf = rot.hf;
     if (RROUNDS == 1 && !unit_live) return;
-    // float32 rows: both operands as two fp16 terms, three MFMA terms; rows already rounded to 16 bits (the
-    // paged form) are exact in one
+    // float32 rows: both operands as two fp16 terms, three MFMA terms; rows already rounded to 16 bits (the paged form) in
+    // one, the row's largest value brought into [2^14, 2^15): what is above 2^-28 of it is exact, the rest to 2^-39 of it (a
+    // largest value in [1, 2) left the coordinates below 2^-14 of it among fp16's subnormals)
+    constexpr int kUp = PAGED ? 14 : 0;
     float mo = 0.0f;
 #pragma unroll
     for (int ob = 0; ob < NOB; ++ob)
@@ -299,7 +301,7 @@ __device__ __forceinline__ void finish_rows(const PrefillParams& p, RotationBloc
     for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
         for (int e = 0; e < 8; e += 2) {
-            const float a0 = O[ks >> 1][8 * (ks & 1) + e] * pow2(-eo), a1 = O[ks >> 1][8 * (ks & 1) + e + 1] * pow2(-eo);
+            const float a0 = O[ks >> 1][8 * (ks & 1) + e] * pow2(kUp - eo), a1 = O[ks >> 1][8 * (ks & 1) + e + 1] * pow2(kUp - eo);
             if (PAGED) {
                 ohi[ks][e] = _Float16(a0); ohi[ks][e + 1] = _Float16(a1);
             } else {
@@ -338,8 +340,8 @@ __device__ __forceinline__ void finish_rows(const PrefillParams& p, RotationBloc
         uint32_t wd[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const float v0 = (hi[2 * i] + lo[2 * i] * (1.0f / 4096.0f)) * pow2(eo);
-            const float v1 = (hi[2 * i + 1] + lo[2 * i + 1] * (1.0f / 4096.0f)) * pow2(eo);
+            const float v0 = (hi[2 * i] + lo[2 * i] * (1.0f / 4096.0f)) * pow2(eo - kUp);
+            const float v1 = (hi[2 * i + 1] + lo[2 * i + 1] * (1.0f / 4096.0f)) * pow2(eo - kUp);
             wd[i] = uint32_t(store_elem<DT>(v0)) | uint32_t(store_elem<DT>(v1)) << 16;
         }
 #pragma unroll
@@ -1026,23 +1028,29 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillPar
 #pragma unroll
             for (int e = 0; e < 4; ++e) a[j][4 * h + e] = v[e];
         }
-    // two fp16 terms, scaled row by row (the rows of a block may differ by any factor): lanes n16 + 16 g hold row n16
+    // fp16 terms as in finish_rows, scaled row by row (the rows of a block may differ by any factor): lanes n16 + 16 g hold
+    // row n16
+    constexpr int kUp = PAGED ? 14 : 0;
     half8 ahi[NJ], alo[NJ];
     float mx = 0.0f;
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
         for (int e = 0; e < 8; ++e) mx = __builtin_fmaxf(mx, __builtin_fabsf(a[j][e]));
-    const int ex = row_exponent(max_xor16(mx));
+    const int ex = row_exponent(max_xor16(mx)) - kUp;
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
         for (int e = 0; e < 8; e += 2) {
             const float a0 = a[j][e] * pow2(-ex), a1 = a[j][e + 1] * pow2(-ex);
-            const auto h2 = __builtin_amdgcn_cvt_pkrtz(a0, a1);
-            const auto l2 = __builtin_amdgcn_cvt_pkrtz((a0 - float(h2[0])) * 4096.0f, (a1 - float(h2[1])) * 4096.0f);
-            ahi[j][e] = h2[0]; ahi[j][e + 1] = h2[1];
-            alo[j][e] = l2[0]; alo[j][e + 1] = l2[1];
+            if (PAGED) {
+                ahi[j][e] = _Float16(a0); ahi[j][e + 1] = _Float16(a1);
+            } else {
+                const auto h2 = __builtin_amdgcn_cvt_pkrtz(a0, a1);
+                const auto l2 = __builtin_amdgcn_cvt_pkrtz((a0 - float(h2[0])) * 4096.0f, (a1 - float(h2[1])) * 4096.0f);
+                ahi[j][e] = h2[0]; ahi[j][e + 1] = h2[1];
+                alo[j][e] = l2[0]; alo[j][e + 1] = l2[1];
+            }
         }
     float up[4];                       // of the result rows 4 g4 + k
 #pragma unroll

@@ -338,3 +338,33 @@ def test_rows_of_very_different_size_in_one_block(nq, d, paged):
     limit = 3 * 2 ** -9 + 2 ** -10 + 2 ** -9
     _rows_close(one, want, limit, "in one piece")
     _rows_close(got, want, limit, "in pieces")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("nq,n", [(2, 1), (2, 2111), (40, 2111), (400, 4100)])
+def test_coordinates_of_very_different_size_in_one_row(nq, n, d, dtype):
+    """Paged rows are rounded to the query dtype and rotated back: with the identity as the matrix every coordinate comes
+    out as it was rounded, also one 2^-20 of the row's largest."""
+    hq, hkv, bs = 4, 1, 16
+    if nq == 400:
+        hq, hkv = 32, 8                                     # the combine launch by workgroups
+    g = torch.Generator().manual_seed(103)
+    c = torch.cat([-2.0 ** -10 * (1 + torch.rand(8, generator=g)), 2.0 ** 10 * (1 + torch.rand(8, generator=g))])
+    token = torch.randint(0, 256, (hkv, d // 2), dtype=torch.uint8, generator=g)
+    pages = (n + bs - 1) // bs
+    cache = torch.zeros(pages, bs, hkv * (d + 8), dtype=torch.uint8)
+    same = token[None].expand(n, hkv, d // 2).contiguous()
+    ones = torch.ones(n, hkv, 1)
+    O.store_rows(cache, torch.arange(n), same, ones, same, ones)
+    q = (torch.randn(nq, hq, d, generator=g) * 1e-3).to(dtype).to(DEV)
+    eye = torch.eye(d, device=DEV)
+    got = K.paged_tq4_prefill(q, torch.tensor([0, nq], dtype=torch.int32, device=DEV), nq, cache.to(DEV),
+                              torch.arange(pages, dtype=torch.int32, device=DEV)[None],
+                              torch.tensor([n], dtype=torch.int32, device=DEV), c.to(DEV), c.to(DEV), eye, hkv, d, bs,
+                              causal=False).cpu().double()
+    value = c[O.nibble_unpack(token).long()].double().repeat_interleave(hq // hkv, 0)      # (heads, D)
+    # held as fp16 (2^-11), the weights' sum as theirs (2^-11), rounded to the query dtype once: nothing more for one key
+    limit = 2 * 2 ** -11 + (2 ** -8 if dtype == torch.bfloat16 else 2 ** -11)
+    err = ((got - value) / value).abs().max()
+    assert err <= limit, f"{err:.2e}, limit {limit:.2e}"
