@@ -5,7 +5,7 @@
 // magnitude.  Nothing on the host knows the lengths, so every workgroup works out from them which piece of the work is
 // its own:
 //   * work is handed out longest first (the workgroups of a KV-head group in the order of their linear index), so that
-//     the short ones fill the end of the launch;
+//     the short ones fill the end of the launch (up to kOrderSeqs sequences);
 //   * where a sequence's keys are long for its few queries (`split_w`, `max_pieces`, set by the host from what it
 //     knows), they are cut into pieces of about the share of a CU; the pieces leave partial results, combined by a
 //     launch of their own.
@@ -30,6 +30,15 @@ namespace fq {
 // 32 heads over 8: 30.2 us with at least 8 tiles a piece, 28.5 with 6, 26.0 with 5 and 25.9 with 4; 1 x 1300 tokens 34.5, 28.5,
 // 27.1 and 25.8; 8 heads over 1 of 256 coordinates, 1 x 2000 tokens, 2 queries 78.5, 72.0, 67.9 and 58.1.
 constexpr int kSplitMinTiles = 4;
+
+// Batches of more sequences than this are not ordered.  Every workgroup finds its own item, and the search for the longest
+// ones reads all lengths some fifteen times: 1 us up to 64 sequences, 40 us at 1024 (a workgroup's own time is 40 to 60).
+// Beyond it a workgroup counts through the sequences once, or, where the grid has at most two places for every workgroup that
+// the batch can need, its place says which sequence it is.  32 query heads over 8 of 128, bf16, in us (grid order of all
+// sequences / ordered / not ordered): 256 sequences, sixteen of them prompts of up to 512 tokens, 1910 / 568 / 547, at one KV
+// head 175 / 98 / 122, 16 heads over 4 of 256 11,400 / 952 / 1014; 384 sequences 2804 / 904 / 751; 1024 single queries
+// 2060 / 2849 / 1630, 4096 8080 / 32,700 / 6400; 2048 prompts of 30 to 300 tokens 7409 / 16,800 / 4823.
+constexpr int kOrderSeqs = 256;
 
 // One sequence as the kernel sees it.
 struct SeqShape {

@@ -92,6 +92,7 @@ struct PrefillParams {
     int round_slots;               // workgroups running at a time (one per CU)
     // order and split of the work (fq_attention_schedule.hpp); workgroups in split pieces leave their rows in `part`
     int num_seqs, max_w, split_w, max_pieces;
+    bool dense;                 // beyond kOrderSeqs sequences: max_w places for each of them
     float* part;                   // slot of a workgroup's piece: PrefillCfg<D>::SLOT floats
     bool out_wide;                 // `out` is 16-byte aligned (its rows are multiples of 128 bytes apart)
 };
@@ -158,11 +159,16 @@ struct WorkItem {
 };
 
 // The item of place `place` (of one KV head) in the order longest piece first: the largest tile count T that more than
-// `place` pieces reach, by bisection with a lane per sequence; then the place among the pieces of exactly T.
+// `place` pieces reach, by bisection with a lane per sequence; then the place among the pieces of exactly T.  Beyond
+// kOrderSeqs sequences the items in the order of the sequences (kOrderSeqs says why).
 template <bool PAGED>
 __device__ __forceinline__ WorkItem find_item(const PrefillParams& p, int place, int lane) {
     const int G = p.G;
     const bool causal = p.causal != 0;
+    if (p.dense) {
+        const int seq = place / p.max_w, x = p.max_w - 1 - place % p.max_w;
+        return seq < p.num_seqs && x < seq_shape<PAGED>(p, seq).W ? WorkItem{seq, x, 0, 1} : WorkItem{-1, 0, 0, 1};
+    }
     const int share = p.max_pieces > 1 ? batch_share<PAGED>(p, lane) : 1;
     const SeqShape none = make_seq_shape(0, 0, 0, G, 0);
     const SeqShape first = lane < p.num_seqs ? seq_shape<PAGED>(p, lane) : none;
@@ -180,15 +186,18 @@ __device__ __forceinline__ WorkItem find_item(const PrefillParams& p, int place,
         return int(wave_add(c));
     };
     WorkItem item{-1, 0, 0, 1};
-    if (place >= count(0)) return item;
-    int lo = 0, hi = 1;               // count(lo) > place >= count(hi)
-    while (count(hi) > place) { lo = hi; hi *= 2; }      // (no sequence has 2^30 tiles: ends)
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (count(mid) > place) lo = mid;
-        else hi = mid;
+    int lo = 0, hi = 0x3fffffff, rem = place;            // tile counts lo .. hi - 1 (no sequence has 2^30 tiles)
+    if (p.num_seqs <= kOrderSeqs) {
+        if (place >= count(0)) return item;
+        hi = 1;                                          // count(lo) > place >= count(hi)
+        while (count(hi) > place) { lo = hi; hi *= 2; }
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (count(mid) > place) lo = mid;
+            else hi = mid;
+        }
+        rem = place - count(hi);
     }
-    int rem = place - count(hi);
     for (int s0 = 0; s0 < p.num_seqs; s0 += kWave) {
         const SeqShape sh = shape(s0);
         const int n = pieces(sh), x0 = first_piece_with(sh, lo, n, G, causal);
@@ -1291,6 +1300,7 @@ extern "C" int fq_fused_tq_attention_split(const void* q, const uint8_t* k_packe
     p.out_wide = fq_host::aligned(out, 16);
     p.num_seqs = B;
     p.max_w = int(wgs);
+    p.dense = false;
     // A launch that fills the chip keeps the plain order, one that leaves CUs idle is split if the lengths allow (here
     // they are known: a plan under which no workgroup would be split is dropped).
     SplitPlan sp = plan_of(B, N_Q, N_KV, H_Q, H_KV, D, p.causal != 0);
@@ -1349,6 +1359,9 @@ extern "C" int fq_paged_tq4_prefill_split(const void* q, const int32_t* cu_seqle
         const int64_t most = (total_q / 32 + num_seqs) * (H_Q / H_KV) / 8 + num_seqs;
         places = most < places ? most : places;
     }
+    // (kOrderSeqs) beyond so many sequences, and where at least half of the places of all sequences are needed, no search
+    const bool dense = num_seqs > kOrderSeqs && sp.max_pieces < 2 && 2 * places >= num_seqs * wgs;
+    if (dense) places = num_seqs * wgs;
     const bool fits = wgs <= 0x7fffffffLL && (places + int64_t(num_seqs) * sp.split_w * (sp.max_pieces - 1)) * H_KV <= 0x7fffffffLL;
     // (the general kernel's grid has no such bound: head_dim 256 runs there beyond it)
     if (fq_host::force_any_dim_attention() || (D == 256 && !fits)) {
@@ -1387,6 +1400,7 @@ extern "C" int fq_paged_tq4_prefill_split(const void* q, const int32_t* cu_seqle
     p.max_w = int(wgs);
     const int st = use_plan(p, sp, D, workspace, workspace_bytes);
     if (st != FQ_OK) return st;
+    p.dense = dense;
     places += int64_t(num_seqs) * p.split_w * (p.max_pieces - 1);
     return launch_prefill<true, true>(p, D, folded_grid(places * H_KV), max_q_len, dtype, static_cast<hipStream_t>(stream));
 }

@@ -368,3 +368,27 @@ def test_coordinates_of_very_different_size_in_one_row(nq, n, d, dtype):
     limit = 2 * 2 ** -11 + (2 ** -8 if dtype == torch.bfloat16 else 2 ** -11)
     err = ((got - value) / value).abs().max()
     assert err <= limit, f"{err:.2e}, limit {limit:.2e}"
+
+
+# more sequences than are ordered: single queries (the grid has a place for every sequence), the same with one long prompt
+# (most places of such a grid would be empty: the sequences are counted), short prompts of one and two workgroups
+MANY = {"single": [1] * 300, "one prompt": [1] * 150 + [700] + [1] * 139 + [0, 40] * 5, "prompts": [(s * 37) % 90 for s in range(330)]}
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("many", list(MANY))
+def test_paged_prefill_of_many_sequences(many, d):
+    """Every row of every sequence is written once; the entry that does not know the number of tokens hands out the same."""
+    ql, hq, hkv, bs, dtype = MANY[many], 8, 2, 16, torch.bfloat16
+    kv = [n + (s * 29) % 50 if s % 7 else n for s, n in enumerate(ql)]
+    c, _, r = book(d)
+    _, cache, table, sl = build_paged_case(kv, hq, hkv, d=d, bs=bs, seed=111, dtype=dtype)
+    q = torch.randn(sum(ql), hq, d, generator=torch.Generator().manual_seed(112)).to(dtype)
+    cu = torch.tensor([0] + list(torch.tensor(ql).cumsum(0)), dtype=torch.int32)
+    want = O.paged_prefill(q, cu, cache, table, sl, c, c, r, hkv, d, bs)
+    args = (q.to(DEV), cu.to(DEV), max(ql), cache.to(DEV), table.to(DEV), sl.to(DEV), c.to(DEV))
+    got = torch.full_like(q, 7.0).to(DEV)
+    K.paged_tq4_prefill(*args, c.to(DEV), r.to(DEV), hkv, d, bs, out=got)
+    # three roundings to bf16 and fp16 keys, a worst row of some thousands: as in _close with the row's own norm
+    _rows_close(got, want, 4 * 2 ** -8)
+    assert torch.equal(prefill_in_one_piece(*args, r.to(DEV), hkv, d, bs), got)
