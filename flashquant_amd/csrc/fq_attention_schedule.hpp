@@ -82,17 +82,48 @@ FQ_HD int first_with(const SeqShape& s, int T, int G, bool causal) {
     return x < s.W ? int(x) : s.W;
 }
 
-// Pieces that every workgroup's keys of this sequence are cut into.
-FQ_HD int pieces_of(const SeqShape& s, int share, int split_w, int max_pieces, int G, bool causal) {
-    if (max_pieces < 2 || s.W == 0 || s.W > split_w) return 1;
-    const int n = (tiles_of(s, s.W - 1, G, causal) + share / 2) / share;
-    return n < 1 ? 1 : (n > max_pieces ? max_pieces : n);
+// What splitting saves and costs, in ns: a tile of 64 keys of the longest workgroup; what a sequence's rows cost in the combine
+// however few they are; a piece of 256 rows, written and read.  Fitted on 1775 paged batches of equal sequences (1, 3 and 8
+// of them, 1 to 1000 queries over 400 to 4000 keys, four head counts), each run in pieces and in one: with 33 queries and more
+// the combine took 3 and 5 us up to 16 workgroups' worth of pieces and 8 and 17 us at 128 (64 and 128 coordinates).  At 256
+// pieces won in nearly all of them: the rotation back of a few workgroups is what the combine spreads over the chip.
+struct SplitCost {
+    int tile, fixed, slot;
+};
+FQ_HD SplitCost split_cost(int D) {
+    return D == 64 ? SplitCost{1400, 3000, 45} : (D == 128 ? SplitCost{2100, 5000, 80} : SplitCost{5200, 0, 0});
 }
 
-// Tiles of the share that one of `slots` CUs would have of the whole batch.
+// What the pieces of a batch follow from: the tiles of a CU's share of all work, and the rows that may have to be combined,
+// in workgroups' worth of 256.
+struct BatchWork {
+    int share, slots;
+};
+
+// Pieces that every workgroup's keys of this sequence are cut into.  The plan allows them by the longest context possible, of
+// which the sequence may have little: with more than 16 queries (those of fewer always gained) pieces have to save more
+// than they cost.  Without this a paged batch with a table of 4096 tokens lost: 3 prompts of 400 tokens, 16 heads over 4
+// of 128, 41 us in one piece and 57 in two; 8 of 400 on one KV head of 64 25 and 36.
+FQ_HD int pieces_of(const SeqShape& s, const BatchWork& b, int split_w, int max_pieces, int G, bool causal, int D) {
+    if (max_pieces < 2 || s.W == 0 || s.W > split_w) return 1;
+    const int tiles = tiles_of(s, s.W - 1, G, causal);
+    int n = (tiles + b.share / 2) / b.share;
+    n = n < max_pieces ? n : max_pieces;
+    if (n < 2) return 1;
+    const SplitCost c = split_cost(D);
+    if (s.NQ > 16 && int64_t(c.tile) * tiles * (n - 1) <= int64_t(n) * (c.fixed + int64_t(c.slot) * b.slots * n)) return 1;
+    return n;
+}
+
+// The share of one of `slots` CUs: `tile_sum` tiles of all workgroups.
 FQ_HD int share_of(uint32_t tile_sum, int slots) {
     const int s = int((tile_sum + uint32_t(slots) - 1) / uint32_t(slots));
     return s > kSplitMinTiles ? s : kSplitMinTiles;
+}
+
+// Whether any batch around this sequence could make it run in pieces.
+FQ_HD bool may_split(const SeqShape& s, int split_w, int max_pieces, int G, bool causal, int D) {
+    return pieces_of(s, BatchWork{kSplitMinTiles, 0}, split_w, max_pieces, G, causal, D) > 1;
 }
 
 // Workgroups x of the sequence whose pieces have at least T tiles: x >= this.
@@ -125,7 +156,7 @@ inline SplitPlan plan_split(int num_seqs, int H_KV, int max_w, int64_t max_tiles
     };
     const int64_t items = int64_t(num_seqs) * H_KV * max_w;
     const int n = pieces(items);
-    const double tile = D == 256 ? 5.2 : (D == 64 ? 1.4 : 2.1), slot = 0.033 * (D / 64), prologue = D == 256 ? 40.0 : 15.0;
+    const double tile = split_cost(D).tile * 1e-3, slot = 0.033 * (D / 64), prologue = D == 256 ? 40.0 : 15.0;
     if (n >= 2) {
         const double saved = tile * double(max_tiles) * (1.0 - 1.0 / n), cost = (D == 256 ? 12.0 : 6.0) + slot * double(items) * n;
         if (saved > 1.3 * cost) return {max_w, n};

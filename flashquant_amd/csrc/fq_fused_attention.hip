@@ -94,6 +94,7 @@ struct PrefillParams {
     int num_seqs, max_w, split_w, max_pieces;
     bool dense;                 // beyond kOrderSeqs sequences: max_w places for each of them
     float* part;                   // slot of a workgroup's piece: PrefillCfg<D>::SLOT floats
+    int* left;                     // paged: pieces in `part` of every workgroup that may be split, 0 if none
     bool out_wide;                 // `out` is 16-byte aligned (its rows are multiples of 128 bytes apart)
 };
 
@@ -139,55 +140,84 @@ __device__ __forceinline__ uint32_t wave_add(uint32_t v) {
     return uint32_t(__builtin_amdgcn_readfirstlane(int(c[0] + c[1])));
 }
 
-// The share of a CU of the whole batch (all KV heads), in tiles.  The sum may wrap on batches beyond any memory: the
-// share is then merely a poor one, and still the same everywhere.
+// The sequences s0 + lane as the lanes of a wavefront hold them; empty ones past the end.
 template <bool PAGED>
-__device__ __forceinline__ int batch_share(const PrefillParams& p, int lane) {
-    uint32_t sum = 0;
+__device__ __forceinline__ SeqShape lane_shape(const PrefillParams& p, int s0, int lane) {
+    return s0 + lane < p.num_seqs ? seq_shape<PAGED>(p, s0 + lane) : make_seq_shape(0, 0, 0, p.G, 0);
+}
+
+// The share of a CU of the whole batch (all KV heads), in tiles, and the rows of the sequences that may be split.  The sums
+// may wrap on batches beyond any memory: the pieces are then merely poor ones, and still the same everywhere.  `first`: the
+// first wavefront's worth of sequences.
+template <bool PAGED>
+__device__ __forceinline__ BatchWork batch_work(const PrefillParams& p, const SeqShape& first, int lane) {
+    uint32_t tiles = 0, rows = 0;
     for (int s0 = 0; s0 < p.num_seqs; s0 += kWave) {
-        if (s0 + lane < p.num_seqs) {
-            const SeqShape sh = seq_shape<PAGED>(p, s0 + lane);
-            if (sh.W > 0)
-                sum += uint32_t(sh.W) * uint32_t(tiles_of(sh, 0, p.G, p.causal) + tiles_of(sh, sh.W - 1, p.G, p.causal) + 1) / 2;
-        }
+        const SeqShape sh = s0 == 0 ? first : lane_shape<PAGED>(p, s0, lane);
+        if (sh.W > 0)
+            tiles += uint32_t(sh.W) * uint32_t(tiles_of(sh, 0, p.G, p.causal) + tiles_of(sh, sh.W - 1, p.G, p.causal) + 1) / 2;
+        if (sh.W <= p.split_w) rows += uint32_t(sh.NQ) * uint32_t(p.G);
     }
-    return share_of(wave_add(sum) * uint32_t(p.H_KV), p.round_slots);
+    return {share_of(wave_add(tiles) * uint32_t(p.H_KV), p.round_slots), int(wave_add(rows) * uint32_t(p.H_KV) >> 8)};
+}
+
+// Pieces of a sequence's workgroups.  Sequences of one length: the host has worked them out.
+template <int D, bool PAGED>
+__device__ __forceinline__ int pieces_in(const PrefillParams& p, const SeqShape& sh, const BatchWork& batch) {
+    if (!PAGED) return p.max_pieces;
+    return pieces_of(sh, batch, p.split_w, p.max_pieces, p.G, p.causal != 0, D);
 }
 
 struct WorkItem {
     int seq, x, piece, pieces;      // seq < 0: none
 };
 
-// The item of place `place` (of one KV head) in the order longest piece first: the largest tile count T that more than
+// What the combine needs to know of its workgroup `at`, so that one without work costs a load (adding up the lengths there
+// took 5 us a launch).  The grid has more workgroups than there are such entries.
+template <int D>
+__device__ __forceinline__ void note_pieces(const PrefillParams& p, const SeqShape& first, const BatchWork& batch, int at, int lane) {
+    if (at >= p.num_seqs * p.H_KV * p.split_w) return;
+    const int x = at % p.split_w, b = at / p.split_w / p.H_KV;
+    auto of_lane = [&](int v) { return __builtin_amdgcn_readlane(v, b); };
+    const SeqShape sh = b < kWave ? make_seq_shape(of_lane(first.NQ), of_lane(first.NKV), of_lane(first.qoff), p.G, p.max_w)
+                                  : seq_shape<true>(p, b);
+    const int n = x < sh.W && sh.W <= p.split_w ? pieces_in<D, true>(p, sh, batch) : 0;
+    if (threadIdx.x == 0) p.left[at] = n > 1 ? n : 0;
+}
+
+// The item of a place (`at` / H_KV, of one KV head) in the order longest piece first: the largest tile count T that more than
 // `place` pieces reach, by bisection with a lane per sequence; then the place among the pieces of exactly T.  Beyond
 // kOrderSeqs sequences the items in the order of the sequences (kOrderSeqs says why).
-template <bool PAGED>
-__device__ __forceinline__ WorkItem find_item(const PrefillParams& p, int place, int lane) {
-    const int G = p.G;
+// `at` is the workgroup's number in the launch.
+template <int D, bool PAGED>
+__device__ __forceinline__ WorkItem find_item(const PrefillParams& p, int at, int lane) {
+    const int G = p.G, place = at / p.H_KV;
     const bool causal = p.causal != 0;
-    if (p.dense) {
+    if (PAGED && p.dense) {
         const int seq = place / p.max_w, x = p.max_w - 1 - place % p.max_w;
         return seq < p.num_seqs && x < seq_shape<PAGED>(p, seq).W ? WorkItem{seq, x, 0, 1} : WorkItem{-1, 0, 0, 1};
     }
-    const int share = p.max_pieces > 1 ? batch_share<PAGED>(p, lane) : 1;
-    const SeqShape none = make_seq_shape(0, 0, 0, G, 0);
-    const SeqShape first = lane < p.num_seqs ? seq_shape<PAGED>(p, lane) : none;
-    auto shape = [&](int s0) {
-        return s0 == 0 ? first : (s0 + lane < p.num_seqs ? seq_shape<PAGED>(p, s0 + lane) : none);
-    };
-    auto pieces = [&](const SeqShape& sh) { return pieces_of(sh, share, p.split_w, p.max_pieces, G, causal); };
+    const SeqShape first = lane_shape<PAGED>(p, 0, lane);
+    // (the lengths of the batch are only summed where a sequence is long enough for the shortest pieces)
+    BatchWork batch{kSplitMinTiles, 0};
+    if (PAGED && p.max_pieces > 1 && (p.num_seqs > kWave || __any(may_split(first, p.split_w, p.max_pieces, G, causal, D))))
+        batch = batch_work<PAGED>(p, first, lane);
+    if (PAGED && p.max_pieces > 1) note_pieces<D>(p, first, batch, at, lane);
+    auto shape = [&](int s0) { return s0 == 0 ? first : lane_shape<PAGED>(p, s0, lane); };
+    const int first_pieces = pieces_in<D, PAGED>(p, first, batch);
+    auto pieces = [&](int s0, const SeqShape& sh) { return s0 == 0 ? first_pieces : pieces_in<D, PAGED>(p, sh, batch); };
     auto count = [&](int T) {
         uint32_t c = 0;
         for (int s0 = 0; s0 < p.num_seqs; s0 += kWave) {
             const SeqShape sh = shape(s0);
-            const int n = pieces(sh);
+            const int n = pieces(s0, sh);
             c += uint32_t(n * (sh.W - first_piece_with(sh, T, n, G, causal)));
         }
         return int(wave_add(c));
     };
     WorkItem item{-1, 0, 0, 1};
     int lo = 0, hi = 0x3fffffff, rem = place;            // tile counts lo .. hi - 1 (no sequence has 2^30 tiles)
-    if (p.num_seqs <= kOrderSeqs) {
+    if (!PAGED || p.num_seqs <= kOrderSeqs) {
         if (place >= count(0)) return item;
         hi = 1;                                          // count(lo) > place >= count(hi)
         while (count(hi) > place) { lo = hi; hi *= 2; }
@@ -200,7 +230,7 @@ __device__ __forceinline__ WorkItem find_item(const PrefillParams& p, int place,
     }
     for (int s0 = 0; s0 < p.num_seqs; s0 += kWave) {
         const SeqShape sh = shape(s0);
-        const int n = pieces(sh), x0 = first_piece_with(sh, lo, n, G, causal);
+        const int n = pieces(s0, sh), x0 = first_piece_with(sh, lo, n, G, causal);
         const int mine = n * (first_piece_with(sh, hi, n, G, causal) - x0);
         int before = mine;            // pieces of the lanes up to this one
 #pragma unroll
@@ -407,7 +437,7 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     if constexpr (SCHED) {
         // the KV heads of a place are neighbours: each XCD serves few of them
         const int at = int(blockIdx.x + gridDim.x * blockIdx.y);
-        const WorkItem it = find_item<PAGED>(p, at / p.H_KV, lane);
+        const WorkItem it = find_item<D, PAGED>(p, at, lane);
         if (it.seq < 0) return;                            // the grid is sized for the most work possible
         b = it.seq; hkv = at % p.H_KV; wg = it.x; piece = it.piece; pieces = it.pieces;
     } else {
@@ -970,14 +1000,14 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillPar
     const int n16 = lane & 15, g4 = lane >> 4;
     const int x = int(blockIdx.x) % p.split_w, pair = int(blockIdx.x) / p.split_w;
     const int b = pair / p.H_KV, hkv = pair % p.H_KV;
+    const int pieces = PAGED ? p.left[blockIdx.x] : p.max_pieces;
+    if (pieces == 0) return;
     const SeqShape sh = seq_shape<PAGED>(p, b);
     const int groups = (int(gridDim.y) + 7) / 8, u = int(blockIdx.y) / groups, row0 = int(blockIdx.y) % groups * rows;
     const int unit = 8 * x + u;
-    if (sh.W == 0 || sh.W > p.split_w || x >= sh.W || unit >= sh.units) return;
+    if (unit >= sh.units) return;
     const int pos0 = 32 * (unit / p.G) + row0;
     if (pos0 >= sh.NQ) return;
-    const int pieces = pieces_of(sh, batch_share<PAGED>(p, lane), p.split_w, p.max_pieces, p.G, p.causal != 0);
-    if (pieces < 2) return;
 
     const float* src = p.part + (int64_t(blockIdx.x) * p.max_pieces) * Cfg::SLOT + u * (32 * D + 64);
     constexpr bool kAhead = D <= 128;             // (256 coordinates: too many registers)
@@ -1012,12 +1042,10 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillPar
             }
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                if (k0 + i < pieces) {
-                    const float wk = of_lane(wgt, k0 + i);
-                    den = __builtin_fmaf(of_lane(l, k0 + i), wk, den);
+                const float wk = of_lane(wgt, k0 + i);          // (past the end 0: the last piece's row again adds nothing)
+                den = __builtin_fmaf(of_lane(l, k0 + i), wk, den);
 #pragma unroll
-                    for (int e = 0; e < CPL; ++e) num[e] = __builtin_fmaf(at[i][e], wk, num[e]);
-                }
+                for (int e = 0; e < CPL; ++e) num[e] = __builtin_fmaf(at[i][e], wk, num[e]);
             }
         }
         const float inv = inverse_sum(den);
@@ -1097,10 +1125,9 @@ __global__ __launch_bounds__(512) void attention_combine_prompts_kernel(const Pr
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wg = int(blockIdx.x) % p.split_w, pair = int(blockIdx.x) / p.split_w;
     const int b = pair / p.H_KV, hkv = pair % p.H_KV;
+    const int pieces = PAGED ? p.left[blockIdx.x] : p.max_pieces;
+    if (pieces == 0) return;
     const SeqShape sh = seq_shape<PAGED>(p, b);
-    if (sh.W == 0 || sh.W > p.split_w || wg >= sh.W) return;
-    const int pieces = pieces_of(sh, batch_share<PAGED>(p, lane), p.split_w, p.max_pieces, p.G, p.causal != 0);
-    if (pieces < 2) return;
     RotationBlocks<D> rot{p.rotation, p.rot_col_major != 0, share, w, lane, m32, hf, {}};
     rot.fetch(true, 0);
 
@@ -1190,22 +1217,29 @@ inline SplitPlan plan_of(int num_seqs, int max_q, int64_t max_kv, int H_Q, int H
     if (prompts && max_kv > max_q) max_kv = max_q;               // the keys beyond the queries are hidden
     return plan_split(num_seqs, H_KV, int(max_w), (max_kv + 63) / 64, fq_host::device_cu_count(), D, prompts);
 }
+// Workgroups that may be split, floats of their pieces' rows, and bytes of both with the number of pieces of each.
+inline size_t split_slots(const SplitPlan& sp, int num_seqs, int H_KV) { return size_t(num_seqs) * H_KV * sp.split_w; }
+inline size_t part_floats(const SplitPlan& sp, int num_seqs, int H_KV, int D) {
+    const int slot = D == 64 ? PrefillCfg<64>::SLOT : (D == 128 ? PrefillCfg<128>::SLOT : PrefillCfg<256>::SLOT);
+    return split_slots(sp, num_seqs, H_KV) * sp.max_pieces * slot;
+}
 inline size_t part_bytes(const SplitPlan& sp, int num_seqs, int H_KV, int D) {
     if (sp.max_pieces < 2) return 0;
-    const int slot = D == 64 ? PrefillCfg<64>::SLOT : (D == 128 ? PrefillCfg<128>::SLOT : PrefillCfg<256>::SLOT);
-    return size_t(num_seqs) * H_KV * sp.split_w * sp.max_pieces * slot * 4;
+    return 4 * (part_floats(sp, num_seqs, H_KV, D) + split_slots(sp, num_seqs, H_KV));
 }
 inline int use_plan(PrefillParams& p, const SplitPlan& sp, int D, void* workspace, size_t workspace_bytes) {
     const size_t need = part_bytes(sp, p.num_seqs, p.H_KV, D);
     p.split_w = 0;
     p.max_pieces = 1;
     p.part = nullptr;
+    p.left = nullptr;
     if (need == 0 || workspace == nullptr) return FQ_OK;         // no workspace: nothing is split
     if (workspace_bytes < need) return FQ_ERR_WORKSPACE;
     if (!fq_host::aligned(workspace, 256)) return FQ_ERR_MISALIGNED;
     p.split_w = sp.split_w;
     p.max_pieces = sp.max_pieces;
     p.part = static_cast<float*>(workspace);
+    p.left = reinterpret_cast<int*>(p.part + part_floats(sp, p.num_seqs, p.H_KV, D));
     return FQ_OK;
 }
 
@@ -1301,13 +1335,16 @@ extern "C" int fq_fused_tq_attention_split(const void* q, const uint8_t* k_packe
     p.num_seqs = B;
     p.max_w = int(wgs);
     p.dense = false;
-    // A launch that fills the chip keeps the plain order, one that leaves CUs idle is split if the lengths allow (here
-    // they are known: a plan under which no workgroup would be split is dropped).
+    // A launch that fills the chip keeps the plain order, one that leaves CUs idle is split if the lengths allow (here they
+    // are known, and with them the pieces).
     SplitPlan sp = plan_of(B, N_Q, N_KV, H_Q, H_KV, D, p.causal != 0);
     if (sp.max_pieces > 1) {
         const SeqShape sh = make_seq_shape(N_Q, N_KV, 0, p.G, p.max_w);
         const uint32_t sum = uint32_t(B) * (uint32_t(sh.W) * uint32_t(tiles_of(sh, 0, p.G, p.causal) + tiles_of(sh, sh.W - 1, p.G, p.causal) + 1) / 2);
-        if (pieces_of(sh, share_of(sum * uint32_t(H_KV), p.round_slots), sp.split_w, sp.max_pieces, p.G, p.causal) < 2) sp = SplitPlan{0, 1};
+        const uint32_t rows = sh.W <= sp.split_w ? uint32_t(B) * uint32_t(N_Q) * uint32_t(H_Q) : 0;
+        const BatchWork batch{share_of(sum * uint32_t(H_KV), p.round_slots), int(rows >> 8)};
+        const int n = pieces_of(sh, batch, sp.split_w, sp.max_pieces, p.G, p.causal, D);
+        sp = n < 2 ? SplitPlan{0, 1} : SplitPlan{sp.split_w, n};
     }
     const int st = use_plan(p, sp, D, workspace, workspace_bytes);
     if (st != FQ_OK) return st;

@@ -392,3 +392,30 @@ def test_paged_prefill_of_many_sequences(many, d):
     # three roundings to bf16 and fp16 keys, a worst row of some thousands: as in _close with the row's own norm
     _rows_close(got, want, 4 * 2 ** -8)
     assert torch.equal(prefill_in_one_piece(*args, r.to(DEV), hkv, d, bs), got)
+
+
+# (queries, keys) per sequence under a block table of 4096 tokens, which allows pieces that the lengths may not be worth:
+# prompts of one and of several workgroups, long and short contexts together, sequences without queries or keys
+UNDER_WIDE = [([400] * 3, [400] * 3), ([200] * 3, [700, 200, 900]), ([40, 1, 300, 0, 5], [2000, 300, 300, 50, 1100]),
+              ([1, 1, 17, 1], [200, 0, 430, 900]), ([700, 64], [700, 1500])]
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(16, 4, 64), (16, 4, 128), (8, 2, 256), (8, 8, 128)])
+@pytest.mark.parametrize("batch", range(len(UNDER_WIDE)))
+def test_paged_prefill_under_a_wide_table(batch, hq, hkv, d):
+    ql, kv = UNDER_WIDE[batch]
+    bs, dtype = 16, torch.bfloat16
+    assert attention_workspace_bytes(len(ql), max(ql), 4096, hq, hkv, d) > 0
+    c, _, r = book(d)
+    _, cache, table, sl = build_paged_case(kv, hq, hkv, d=d, bs=bs, seed=121, dtype=dtype)
+    q = torch.randn(sum(ql), hq, d, generator=torch.Generator().manual_seed(122)).to(dtype)
+    cu = torch.tensor([0] + list(torch.tensor(ql).cumsum(0)), dtype=torch.int32)
+    want = O.paged_prefill(q, cu, cache, table, sl, c, c, r, hkv, d, bs)
+    wide = torch.randint(-3, 1 << 20, (len(ql), 256), dtype=torch.int32, generator=torch.Generator().manual_seed(123))
+    wide[:, :table.shape[1]] = table
+    got = torch.full_like(q, 7.0).to(DEV)
+    K.paged_tq4_prefill(q.to(DEV), cu.to(DEV), max(ql), cache.to(DEV), wide.to(DEV), sl.to(DEV), c.to(DEV), c.to(DEV), r.to(DEV),
+                        hkv, d, bs, out=got)
+    keyless = torch.cat([torch.full((n,), m == 0) for n, m in zip(ql, kv)])
+    assert (got.cpu()[keyless] == 0).all()
+    _rows_close(got.cpu()[~keyless], want[~keyless], 4 * 2 ** -8)
