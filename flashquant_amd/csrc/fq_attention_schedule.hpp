@@ -86,7 +86,7 @@ FQ_HD int first_with(const SeqShape& s, int T, int G, bool causal) {
 // however few they are; a piece of 256 rows, written and read.  Fitted on 1775 paged batches of equal sequences (1, 3 and 8
 // of them, 1 to 1000 queries over 400 to 4000 keys, four head counts), each run in pieces and in one: with 33 queries and more
 // the combine took 3 and 5 us up to 16 workgroups' worth of pieces and 8 and 17 us at 128 (64 and 128 coordinates).  At 256
-// pieces won in nearly all of them: the rotation back of a few workgroups is what the combine spreads over the chip.
+// pieces won in all of them: the rows go through the combine there whether they are split or not.
 struct SplitCost {
     int tile, fixed, slot;
 };

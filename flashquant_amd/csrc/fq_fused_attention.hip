@@ -93,6 +93,7 @@ struct PrefillParams {
     // order and split of the work (fq_attention_schedule.hpp); workgroups in split pieces leave their rows in `part`
     int num_seqs, max_w, split_w, max_pieces;
     bool dense;                 // beyond kOrderSeqs sequences: max_w places for each of them
+    bool all_in_part;           // workgroups that are not split leave their rows in `part` too
     float* part;                   // slot of a workgroup's piece: PrefillCfg<D>::SLOT floats
     int* left;                     // paged: pieces in `part` of every workgroup that may be split, 0 if none
     bool out_wide;                 // `out` is 16-byte aligned (its rows are multiples of 128 bytes apart)
@@ -182,14 +183,14 @@ __device__ __forceinline__ void note_pieces(const PrefillParams& p, const SeqSha
     const SeqShape sh = b < kWave ? make_seq_shape(of_lane(first.NQ), of_lane(first.NKV), of_lane(first.qoff), p.G, p.max_w)
                                   : seq_shape<true>(p, b);
     const int n = x < sh.W && sh.W <= p.split_w ? pieces_in<D, true>(p, sh, batch) : 0;
-    if (threadIdx.x == 0) p.left[at] = n > 1 ? n : 0;
+    if (threadIdx.x == 0) p.left[at] = n > 1 || p.all_in_part ? n : 0;
 }
 
 // The item of a place (`at` / H_KV, of one KV head) in the order longest piece first: the largest tile count T that more than
 // `place` pieces reach, by bisection with a lane per sequence; then the place among the pieces of exactly T.  Beyond
 // kOrderSeqs sequences the items in the order of the sequences (kOrderSeqs says why).
-// `at` is the workgroup's number in the launch.
-template <int D, bool PAGED>
+// SPLIT: `at` is the workgroup's number in the launch.
+template <int D, bool PAGED, bool SPLIT>
 __device__ __forceinline__ WorkItem find_item(const PrefillParams& p, int at, int lane) {
     const int G = p.G, place = at / p.H_KV;
     const bool causal = p.causal != 0;
@@ -200,12 +201,12 @@ __device__ __forceinline__ WorkItem find_item(const PrefillParams& p, int at, in
     const SeqShape first = lane_shape<PAGED>(p, 0, lane);
     // (the lengths of the batch are only summed where a sequence is long enough for the shortest pieces)
     BatchWork batch{kSplitMinTiles, 0};
-    if (PAGED && p.max_pieces > 1 && (p.num_seqs > kWave || __any(may_split(first, p.split_w, p.max_pieces, G, causal, D))))
+    if (PAGED && SPLIT && (p.num_seqs > kWave || __any(may_split(first, p.split_w, p.max_pieces, G, causal, D))))
         batch = batch_work<PAGED>(p, first, lane);
-    if (PAGED && p.max_pieces > 1) note_pieces<D>(p, first, batch, at, lane);
+    if (PAGED && SPLIT) note_pieces<D>(p, first, batch, at, lane);
     auto shape = [&](int s0) { return s0 == 0 ? first : lane_shape<PAGED>(p, s0, lane); };
-    const int first_pieces = pieces_in<D, PAGED>(p, first, batch);
-    auto pieces = [&](int s0, const SeqShape& sh) { return s0 == 0 ? first_pieces : pieces_in<D, PAGED>(p, sh, batch); };
+    const int first_pieces = SPLIT ? pieces_in<D, PAGED>(p, first, batch) : 1;
+    auto pieces = [&](int s0, const SeqShape& sh) { return s0 == 0 || !SPLIT ? first_pieces : pieces_in<D, PAGED>(p, sh, batch); };
     auto count = [&](int T) {
         uint32_t c = 0;
         for (int s0 = 0; s0 < p.num_seqs; s0 += kWave) {
@@ -404,18 +405,29 @@ __device__ __forceinline__ void finish_rows(const PrefillParams& p, RotationBloc
     }
 }
 
+// Where a workgroup's work comes from and what becomes of its rows.  At 256 coordinates the end of a workgroup beside the
+// branch that leaves its rows to the combine costs 170 to 260 spilled registers, some of them inside the tile loop, either
+// one alone 30 to 40: 8 sequences of 120 queries over 1500 keys, 32 heads, 226 us with both compiled in, 170 with one.
+enum Work {
+    kGrid,            // one workgroup per grid position, rows finished in the kernel
+    kOrdered,         // find_item, the same
+    kPieces,          // find_item, rows of a piece left to the combine, other rows finished in the kernel
+    kAllPieces        // find_item, all rows left to the combine
+};
+
 // PAGED: the sequences' queries are packed along the token axis of q (tokens, H_Q, 128), the keys
 // and values come from the paged TQ4 cache through the block table, query j of a sequence with
 // n queries and L keys sits at position L - n + j (the new tokens are the last ones), and the
 // attention result is rounded to the query dtype before the rotation back, as the attention
 // library's output is in the path this replaces (src/flashquant/vllm/impl.py:265-336, 470-512).
-// SCHED: workgroups take their work from find_item; else one workgroup per grid position, in the order below.
-template <int D, int DT, bool PAGED, bool SCHED>
+// WORK: how the workgroups take their work and where it ends (below).
+template <int D, int DT, bool PAGED, int WORK>
 __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillParams p) {
     using Cfg = PrefillCfg<D>;
     constexpr int kPfKStride = Cfg::KSTRIDE, kPfKBytes = Cfg::KBYTES, kPfBufBytes = Cfg::BUF;
     constexpr int NKS = Cfg::NKS, NOB = Cfg::NOB, PB = Cfg::PB, TS = Cfg::TS, TT = Cfg::TT;
     constexpr int NTB = TT / 32, NVS = TT / 16;    // 32-token blocks of the scores, k-steps of the second product
+    constexpr bool kFind = WORK != kGrid, kSplit = WORK == kPieces || WORK == kAllPieces;
     __shared__ __attribute__((aligned(256))) uint32_t lut[256 * 64];
     extern __shared__ __attribute__((aligned(16))) uint8_t bufs[];   // 2 x (K tile | V^T tile)
     // Rows whose norm times a centroid would not fit fp16 are stored divided by a power of two.
@@ -434,10 +446,10 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     // slow, and the position order reversed in every other round over the chip: whichever way the
     // rounds land on the CUs, each CU sees long and short workgroups alternate.
     int b, hkv, wg, piece = 0, pieces = 1;
-    if constexpr (SCHED) {
+    if constexpr (kFind) {
         // the KV heads of a place are neighbours: each XCD serves few of them
         const int at = int(blockIdx.x + gridDim.x * blockIdx.y);
-        const WorkItem it = find_item<D, PAGED>(p, at, lane);
+        const WorkItem it = find_item<D, PAGED, kSplit>(p, at, lane);
         if (it.seq < 0) return;                            // the grid is sized for the most work possible
         b = it.seq; hkv = at % p.H_KV; wg = it.x; piece = it.piece; pieces = it.pieces;
     } else {
@@ -487,7 +499,7 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     // this piece's tiles: first_tile .. ntiles - 1 (of this wavefront: .. my_tiles - 1).  Pieces are cut between the
     // schedule's tiles of 64 keys.
     int first_tile = 0;
-    if (SCHED && pieces > 1) {
+    if (kSplit && pieces > 1) {
         constexpr int SH = 6 - TS;
         const int whole = (ntiles + (1 << SH) - 1) >> SH;
         first_tile = int(int64_t(whole) * piece / pieces) << SH;
@@ -953,7 +965,7 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     // ---- a piece of a workgroup's keys: the rows as they are, for the combine launch ------------------------
     // Only rows that hold a query: a unit of one query left 31 rows of padding, 64 KB a piece at 4 heads of 128 (one query
     // over 4 x 2500 tokens of a ring buffer 33.5 -> 30.2 us, a mixed batch of 12 sequences 381 -> 373 us).
-    if (SCHED && pieces > 1) {
+    if (WORK == kAllPieces || (WORK == kPieces && pieces > 1)) {
         const float l_piece = l_run + xor_shuffle(l_run, 32);
         if (!unit_live || pos0 + m32 >= NQ) return;
         const int64_t slot = ((int64_t(b) * p.H_KV + hkv) * p.split_w + wg) * p.max_pieces + piece;
@@ -969,13 +981,15 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     }
 
     // ---- normalise, rotate back, store -------------------------------------------------------------------
-    const float l_tot = l_run + xor_shuffle(l_run, 32);
-    const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-    rot.fetch(true, 0);
-    __syncthreads();                // every wavefront is done with the lookup tables
-    rot.put();
-    __syncthreads();
-    finish_rows<D, DT, PAGED>(p, rot, O, inv, unit_live, pos0, hq, NQ, q_row0, q_stride);
+    if constexpr (WORK != kAllPieces) {
+        const float l_tot = l_run + xor_shuffle(l_run, 32);
+        const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+        rot.fetch(true, 0);
+        __syncthreads();                // every wavefront is done with the lookup tables
+        rot.put();
+        __syncthreads();
+        finish_rows<D, DT, PAGED>(p, rot, O, inv, unit_live, pos0, hq, NQ, q_row0, q_stride);
+    }
 }
 
 // The weight 2^(m - top) of a piece's row.  A piece without a visible key has m = -inf, a sum of 0 and rows of zeros; one whose
@@ -1166,40 +1180,55 @@ __global__ __launch_bounds__(512) void attention_combine_prompts_kernel(const Pr
                               PAGED ? p.H_Q * D : D);
 }
 
-template <int D, int DT, bool PAGED, bool SCHED>
+template <int D, int DT, bool PAGED, int WORK>
 int launch_prefill_as(const PrefillParams& p, dim3 grid, int max_q, hipStream_t s) {
     const size_t lds = 2 * size_t(PrefillCfg<D>::BUF);
-    auto kern = fused_tq_attention_kernel<D, DT, PAGED, SCHED>;
+    auto kern = fused_tq_attention_kernel<D, DT, PAGED, WORK>;
     if (!fq_host::lds_limit_raised(reinterpret_cast<const void*>(kern), lds)) return FQ_ERR_LAUNCH;
     hipLaunchKernelGGL(kern, grid, dim3(512), lds, s, p);
     const int st = fq_host::check_launch();
-    if constexpr (SCHED) {
-        if (st == FQ_OK && p.max_pieces > 1) {
-            const int64_t slots = int64_t(p.num_seqs) * p.H_KV * p.split_w;
-            if (p.split_w > 1 && 2 * slots >= p.round_slots) {
-                hipLaunchKernelGGL((attention_combine_prompts_kernel<D, DT, PAGED>), dim3(unsigned(slots)), dim3(512), 0, s, p);
-                return fq_host::check_launch();
-            }
-            const int rows = max_q <= 4 ? 4 : 16;
-            const int groups = max_q <= 16 ? 1 : 2;             // 32 rows a unit at most
-            hipLaunchKernelGGL((attention_combine_kernel<D, DT, PAGED>),
-                               dim3(unsigned(slots), 8 * groups), dim3(256), 0, s, p, rows);
+    if constexpr (WORK == kPieces || WORK == kAllPieces) {
+        if (st != FQ_OK) return st;
+        const int64_t slots = int64_t(p.num_seqs) * p.H_KV * p.split_w;
+        if (p.split_w > 1 && 2 * slots >= p.round_slots) {
+            hipLaunchKernelGGL((attention_combine_prompts_kernel<D, DT, PAGED>), dim3(unsigned(slots)), dim3(512), 0, s, p);
             return fq_host::check_launch();
         }
+        const int rows = max_q <= 4 ? 4 : 16;
+        const int groups = max_q <= 16 ? 1 : 2;             // 32 rows a unit at most
+        hipLaunchKernelGGL((attention_combine_kernel<D, DT, PAGED>), dim3(unsigned(slots), 8 * groups), dim3(256), 0, s, p, rows);
+        return fq_host::check_launch();
     }
     return st;
 }
 
-template <bool PAGED, bool SCHED>
-int launch_prefill(const PrefillParams& p, int D, dim3 grid, int max_q, int dtype, hipStream_t s) {
-    if (D == 64)
-        return dtype == FQ_F16 ? launch_prefill_as<64, FQ_F16, PAGED, SCHED>(p, grid, max_q, s)
-                               : launch_prefill_as<64, FQ_BF16, PAGED, SCHED>(p, grid, max_q, s);
-    if (D == 256)
-        return dtype == FQ_F16 ? launch_prefill_as<256, FQ_F16, PAGED, SCHED>(p, grid, max_q, s)
-                               : launch_prefill_as<256, FQ_BF16, PAGED, SCHED>(p, grid, max_q, s);
-    return dtype == FQ_F16 ? launch_prefill_as<128, FQ_F16, PAGED, SCHED>(p, grid, max_q, s)
-                           : launch_prefill_as<128, FQ_BF16, PAGED, SCHED>(p, grid, max_q, s);
+template <int D, bool PAGED, int WORK>
+int launch_prefill_dtype(const PrefillParams& p, dim3 grid, int max_q, int dtype, hipStream_t s) {
+    return dtype == FQ_F16 ? launch_prefill_as<D, FQ_F16, PAGED, WORK>(p, grid, max_q, s)
+                           : launch_prefill_as<D, FQ_BF16, PAGED, WORK>(p, grid, max_q, s);
+}
+
+// The forms that are built: contiguous launches are all in pieces or not at all; of the paged ones a batch whose every
+// workgroup has a place in `part` leaves all rows there at 256 coordinates (Work says why).
+template <int D, bool PAGED>
+int launch_prefill_dim(PrefillParams& p, dim3 grid, int max_q, int dtype, hipStream_t s) {
+    p.all_in_part = p.max_pieces > 1 && (!PAGED || (D == 256 && p.split_w == p.max_w));
+    if (p.all_in_part) {
+        if constexpr (!PAGED || D == 256) return launch_prefill_dtype<D, PAGED, kAllPieces>(p, grid, max_q, dtype, s);
+    }
+    if constexpr (!PAGED) {
+        return launch_prefill_dtype<D, PAGED, kGrid>(p, grid, max_q, dtype, s);
+    } else {
+        if (p.max_pieces > 1) return launch_prefill_dtype<D, PAGED, kPieces>(p, grid, max_q, dtype, s);
+        return launch_prefill_dtype<D, PAGED, kOrdered>(p, grid, max_q, dtype, s);
+    }
+}
+
+template <bool PAGED>
+int launch_prefill(PrefillParams& p, int D, dim3 grid, int max_q, int dtype, hipStream_t s) {
+    if (D == 64) return launch_prefill_dim<64, PAGED>(p, grid, max_q, dtype, s);
+    if (D == 256) return launch_prefill_dim<256, PAGED>(p, grid, max_q, dtype, s);
+    return launch_prefill_dim<128, PAGED>(p, grid, max_q, dtype, s);
 }
 
 // n workgroups in rows of at most 2^20 (a grid row holds fewer than 2^32 threads); the last row's surplus finds no work.
@@ -1348,9 +1377,7 @@ extern "C" int fq_fused_tq_attention_split(const void* q, const uint8_t* k_packe
     }
     const int st = use_plan(p, sp, D, workspace, workspace_bytes);
     if (st != FQ_OK) return st;
-    if (p.max_pieces > 1)
-        return launch_prefill<false, true>(p, D, folded_grid(int64_t(B) * H_KV * wgs * p.max_pieces), N_Q, dtype, s);
-    return launch_prefill<false, false>(p, D, grid, N_Q, dtype, s);
+    return launch_prefill<false>(p, D, p.max_pieces > 1 ? folded_grid(int64_t(B) * H_KV * wgs * p.max_pieces) : grid, N_Q, dtype, s);
 }
 
 extern "C" int fq_paged_tq4_prefill(const void* q, const int32_t* cu_seqlens_q, const uint8_t* kv_cache,
@@ -1439,5 +1466,5 @@ extern "C" int fq_paged_tq4_prefill_split(const void* q, const int32_t* cu_seqle
     if (st != FQ_OK) return st;
     p.dense = dense;
     places += int64_t(num_seqs) * p.split_w * (p.max_pieces - 1);
-    return launch_prefill<true, true>(p, D, folded_grid(places * H_KV), max_q_len, dtype, static_cast<hipStream_t>(stream));
+    return launch_prefill<true>(p, D, folded_grid(places * H_KV), max_q_len, dtype, static_cast<hipStream_t>(stream));
 }
