@@ -619,21 +619,22 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> prod_compress(const at::Tensor& x
     return {packed, norms, gam};
 }
 
-void prod_store_rows(const at::Tensor& kv_cache, const at::Tensor& slot_mapping, const at::Tensor& k_packed,
+// False, with nothing done, where the operands are not what the kernel takes as they are: uint8 rows and float32 norms, one
+// slot per token, the bytes of a cache row side by side and its rows not over one another.
+bool prod_store_rows(const at::Tensor& kv_cache, const at::Tensor& slot_mapping, const at::Tensor& k_packed,
                      const at::Tensor& k_norms, const at::Tensor& k_gamma, const at::Tensor& v_packed,
                      const at::Tensor& v_norms) {
     fqbind::require_gpu(kv_cache, "kv_cache");
-    require(k_packed.dim() == 3 && k_packed.scalar_type() == at::kByte && k_packed.size(2) > 0 && k_packed.size(1) > 0,
-            "k_packed must be uint8 of shape (N, H, D/2)");
+    if (k_packed.dim() != 3 || k_packed.numel() == 0 || slot_mapping.dim() != 1 || slot_mapping.numel() != k_packed.size(0)) return false;
     const int64_t N = k_packed.size(0), H = k_packed.size(1), half = k_packed.size(2), row_bytes = H * (2 * half + 12);
-    require(v_packed.scalar_type() == at::kByte && v_packed.numel() == k_packed.numel(), "v_packed must be uint8 with the size of k_packed");
+    if (H > 65535 || half > 2048 || kv_cache.numel() % row_bytes != 0) return false;
+    for (const at::Tensor* t : {&kv_cache, &k_packed, &v_packed})
+        if (t->scalar_type() != at::kByte) return false;
     for (const at::Tensor* t : {&k_norms, &k_gamma, &v_norms})
-        require(t->scalar_type() == at::kFloat && t->numel() == N * H, "norms must be float32 with one value per (token, head)");
-    require(kv_cache.scalar_type() == at::kByte && kv_cache.numel() % row_bytes == 0,
-            "kv_cache must be a uint8 tensor of token rows of H * (D + 12) bytes");
+        if (t->scalar_type() != at::kFloat || t->numel() != N * H) return false;
+    if (v_packed.numel() != k_packed.numel()) return false;
     const at::Tensor rows = kv_cache.view({kv_cache.numel() / row_bytes, row_bytes});     // the rows may lie apart, not their bytes
-    require(rows.stride(1) == 1 && (rows.size(0) <= 1 || rows.stride(0) >= row_bytes), "the bytes of a row of kv_cache must be contiguous");
-    require(slot_mapping.numel() == N, "slot_mapping must hold one slot per token");
+    if (rows.stride(1) != 1 || (rows.size(0) > 1 && rows.stride(0) < row_bytes)) return false;
     c10::DeviceGuard guard(kv_cache.device());
     const auto dev = kv_cache.device();
     const at::Tensor sm = slot_mapping.to(dev, at::kLong).contiguous();
@@ -643,6 +644,7 @@ void prod_store_rows(const at::Tensor& kv_cache, const at::Tensor& slot_mapping,
                                       kn.data_ptr<float>(), kg.data_ptr<float>(), vp.data_ptr<uint8_t>(), vn.data_ptr<float>(),
                                       N, rows.size(0), int(H), int(2 * half), fqbind::current_stream(kv_cache));
     fqbind::raise_on_error(st, "prod_store_rows");
+    return true;
 }
 
 at::Tensor prod_paged_decode(const at::Tensor& q, const at::Tensor& kv_cache, const at::Tensor& block_table,
@@ -925,7 +927,7 @@ void bind_kernels(py::module_& m) {
           "Variable-length prefill over the packed paged TQ4 cache: un-rotated q (tokens, H_Q, D), original-space output");
     m.def("prod_store_rows", &prod_store_rows, py::arg("kv_cache"), py::arg("slot_mapping"), py::arg("k_packed"),
           py::arg("k_norms"), py::arg("k_gamma"), py::arg("v_packed"), py::arg("v_norms"),
-          "Write TurboQuantProd token rows into the paged cache at the flat slots of slot_mapping.");
+          "Write TurboQuantProd token rows into the paged cache at the flat slots of slot_mapping; False if it does not take the operands' form.");
     m.def("prod_compress", &prod_compress, py::arg("x"), py::arg("rotation"), py::arg("sketch_rot"),
           py::arg("boundaries"), py::arg("centroids"),
           "TurboQuantProd key compress: (packed nibbles sign<<3|idx (N,H,D/2), norms (N,H,1), residual norms (N,H,1))");

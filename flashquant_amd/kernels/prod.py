@@ -57,9 +57,22 @@ def prod_store_rows(
     v_norms: torch.Tensor,
 ) -> None:
     """Write the tokens' rows into the paged cache (num_blocks, block_size,
-    H*(D+12)) at the flat slots of ``slot_mapping`` (device tensors), one launch."""
+    H*(D+12)) at the flat slots of ``slot_mapping`` (device tensors), one launch;
+    a slot outside the cache is not stored.  Forms that the kernel does not take
+    (other integer types, one row for several slots, strided bytes) are assembled
+    into rows and stored by index."""
     require_gpu(kv_cache, "kv_cache")
-    native().prod_store_rows(kv_cache, slot_mapping, k_packed, k_norms, k_gamma, v_packed, v_norms)
+    if native().prod_store_rows(kv_cache, slot_mapping, k_packed, k_norms, k_gamma, v_packed, v_norms):
+        return
+    n, h, half = k_packed.shape
+    k_norm, k_gamma_off, v_idx, v_norm, row_bytes = prod_page_layout(h, 2 * half)
+    row = torch.empty(n, row_bytes, dtype=torch.uint8, device=kv_cache.device)
+    row[:, :k_norm] = k_packed.reshape(n, -1)
+    row[:, k_norm:k_gamma_off] = k_norms.reshape(n, h).contiguous().view(torch.uint8)
+    row[:, k_gamma_off:v_idx] = k_gamma.reshape(n, h).contiguous().view(torch.uint8)
+    row[:, v_idx:v_norm] = v_packed.reshape(n, -1)
+    row[:, v_norm:] = v_norms.reshape(n, h).contiguous().view(torch.uint8)
+    kv_cache.view(-1, row_bytes)[slot_mapping.long()] = row
 
 
 def prod_paged_decode(

@@ -115,3 +115,46 @@ def test_decompress_cache_at_an_odd_byte():
         for a, b in zip(layer.decompress_cache(moved, torch.bfloat16, apply_rotation=rotate),
                         layer.decompress_cache(cache, torch.bfloat16, apply_rotation=rotate)):
             assert torch.equal(a, b)
+
+
+def _prod_rows(n, h, d, seed):
+    g = torch.Generator().manual_seed(seed)
+    packed = [torch.randint(0, 256, (n, h, d // 2), dtype=torch.uint8, generator=g) for _ in range(2)]
+    norms = [torch.rand(n, h, 1, generator=g) for _ in range(3)]
+    row = torch.cat([packed[0].view(n, -1), norms[0].view(n, h).view(torch.uint8), norms[1].view(n, h).view(torch.uint8),
+                     packed[1].view(n, -1), norms[2].view(n, h).view(torch.uint8)], dim=1)
+    return (packed[0], norms[0], norms[1], packed[1], norms[2]), row
+
+
+@pytest.mark.parametrize("form", ["one row", "slots in rows", "int packed", "strided bytes", "two-dimensional slots"])
+def test_prod_store_rows_of_unusual_forms(form):
+    """What an indexed store of assembled rows takes: one row for several slots, slots of more dimensions, indices of another
+    integer type, a cache whose bytes lie apart."""
+    h, d, pages, page = 4, 64, 3, 16
+    n = 1 if form == "one row" else 6
+    operands, row = _prod_rows(n, h, d, 7)
+    slots = torch.tensor([3, 41, 17, -1, 8, 30])
+    if form in ("slots in rows", "two-dimensional slots"):
+        slots = slots[None] if form == "slots in rows" else torch.stack([slots, (slots + 1) % 48])
+    gap = 2 if form == "strided bytes" else 1
+    buf = torch.randint(0, 256, (pages, page, row.shape[1] * gap), dtype=torch.uint8, generator=torch.Generator().manual_seed(8))
+    want = buf.clone()
+    want[..., ::gap].view(-1, row.shape[1])[slots] = row
+    got = buf.to(DEV)
+    dev = [t.to(DEV) for t in operands]
+    if form == "int packed":
+        dev[0], dev[3] = dev[0].int(), dev[3].long()
+    K.prod_store_rows(got[..., ::gap], slots.to(DEV), *dev)
+    assert torch.equal(got.cpu(), want)
+
+
+def test_prod_store_rows_skips_slots_outside_the_cache():
+    h, d, pages, page = 2, 64, 2, 16
+    operands, row = _prod_rows(5, h, d, 9)
+    slots = torch.tensor([32, 4, -33, 1 << 40, 31])
+    cache = torch.randint(0, 256, (pages, page, row.shape[1]), dtype=torch.uint8, generator=torch.Generator().manual_seed(10))
+    want = cache.clone()
+    want.view(-1, row.shape[1])[slots[[1, 4]]] = row[[1, 4]]
+    got = cache.to(DEV)
+    K.prod_store_rows(got, slots.to(DEV), *[t.to(DEV) for t in operands])
+    assert torch.equal(got.cpu(), want)
