@@ -139,7 +139,7 @@ extern "C" int fq_tq4_decompress_cache(const uint8_t* kv_cache, const float* cen
                                        int rotation_col_major, void* out_k, void* out_v, int out_dtype, int64_t num_slots,
                                        int H, int D, void* stream) {
     using namespace fq;
-    if (num_slots < 0 || H <= 0 || H > 65535) return FQ_ERR_BAD_SHAPE;
+    if (num_slots < 0 || H <= 0 || H > (1 << 20)) return FQ_ERR_BAD_SHAPE;      // the kernels divide by H in float32
     if (!fq_host::supported_dim(D)) return FQ_ERR_UNSUPPORTED_DIM;
     if (out_dtype != FQ_F16 && out_dtype != FQ_BF16 && (out_dtype != FQ_F32 || rotation)) return FQ_ERR_UNSUPPORTED_DTYPE;
     if (num_slots == 0) return FQ_OK;

@@ -26,8 +26,9 @@ def random_cache(pages, page, h, d, seed):
     return cache.to(DEV), [t.to(DEV) for t in sections]
 
 
-# one token, a tile that ends inside a token, several tiles of a workgroup, heads that do not divide a tile
-@pytest.mark.parametrize("pages,page,h", [(1, 1, 1), (3, 16, 1), (1, 8, 3), (5, 16, 8), (200, 32, 8), (7, 16, 40), (40, 16, 5)])
+# one token, a tile that ends inside a token, several tiles of a workgroup, heads that do not divide a tile, more heads than
+# 16 bits count
+@pytest.mark.parametrize("pages,page,h", [(1, 1, 1), (3, 16, 1), (1, 8, 3), (5, 16, 8), (200, 32, 8), (7, 16, 40), (40, 16, 5), (2, 3, 70001)])
 @pytest.mark.parametrize("d", [64, 128, 256])
 def test_decompress_cache_equals_decompress_of_its_sections(pages, page, h, d):
     layer = TQ4AttentionKernels(h, d, 1.0 / math.sqrt(d), torch.device(DEV))
