@@ -287,3 +287,35 @@ def test_shape_limits_of_the_staged_and_prod_decodes(lib):
     g.argtypes = ([ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int] + [ctypes.c_void_p] * 8 + [ctypes.c_int] * 6 +
                   [ctypes.c_int64, ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_void_p])
     assert g(_p(4096), _p(4096), 0, *([_p(4096)] * 8), 2, 16, 4, 128, 16, 4, 64, 0.088, 1, 1, _p()) == FQ_SHAPE
+
+
+def test_attention_workspace_errors(lib):
+    """The entries with a workspace refuse one that is too small or not aligned (none at all is allowed: nothing is split)."""
+    size = lib.fq_attention_workspace_bytes
+    size.restype = ctypes.c_size_t
+    size.argtypes = [ctypes.c_int] * 2 + [ctypes.c_int64] + [ctypes.c_int] * 4
+    p, i, v = ctypes.c_void_p, ctypes.c_int, _p(4096)
+    f = lib.fq_fused_tq_attention_split
+    f.argtypes = [p] * 8 + [i, p] + [i] * 5 + [ctypes.c_int64] * 2 + [i, ctypes.c_float, i, i, p, ctypes.c_size_t, p]
+    paged = lib.fq_paged_tq4_prefill_split
+    paged.argtypes = [p] * 8 + [i, p] + [i] * 7 + [ctypes.c_int64, ctypes.c_float, i, i, ctypes.c_int64, p, ctypes.c_size_t, p]
+    for d in (64, 128, 256):
+        need = size(4, 1, 2500, 32, 8, d, 0)
+        assert need > 0
+
+        def call(ws, n):
+            return f(*[v] * 8, 0, v, 4, 32, 8, 1, 2500, 2500, 2500, d, 0.1, 0, 1, _p(ws), n, _p())
+
+        # (the plan of one call may use less than the size that holds for all calls of its sizes)
+        assert call(8192, 0) == FQ_WS and call(8192, 4096) == FQ_WS
+        assert call(8192 + 128, need) == FQ_ALIGN
+        need = size(3, 40, 200 * 16, 32, 8, d, 0)
+        assert need > 0
+
+        def call_paged(ws, n):
+            return paged(*[v] * 8, 0, v, 3, 40, 32, 8, d, 16, 200, 4096, 0.1, 1, 1, 42, _p(ws), n, _p())
+
+        assert call_paged(8192, need - 1) == FQ_WS and call_paged(8192, 0) == FQ_WS
+        assert call_paged(8192 + 128, need) == FQ_ALIGN
+    # sizes that are never split, or that no call can have
+    assert size(1, 1, 300, 32, 8, 128, 0) == 0 and size(0, 1, 9000, 32, 8, 128, 0) == 0 and size(1, 1, 9000, 30, 8, 128, 0) == 0
