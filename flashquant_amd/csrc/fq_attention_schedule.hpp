@@ -9,9 +9,12 @@
 //   * where a sequence's keys are long for its few queries (`split_w`, `max_pieces`, set by the host from what it
 //     knows), they are cut into pieces of about the share of a CU; the pieces leave partial results, combined by a
 //     launch of their own.
+// So the bits of a row depend on the batch around it (the pieces on the lengths, their sum, the longest context that the host
+// allows for and the number of CUs): within rounding, and the same for the same call.
 // Measured (MI355X, bf16, 32 query heads over 8 KV heads of 128): a batch of 12 with six prompts, three later chunks and
 // three single queries, 10,556 new tokens, 467 us in grid order and 385 us longest first; one query over 4 x 2500 tokens of a
-// ring buffer 67 us in one workgroup per KV head and 34 us in 5 pieces, over 1 x 16,384 tokens 390 and 39 us (32 pieces).
+// ring buffer 67 us in one workgroup per KV head, 24 to 26 us in 8 pieces, over 1 x 16,384 tokens 31 us in 32 pieces (369 us
+// before the kernel cut contexts).
 // Everything here is arithmetic on the lengths alone: the same in every workgroup and in the combine launch.
 #pragma once
 
@@ -28,7 +31,8 @@ namespace fq {
 // The shortest piece, in tiles of 64 keys.  Pieces go to CUs that have nothing else to do, so a piece costs its rows in
 // the combine (2 KB a query head block of few queries) and not its prologue.  One query over a ring buffer of 4 x 2500 tokens,
 // 32 heads over 8: 30.2 us with at least 8 tiles a piece, 28.5 with 6, 26.0 with 5 and 25.9 with 4; 1 x 1300 tokens 34.5, 28.5,
-// 27.1 and 25.8; 8 heads over 1 of 256 coordinates, 1 x 2000 tokens, 2 queries 78.5, 72.0, 67.9 and 58.1.
+// 27.1 and 25.8; 8 heads over 1 of 256 coordinates, 1 x 2000 tokens, 2 queries 78.5, 72.0, 67.9 and 58.1.  (Each is 1.5 to 2.5
+// us less now that the host works out the pieces of contiguous keys.)
 constexpr int kSplitMinTiles = 4;
 
 // Batches of more sequences than this are not ordered.  Every workgroup finds its own item, and the search for the longest
@@ -141,8 +145,8 @@ FQ_HD int first_piece_with(const SeqShape& s, int T, int pieces, int G, bool cau
 // of one known length under a causal mask) is about one round of workgroups, the longest with twice the average work: two
 // pieces, if half of the longest workgroup outweighs that traffic and the second prologues too.  (Whether the shares are
 // uneven enough pieces_of decides; more workgroups than 4/3 of a round never are.)  8 heads x 6000 tokens of 256 coordinates,
-// one KV head, 188 workgroups: 538 us in one piece, 347 us in two; 16 heads x 3001 tokens on 4 KV heads 307 and 240 us.  Else only sequences of one workgroup
-// (single queries of a mixed batch) are.
+// one KV head, 188 workgroups: 538 us in one piece, 336 us in two; 16 heads x 3001 tokens on 4 KV heads 307 and 220 us.  Else only
+// sequences of one workgroup (single queries of a mixed batch) are.
 struct SplitPlan {
     int split_w, max_pieces;
 };

@@ -57,7 +57,7 @@ __device__ __forceinline__ int row_to_coord(int r) { return 16 * ((r >> 2) & 1) 
 // [K idx H*D/2 | K norm H*4 | V idx H*D/2 | V norm H*4], read where they are; row (t, h) of either lies
 // t * row_bytes + h * D/2 (norm: + 4 h) behind its section's start.  Bound by the launch's start and end (about 8 tiles
 // a workgroup) and then by HBM: 24,016 tokens x 8 heads of 128 in bf16 took 89 us as four strided copies of the
-// sections and a launch each for keys and values, 38 us this way (124 MB: 25 us at the rate of a plain copy).
+// sections and a launch each for keys and values, 40 us this way (124 MB: 25 us at the rate of a plain copy).
 struct DecRotSource {
     const uint8_t* packed;
     const float* norms;

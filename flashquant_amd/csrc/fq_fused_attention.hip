@@ -32,11 +32,12 @@
 // permutation on the coordinates, and the query operand is read to match.
 //
 // head_dim 256: tiles of 32 tokens (the accumulators of 32 rows, their query operand and the scores are 208 of a lane's
-// 256 registers), the second product in groups of two coordinate blocks, the rotation matrix in four rounds through LDS
-// (it is 256 KB in two terms).  Per flop the tile loop costs what it costs at 128: 2.6 us for 256 rows x 32 tokens, bound
-// like it by the chain K reads - scores - weights - V reads - output.  The general kernel (fq_attention_any_dim.hip), which
-// served this dimension with 16 rows a wavefront, read twice the LDS bytes per row: 16 heads x 3001 tokens fp16 516 -> 308 us,
-// 2 x 32 x 700 tokens bf16 260 -> 114 us, 16 x 65 tokens 93 -> 53 us; one query over 3 x 3500 tokens 369 -> 85 us (in pieces).
+// 256 registers, and 20 to 40 are spilled around the ends), the second product in groups of two coordinate blocks, the rotation
+// matrix in four rounds through LDS (it is 256 KB in two terms).  Per flop the tile loop costs what it costs at 128: 2.6 us for
+// 256 rows x 32 tokens, bound like it by the chain K reads - scores - weights - V reads - output.  The general kernel
+// (fq_attention_any_dim.hip), which served this dimension with 16 rows a wavefront, read twice the LDS bytes per row: 2 x 32 x
+// 700 tokens bf16 260 -> 110 us, 16 x 65 tokens 92 -> 51 us, 2 x 16 x 8192 tokens 4.11 -> 1.97 ms; in pieces 16 heads x 3001
+// tokens fp16 516 -> 220 us, one query over 3 x 3500 tokens 350 -> 57 us.
 //
 // The two head rotations run inside the kernel (prologue and epilogue) on the fp16 MFMA
 // with operands split into two fp16 terms, staged through the tile buffers.
@@ -263,7 +264,7 @@ __device__ __forceinline__ WorkItem find_item(const PrefillParams& p, int at, in
 //
 // What it replaced staged the rows through LDS for the 16x16x32 MFMA (16 to 32 lanes on a bank) and stored the
 // results 2 bytes a lane: a workgroup per CU on 64 tokens of 32 heads over 64 keys took 33 us and 27 us with one
-// query row, 24 and 15.5 us this way (the tile itself: 2 us); 4 x 32 heads x 8192 tokens 2.94 -> 2.77 ms.
+// query row, 24 and 15.5 us this way (the tile itself: 2 us); 4 x 32 heads x 8192 tokens 2.89 -> 2.81 ms.
 template <int D>
 struct RotationBlocks {
     using Cfg = PrefillCfg<D>;
@@ -964,7 +965,7 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
 
     // ---- a piece of a workgroup's keys: the rows as they are, for the combine launch ------------------------
     // Only rows that hold a query: a unit of one query left 31 rows of padding, 64 KB a piece at 4 heads of 128 (one query
-    // over 4 x 2500 tokens of a ring buffer 33.5 -> 30.2 us, a mixed batch of 12 sequences 381 -> 373 us).
+    // over 4 x 2500 tokens of a ring buffer 33.5 -> 30.2 us).
     if (WORK == kAllPieces || (WORK == kPieces && pieces > 1)) {
         const float l_piece = l_run + xor_shuffle(l_run, 32);
         if (!unit_live || pos0 + m32 >= NQ) return;
@@ -1004,7 +1005,7 @@ __device__ __forceinline__ float inverse_sum(float den) { return den == 0.0f ? 0
 // Rows of the workgroups that ran in pieces: the pieces' rows weighted by 2^(m - max m), summed and normalised, rounded
 // as the kernel above rounds, rotated back.  A workgroup takes `rows` (4 or 16) rows of a unit, a wavefront a row at a
 // time; blockIdx.x numbers the (sequence, KV head, workgroup) triples that may have been split, blockIdx.y their row
-// groups.  Bound by the launch and two round trips (partials and matrix are asked for together): about 6 us.
+// groups.  Bound by the launch and two round trips (partials and matrix are asked for together): 5.6 us.
 template <int D, int DT, bool PAGED>
 __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillParams p, int rows) {
     using Cfg = PrefillCfg<D>;
@@ -1126,10 +1127,10 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillPar
 
 // The same for whole prompts in pieces, where the rotation is the work: a workgroup as the one that left the pieces, its
 // wavefronts gather their 32 rows in the accumulators and end as that kernel does (the kernel above fetches and splits the
-// matrix for every 16 rows).  16 heads x 3001 tokens of 256 coordinates, 188 workgroups in two pieces: 298 us with the kernel
-// above, 240 with this one; 8 heads x 5000 tokens of 128, 157 workgroups: 140 and 121; 16 heads x 2000 tokens of 64, 128
-// workgroups: 54.6 and 48.3.  With 63 workgroups in four pieces the smaller workgroups above are faster (128 and 148 us at 256
-// coordinates, 55 and 68 at 128): this one runs from half a round of workgroups on.
+// matrix for every 16 rows).  When it was added, 16 heads x 3001 tokens of 256 coordinates, 188 workgroups in two pieces: 298 us
+// with the kernel above, 240 with this one (220 now); 8 heads x 5000 tokens of 128, 157 workgroups: 140 and 121; 16 heads x
+// 2000 tokens of 64, 128 workgroups: 54.6 and 48.3 (45.8 now).  With 63 workgroups in four pieces the smaller workgroups above
+// are faster (128 and 148 us at 256 coordinates, 55 and 68 at 128): this one runs from half a round of workgroups on.
 template <int D, int DT, bool PAGED>
 __global__ __launch_bounds__(512) void attention_combine_prompts_kernel(const PrefillParams p) {
     using Cfg = PrefillCfg<D>;

@@ -142,8 +142,8 @@ __global__ __launch_bounds__(256) void prod_compress_kernel(
 // One wavefront per token: its row [K nibbles | K norm | K residual norm | V idx | V norm] assembled from the five
 // operands and written where its slot says, 4 bytes a lane (W = uint32_t; single bytes where the cache, its row stride
 // or an operand is not aligned to 4).  Bound by the launch at a decode step's size and by HBM beyond it.  As torch
-// copies into a row buffer and an indexed store it was six launches and twice the bytes: 8 tokens of 8 heads 30 us,
-// one launch 4 us.  `kw`, `nw`: units of one index section and of one section of norms.
+// copies into a row buffer and an indexed store it was six launches and twice the bytes: a generated token of 8 sequences
+// with its attention 207.7 us, 192.5 with this launch of 5 us.  `kw`, `nw`: units of one index section and of one section of norms.
 template <typename W>
 __global__ __launch_bounds__(256) void prod_store_rows_kernel(
     W* __restrict__ cache, const int64_t* __restrict__ slots, const W* __restrict__ k_packed, const W* __restrict__ k_norms,

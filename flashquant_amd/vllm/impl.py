@@ -105,8 +105,9 @@ def _make_impl_class() -> type:
 
         Where the reference decompresses the whole cache and hands it to a FlashAttention library
         (src/flashquant/vllm/impl.py:395-512), a batch of single-token queries runs the split-K paged
-        decode and everything else the paged prefill, both reading the packed pages; neither
-        allocates, so a decode step can be captured in a graph."""
+        decode and everything else the paged prefill, both reading the packed pages.  Their scratch
+        memory (split partials; of the prefill at most 65 MiB) comes from torch's caching
+        allocator, so either can be captured in a graph."""
 
         def __init__(self, *args, **kwargs) -> None:
             super().__init__(*args, **kwargs)

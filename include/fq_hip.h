@@ -239,7 +239,7 @@ int fq_tq4_decompress_rotated(const uint8_t* packed, const float* norms, const f
  * product with the rotation).
  *   kv_cache   (num_slots, H*(D+8)) u8 token rows; num_slots = num_blocks * block_size
  *   rotation   (D, D) f32, or NULL: the output stays in rotated space
- *   out_k/v    (num_slots, H, D) out_dtype (FQ_F32 only without rotation), 16-byte aligned
+ *   out_k/v    (num_slots, H, D) out_dtype (FQ_F32 only without rotation), 16-byte aligned; H at most 2^20
  */
 int fq_tq4_decompress_cache(const uint8_t* kv_cache, const float* centroids, const float* rotation, int rotation_col_major,
                             void* out_k, void* out_v, int out_dtype, int64_t num_slots, int H, int D, void* stream);
@@ -324,9 +324,11 @@ int fq_paged_tq4_prefill(const void* q, const int32_t* cu_seqlens_q, const uint8
 /*
  * The two operators above with a workspace.  Where a batch has long contexts for its few queries (a single query over a
  * ring buffer, the decode steps of a mixed batch, the chunks of a few prompts) its keys are cut into pieces that run on
- * different CUs, and a second launch combines their results (rounded as the unsplit result is).
- *   workspace        256-byte aligned, at least fq_attention_workspace_bytes bytes (0: these sizes are never split);
- *                    NULL: nothing is split
+ * different CUs, and a second launch combines their results (rounded as the unsplit result is; rows that are no numbers in
+ * one piece are none in several).  The pieces follow from the whole batch, the longest context possible and the number of
+ * CUs: the last bits of a row may differ with the batch that it is in.
+ *   workspace        256-byte aligned, at least fq_attention_workspace_bytes bytes (0: these sizes are never split; at
+ *                    most 65 MiB paged, 172 MiB for whole prompts); NULL: nothing is split
  *   max_kv_len       the longest context possible: N_KV, or max_blocks_per_seq * block_size
  *   prompts          1: for fq_fused_tq_attention_split with is_causal (all sequences have these very lengths), else 0
  *   total_q          cu_seqlens_q[num_seqs] where the caller knows it (sizes the grid), else 0
@@ -335,21 +337,21 @@ size_t fq_attention_workspace_bytes(int num_seqs, int max_q_len, int64_t max_kv_
                                     int prompts);
 
 int fq_fused_tq_attention_split(const void* q, const uint8_t* k_packed, const float* k_norms,
-                                  const uint8_t* v_packed, const float* v_norms,
-                                  const float* centroids_k, const float* centroids_v,
-                                  const float* rotation, int rotation_col_major, void* out,
-                                  int B, int H_Q, int H_KV, int N_Q, int N_KV,
-                                  int64_t k_capacity, int64_t v_capacity, int D,
-                                  float sm_scale, int is_causal, int dtype, void* workspace,
+                                const uint8_t* v_packed, const float* v_norms,
+                                const float* centroids_k, const float* centroids_v,
+                                const float* rotation, int rotation_col_major, void* out,
+                                int B, int H_Q, int H_KV, int N_Q, int N_KV,
+                                int64_t k_capacity, int64_t v_capacity, int D,
+                                float sm_scale, int is_causal, int dtype, void* workspace,
                                 size_t workspace_bytes, void* stream);
 
 int fq_paged_tq4_prefill_split(const void* q, const int32_t* cu_seqlens_q, const uint8_t* kv_cache,
-                         const int32_t* block_table, const int32_t* seq_lens,
-                         const float* centroids_k, const float* centroids_v,
-                         const float* rotation, int rotation_col_major, void* out,
-                         int num_seqs, int max_q_len, int H_Q, int H_KV, int D, int block_size,
-                         int max_blocks_per_seq, int64_t num_blocks, float sm_scale, int is_causal,
-                         int dtype, int64_t total_q, void* workspace, size_t workspace_bytes, void* stream);
+                               const int32_t* block_table, const int32_t* seq_lens,
+                               const float* centroids_k, const float* centroids_v,
+                               const float* rotation, int rotation_col_major, void* out,
+                               int num_seqs, int max_q_len, int H_Q, int H_KV, int D, int block_size,
+                               int max_blocks_per_seq, int64_t num_blocks, float sm_scale, int is_causal,
+                               int dtype, int64_t total_q, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * Split-K paged decode from the packed TQ4 cache, un-rotated query in,
