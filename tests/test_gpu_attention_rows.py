@@ -428,3 +428,30 @@ def test_paged_prefill_under_a_wide_table(batch, hq, hkv, d):
     keyless = torch.cat([torch.full((n,), m == 0) for n, m in zip(ql, kv)])
     assert (got.cpu()[keyless] == 0).all()
     _rows_close(got.cpu()[~keyless], want[~keyless], 4 * 2 ** -8)
+
+
+def test_paged_attention_under_capture_with_other_lengths():
+    """One captured call: the pieces follow from the lengths that each replay finds on the device."""
+    hq, hkv, d, bs, dtype = 16, 4, 128, 16, torch.bfloat16
+    kv, ql = [3000, 900, 2500, 60], [1, 40, 200, 5]
+    c, _, r = book(d)
+    _, cache, table, sl = build_paged_case(kv, hq, hkv, d=d, bs=bs, seed=131, dtype=dtype)
+    q = torch.randn(sum(ql), hq, d, generator=torch.Generator().manual_seed(132)).to(dtype).to(DEV)
+    cu = torch.tensor([0] + list(torch.tensor(ql).cumsum(0)), dtype=torch.int32).to(DEV)
+    sl = sl.to(DEV)
+    out = torch.zeros_like(q)
+    args = (cu, max(ql), cache.to(DEV), table.to(DEV), sl, c.to(DEV), c.to(DEV), r.to(DEV), hkv, d, bs)
+    K.paged_tq4_prefill(q, *args, out=out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        K.paged_tq4_prefill(q, *args, out=out)
+    for lens in (kv, [200, 900, 200, 5], [3000, 40, 2400, 60], [1, 41, 201, 6], kv):
+        sl.copy_(torch.tensor(lens, dtype=torch.int32))
+        eager = K.paged_tq4_prefill(q, *args)
+        out.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+        want = O.paged_prefill(q.cpu(), cu.cpu(), cache, table, sl.cpu(), c, c, r, hkv, d, bs)
+        _rows_close(out, want, 4 * 2 ** -8)
