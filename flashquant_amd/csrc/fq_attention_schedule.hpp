@@ -87,15 +87,15 @@ FQ_HD int first_with(const SeqShape& s, int T, int G, bool causal) {
 }
 
 // What splitting saves and costs, in ns: a tile of 64 keys of the longest workgroup; what a sequence's rows cost in the combine
-// however few they are; a piece of 256 rows, written and read.  Fitted on 1775 paged batches of equal sequences (1, 3 and 8
+// however few they are; 256 rows that are combined, and each of their pieces, written and read.  Fitted on 1775 paged batches of equal sequences (1, 3 and 8
 // of them, 1 to 1000 queries over 400 to 4000 keys, four head counts), each run in pieces and in one: with 33 queries and more
 // the combine took 3 and 5 us up to 16 workgroups' worth of pieces and 8 and 17 us at 128 (64 and 128 coordinates).  At 256
 // pieces won in all of them: the rows go through the combine there whether they are split or not.
 struct SplitCost {
-    int tile, fixed, slot;
+    int tile, fixed, rows, piece;
 };
 FQ_HD SplitCost split_cost(int D) {
-    return D == 64 ? SplitCost{1400, 3000, 45} : (D == 128 ? SplitCost{2100, 5000, 80} : SplitCost{5200, 0, 0});
+    return D == 64 ? SplitCost{1400, 3000, 60, 15} : (D == 128 ? SplitCost{2100, 5000, 20, 70} : SplitCost{5200, 0, 0, 0});
 }
 
 // What the pieces of a batch follow from: the tiles of a CU's share of all work, and the rows that may have to be combined,
@@ -115,7 +115,7 @@ FQ_HD int pieces_of(const SeqShape& s, const BatchWork& b, int split_w, int max_
     n = n < max_pieces ? n : max_pieces;
     if (n < 2) return 1;
     const SplitCost c = split_cost(D);
-    if (s.NQ > 16 && int64_t(c.tile) * tiles * (n - 1) <= int64_t(n) * (c.fixed + int64_t(c.slot) * b.slots * n)) return 1;
+    if (s.NQ > 16 && int64_t(c.tile) * tiles * (n - 1) <= int64_t(n) * (c.fixed + int64_t(b.slots) * (c.rows + c.piece * n))) return 1;
     return n;
 }
 
