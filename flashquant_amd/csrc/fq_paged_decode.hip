@@ -728,10 +728,18 @@ __global__ __launch_bounds__(512 + 64 * CW) void paged_decode_staged_kernel(cons
     // out, [3 + s] tiles written to slot s (one count per copy wavefront and tile), [5 + s] tiles read
     // from slot s (one count per computing wavefront and tile)
     // STORE: [7] computing wavefronts whose part of the new token's row has reached the cache
-    __shared__ uint32_t flags[8];
+    // [8] query and new-token rows staged
+    __shared__ uint32_t flags[9];
     // D256: [h] score halves posted by wavefront h, [8 + h] partner halves read by wavefront h (counts of tiles)
     // LINEAR: [16] computing wavefronts that have posted their partial for the merge at the end
     __shared__ uint32_t xflags[17];
+    // The first 32 query heads and the new token's rows (16 at most) as loaded, for the rotation: every computing wavefront
+    // needs all of them as operands, and fetches a part.  Each fetching all of them was most of the requests of the
+    // prologue, and the matrix columns and the first tiles waited behind them: one sequence of 777 tokens, 32 heads over 8,
+    // 19.2 -> 17.6 us, 24 sequences of 200 to 4000 at head_dim 64 27.7 -> 26.7.
+    constexpr int kQBytes = 2 * (D64 ? 64 : 128), kQStride = kQBytes + 16, kNewStride = 256 + 16;
+    constexpr int kQStage = D256 ? 0 : 32 * kQStride, kNewStage = STORE ? 16 * kNewStride : 0;
+    __shared__ __attribute__((aligned(16))) uint8_t stage[kQStage + kNewStage + 16];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -900,15 +908,31 @@ __global__ __launch_bounds__(512 + 64 * CW) void paged_decode_staged_kernel(cons
             return (v >> 6) == row_sub ? x : uint4v{0u, 0u, 0u, 0u};
         }
     };
-    uint4v q_pre[2][4];
+    // this wavefront's part of the rows that go through `stage`: 16 bytes a lane of each kind
+    uint4v q_part = {0u, 0u, 0u, 0u}, new_part = {0u, 0u, 0u, 0u};
+    constexpr int kPerRow = kQBytes / 16, kParts = 32 * kPerRow;
     auto load_first_heads = [&]() {
+        if (p.rotation != nullptr && !copier && tid < kParts) {
+            const int row = tid / kPerRow < HQG ? tid / kPerRow : HQG - 1;
+            q_part = *reinterpret_cast<const uint4v*>(qseq + row * (kQBytes / 2) + 8 * (tid % kPerRow));
+        }
+    };
+    auto stage_rows = [&]() {
         if (p.rotation != nullptr && !copier) {
-#pragma unroll
-            for (int rb = 0; rb < 2; ++rb) {
-                const int row = 16 * rb + n < HQG ? 16 * rb + n : HQG - 1;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) q_pre[rb][j] = q_chunk(row, 32 * j + 8 * g);
-            }
+            if (tid < kParts) *reinterpret_cast<uint4v*>(stage + (tid / kPerRow) * kQStride + 16 * (tid % kPerRow)) = q_part;
+            if (STORE && tid < 256) *reinterpret_cast<uint4v*>(stage + kQStage + (tid >> 4) * kNewStride + 16 * (tid & 15)) = new_part;
+            if constexpr (CW > 0) lds_flag_signal(&flags[8], lane);
+        }
+    };
+    // eight elements, from element v, of staged query row `row` (as q_chunk)
+    auto staged_chunk = [&](int row, int v) -> uint4v {
+        if constexpr (!D64) {
+            return *reinterpret_cast<const uint4v*>(stage + row * kQStride + 2 * v);
+        } else {
+            const int in_group = row - (row / p.G) * p.G;
+            const int row_sub = in_group >= p.G / 2 ? 1 : 0;
+            const uint4v x = *reinterpret_cast<const uint4v*>(stage + row * kQStride + 2 * (v & 63));
+            return (v >> 6) == row_sub ? x : uint4v{0u, 0u, 0u, 0u};
         }
     };
     if constexpr (CW == 0) load_first_heads();
@@ -934,30 +958,29 @@ __global__ __launch_bounds__(512 + 64 * CW) void paged_decode_staged_kernel(cons
         // The flags are cleared behind a barrier placed where nobody waits for anybody: every
         // wavefront has just asked for its sequence length and page ids and none has used them yet
         // (the barrier does not wait for loads from global memory).
-        if (tid < 8) flags[tid] = 0u;
+        if (tid < 9) flags[tid] = 0u;
         if ((D256 || LINEAR) && tid < 17) xflags[tid] = 0u;
         __syncthreads();
-        load_matrix_columns();
         load_first_heads();
     }
     // STORE: the new token's rows and slot are asked for with the other prologue loads, by every workgroup
     // (which one needs them depends on the sequence length, which is on its way)
     constexpr int kNewHeads = HPR;                          // KV heads of this workgroup
-    uint4v new_raw[4];
     int64_t new_slot = -1;
     float bnd_mine = 0.0f;      // boundary `lane` of the 15 (asked for here: at its use it would be a round trip of its own)
     if constexpr (STORE) {
         if (!copier) {
             const int kv_heads = MULTI > 0 ? HPR : p.H_KV;       // (head_dim 64: pairs of heads, 128 elements together)
-            const int nr = n < 2 * kNewHeads ? n : 2 * kNewHeads - 1;     // block row: key head nr, or value head nr - KH
+            // block row: key head nr, or value head nr - KH; 16 lanes a row
+            const int nr = (tid >> 4) < 2 * kNewHeads ? tid >> 4 : 2 * kNewHeads - 1;
             const uint16_t* xrow = reinterpret_cast<const uint16_t*>(nr < kNewHeads ? p.new_key : p.new_value) +
                                    (int64_t(seq) * kv_heads + kNewHeads * hgrp + (nr & (kNewHeads - 1))) * 128;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) new_raw[j] = *reinterpret_cast<const uint4v*>(xrow + 32 * j + 8 * g);
+            if (tid < 256) new_part = *reinterpret_cast<const uint4v*>(xrow + 8 * (tid & 15));
             new_slot = p.new_slots[seq];
             bnd_mine = p.boundaries[lane < 15 ? lane : 14];
         }
     }
+    if constexpr (CW > 0) load_matrix_columns();
     L = L < 0 ? 0 : L;
     L = L > p.max_blocks * BS * TPR ? p.max_blocks * BS * TPR : L;
     // MULTI > 0: from here on L counts rows (of TPR tokens); the last row may hold no token of this wavefront
@@ -1004,7 +1027,7 @@ __global__ __launch_bounds__(512 + 64 * CW) void paged_decode_staged_kernel(cons
     };
     // the table is filled while the page ids are on their way
     if (!copier) fill_pair_tables<8>(lut, cent_k_mine, cent_v_mine, PROD ? 7 : 15, h, lane);
-
+    stage_rows();
 
     uint4v stage_reg[ROUNDS];
     auto issue_loads = [&](int t0) {
@@ -1199,12 +1222,17 @@ __global__ __launch_bounds__(512 + 64 * CW) void paged_decode_staged_kernel(cons
                 split_rotation_block<D>(rot_b, rot_hi, rot_lo);
                 if constexpr (PROD) split_rotation_block<D>(rot_s, sk_hi, sk_lo);
             }
+            if constexpr (CW > 0) {
+                if (!lds_flag_wait(&flags[8], 8u, p.spin_limit)) { flags[2] = 1u; handoff_failed = true; }
+            } else {
+                __syncthreads();
+            }
             for (int rb = 0; 16 * rb < HQG; ++rb) {
                 const int row = 16 * rb + n < HQG ? 16 * rb + n : HQG - 1;
                 uint4v raw[KS];
 #pragma unroll
                 for (int j = 0; j < KS; ++j)
-                    raw[j] = rb < 2 ? q_pre[rb & 1][j] : q_chunk(row, 32 * j + 8 * g);
+                    raw[j] = rb < 2 ? staged_chunk(row, 32 * j + 8 * g) : q_chunk(row, 32 * j + 8 * g);
                 float4v acc, acc2 = {0.f, 0.f, 0.f, 0.f};
                 float up = 1.0f;
                 if constexpr (kRawBf16) {
@@ -1245,7 +1273,7 @@ __global__ __launch_bounds__(512 + 64 * CW) void paged_decode_staged_kernel(cons
                     const int64_t slot = new_slot;
                     uint4v raw[KS];
 #pragma unroll
-                    for (int j = 0; j < KS; ++j) raw[j] = new_raw[j];
+                    for (int j = 0; j < KS; ++j) raw[j] = *reinterpret_cast<const uint4v*>(stage + kQStage + n * kNewStride + 64 * j + 16 * g);
                     // sum of squares of row n: this lane's 32 elements, then over g.  head_dim 64: a row is a pair of heads,
                     // elements 0..63 the first and 64..127 the second; wavefront h holds columns of head h / 4 of the pair
                     float ss = 0.0f;
