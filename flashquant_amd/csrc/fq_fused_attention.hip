@@ -145,7 +145,13 @@ __device__ __forceinline__ uint32_t wave_add(uint32_t v) {
 // The sequences s0 + lane as the lanes of a wavefront hold them; empty ones past the end.
 template <bool PAGED>
 __device__ __forceinline__ SeqShape lane_shape(const PrefillParams& p, int s0, int lane) {
-    return s0 + lane < p.num_seqs ? seq_shape<PAGED>(p, s0 + lane) : make_seq_shape(0, 0, 0, p.G, 0);
+    // (no branch around the loads: the caller has other requests to send before it needs them)
+    const bool some = s0 + lane < p.num_seqs;
+    SeqShape sh = seq_shape<PAGED>(p, some ? s0 + lane : p.num_seqs - 1);
+    sh.NQ = some ? sh.NQ : 0;
+    sh.NKV = some ? sh.NKV : 0;
+    sh.qoff = some ? sh.qoff : 0;
+    return make_seq_shape(sh.NQ, sh.NKV, sh.qoff, p.G, some ? p.max_w : 0);
 }
 
 // The share of a CU of the whole batch (all KV heads), in tiles, and the rows of the sequences that may be split.  The sums
@@ -187,19 +193,26 @@ __device__ __forceinline__ void note_pieces(const PrefillParams& p, const SeqSha
     if (threadIdx.x == 0) p.left[at] = n > 1 || p.all_in_part ? n : 0;
 }
 
-// The item of a place (`at` / H_KV, of one KV head) in the order longest piece first: the largest tile count T that more than
-// `place` pieces reach, by bisection with a lane per sequence; then the place among the pieces of exactly T.  Beyond
-// kOrderSeqs sequences the items in the order of the sequences (kOrderSeqs says why).
-// SPLIT: `at` is the workgroup's number in the launch.
+// The item of a place (`at` / H_KV, of one KV head) in the order longest piece first.  Sequences of one shape: the workgroups
+// of all of them from the last one down.  Else the largest tile count T that more than `place` pieces reach, a lane per
+// sequence, three counts at a time (they do not wait for one another) between 0 and the longest context; then the place among
+// the pieces of exactly T.  Beyond kOrderSeqs sequences the items in the order of the sequences (kOrderSeqs says why).
+// SPLIT: `at` is the workgroup's number in the launch.  `first`: the first wavefront's worth of sequences.
 template <int D, bool PAGED, bool SPLIT>
-__device__ __forceinline__ WorkItem find_item(const PrefillParams& p, int at, int lane) {
+__device__ __forceinline__ WorkItem find_item(const PrefillParams& p, int at, const SeqShape& first, int lane) {
     const int G = p.G, place = at / p.H_KV;
     const bool causal = p.causal != 0;
+    if constexpr (!PAGED) {
+        const int per = p.num_seqs * (SPLIT ? p.max_pieces : 1), down = place / per, rest = place % per;
+        const int W = seq_shape<PAGED>(p, 0).W;
+        if (down >= W) return WorkItem{-1, 0, 0, 1};
+        if (!SPLIT) return WorkItem{rest, W - 1 - down, 0, 1};
+        return WorkItem{rest / p.max_pieces, W - 1 - down, rest % p.max_pieces, p.max_pieces};
+    }
     if (PAGED && p.dense) {
         const int seq = place / p.max_w, x = p.max_w - 1 - place % p.max_w;
         return seq < p.num_seqs && x < seq_shape<PAGED>(p, seq).W ? WorkItem{seq, x, 0, 1} : WorkItem{-1, 0, 0, 1};
     }
-    const SeqShape first = lane_shape<PAGED>(p, 0, lane);
     // (the lengths of the batch are only summed where a sequence is long enough for the shortest pieces)
     BatchWork batch{kSplitMinTiles, 0};
     if (PAGED && SPLIT && (p.num_seqs > kWave || __any(may_split(first, p.split_w, p.max_pieces, G, causal, D))))
@@ -208,27 +221,37 @@ __device__ __forceinline__ WorkItem find_item(const PrefillParams& p, int at, in
     auto shape = [&](int s0) { return s0 == 0 ? first : lane_shape<PAGED>(p, s0, lane); };
     const int first_pieces = SPLIT ? pieces_in<D, PAGED>(p, first, batch) : 1;
     auto pieces = [&](int s0, const SeqShape& sh) { return s0 == 0 || !SPLIT ? first_pieces : pieces_in<D, PAGED>(p, sh, batch); };
-    auto count = [&](int T) {
-        uint32_t c = 0;
+    struct Counts { int c[3]; };
+    auto count = [&](int t0, int t1, int t2) {           // pieces of at least so many tiles
+        uint32_t c0 = 0, c1 = 0, c2 = 0;
         for (int s0 = 0; s0 < p.num_seqs; s0 += kWave) {
             const SeqShape sh = shape(s0);
             const int n = pieces(s0, sh);
-            c += uint32_t(n * (sh.W - first_piece_with(sh, T, n, G, causal)));
+            c0 += uint32_t(n * (sh.W - first_piece_with(sh, t0, n, G, causal)));
+            c1 += uint32_t(n * (sh.W - first_piece_with(sh, t1, n, G, causal)));
+            c2 += uint32_t(n * (sh.W - first_piece_with(sh, t2, n, G, causal)));
         }
-        return int(wave_add(c));
+        return Counts{{int(wave_add(c0)), int(wave_add(c1)), int(wave_add(c2))}};
     };
     WorkItem item{-1, 0, 0, 1};
     int lo = 0, hi = 0x3fffffff, rem = place;            // tile counts lo .. hi - 1 (no sequence has 2^30 tiles)
-    if (!PAGED || p.num_seqs <= kOrderSeqs) {
-        if (place >= count(0)) return item;
-        hi = 1;                                          // count(lo) > place >= count(hi)
-        while (count(hi) > place) { lo = hi; hi *= 2; }
+    if (p.num_seqs <= kOrderSeqs) {
+        float most = 0.0f;                               // (rounded up past 2^24)
+        for (int s0 = 0; s0 < p.num_seqs; s0 += kWave) most = __builtin_fmaxf(most, float(shape(s0).all_tiles));
+        hi = __builtin_amdgcn_readfirstlane(int(wave_max(most) * 1.000001f)) + 1;
+        int at_hi = 0;                                   // count(lo) > place >= count(hi)
+        if (place >= count(0, 0, 0).c[0]) return item;
         while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (count(mid) > place) lo = mid;
-            else hi = mid;
+            const int m1 = (lo + hi) >> 1, m0 = (lo + m1) >> 1, m2 = (m1 + hi) >> 1;
+            const Counts c = count(m0, m1, m2);
+            const int below = c.c[1] > place ? 2 : 0;    // which half, then which quarter
+            const int mid = c.c[1] > place ? m2 : m0, at_mid = c.c[below];
+            if (c.c[1] > place) lo = m1;
+            else { hi = m1; at_hi = c.c[1]; }
+            if (at_mid > place) lo = mid;
+            else { hi = mid; at_hi = at_mid; }
         }
-        rem = place - count(hi);
+        rem = place - at_hi;
     }
     for (int s0 = 0; s0 < p.num_seqs; s0 += kWave) {
         const SeqShape sh = shape(s0);
@@ -269,9 +292,11 @@ template <int D>
 struct RotationBlocks {
     using Cfg = PrefillCfg<D>;
     static constexpr int NKS = Cfg::NKS, RBLK = Cfg::RBLK, BPW = RBLK * NKS / 8;
+    static constexpr int RROUNDS = Cfg::RROUNDS;
     const float* rotation;
     bool col_major;
-    uint8_t* share;               // 2 x RTERM bytes of LDS
+    uint8_t* share;               // 2 x RTERM bytes of LDS: the last round's operands, and every second one's before it
+    uint8_t* other;               // as many again for the rounds between (unused with one round)
     int w, lane, m32, hf;
     float rbv[BPW][8];
     // `back`: x @ R with the contraction index in the order of the accumulator registers (element 4 a + c of half
@@ -292,17 +317,57 @@ struct RotationBlocks {
             }
         }
     }
-    __device__ __forceinline__ void put() {
+    __device__ __forceinline__ uint8_t* at(int round) const { return ((RROUNDS - 1 - round) & 1) == 0 ? share : other; }
+    __device__ __forceinline__ void put(int round) {
+        uint8_t* dst = at(round);
         half8 rhi[BPW], rlo[BPW];
         split_rotation_block<32 * BPW>(rbv, rhi, rlo);
 #pragma unroll
         for (int i = 0; i < BPW; ++i) {
-            *reinterpret_cast<half8*>(share + ((BPW * w + i) * 64 + lane) * 16) = rhi[i];
-            *reinterpret_cast<half8*>(share + Cfg::RTERM + ((BPW * w + i) * 64 + lane) * 16) = rlo[i];
+            *reinterpret_cast<half8*>(dst + ((BPW * w + i) * 64 + lane) * 16) = rhi[i];
+            *reinterpret_cast<half8*>(dst + Cfg::RTERM + ((BPW * w + i) * 64 + lane) * 16) = rlo[i];
         }
     }
-    __device__ __forceinline__ half8 term(int t, int jb, int ks) const {
-        return *reinterpret_cast<const half8*>(share + t * Cfg::RTERM + ((jb * NKS + ks) * 64 + lane) * 16);
+    // The products of a round with this wavefront's 32 rows (`a`, and with ROWS_LO `alo`, 2^12 times what `a` leaves of
+    // them); done(block of the round, high sums, low sums times 2^12).  The matrix operands are read two groups of two k-steps
+    // (one at 256 coordinates, where registers are few) ahead of their products: the compiler on its own reads one product
+    // ahead.  The fences hold LDS reads and products in this order and let the vector instructions of the block before pass.
+    // Bound by LDS: eight wavefronts read the 64 KB of a round each, 3.4 us at the 150 bytes a ns that a CU's LDS gives here.
+    template <bool ROWS_LO, class Done>
+    __device__ __forceinline__ void products(int round, const half8 (&a)[NKS], const half8 (&alo)[NKS], const Done& done) const {
+        constexpr int GK = D == 256 ? 1 : 2, GROUPS = NKS / GK, ALL = RBLK * GROUPS, kFence = 0x76;
+        const uint8_t* src = at(round) + 16 * lane;
+        half8 t[ALL][2][GK];
+        auto read = [&](int g) {
+#pragma unroll
+            for (int k = 0; k < GK; ++k)
+#pragma unroll
+                for (int term = 0; term < 2; ++term)
+                    t[g][term][k] = *reinterpret_cast<const half8*>(src + term * Cfg::RTERM + (GK * g + k) * 1024);
+        };
+        read(0);
+        read(1);
+        __builtin_amdgcn_sched_barrier(kFence);
+        float16v hi, lo;
+#pragma unroll
+        for (int g = 0; g < ALL; ++g) {
+            if (g + 2 < ALL) {
+                read(g + 2);
+                __builtin_amdgcn_sched_barrier(kFence);
+            }
+            if (g % GROUPS == 0)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) { hi[r] = 0.0f; lo[r] = 0.0f; }
+#pragma unroll
+            for (int k = 0; k < GK; ++k) {
+                const int ks = GK * (g % GROUPS) + k;
+                hi = __builtin_amdgcn_mfma_f32_32x32x16_f16(t[g][0][k], a[ks], hi, 0, 0, 0);
+                lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(t[g][1][k], a[ks], lo, 0, 0, 0);
+                if (ROWS_LO) lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(t[g][0][k], alo[ks], lo, 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(kFence);
+            if (g % GROUPS == GROUPS - 1) done(g / GROUPS, hi, lo);
+        }
     }
 };
 
@@ -323,6 +388,7 @@ __device__ __forceinline__ void finish_rows(const PrefillParams& p, RotationBloc
     constexpr int NKS = Cfg::NKS, NOB = Cfg::NOB, RROUNDS = Cfg::RROUNDS, RBLK = Cfg::RBLK;
     const int m32 = rot.m32, hf = rot.hf;
     if (RROUNDS == 1 && !unit_live) return;
+    if (RROUNDS > 1) rot.fetch(true, 1);
     // float32 rows: both operands as two fp16 terms, three MFMA terms; rows already rounded to 16 bits (the paged form) in
     // one, the row's largest value brought into [2^14, 2^15): what is above 2^-28 of it is exact, the rest to 2^-39 of it (a
     // largest value in [1, 2) left the coordinates below 2^-14 of it among fp16's subnormals)
@@ -356,26 +422,12 @@ __device__ __forceinline__ void finish_rows(const PrefillParams& p, RotationBloc
     uint16_t* obase = PAGED ? p.out + (q_row0 + hq) * D : p.out + (q_row0 + int64_t(hq) * NQ) * D;
     uint16_t* orow = obase + int64_t(opos) * q_stride;
 #pragma unroll
-    for (int cb = 0; cb < NOB; ++cb) {
-        const int cr = cb % RBLK;                      // within the round
-        if (RROUNDS > 1 && cr == 0) {
-            if (cb > 0) {
-                __syncthreads();
-                rot.put();
-                __syncthreads();
-            }
-            if (cb + RBLK < NOB) rot.fetch(true, cb / RBLK + 1);
-        }
-        float16v hi, lo;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) { hi[r] = 0.0f; lo[r] = 0.0f; }
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) {
-            const half8 rh = rot.term(0, cr, ks);
-            hi = __builtin_amdgcn_mfma_f32_32x32x16_f16(rh, ohi[ks], hi, 0, 0, 0);
-            lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(rot.term(1, cr, ks), ohi[ks], lo, 0, 0, 0);
-            if (!PAGED) lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(rh, olo[ks], lo, 0, 0, 0);
-        }
+    for (int round = 0; round < RROUNDS; ++round) {
+        if (round > 0) __syncthreads();                // this round's operands are there, the ones before are done with
+        if (round + 1 < RROUNDS) rot.put(round + 1);
+        if (round + 2 < RROUNDS) rot.fetch(true, round + 2);
+        rot.template products<!PAGED>(round, ohi, olo, [&](int cr, const float16v& hi, const float16v& lo) {
+        const int cb = RBLK * round + cr;
         // registers 4 q + c of half hf = coordinate 32 cb + 8 q + 4 hf + c; the halves exchange a quad of every two,
         // so that a lane stores eight neighbours at a time
         uint32_t wd[8];
@@ -403,6 +455,7 @@ __device__ __forceinline__ void finish_rows(const PrefillParams& p, RotationBloc
                 }
             }
         }
+        });
     }
 }
 
@@ -447,10 +500,21 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     // slow, and the position order reversed in every other round over the chip: whichever way the
     // rounds land on the CUs, each CU sees long and short workgroups alternate.
     int b, hkv, wg, piece = 0, pieces = 1;
+    // What does not depend on the workgroup's work is asked for before it looks for it.  The start of a workgroup is one serial
+    // chain (its work, the query rows, the rotation, the first tile); with the matrix fetched under the search, its operands
+    // where the tiles will be, so that the tables are filled meanwhile, and wavefronts without a unit out of the
+    // products, the first tile of one query over 4 x 2500 ring-buffer tokens begins after 6.5 us instead of 9.7 (24.3 -> 21.9 us
+    // in all), 16 heads x 3001 tokens of 256 coordinates 219 -> 208 us.
+    SeqShape first{};
+    if constexpr (kFind) first = lane_shape<PAGED>(p, 0, lane);
+    const float cent_k = p.centroids_k[lane & 15], cent_v = p.centroids_v[lane & 15];
+    constexpr int RROUNDS = Cfg::RROUNDS, RBLK = Cfg::RBLK;
+    RotationBlocks<D> rot{p.rotation, p.rot_col_major != 0, bufs, reinterpret_cast<uint8_t*>(lut), w, lane, m32, hf, {}};
+    rot.fetch(false, 0);
     if constexpr (kFind) {
         // the KV heads of a place are neighbours: each XCD serves few of them
         const int at = int(blockIdx.x + gridDim.x * blockIdx.y);
-        const WorkItem it = find_item<D, PAGED, kSplit>(p, at, lane);
+        const WorkItem it = find_item<D, PAGED, kSplit>(p, at, first, lane);
         if (it.seq < 0) return;                            // the grid is sized for the most work possible
         b = it.seq; hkv = at % p.H_KV; wg = it.x; piece = it.piece; pieces = it.pieces;
     } else {
@@ -510,8 +574,8 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     }
     if (!unit_live) my_tiles = 0;
 
-    // ---- tables: filled after the query stage, whose rotation operands use their place ----------
-    static_assert(2 * Cfg::RTERM <= int(sizeof(lut)), "the rotation operands fit where the tables are");
+    static_assert(2 * Cfg::RTERM <= int(sizeof(lut)) && 2 * Cfg::RTERM <= 2 * kPfBufBytes,
+                  "the rotation operands fit where the tiles are, and at 256 coordinates every second round's where the tables are");
     // cleared here: the barriers of the query stage order this before the first dequantisation
     if (tid < 2) big_tile[tid] = 0;
     if (tid < 256) (&scale_exp[0][0])[tid] = 0;
@@ -679,11 +743,6 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
         }
     };
 
-    issue_loads(first_tile);
-
-    constexpr int RROUNDS = Cfg::RROUNDS, RBLK = Cfg::RBLK;
-    RotationBlocks<D> rot{p.rotation, p.rot_col_major != 0, reinterpret_cast<uint8_t*>(lut), w, lane, m32, hf, {}};
-
     // ---- query: rotate this wavefront's 32 rows, round to the query dtype, scale to fp16 ----------
     half8 qb[NKS];
     float krow = 0.0f;
@@ -694,7 +753,12 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks)
             raw[ks] = *reinterpret_cast<const uint4v*>(qbase + int64_t(pos) * q_stride + 16 * ks + 8 * hf);
-        rot.fetch(false, 0);
+        issue_loads(first_tile);
+        // The matrix lies where the tiles will be, so the tables are there before the products begin; at 256 coordinates they
+        // take turns with the rounds of the matrix and are filled under the last one.
+        if (RROUNDS == 1) fill_pair_tables<8>(lut, cent_k, cent_v, 15, w, lane);
+        rot.put(0);
+        if (RROUNDS > 1) rot.fetch(false, 1);
         // the rows are exact in fp16 up to a power of two
         half8 qa[NKS];
         float mx = 0.0f;
@@ -712,26 +776,20 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
                 qa[ks][2 * i] = _Float16(load_elem<DT>(uint16_t(raw[ks][i] & 0xffffu)) * pow2(-ex));
                 qa[ks][2 * i + 1] = _Float16(load_elem<DT>(uint16_t(raw[ks][i] >> 16)) * pow2(-ex));
             }
-        float16v rows[D == 256 ? 1 : NOB];
-        uint32_t rows16[D == 256 ? NOB : 1][8];          // 256 coordinates: held as the 16-bit pairs they are rounded to
+        float16v rows[D == 256 ? 1 : NOB] = {};
+        uint32_t rows16[D == 256 ? NOB : 1][8] = {};     // 256 coordinates: held as the 16-bit pairs they are rounded to
         float mr = 0.0f;
 #pragma unroll
         for (int round = 0; round < RROUNDS; ++round) {
-            if (round > 0) __syncthreads();             // every wavefront is done with the round before
-            rot.put();
-            __syncthreads();
-            if (round + 1 < RROUNDS) rot.fetch(false, round + 1);
-#pragma unroll
-            for (int jr = 0; jr < RBLK; ++jr) {
+            __syncthreads();                            // this round's operands are there, the ones before are done with
+            if (round + 1 < RROUNDS) rot.put(round + 1);
+            if (round + 2 < RROUNDS) rot.fetch(false, round + 2);
+            if (RROUNDS > 1 && round == RROUNDS - 1) fill_pair_tables<8>(lut, cent_k, cent_v, 15, w, lane);
+            // (a wavefront without a unit leaves the LDS and the matrix cores to the others: half of them where one query of
+            // four heads shares its keys)
+            if (!unit_live) continue;
+            rot.template products<false>(round, qa, qa, [&](int jr, const float16v& hi, const float16v& lo) {
                 const int jb = RBLK * round + jr;
-                float16v hi, lo;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) { hi[r] = 0.0f; lo[r] = 0.0f; }
-#pragma unroll
-                for (int ks = 0; ks < NKS; ++ks) {
-                    hi = __builtin_amdgcn_mfma_f32_32x32x16_f16(rot.term(0, jr, ks), qa[ks], hi, 0, 0, 0);
-                    lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(rot.term(1, jr, ks), qa[ks], lo, 0, 0, 0);
-                }
                 if constexpr (D == 256) {
 #pragma unroll
                     for (int i = 0; i < 8; ++i) {
@@ -747,7 +805,7 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
                         mr = __builtin_fmaxf(mr, __builtin_fabsf(rows[jb][r]));
                     }
                 }
-            }
+            });
         }
         const int er = row_exponent(mr);
         krow = p.scale_log2e * pow2(er);
@@ -761,10 +819,8 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
                 else v = rows[ks >> 1][8 * (ks & 1) + e];
                 qb[ks][e] = _Float16(v * pow2(-er));
             }
-        __syncthreads();   // the rotation operands become lookup tables
+        __syncthreads();   // the rotation operands become tiles
     }
-    fill_pair_tables<8>(lut, p.centroids_k[lane & 15], p.centroids_v[lane & 15], 15, w, lane);
-    __syncthreads();
 
     // ---- lane-constant LDS read offsets ----------------------------------------------------------
     const int k_rd = m32 * kPfKStride + 16 * hf;
@@ -986,8 +1042,8 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
         const float l_tot = l_run + xor_shuffle(l_run, 32);
         const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
         rot.fetch(true, 0);
-        __syncthreads();                // every wavefront is done with the lookup tables
-        rot.put();
+        __syncthreads();                // every wavefront is done with the tiles and the tables
+        rot.put(0);
         __syncthreads();
         finish_rows<D, DT, PAGED>(p, rot, O, inv, unit_live, pos0, hq, NQ, q_row0, q_stride);
     }
@@ -1135,7 +1191,7 @@ template <int D, int DT, bool PAGED>
 __global__ __launch_bounds__(512) void attention_combine_prompts_kernel(const PrefillParams p) {
     using Cfg = PrefillCfg<D>;
     constexpr int NOB = Cfg::NOB;
-    __shared__ __attribute__((aligned(16))) uint8_t share[2 * Cfg::RTERM];
+    __shared__ __attribute__((aligned(16))) uint8_t share[(Cfg::RROUNDS > 1 ? 4 : 2) * Cfg::RTERM];
     const int tid = threadIdx.x, lane = tid & 63, m32 = lane & 31, hf = lane >> 5;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wg = int(blockIdx.x) % p.split_w, pair = int(blockIdx.x) / p.split_w;
@@ -1143,7 +1199,7 @@ __global__ __launch_bounds__(512) void attention_combine_prompts_kernel(const Pr
     const int pieces = PAGED ? p.left[blockIdx.x] : p.max_pieces;
     if (pieces == 0) return;
     const SeqShape sh = seq_shape<PAGED>(p, b);
-    RotationBlocks<D> rot{p.rotation, p.rot_col_major != 0, share, w, lane, m32, hf, {}};
+    RotationBlocks<D> rot{p.rotation, p.rot_col_major != 0, share, share + (Cfg::RROUNDS > 1 ? 2 * Cfg::RTERM : 0), w, lane, m32, hf, {}};
     rot.fetch(true, 0);
 
     const bool unit_live = 8 * wg + w < sh.units;              // a dead unit left no rows
@@ -1174,7 +1230,7 @@ __global__ __launch_bounds__(512) void attention_combine_prompts_kernel(const Pr
                 }
         }
     }
-    rot.put();
+    rot.put(0);
     __syncthreads();
     const int64_t q_row0 = PAGED ? int64_t(p.cu_seqlens_q[b]) * p.H_Q : int64_t(b) * p.H_Q * p.N_Q;
     finish_rows<D, DT, PAGED>(p, rot, O, inverse_sum(den), unit_live, pos0, hq, sh.NQ, q_row0,

@@ -455,3 +455,24 @@ def test_paged_attention_under_capture_with_other_lengths():
         assert torch.equal(out, eager)
         want = O.paged_prefill(q.cpu(), cu.cpu(), cache, table, sl.cpu(), c, c, r, hkv, d, bs)
         _rows_close(out, want, 4 * 2 ** -8)
+
+
+# (queries, keys): contexts of one tile, of tile counts that halve and quarter evenly and not, all alike, one long among short
+SEARCH = [([1, 2, 3], [1, 64, 63]), ([33] * 4, [64, 128, 256, 512]), ([20, 300, 1], [65, 321, 449]), ([40] * 9, [200] * 9),
+          ([1] * 64 + [500], [1] * 64 + [1700])]
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(3, 1, 128), (8, 2, 64), (2, 1, 256)])
+@pytest.mark.parametrize("batch", range(len(SEARCH)))
+def test_every_row_once_at_the_edges_of_the_search(batch, hq, hkv, d):
+    """Workgroups find their work by the tile counts; with fewer than eight units some of their wavefronts have none."""
+    ql, kv = SEARCH[batch]
+    bs, dtype = 16, torch.float16
+    c, _, r = book(d)
+    _, cache, table, sl = build_paged_case(kv, hq, hkv, d=d, bs=bs, seed=91, dtype=dtype)
+    q = torch.randn(sum(ql), hq, d, generator=torch.Generator().manual_seed(92)).to(dtype)
+    cu = torch.tensor([0] + list(torch.tensor(ql).cumsum(0)), dtype=torch.int32)
+    want = O.paged_prefill(q, cu, cache, table, sl, c, c, r, hkv, d, bs)
+    got = K.paged_tq4_prefill(q.to(DEV), cu.to(DEV), max(ql), cache.to(DEV), table.to(DEV), sl.to(DEV), c.to(DEV), c.to(DEV),
+                              r.to(DEV), hkv, d, bs, out=torch.full_like(q, 7.0).to(DEV))
+    _close(got, want, dtype)
