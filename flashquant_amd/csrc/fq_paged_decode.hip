@@ -2012,12 +2012,23 @@ inline WorkspaceLayout workspace_layout(int S, int H_Q, int D, int NS) {
 }
 
 
+// Rows of a split when the chunks follow from the longest possible context.
+inline int64_t chunk_of(int64_t max_rows, int num_splits) { return ((max_rows + num_splits - 1) / num_splits + 63) & ~int64_t(63); }
+
 // Workgroups that run at a time (one per CU) when the staged kernel should size its chunks from
 // the actual sequence lengths, 0 when the fixed chunks already fill the chip in one round or the
-// batch is too large for one lane per sequence.
-inline int staged_balance_slots(int num_seqs, int num_splits) {
+// batch is too large for four sequences a lane.
+// Beyond 64 sequences from chunks of 384 rows on: the search costs every workgroup, the shortest ones most.  Serving step, bf16,
+// fixed chunks and sized ones in us: 32 query heads over 8 of 128, 96 sequences of 1000 to 7000 tokens 129 and 106, 96 x 4000
+// 138 and 109, 200 of 100 to 2000 88 and 74; of 256, 72 of 300 to 6000 207 and 195; 16 over 2 of 128, 128 of 500 to 4000 37.4
+// and 36.8.  With chunks of 320 rows (8 over 1, 96 sequences) a batch of equal lengths still gains, 45.5 and 37.8, and one of
+// 1000 to 7000 tokens, which makes one round either way, loses: 29.2 and 29.6.
+// Rows of tokens at 256 coordinates (`chunk` 0) keep the fixed ones: 8 over 1, 200 of 500 to 10,000 146 and 152.
+inline int staged_balance_slots(int num_seqs, int num_splits, int64_t chunk) {
     const int cus = fq_host::device_cu_count();
-    return (num_seqs <= 64 && int64_t(num_seqs) * num_splits > cus) ? cus : 0;
+    const int64_t pairs = int64_t(num_seqs) * num_splits;
+    const bool few = num_seqs <= kWave, many = num_seqs <= kBalanceSeqs && pairs < 65536 && chunk >= 384;
+    return pairs > cus && (few || many) ? cus : 0;
 }
 
 // The kernel-variant switches as one decode call sees them.  They are process-wide and may be changed
@@ -2253,7 +2264,7 @@ int launch_partials(const DecodeParams& p, int S, int BS, hipStream_t stream, co
     if constexpr (D == 256) {
         if (p.new_key == nullptr && p.rotation == nullptr && staged_d256_linear_applies(D, p.H_KV, BS, var)) {
             DecodeParams ps = p;
-            ps.balance_slots = staged_balance_slots(S, p.num_splits);
+            ps.balance_slots = staged_balance_slots(S, p.num_splits, 0);
             return launch_staged_d256_linear<DT>(ps, S, BS * p.H_KV / 4, stream);
         }
         if (p.new_key == nullptr && p.rotation == nullptr && staged_d256_applies(D, p.H_KV, var)) {
@@ -2261,7 +2272,7 @@ int launch_partials(const DecodeParams& p, int S, int BS, hipStream_t stream, co
             const int64_t chunk = (((max_ctx + p.num_splits - 1) / p.num_splits) + 63) & ~int64_t(63);
             DecodeParams ps = p;
             const int groups = p.H_KV / 4;
-            ps.balance_slots = staged_balance_slots(S, p.num_splits * groups);
+            ps.balance_slots = staged_balance_slots(S, p.num_splits * groups, chunk);
             if (ps.balance_slots > 0) ps.balance_slots = ps.balance_slots / groups > 0 ? ps.balance_slots / groups : 1;
             const bool wide = chunk / BS > 64 || ps.balance_slots > 0 || (p.max_blocks > 64 && p.max_blocks <= 256);
             return launch_staged_d256<DT>(ps, S, BS, wide, stream);
@@ -2276,7 +2287,7 @@ int launch_partials(const DecodeParams& p, int S, int BS, hipStream_t stream, co
             DecodeParams ps = p;
             ps.G = 2 * p.G;                 // query heads of a pair of KV heads
             const int groups = d64_half ? 1 : p.H_KV / 16;
-            ps.balance_slots = staged_balance_slots(S, p.num_splits * groups);
+            ps.balance_slots = staged_balance_slots(S, p.num_splits * groups, chunk_rows);
             if (ps.balance_slots > 0) ps.balance_slots = ps.balance_slots / groups > 0 ? ps.balance_slots / groups : 1;
             const bool wide_rows = chunk_rows / rows_per_page > 64 || ps.balance_slots > 0 || (p.max_blocks > 64 && p.max_blocks <= 256);
             return launch_staged_d64<DT>(ps, S, rows_per_page, wide_rows, d64_half, stream);
@@ -2285,7 +2296,7 @@ int launch_partials(const DecodeParams& p, int S, int BS, hipStream_t stream, co
     if (staged_linear_applies(D, p.H_KV, BS, var)) {     // (one partial per split: also for callers that bring their own partial buffers)
         const int rows_per_page = BS * p.H_KV / 8;
         DecodeParams ps = p;
-        ps.balance_slots = staged_balance_slots(S, p.num_splits);
+        ps.balance_slots = staged_balance_slots(S, p.num_splits, chunk_of(int64_t(p.max_blocks) * rows_per_page, p.num_splits));
         return launch_staged_linear<DT>(ps, S, rows_per_page, stream);
     }
     // pages a split can span: its tokens are ceil(max_ctx / splits) rounded up to a tile
@@ -2298,7 +2309,7 @@ int launch_partials(const DecodeParams& p, int S, int BS, hipStream_t stream, co
         DecodeParams ps = p;
         // every group of 8 heads is a slice of the grid with the same (sequence, split) pairs
         const int groups = p.H_KV / 8;
-        ps.balance_slots = staged_balance_slots(S, p.num_splits * groups);
+        ps.balance_slots = staged_balance_slots(S, p.num_splits * groups, chunk);
         if (ps.balance_slots > 0) ps.balance_slots = ps.balance_slots / groups > 0 ? ps.balance_slots / groups : 1;
         // a chosen chunk may span up to 256 pages: four page-id registers
         if (var.ring && p.new_key != nullptr) return FQ_ERR_LAUNCH;
@@ -2827,7 +2838,7 @@ extern "C" int fq_prod_paged_decode(const void* q, const uint8_t* kv_cache, cons
     p.scale_log2e = sm_scale * kLog2e;
     // every group of 8 heads is a slice of the grid with the same (sequence, split) pairs
     const int groups = H_KV / 8;
-    p.balance_slots = staged_balance_slots(num_seqs, num_splits * groups);
+    p.balance_slots = staged_balance_slots(num_seqs, num_splits * groups, chunk_of(int64_t(max_blocks_per_seq) * block_size, num_splits));
     if (p.balance_slots > 0) p.balance_slots = p.balance_slots / groups > 0 ? p.balance_slots / groups : 1;
     p.heads_per_wg = 0;
     p.spin_limit = fq_host::option(FQ_OPT_DECODE_TINY_SPIN) != 0 ? 2 : (1 << 20);

@@ -29,7 +29,7 @@ struct DecodeParams {
     int heads_per_wg;           // direct kernel: KV heads a workgroup serves; its other wavefronts take further splits
     int spin_limit;             // staged kernel: polls of a bounded wait between wavefronts before it gives up
     int balance_slots;          // staged kernel: > 0 lets the workgroups size the token chunks from the actual
-                                // sequence lengths, for this many workgroups running at a time (num_seqs <= 64)
+                                // sequence lengths, for this many workgroups running at a time (num_seqs <= kBalanceSeqs)
     // Staged kernel instantiated with STORE: the serving step in one launch.  The workgroup whose split
     // holds a sequence's last token first compresses that token's new key and value rows into their
     // cache row (slot new_slots[seq]; negative: not stored), then reads the row back with its tile.
@@ -42,7 +42,114 @@ struct DecodeParams {
 };
 
 
-// Ragged batches of long contexts (at most 64 sequences, one lane each).  With the chunk
+__device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
+    int i = int(v);
+    i += __builtin_amdgcn_update_dpp(0, i, 0x121, 0xf, 0xf, false);   // row_ror:1, 2, 4, 8
+    i += __builtin_amdgcn_update_dpp(0, i, 0x122, 0xf, 0xf, false);
+    i += __builtin_amdgcn_update_dpp(0, i, 0x124, 0xf, 0xf, false);
+    i += __builtin_amdgcn_update_dpp(0, i, 0x128, 0xf, 0xf, false);
+    const auto a = __builtin_amdgcn_permlane16_swap(uint32_t(i), uint32_t(i), false, false);
+    const uint32_t b = a[0] + a[1];
+    const auto c = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    return uint32_t(__builtin_amdgcn_readfirstlane(int(c[0] + c[1])));
+}
+
+// balance_chunks for 65 to 256 sequences, four a lane: eight candidates (to 1.9 times the smallest chunk; lane j holds the
+// j-th), the workgroups of two of them added up at a time.  Every workgroup pays for this, also one without work: a first form
+// with 16 candidates, each one's cost worked out in all lanes, took 3.4 us (80 sequences of 60 to 1200 tokens, 8 KV heads of 64:
+// 23.5 -> 26.9 us).  Where the smallest chunk makes one round, nothing is better and all stays as it was.
+template <int TPR>
+__device__ __forceinline__ void balance_chunks_many(const DecodeParams& p, int lane, int NS, int cap, int max_tokens, int& chunk,
+                                                    int& seq, int& split, int& L_known) {
+    constexpr int K = 4, CANDS = 8;
+    const int nseq = int(gridDim.x);
+    int l_real[K];
+    float rows[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int at = K * lane + k;
+        const int l = p.seq_lens[at < nseq ? at : nseq - 1];
+        l_real[k] = at >= nseq || l < 0 ? 0 : (l > max_tokens ? max_tokens : l);
+        rows[k] = float((l_real[k] + TPR - 1) / TPR);
+    }
+    int cand = chunk + (lane & (CANDS - 1)) * (((chunk >> 3) + 63) & ~63);
+    cand = cand < cap ? cand : cap;
+    cand = cand > chunk ? cand : chunk;
+    const int rc_mine = int(__builtin_bit_cast(uint32_t, __builtin_amdgcn_rcpf(float(cand))));
+    auto groups_of = [&](int j) {                              // (the host sees to it that 16 bits hold the sum)
+        const float rc = __builtin_bit_cast(float, __builtin_amdgcn_readlane(rc_mine, j));
+        float n = 0.0f;
+#pragma unroll
+        for (int k = 0; k < K; ++k) n += __builtin_ceilf(rows[k] * rc - 0.0009765625f);
+        return uint32_t(n);
+    };
+    auto length_of = [&](int sq) {
+        int l = 0;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int lk = __builtin_amdgcn_readlane(l_real[k], sq / K);
+            l = sq % K == k ? lk : l;
+        }
+        return l;
+    };
+    if (int(wave_sum(groups_of(0))) <= p.balance_slots) {
+        L_known = length_of(seq);
+        return;
+    }
+    uint32_t mine = 0;
+#pragma unroll
+    for (int j = 0; j < CANDS; j += 2) {
+        const uint32_t both = wave_sum(groups_of(j) | groups_of(j + 1) << 16);
+        mine = lane == j ? both & 0xffffu : (lane == j + 1 ? both >> 16 : mine);
+    }
+    const float rounds = __builtin_ceilf(float(mine) * __builtin_amdgcn_rcpf(float(p.balance_slots)) - 0.0009765625f);
+    const float cost = lane < CANDS ? (rounds < 1.0f ? 1.0f : rounds) * float(cand + 96) : __builtin_inff();
+    const uint64_t cheapest = __ballot(cost == -wave_max(-cost));
+    chunk = __builtin_amdgcn_readlane(cand, __ffsll(static_cast<unsigned long long>(cheapest)) - 1);
+    int n[K], live = 0, dead = 0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        n[k] = ((l_real[k] + TPR - 1) / TPR + chunk - 1) / chunk;
+        n[k] = n[k] < NS ? n[k] : NS;
+        live += n[k];
+        dead += K * lane + k < nseq ? NS - n[k] : 0;
+    }
+    auto scan = [&](int v) {
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int t = __shfl_up(v, d, kWave);
+            v += lane >= d ? t : 0;
+        }
+        return v;
+    };
+    // the w-th of the live pairs, else of the empty ones: the lane that holds it, then which of its sequences
+    const int live_incl = scan(live);
+    const int total_live = __builtin_amdgcn_readlane(live_incl, 63);
+    const int w = int(blockIdx.x) + int(gridDim.x) * int(blockIdx.y);
+    const bool is_live = w < total_live;
+    const int incl = is_live ? live_incl : scan(dead), e = is_live ? w : w - total_live;
+    int sl = __builtin_popcountll(__ballot(incl <= e));
+    sl = sl < (nseq - 1) / K ? sl : (nseq - 1) / K;
+    int rem = e - __builtin_amdgcn_readlane(incl - (is_live ? live : dead), sl);
+    seq = -1;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int nk = __builtin_amdgcn_readlane(n[k], sl), have = is_live ? nk : NS - nk;
+        const bool last = K * sl + k >= nseq - 1 || k == K - 1;
+        if (seq < 0 && (rem < have || last)) {
+            seq = K * sl + k;
+            split = is_live ? rem : nk + rem;
+        }
+        rem -= have;
+    }
+    split = split < NS ? split : NS - 1;
+    L_known = length_of(seq);
+}
+
+// Most sequences of a batch whose chunks follow from the actual lengths. 
+constexpr int kBalanceSeqs = 256;
+
+// Ragged batches of long contexts (at most 64 sequences here, one lane each; more above).  With the chunk
 // of the longest possible context the live workgroups are all the same size and their
 // count is whatever the lengths add up to, e.g. 2.1 rounds over the chip, which costs 3.
 // Every workgroup evaluates the same 64 candidate chunk sizes (one per lane) on the
@@ -55,6 +162,8 @@ template <int PVR, int BS, int TPR>
 __device__ __forceinline__ void balance_chunks(const DecodeParams& p, int lane, int NS, bool rowwide, int& chunk, int& seq,
                                                int& split, int& L_known) {
     const int cap = rowwide ? chunk * NS : 64 * PVR * BS;       // page ids of a split: 64 * PVR lanes
+    if (int(gridDim.x) > kWave)
+        return balance_chunks_many<TPR>(p, lane, NS, cap, p.max_blocks * BS * TPR, chunk, seq, split, L_known);
     const int step = ((chunk >> 4) + 63) & ~63;
     int cand = chunk + lane * step;
     cand = cand < cap ? cand : cap;
