@@ -2022,7 +2022,8 @@ inline int64_t chunk_of(int64_t max_rows, int num_splits) { return ((max_rows + 
 // fixed chunks and sized ones in us: 32 query heads over 8 of 128, 96 sequences of 1000 to 7000 tokens 129 and 106, 96 x 4000
 // 138 and 109, 200 of 100 to 2000 88 and 74; of 256, 72 of 300 to 6000 207 and 195; 16 over 2 of 128, 128 of 500 to 4000 37.4
 // and 36.8.  With chunks of 320 rows (8 over 1, 96 sequences) a batch of equal lengths still gains, 45.5 and 37.8, and one of
-// 1000 to 7000 tokens, which makes one round either way, loses: 29.2 and 29.6.
+// 1000 to 7000 tokens, which makes one round either way, loses: 29.2 and 29.6.  A batch of equal lengths that fills its rounds
+// exactly pays for the search too, 128 x 4096 on 8 KV heads 125.7 and 129.3; 128 of 300 to 8192 198 and 143.
 // Rows of tokens at 256 coordinates (`chunk` 0) keep the fixed ones: 8 over 1, 200 of 500 to 10,000 146 and 152.
 inline int staged_balance_slots(int num_seqs, int num_splits, int64_t chunk) {
     const int cus = fq_host::device_cu_count();
