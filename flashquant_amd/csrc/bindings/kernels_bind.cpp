@@ -961,7 +961,7 @@ void bind_kernels(py::module_& m) {
               return before;
           }, py::arg("name"), py::arg("value"),
           "Set a kernel-variant switch ('decode_copy_waves', 'decode_direct', 'decode_ring', 'attention_any_dim', "
-          "'compress_three_terms': 0 / 1; 'reduce_rows': 0, 4, 8 or 16); returns the old value");
+          "'compress_three_terms': 0 / 1; 'decode_tiny_spin': 0, 1 or 2; 'reduce_rows': 0, 4, 8 or 16); returns the old value");
     m.def("get_option", [](const std::string& name) { return fq_get_option(option_id(name)); }, py::arg("name"));
     m.def("paged_decode_fault_count", []() {
               unsigned int n = 0;

@@ -51,7 +51,9 @@ extern "C" int fq_get_option(int option) {
 extern "C" int fq_set_option(int option, int value) {
     if (option < 0 || option >= FQ_OPTION_COUNT) return FQ_ERR_BAD_SHAPE;
     init_options();
-    g_options[option].store(option == FQ_OPT_REDUCE_ROWS ? value : (value != 0 ? 1 : 0), std::memory_order_relaxed);
+    if (option == FQ_OPT_DECODE_TINY_SPIN) value = value >= 2 ? 2 : (value != 0 ? 1 : 0);
+    else if (option != FQ_OPT_REDUCE_ROWS) value = value != 0 ? 1 : 0;
+    g_options[option].store(value, std::memory_order_relaxed);
     return FQ_OK;
 }
 

@@ -968,14 +968,16 @@ __global__ __launch_bounds__(512 + 64 * CW) void paged_decode_staged_kernel(cons
     constexpr int kNewHeads = HPR;                          // KV heads of this workgroup
     int64_t new_slot = -1;
     float bnd_mine = 0.0f;      // boundary `lane` of the 15 (asked for here: at its use it would be a round trip of its own)
+    // row r of the block of new rows: key head r, or value head r - KH (the last one again beyond them)
+    auto new_row = [&](int r) {
+        const int kv_heads = MULTI > 0 ? HPR : p.H_KV;           // (head_dim 64: pairs of heads, 128 elements together)
+        const int nr = r < 2 * kNewHeads ? r : 2 * kNewHeads - 1;
+        return reinterpret_cast<const uint16_t*>(nr < kNewHeads ? p.new_key : p.new_value) +
+               (int64_t(seq) * kv_heads + kNewHeads * hgrp + (nr & (kNewHeads - 1))) * 128;
+    };
     if constexpr (STORE) {
         if (!copier) {
-            const int kv_heads = MULTI > 0 ? HPR : p.H_KV;       // (head_dim 64: pairs of heads, 128 elements together)
-            // block row: key head nr, or value head nr - KH; 16 lanes a row
-            const int nr = (tid >> 4) < 2 * kNewHeads ? tid >> 4 : 2 * kNewHeads - 1;
-            const uint16_t* xrow = reinterpret_cast<const uint16_t*>(nr < kNewHeads ? p.new_key : p.new_value) +
-                                   (int64_t(seq) * kv_heads + kNewHeads * hgrp + (nr & (kNewHeads - 1))) * 128;
-            if (tid < 256) new_part = *reinterpret_cast<const uint4v*>(xrow + 8 * (tid & 15));
+            if (tid < 256) new_part = *reinterpret_cast<const uint4v*>(new_row(tid >> 4) + 8 * (tid & 15));     // 16 lanes a row
             new_slot = p.new_slots[seq];
             bnd_mine = p.boundaries[lane < 15 ? lane : 14];
         }
@@ -1274,6 +1276,12 @@ __global__ __launch_bounds__(512 + 64 * CW) void paged_decode_staged_kernel(cons
                     uint4v raw[KS];
 #pragma unroll
                     for (int j = 0; j < KS; ++j) raw[j] = *reinterpret_cast<const uint4v*>(stage + kQStage + n * kNewStride + 64 * j + 16 * g);
+                    // Later steps read what is stored here, also when this one's output is NaN: rows that may not be in `stage`
+                    // yet are fetched from where they came.
+                    if (__builtin_expect(handoff_failed, 0)) {
+#pragma unroll
+                        for (int j = 0; j < KS; ++j) raw[j] = *reinterpret_cast<const uint4v*>(new_row(n) + 32 * j + 8 * g);
+                    }
                     // sum of squares of row n: this lane's 32 elements, then over g.  head_dim 64: a row is a pair of heads,
                     // elements 0..63 the first and 64..127 the second; wavefront h holds columns of head h / 4 of the pair
                     float ss = 0.0f;
@@ -2032,6 +2040,12 @@ inline int staged_balance_slots(int num_seqs, int num_splits, int64_t chunk) {
     return pairs > cus && (few || many) ? cus : 0;
 }
 
+// Polls of a bounded wait between the wavefronts of the staged kernel.
+inline int handoff_polls() {
+    const int tiny = fq_host::option(FQ_OPT_DECODE_TINY_SPIN);
+    return tiny == 0 ? 1 << 20 : (tiny == 1 ? 2 : 0);
+}
+
 // The kernel-variant switches as one decode call sees them.  They are process-wide and may be changed
 // by another thread at any time (fq_set_option): a call reads them once, here, and everything that
 // depends on them (which kernel runs, how many partials it writes, how the workspace is laid out, how
@@ -2564,7 +2578,7 @@ int decode_partials(const void* q, const float* rotation, int rotation_col_major
     p.scale_log2e = sm_scale * kLog2e;
     p.balance_slots = 0;
     p.heads_per_wg = 0;
-    p.spin_limit = fq_host::option(FQ_OPT_DECODE_TINY_SPIN) != 0 ? 2 : (1 << 20);
+    p.spin_limit = handoff_polls();
     p.cache_rw = token ? token->cache : nullptr;
     p.new_key = token ? token->key : nullptr;
     p.new_value = token ? token->value : nullptr;
@@ -2842,7 +2856,7 @@ extern "C" int fq_prod_paged_decode(const void* q, const uint8_t* kv_cache, cons
     p.balance_slots = staged_balance_slots(num_seqs, num_splits * groups, chunk_of(int64_t(max_blocks_per_seq) * block_size, num_splits));
     if (p.balance_slots > 0) p.balance_slots = p.balance_slots / groups > 0 ? p.balance_slots / groups : 1;
     p.heads_per_wg = 0;
-    p.spin_limit = fq_host::option(FQ_OPT_DECODE_TINY_SPIN) != 0 ? 2 : (1 << 20);
+    p.spin_limit = handoff_polls();
     p.cache_rw = nullptr; p.new_key = nullptr; p.new_value = nullptr; p.new_slots = nullptr; p.boundaries = nullptr;
     p.num_slots = 0;
     hipStream_t s = static_cast<hipStream_t>(stream);

@@ -46,7 +46,7 @@ typedef enum fq_dtype {
 /*
  * Kernel-variant switches, for tests and measurements.  Each takes its first value from an
  * environment variable that is read once per process; fq_set_option changes it afterwards
- * (value 0 or 1), fq_get_option reads it (-1 for an unknown option).  Every entry point reads the
+ * (value 0 or 1 unless an option says otherwise), fq_get_option reads it (-1 for an unknown option).  Every entry point reads the
  * switches once, when it is called, so one call never mixes two settings; fq_set_option itself is not
  * ordered against calls running on other host threads, so change a switch only while no other thread
  * is inside the library.
@@ -59,8 +59,8 @@ typedef enum fq_option {
     FQ_OPT_ATTENTION_ANY_DIM = 2, /* FQ_ATTENTION_ANY_DIM, default 0: 1 sends every head_dim to the
                                      general attention kernel                                           */
     FQ_OPT_DECODE_TINY_SPIN = 3,  /* default 0: 1 makes the bounded waits between the wavefronts of the staged
-                                     decode kernel give up after two polls, to exercise the failure path
-                                     (NaN rows, fault counter) without hanging anything                */
+                                     decode kernel give up after two polls, 2 without a poll, to exercise
+                                     the failure path (NaN rows, fault counter) without hanging anything */
     FQ_OPT_COMPRESS_THREE_TERMS = 4, /* FQ_COMPRESS_THREE_TERMS, default 0: bf16 rows of head_dim 64 / 128 are
                                      rotated against the matrix as two bf16 terms (|error| <= 2^-18 per
                                      element: about 6 indices in a million differ from the float32 result);

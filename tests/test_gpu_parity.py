@@ -1124,6 +1124,36 @@ def test_store_and_decode_in_a_captured_graph(hq, hkv):
         assert torch.equal(cache_g, cache_e), rep
 
 
+@pytest.mark.parametrize("hq,hkv,d,dtype", [(32, 8, 128, torch.bfloat16), (32, 16, 128, torch.float16), (8, 1, 128, torch.bfloat16),
+                                            (16, 4, 128, torch.float16), (32, 8, 64, torch.bfloat16)])
+@pytest.mark.parametrize("polls", [1, 2])
+def test_a_failed_handoff_leaves_the_cache_right(polls, hq, hkv, d, dtype, kernel_option):
+    """The serving step with the bounded waits forced to give up from the host, after two polls or at once: every workgroup
+    runs to its end, the cache holds what the step writes when nothing fails, byte for byte (the new token's row is what
+    later steps read), a row of the output is right or NaN, and the fault counter moves."""
+    C = load_native()
+    c, b, r = book(d)
+    lens = [37, 1, 300, 65, 64, 1500, 0, 33]
+    q, cache, table, sl, key, value, slots = _serving_case(lens, hq, hkv, d, 16, dtype, seed=411)
+    q_d, table_d, sl_d, key_d, value_d, slots_d, c_d, b_d, r_d = [t.to(DEV) for t in (q, table, sl, key, value, slots, c, b, r)]
+
+    def step():
+        cache_d = cache.clone().to(DEV)
+        out = K.tq4_store_and_decode(key_d, value_d, slots_d, q_d, cache_d, table_d, sl_d, c_d, c_d, r_d, b_d, hkv, d, 16, num_splits=3)
+        torch.cuda.synchronize()
+        return out.float(), cache_d
+
+    want, cache_want = step()
+    before = C.paged_decode_fault_count()
+    kernel_option("decode_tiny_spin", polls)
+    got, cache_got = step()
+    assert torch.equal(cache_got, cache_want)
+    assert (torch.isnan(got) | (got == want)).all()
+    if polls == 2:
+        assert C.paged_decode_fault_count() > before
+        assert torch.isnan(got[sl_d > 0]).all() and (got[sl_d == 0] == 0).all()
+
+
 def test_store_and_decode_over_several_steps():
     """Three decode steps in a row on one cache: every step's token is there for the next."""
     c, b, r = book(128)
