@@ -380,15 +380,15 @@ __device__ __forceinline__ int row_exponent(float mx) {
 __device__ __forceinline__ float pow2(int e) { return bits_to_float(uint32_t(127 + e) << 23); }
 
 // The end of a workgroup: the rows in the accumulators normalised, rotated back (the first round of the matrix already lies
-// in LDS) and stored.
-template <int D, int DT, bool PAGED>
+// in LDS) and stored.  EARLY: the second round is asked for before the rows are converted, else after.
+template <int D, int DT, bool PAGED, bool EARLY>
 __device__ __forceinline__ void finish_rows(const PrefillParams& p, RotationBlocks<D>& rot, float16v (&O)[D / 32], float inv,
                                             bool unit_live, int pos0, int hq, int NQ, int64_t q_row0, int q_stride) {
     using Cfg = PrefillCfg<D>;
     constexpr int NKS = Cfg::NKS, NOB = Cfg::NOB, RROUNDS = Cfg::RROUNDS, RBLK = Cfg::RBLK;
     const int m32 = rot.m32, hf = rot.hf;
     if (RROUNDS == 1 && !unit_live) return;
-    if (RROUNDS > 1) rot.fetch(true, 1);
+    if (RROUNDS > 1 && EARLY) rot.fetch(true, 1);
     // float32 rows: both operands as two fp16 terms, three MFMA terms; rows already rounded to 16 bits (the paged form) in
     // one, the row's largest value brought into [2^14, 2^15): what is above 2^-28 of it is exact, the rest to 2^-39 of it (a
     // largest value in [1, 2) left the coordinates below 2^-14 of it among fp16's subnormals)
@@ -418,6 +418,7 @@ __device__ __forceinline__ void finish_rows(const PrefillParams& p, RotationBloc
                 olo[ks][e] = l2[0]; olo[ks][e + 1] = l2[1];
             }
         }
+    if (RROUNDS > 1 && !EARLY) rot.fetch(true, 1);
     const int opos = pos0 + m32;
     uint16_t* obase = PAGED ? p.out + (q_row0 + hq) * D : p.out + (q_row0 + int64_t(hq) * NQ) * D;
     uint16_t* orow = obase + int64_t(opos) * q_stride;
@@ -482,6 +483,13 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     constexpr int NKS = Cfg::NKS, NOB = Cfg::NOB, PB = Cfg::PB, TS = Cfg::TS, TT = Cfg::TT;
     constexpr int NTB = TT / 32, NVS = TT / 16;    // 32-token blocks of the scores, k-steps of the second product
     constexpr bool kFind = WORK != kGrid, kSplit = WORK == kPieces || WORK == kAllPieces;
+    // In grid order there is no search to hide the matrix behind, and at 64 coordinates the values held meanwhile and the way
+    // round the products cost more than they give: bf16, causal, 32 heads over 8, 2 x 8192 tokens 949 us with them and 927
+    // without, 4 x 1500 106.8 and 104.6, 16 x 300 42.9 and 42.0.  At 256 the second round of the matrix at the end is asked for
+    // behind the conversions, not before them (2 x 8192 tokens, 16 heads over 4, 2.00 ms with 56 spilled registers and 1.92 with
+    // 26, one prompt of them 1175 and 1154, 8 x 500 of 32 over 8 165 and 156); the other forms spill 7 to 37 either way and
+    // gain by it (one prompt of 3001 in pieces 381 and 377).
+    constexpr bool kEarlyFetch = kFind || D != 64, kSkipDead = kFind || D != 64, kEarlyFinish = kFind;
     __shared__ __attribute__((aligned(256))) uint32_t lut[256 * 64];
     extern __shared__ __attribute__((aligned(16))) uint8_t bufs[];   // 2 x (K tile | V^T tile)
     // Rows whose norm times a centroid would not fit fp16 are stored divided by a power of two.
@@ -510,7 +518,7 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     const float cent_k = p.centroids_k[lane & 15], cent_v = p.centroids_v[lane & 15];
     constexpr int RROUNDS = Cfg::RROUNDS, RBLK = Cfg::RBLK;
     RotationBlocks<D> rot{p.rotation, p.rot_col_major != 0, bufs, reinterpret_cast<uint8_t*>(lut), w, lane, m32, hf, {}};
-    rot.fetch(false, 0);
+    if constexpr (kEarlyFetch) rot.fetch(false, 0);
     if constexpr (kFind) {
         // the KV heads of a place are neighbours: each XCD serves few of them
         const int at = int(blockIdx.x + gridDim.x * blockIdx.y);
@@ -753,6 +761,7 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks)
             raw[ks] = *reinterpret_cast<const uint4v*>(qbase + int64_t(pos) * q_stride + 16 * ks + 8 * hf);
+        if constexpr (!kEarlyFetch) rot.fetch(false, 0);
         issue_loads(first_tile);
         // The matrix lies where the tiles will be, so the tables are there before the products begin; at 256 coordinates they
         // take turns with the rounds of the matrix and are filled under the last one.
@@ -779,15 +788,27 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
         float16v rows[D == 256 ? 1 : NOB] = {};
         uint32_t rows16[D == 256 ? NOB : 1][8] = {};     // 256 coordinates: held as the 16-bit pairs they are rounded to
         float mr = 0.0f;
+        // A wavefront without a unit leaves the LDS and the matrix cores to the others: half of them where one query of four
+        // heads shares its keys.  In the forms without pieces the branch is opaque: the compiler took it for a reason to hold
+        // two copies of the tile loop (64 coordinates 193 registers instead of 170, 40 queries over 100 to 4000 keys 88.0 and
+        // 83.9 us, 85.2 before there was a branch; 16 x 300 tokens of 128, grid order, 106 scalar registers and 5 spilled instead of
+        // 65).  With pieces it does not, and opaque costs 1 % (mixed batch of 12 at 64 coordinates 266 and 270 us).
+        int live = 1;
+        if constexpr (kSkipDead && WORK != kPieces) {
+            live = __builtin_amdgcn_readfirstlane(unit_live ? 1 : 0);
+            asm volatile("" : "+s"(live));
+        }
 #pragma unroll
         for (int round = 0; round < RROUNDS; ++round) {
             __syncthreads();                            // this round's operands are there, the ones before are done with
             if (round + 1 < RROUNDS) rot.put(round + 1);
             if (round + 2 < RROUNDS) rot.fetch(false, round + 2);
             if (RROUNDS > 1 && round == RROUNDS - 1) fill_pair_tables<8>(lut, cent_k, cent_v, 15, w, lane);
-            // (a wavefront without a unit leaves the LDS and the matrix cores to the others: half of them where one query of
-            // four heads shares its keys)
-            if (!unit_live) continue;
+            if constexpr (WORK == kPieces) {
+                if (!unit_live) continue;
+            } else if constexpr (kSkipDead) {
+                if (live == 0) continue;
+            }
             rot.template products<false>(round, qa, qa, [&](int jr, const float16v& hi, const float16v& lo) {
                 const int jb = RBLK * round + jr;
                 if constexpr (D == 256) {
@@ -1002,6 +1023,9 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
 
     // ---- tiles ----------------------------------------------------------------------------------------
     dequant(first_tile & 1, first_tile);
+    // (at 256 coordinates the scheduler drew the first tile's end into the loop of this form: one prompt of 8192 tokens, 16 heads
+    // over 4, 962 us without the fence and 951 with it, 4 prompts of 4096 1031 and 1026)
+    if constexpr (D == 256 && WORK == kOrdered) __builtin_amdgcn_sched_barrier(0);
     issue_loads(first_tile + 1);
     // The dequantisation of tile i + 1 and the products of tile i sit in one basic block (no
     // conditions between them), so that the lookups and LDS writes of the one interleave with
@@ -1045,7 +1069,7 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
         __syncthreads();                // every wavefront is done with the tiles and the tables
         rot.put(0);
         __syncthreads();
-        finish_rows<D, DT, PAGED>(p, rot, O, inv, unit_live, pos0, hq, NQ, q_row0, q_stride);
+        finish_rows<D, DT, PAGED, kEarlyFinish>(p, rot, O, inv, unit_live, pos0, hq, NQ, q_row0, q_stride);
     }
 }
 
@@ -1233,7 +1257,7 @@ __global__ __launch_bounds__(512) void attention_combine_prompts_kernel(const Pr
     rot.put(0);
     __syncthreads();
     const int64_t q_row0 = PAGED ? int64_t(p.cu_seqlens_q[b]) * p.H_Q : int64_t(b) * p.H_Q * p.N_Q;
-    finish_rows<D, DT, PAGED>(p, rot, O, inverse_sum(den), unit_live, pos0, hq, sh.NQ, q_row0,
+    finish_rows<D, DT, PAGED, true>(p, rot, O, inverse_sum(den), unit_live, pos0, hq, sh.NQ, q_row0,
                               PAGED ? p.H_Q * D : D);
 }
 
