@@ -61,8 +61,8 @@ struct PrefillCfg {
     static constexpr int NOB = D / 32;                    // 32-coordinate blocks of the output
     static constexpr int PB = D / 2;                      // packed bytes per token and head
     // The rotation matrix as MFMA operands (two fp16 terms), shared by the wavefronts of a workgroup:
-    // a block of 32 x 16 holds one 16-byte operand per lane and term.  They lie where the lookup
-    // tables are between the query stage and the end of the tile loop (64 KB), at D = 256 a quarter at a time.
+    // a block of 32 x 16 holds one 16-byte operand per lane and term.  They lie where the tiles are between the query
+    // stage and the end of the tile loop (64 KB), at D = 256 a quarter at a time, there and where the lookup tables are by turns.
     static constexpr int SLOT = 8 * (32 * D + 64);        // floats: per unit 32 rows un-normalised, 32 maxima, 32 sums
     static constexpr int RROUNDS = D == 256 ? 4 : 1;
     static constexpr int RBLK = NOB / RROUNDS;            // blocks of 32 result coordinates in a round
@@ -288,7 +288,10 @@ __device__ __forceinline__ WorkItem find_item(const PrefillParams& p, int at, co
 // What it replaced staged the rows through LDS for the 16x16x32 MFMA (16 to 32 lanes on a bank) and stored the
 // results 2 bytes a lane: a workgroup per CU on 64 tokens of 32 heads over 64 keys took 33 us and 27 us with one
 // query row, 24 and 15.5 us this way (the tile itself: 2 us); 4 x 32 heads x 8192 tokens 2.89 -> 2.81 ms.
-template <int D>
+//
+// At 256 coordinates the matrix comes in rounds.  AREAS: 2 where they take turns in two places, 1 where each waits for the one
+// before to be done with (attention_combine_prompts_kernel).
+template <int D, int AREAS = 2>
 struct RotationBlocks {
     using Cfg = PrefillCfg<D>;
     static constexpr int NKS = Cfg::NKS, RBLK = Cfg::RBLK, BPW = RBLK * NKS / 8;
@@ -296,7 +299,7 @@ struct RotationBlocks {
     const float* rotation;
     bool col_major;
     uint8_t* share;               // 2 x RTERM bytes of LDS: the last round's operands, and every second one's before it
-    uint8_t* other;               // as many again for the rounds between (unused with one round)
+    uint8_t* other;               // as many again for the rounds between (unused with one round, or one area)
     int w, lane, m32, hf;
     float rbv[BPW][8];
     // `back`: x @ R with the contraction index in the order of the accumulator registers (element 4 a + c of half
@@ -317,7 +320,7 @@ struct RotationBlocks {
             }
         }
     }
-    __device__ __forceinline__ uint8_t* at(int round) const { return ((RROUNDS - 1 - round) & 1) == 0 ? share : other; }
+    __device__ __forceinline__ uint8_t* at(int round) const { return AREAS == 1 || ((RROUNDS - 1 - round) & 1) == 0 ? share : other; }
     __device__ __forceinline__ void put(int round) {
         uint8_t* dst = at(round);
         half8 rhi[BPW], rlo[BPW];
@@ -380,15 +383,15 @@ __device__ __forceinline__ int row_exponent(float mx) {
 __device__ __forceinline__ float pow2(int e) { return bits_to_float(uint32_t(127 + e) << 23); }
 
 // The end of a workgroup: the rows in the accumulators normalised, rotated back (the first round of the matrix already lies
-// in LDS) and stored.  EARLY: the second round is asked for before the rows are converted, else after.
-template <int D, int DT, bool PAGED, bool EARLY>
-__device__ __forceinline__ void finish_rows(const PrefillParams& p, RotationBlocks<D>& rot, float16v (&O)[D / 32], float inv,
+// in LDS) and stored.  EARLY: with two areas the second round is asked for before the rows are converted, else after.
+template <int D, int DT, bool PAGED, bool EARLY, int AREAS>
+__device__ __forceinline__ void finish_rows(const PrefillParams& p, RotationBlocks<D, AREAS>& rot, float16v (&O)[D / 32], float inv,
                                             bool unit_live, int pos0, int hq, int NQ, int64_t q_row0, int q_stride) {
     using Cfg = PrefillCfg<D>;
     constexpr int NKS = Cfg::NKS, NOB = Cfg::NOB, RROUNDS = Cfg::RROUNDS, RBLK = Cfg::RBLK;
     const int m32 = rot.m32, hf = rot.hf;
     if (RROUNDS == 1 && !unit_live) return;
-    if (RROUNDS > 1 && EARLY) rot.fetch(true, 1);
+    if (RROUNDS > 1 && AREAS > 1 && EARLY) rot.fetch(true, 1);
     // float32 rows: both operands as two fp16 terms, three MFMA terms; rows already rounded to 16 bits (the paged form) in
     // one, the row's largest value brought into [2^14, 2^15): what is above 2^-28 of it is exact, the rest to 2^-39 of it (a
     // largest value in [1, 2) left the coordinates below 2^-14 of it among fp16's subnormals)
@@ -418,15 +421,23 @@ __device__ __forceinline__ void finish_rows(const PrefillParams& p, RotationBloc
                 olo[ks][e] = l2[0]; olo[ks][e + 1] = l2[1];
             }
         }
-    if (RROUNDS > 1 && !EARLY) rot.fetch(true, 1);
+    if (RROUNDS > 1 && AREAS > 1 && !EARLY) rot.fetch(true, 1);
     const int opos = pos0 + m32;
     uint16_t* obase = PAGED ? p.out + (q_row0 + hq) * D : p.out + (q_row0 + int64_t(hq) * NQ) * D;
     uint16_t* orow = obase + int64_t(opos) * q_stride;
 #pragma unroll
     for (int round = 0; round < RROUNDS; ++round) {
-        if (round > 0) __syncthreads();                // this round's operands are there, the ones before are done with
-        if (round + 1 < RROUNDS) rot.put(round + 1);
-        if (round + 2 < RROUNDS) rot.fetch(true, round + 2);
+        if (round > 0) __syncthreads();                // the operands before are done with; with two areas this round's are there
+        if constexpr (AREAS == 1) {
+            if (round > 0) {
+                rot.put(round);
+                __syncthreads();
+            }
+            if (round + 1 < RROUNDS) rot.fetch(true, round + 1);
+        } else {
+            if (round + 1 < RROUNDS) rot.put(round + 1);
+            if (round + 2 < RROUNDS) rot.fetch(true, round + 2);
+        }
         rot.template products<!PAGED>(round, ohi, olo, [&](int cr, const float16v& hi, const float16v& lo) {
         const int cb = RBLK * round + cr;
         // registers 4 q + c of half hf = coordinate 32 cb + 8 q + 4 hf + c; the halves exchange a quad of every two,
@@ -1210,12 +1221,14 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillPar
 // matrix for every 16 rows).  When it was added, 16 heads x 3001 tokens of 256 coordinates, 188 workgroups in two pieces: 298 us
 // with the kernel above, 240 with this one (208 now); 8 heads x 5000 tokens of 128, 157 workgroups: 140 and 121; 16 heads x
 // 2000 tokens of 64, 128 workgroups: 54.6 and 48.3 (45.8 now).  With 63 workgroups in four pieces the smaller workgroups above
-// are faster (128 and 148 us at 256 coordinates, 55 and 68 at 128): this one runs from half a round of workgroups on.
+// are faster (128 and 148 us at 256 coordinates, 55 and 68 at 128): this one runs from half a round of workgroups on.  At 256
+// coordinates the rounds of the matrix share one area (64 KB, so that two workgroups fit a CU): with two of them 14 registers
+// were spilled and 16 heads x 3001 tokens took 209 us, 202 with one.
 template <int D, int DT, bool PAGED>
 __global__ __launch_bounds__(512) void attention_combine_prompts_kernel(const PrefillParams p) {
     using Cfg = PrefillCfg<D>;
     constexpr int NOB = Cfg::NOB;
-    __shared__ __attribute__((aligned(16))) uint8_t share[(Cfg::RROUNDS > 1 ? 4 : 2) * Cfg::RTERM];
+    __shared__ __attribute__((aligned(16))) uint8_t share[2 * Cfg::RTERM];
     const int tid = threadIdx.x, lane = tid & 63, m32 = lane & 31, hf = lane >> 5;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wg = int(blockIdx.x) % p.split_w, pair = int(blockIdx.x) / p.split_w;
@@ -1223,7 +1236,7 @@ __global__ __launch_bounds__(512) void attention_combine_prompts_kernel(const Pr
     const int pieces = PAGED ? p.left[blockIdx.x] : p.max_pieces;
     if (pieces == 0) return;
     const SeqShape sh = seq_shape<PAGED>(p, b);
-    RotationBlocks<D> rot{p.rotation, p.rot_col_major != 0, share, share + (Cfg::RROUNDS > 1 ? 2 * Cfg::RTERM : 0), w, lane, m32, hf, {}};
+    RotationBlocks<D, 1> rot{p.rotation, p.rot_col_major != 0, share, nullptr, w, lane, m32, hf, {}};
     rot.fetch(true, 0);
 
     const bool unit_live = 8 * wg + w < sh.units;              // a dead unit left no rows
