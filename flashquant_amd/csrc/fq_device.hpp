@@ -304,6 +304,19 @@ __device__ __forceinline__ float wave_max(float v) {
     return max_xor32(max_xor16(v));
 }
 
+// The same for the sum, modulo 2^32.
+__device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
+    int i = int(v);
+    i += __builtin_amdgcn_update_dpp(0, i, 0x121, 0xf, 0xf, false);   // row_ror:1, 2, 4, 8
+    i += __builtin_amdgcn_update_dpp(0, i, 0x122, 0xf, 0xf, false);
+    i += __builtin_amdgcn_update_dpp(0, i, 0x124, 0xf, 0xf, false);
+    i += __builtin_amdgcn_update_dpp(0, i, 0x128, 0xf, 0xf, false);
+    const auto a = __builtin_amdgcn_permlane16_swap(uint32_t(i), uint32_t(i), false, false);
+    const uint32_t b = a[0] + a[1];
+    const auto c = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    return uint32_t(__builtin_amdgcn_readfirstlane(int(c[0] + c[1])));
+}
+
 // 16-bit rows (fp16 / bf16 raw words, lane (m, g) holding k = 32 j + 8 g + e) as the fp16 A
 // operand, scaled by one power of two for the whole 16-row block so that the largest
 // element lies in [1, 2); `up` undoes the scaling on the result.

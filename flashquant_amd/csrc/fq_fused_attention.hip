@@ -130,24 +130,11 @@ __device__ __forceinline__ SeqShape seq_shape(const PrefillParams& p, int s) {
     return make_seq_shape(NQ, NKV, qoff, p.G, p.max_w);
 }
 
-__device__ __forceinline__ uint32_t wave_add(uint32_t v) {
-    int i = int(v);
-    i += __builtin_amdgcn_update_dpp(0, i, 0x121, 0xf, 0xf, false);   // row_ror:1, 2, 4, 8
-    i += __builtin_amdgcn_update_dpp(0, i, 0x122, 0xf, 0xf, false);
-    i += __builtin_amdgcn_update_dpp(0, i, 0x124, 0xf, 0xf, false);
-    i += __builtin_amdgcn_update_dpp(0, i, 0x128, 0xf, 0xf, false);
-    const auto a = __builtin_amdgcn_permlane16_swap(uint32_t(i), uint32_t(i), false, false);
-    const uint32_t b = a[0] + a[1];
-    const auto c = __builtin_amdgcn_permlane32_swap(b, b, false, false);
-    return uint32_t(__builtin_amdgcn_readfirstlane(int(c[0] + c[1])));
-}
-
 // The sequences s0 + lane as the lanes of a wavefront hold them; empty ones past the end.
-template <bool PAGED>
 __device__ __forceinline__ SeqShape lane_shape(const PrefillParams& p, int s0, int lane) {
     // (no branch around the loads: the caller has other requests to send before it needs them)
     const bool some = s0 + lane < p.num_seqs;
-    SeqShape sh = seq_shape<PAGED>(p, some ? s0 + lane : p.num_seqs - 1);
+    SeqShape sh = seq_shape<true>(p, some ? s0 + lane : p.num_seqs - 1);
     sh.NQ = some ? sh.NQ : 0;
     sh.NKV = some ? sh.NKV : 0;
     sh.qoff = some ? sh.qoff : 0;
@@ -157,22 +144,20 @@ __device__ __forceinline__ SeqShape lane_shape(const PrefillParams& p, int s0, i
 // The share of a CU of the whole batch (all KV heads), in tiles, and the rows of the sequences that may be split.  The sums
 // may wrap on batches beyond any memory: the pieces are then merely poor ones, and still the same everywhere.  `first`: the
 // first wavefront's worth of sequences.
-template <bool PAGED>
 __device__ __forceinline__ BatchWork batch_work(const PrefillParams& p, const SeqShape& first, int lane) {
     uint32_t tiles = 0, rows = 0;
     for (int s0 = 0; s0 < p.num_seqs; s0 += kWave) {
-        const SeqShape sh = s0 == 0 ? first : lane_shape<PAGED>(p, s0, lane);
+        const SeqShape sh = s0 == 0 ? first : lane_shape(p, s0, lane);
         if (sh.W > 0)
             tiles += uint32_t(sh.W) * uint32_t(tiles_of(sh, 0, p.G, p.causal) + tiles_of(sh, sh.W - 1, p.G, p.causal) + 1) / 2;
         if (sh.W <= p.split_w) rows += uint32_t(sh.NQ) * uint32_t(p.G);
     }
-    return {share_of(wave_add(tiles) * uint32_t(p.H_KV), p.round_slots), int(wave_add(rows) * uint32_t(p.H_KV) >> 8)};
+    return {share_of(wave_sum(tiles) * uint32_t(p.H_KV), p.round_slots), int(wave_sum(rows) * uint32_t(p.H_KV) >> 8)};
 }
 
-// Pieces of a sequence's workgroups.  Sequences of one length: the host has worked them out.
-template <int D, bool PAGED>
+// Pieces of a sequence's workgroups.
+template <int D>
 __device__ __forceinline__ int pieces_in(const PrefillParams& p, const SeqShape& sh, const BatchWork& batch) {
-    if (!PAGED) return p.max_pieces;
     return pieces_of(sh, batch, p.split_w, p.max_pieces, p.G, p.causal != 0, D);
 }
 
@@ -189,38 +174,40 @@ __device__ __forceinline__ void note_pieces(const PrefillParams& p, const SeqSha
     auto of_lane = [&](int v) { return __builtin_amdgcn_readlane(v, b); };
     const SeqShape sh = b < kWave ? make_seq_shape(of_lane(first.NQ), of_lane(first.NKV), of_lane(first.qoff), p.G, p.max_w)
                                   : seq_shape<true>(p, b);
-    const int n = x < sh.W && sh.W <= p.split_w ? pieces_in<D, true>(p, sh, batch) : 0;
+    const int n = x < sh.W && sh.W <= p.split_w ? pieces_in<D>(p, sh, batch) : 0;
     if (threadIdx.x == 0) p.left[at] = n > 1 || p.all_in_part ? n : 0;
 }
 
-// The item of a place (`at` / H_KV, of one KV head) in the order longest piece first.  Sequences of one shape: the workgroups
-// of all of them from the last one down.  Else the largest tile count T that more than `place` pieces reach, a lane per
-// sequence, three counts at a time (they do not wait for one another) between 0 and the longest context; then the place among
-// the pieces of exactly T.  Beyond kOrderSeqs sequences the items in the order of the sequences (kOrderSeqs says why).
-// SPLIT: `at` is the workgroup's number in the launch.  `first`: the first wavefront's worth of sequences.
-template <int D, bool PAGED, bool SPLIT>
+// Contiguous sequences, all of one shape and in as many pieces as the host has worked out: the workgroups of all of them from
+// the last one down.
+__device__ __forceinline__ WorkItem find_prompt_item(const PrefillParams& p, int at) {
+    const int place = at / p.H_KV, per = p.num_seqs * p.max_pieces, down = place / per, rest = place % per;
+    const int W = seq_shape<false>(p, 0).W;
+    if (down >= W) return WorkItem{-1, 0, 0, 1};
+    return WorkItem{rest / p.max_pieces, W - 1 - down, rest % p.max_pieces, p.max_pieces};
+}
+
+// The item of a place (`at` / H_KV, of one KV head) of a paged batch in the order longest piece first: the largest tile count
+// T that more than `place` pieces reach, a lane per sequence, three counts at a time (they do not wait for one another) between
+// 0 and the longest context; then the place among the pieces of exactly T.  Beyond kOrderSeqs sequences the items in the order
+// of the sequences (kOrderSeqs says why).  SPLIT: `at` is the workgroup's number in the launch.  `first`: the first wavefront's
+// worth of sequences.
+template <int D, bool SPLIT>
 __device__ __forceinline__ WorkItem find_item(const PrefillParams& p, int at, const SeqShape& first, int lane) {
     const int G = p.G, place = at / p.H_KV;
     const bool causal = p.causal != 0;
-    if constexpr (!PAGED) {
-        const int per = p.num_seqs * (SPLIT ? p.max_pieces : 1), down = place / per, rest = place % per;
-        const int W = seq_shape<PAGED>(p, 0).W;
-        if (down >= W) return WorkItem{-1, 0, 0, 1};
-        if (!SPLIT) return WorkItem{rest, W - 1 - down, 0, 1};
-        return WorkItem{rest / p.max_pieces, W - 1 - down, rest % p.max_pieces, p.max_pieces};
-    }
-    if (PAGED && p.dense) {
+    if (p.dense) {
         const int seq = place / p.max_w, x = p.max_w - 1 - place % p.max_w;
-        return seq < p.num_seqs && x < seq_shape<PAGED>(p, seq).W ? WorkItem{seq, x, 0, 1} : WorkItem{-1, 0, 0, 1};
+        return seq < p.num_seqs && x < seq_shape<true>(p, seq).W ? WorkItem{seq, x, 0, 1} : WorkItem{-1, 0, 0, 1};
     }
     // (the lengths of the batch are only summed where a sequence is long enough for the shortest pieces)
     BatchWork batch{kSplitMinTiles, 0};
-    if (PAGED && SPLIT && (p.num_seqs > kWave || __any(may_split(first, p.split_w, p.max_pieces, G, causal, D))))
-        batch = batch_work<PAGED>(p, first, lane);
-    if (PAGED && SPLIT) note_pieces<D>(p, first, batch, at, lane);
-    auto shape = [&](int s0) { return s0 == 0 ? first : lane_shape<PAGED>(p, s0, lane); };
-    const int first_pieces = SPLIT ? pieces_in<D, PAGED>(p, first, batch) : 1;
-    auto pieces = [&](int s0, const SeqShape& sh) { return s0 == 0 || !SPLIT ? first_pieces : pieces_in<D, PAGED>(p, sh, batch); };
+    if (SPLIT && (p.num_seqs > kWave || __any(may_split(first, p.split_w, p.max_pieces, G, causal, D))))
+        batch = batch_work(p, first, lane);
+    if (SPLIT) note_pieces<D>(p, first, batch, at, lane);
+    auto shape = [&](int s0) { return s0 == 0 ? first : lane_shape(p, s0, lane); };
+    const int first_pieces = SPLIT ? pieces_in<D>(p, first, batch) : 1;
+    auto pieces = [&](int s0, const SeqShape& sh) { return s0 == 0 || !SPLIT ? first_pieces : pieces_in<D>(p, sh, batch); };
     struct Counts { int c[3]; };
     auto count = [&](int t0, int t1, int t2) {           // pieces of at least so many tiles
         uint32_t c0 = 0, c1 = 0, c2 = 0;
@@ -231,7 +218,7 @@ __device__ __forceinline__ WorkItem find_item(const PrefillParams& p, int at, co
             c1 += uint32_t(n * (sh.W - first_piece_with(sh, t1, n, G, causal)));
             c2 += uint32_t(n * (sh.W - first_piece_with(sh, t2, n, G, causal)));
         }
-        return Counts{{int(wave_add(c0)), int(wave_add(c1)), int(wave_add(c2))}};
+        return Counts{{int(wave_sum(c0)), int(wave_sum(c1)), int(wave_sum(c2))}};
     };
     WorkItem item{-1, 0, 0, 1};
     int lo = 0, hi = 0x3fffffff, rem = place;            // tile counts lo .. hi - 1 (no sequence has 2^30 tiles)
@@ -476,9 +463,9 @@ __device__ __forceinline__ void finish_rows(const PrefillParams& p, RotationBloc
 // one alone 8 to 58: 8 sequences of 120 queries over 1500 keys, 32 heads, 226 us with both compiled in, 170 with one.
 enum Work {
     kGrid,            // one workgroup per grid position, rows finished in the kernel
-    kOrdered,         // find_item, the same
-    kPieces,          // find_item, rows of a piece left to the combine, other rows finished in the kernel
-    kAllPieces        // find_item, all rows left to the combine
+    kOrdered,         // find_item, the same (paged)
+    kPieces,          // find_item, rows of a piece left to the combine, other rows finished in the kernel (paged)
+    kAllPieces        // find_item or find_prompt_item, all rows left to the combine
 };
 
 // PAGED: the sequences' queries are packed along the token axis of q (tokens, H_Q, 128), the keys
@@ -525,7 +512,7 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     // products, the first tile of one query over 4 x 2500 ring-buffer tokens begins after 6.5 us instead of 9.7 (24.3 -> 21.9 us
     // in all), 16 heads x 3001 tokens of 256 coordinates 219 -> 208 us.
     SeqShape first{};
-    if constexpr (kFind) first = lane_shape<PAGED>(p, 0, lane);
+    if constexpr (kFind && PAGED) first = lane_shape(p, 0, lane);
     const float cent_k = p.centroids_k[lane & 15], cent_v = p.centroids_v[lane & 15];
     constexpr int RROUNDS = Cfg::RROUNDS, RBLK = Cfg::RBLK;
     RotationBlocks<D> rot{p.rotation, p.rot_col_major != 0, bufs, reinterpret_cast<uint8_t*>(lut), w, lane, m32, hf, {}};
@@ -533,7 +520,10 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     if constexpr (kFind) {
         // the KV heads of a place are neighbours: each XCD serves few of them
         const int at = int(blockIdx.x + gridDim.x * blockIdx.y);
-        const WorkItem it = find_item<D, PAGED, kSplit>(p, at, first, lane);
+        static_assert(PAGED || WORK == kAllPieces, "contiguous launches are in grid order or all in pieces");
+        WorkItem it;
+        if constexpr (PAGED) it = find_item<D, kSplit>(p, at, first, lane);
+        else it = find_prompt_item(p, at);
         if (it.seq < 0) return;                            // the grid is sized for the most work possible
         b = it.seq; hkv = at % p.H_KV; wg = it.x; piece = it.piece; pieces = it.pieces;
     } else {

@@ -42,18 +42,6 @@ struct DecodeParams {
 };
 
 
-__device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
-    int i = int(v);
-    i += __builtin_amdgcn_update_dpp(0, i, 0x121, 0xf, 0xf, false);   // row_ror:1, 2, 4, 8
-    i += __builtin_amdgcn_update_dpp(0, i, 0x122, 0xf, 0xf, false);
-    i += __builtin_amdgcn_update_dpp(0, i, 0x124, 0xf, 0xf, false);
-    i += __builtin_amdgcn_update_dpp(0, i, 0x128, 0xf, 0xf, false);
-    const auto a = __builtin_amdgcn_permlane16_swap(uint32_t(i), uint32_t(i), false, false);
-    const uint32_t b = a[0] + a[1];
-    const auto c = __builtin_amdgcn_permlane32_swap(b, b, false, false);
-    return uint32_t(__builtin_amdgcn_readfirstlane(int(c[0] + c[1])));
-}
-
 // balance_chunks for 65 to 256 sequences, four a lane: eight candidates (to 1.9 times the smallest chunk; lane j holds the
 // j-th), the workgroups of two of them added up at a time.  Every workgroup pays for this, also one without work: a first form
 // with 16 candidates, each one's cost worked out in all lanes, took 3.4 us (80 sequences of 60 to 1200 tokens, 8 KV heads of 64:
