@@ -2023,21 +2023,32 @@ inline WorkspaceLayout workspace_layout(int S, int H_Q, int D, int NS) {
 // Rows of a split when the chunks follow from the longest possible context.
 inline int64_t chunk_of(int64_t max_rows, int num_splits) { return ((max_rows + num_splits - 1) / num_splits + 63) & ~int64_t(63); }
 
-// Workgroups that run at a time (one per CU) when the staged kernel should size its chunks from
-// the actual sequence lengths, 0 when the fixed chunks already fill the chip in one round or the
-// batch is too large for four sequences a lane.
-// Beyond 64 sequences from chunks of 384 rows on: the search costs every workgroup, the shortest ones most.  Serving step, bf16,
-// fixed chunks and sized ones in us: 32 query heads over 8 of 128, 96 sequences of 1000 to 7000 tokens 129 and 106, 96 x 4000
-// 138 and 109, 200 of 100 to 2000 88 and 74; of 256, 72 of 300 to 6000 207 and 195; 16 over 2 of 128, 128 of 500 to 4000 37.4
-// and 36.8.  With chunks of 320 rows (8 over 1, 96 sequences) a batch of equal lengths still gains, 45.5 and 37.8, and one of
-// 1000 to 7000 tokens, which makes one round either way, loses: 29.2 and 29.6.  A batch of equal lengths that fills its rounds
-// exactly pays for the search too, 128 x 4096 on 8 KV heads 125.7 and 129.3; 128 of 300 to 8192 198 and 143.
-// Rows of tokens at 256 coordinates (`chunk` 0) keep the fixed ones: 8 over 1, 200 of 500 to 10,000 146 and 152.
-inline int staged_balance_slots(int num_seqs, int num_splits, int64_t chunk) {
+// Workgroups that run at a time (one per CU and `groups` slices of the grid) when the staged kernel should size its chunks from
+// the actual sequence lengths; 0 when the fixed chunks already fill the chip in one round, or where the search does not pay.
+// Beyond 64 sequences it costs every workgroup about a microsecond, and gives what fits the rounds better; in us, fixed chunks
+// and sized ones, serving step, bf16, 32 query heads over 8 of 128 unless said:
+//   65 x 4096 tokens 111 and 77, 96 x 4096 116 and 108, 128 x 4096, whose two rounds are full, 124 and 120, 128 of 512 to 4096
+//   111 and 87, 200 of 250 to 2000 107 and 87, 112 of 1024 to 8192 155 and 140; one of 2048 among 255 short ones 74 and 58;
+//   nothing helps 192 x 4096, three full rounds, 189 and 191, 96 x 9000 of 16 heads over 2 88 and 90, 128 of 256 coordinates, one
+//   of 4096 tokens among short ones, 16 heads over 4, 92 and 94.
+// Not where no chunk can be larger than the smallest (`room`) and at most two rounds are there to be ordered: 128 x 16,384, 16 heads
+// over 2, 137 and 140, of 2048 to 16,384 127 and 129.
+// Not with chunks below 384 rows: short workgroups feel the search most.  80 x 1200 tokens would gain, 45 and 37, but of 150 to 1200,
+// one round either way, 43.4 become 44.7; 96 x 7000 on one KV head 46 and 38, of 900 to 7000 28.9 and 29.8.
+// `many` false: not at all beyond 64 sequences.  That is so for rows of tokens at 256 coordinates: one KV head, 96 x 16,000 136
+// and 139, 200 of 1250 to 10,000 131 and 136; two, 128 x 9000 158 and 163, though of 1125 to 9000 153 and 133.
+inline int staged_balance_slots(int num_seqs, int num_splits, int groups, int max_blocks, int rows_per_page, bool many = true) {
     const int cus = fq_host::device_cu_count();
-    const int64_t pairs = int64_t(num_seqs) * num_splits;
-    const bool few = num_seqs <= kWave, many = num_seqs <= kBalanceSeqs && pairs < 65536 && chunk >= 384;
-    return pairs > cus && (few || many) ? cus : 0;
+    const int64_t pairs = int64_t(num_seqs) * num_splits * groups;
+    if (pairs <= cus) return 0;
+    if (num_seqs > kWave) {
+        const int64_t chunk = chunk_of(int64_t(max_blocks) * rows_per_page, num_splits);
+        // (a split keeps at most 256 page ids, or the whole row of the block table)
+        const int64_t room = max_blocks <= 4 * kWave ? chunk * num_splits : int64_t(4 * kWave) * rows_per_page;
+        const bool helps = room > chunk || pairs > 2 * int64_t(cus);
+        if (!many || num_seqs > kBalanceSeqs || pairs >= 65536 || chunk < 384 || !helps) return 0;
+    }
+    return cus / groups > 0 ? cus / groups : 1;
 }
 
 // Polls of a bounded wait between the wavefronts of the staged kernel.
@@ -2279,16 +2290,16 @@ int launch_partials(const DecodeParams& p, int S, int BS, hipStream_t stream, co
     if constexpr (D == 256) {
         if (p.new_key == nullptr && p.rotation == nullptr && staged_d256_linear_applies(D, p.H_KV, BS, var)) {
             DecodeParams ps = p;
-            ps.balance_slots = staged_balance_slots(S, p.num_splits, 0);
-            return launch_staged_d256_linear<DT>(ps, S, BS * p.H_KV / 4, stream);
+            const int rows_per_page = BS * p.H_KV / 4;
+            ps.balance_slots = staged_balance_slots(S, p.num_splits, 1, p.max_blocks, rows_per_page, /*many=*/false);
+            return launch_staged_d256_linear<DT>(ps, S, rows_per_page, stream);
         }
         if (p.new_key == nullptr && p.rotation == nullptr && staged_d256_applies(D, p.H_KV, var)) {
             const int64_t max_ctx = int64_t(p.max_blocks) * BS;
             const int64_t chunk = (((max_ctx + p.num_splits - 1) / p.num_splits) + 63) & ~int64_t(63);
             DecodeParams ps = p;
             const int groups = p.H_KV / 4;
-            ps.balance_slots = staged_balance_slots(S, p.num_splits * groups, chunk);
-            if (ps.balance_slots > 0) ps.balance_slots = ps.balance_slots / groups > 0 ? ps.balance_slots / groups : 1;
+            ps.balance_slots = staged_balance_slots(S, p.num_splits, groups, p.max_blocks, BS);
             const bool wide = chunk / BS > 64 || ps.balance_slots > 0 || (p.max_blocks > 64 && p.max_blocks <= 256);
             return launch_staged_d256<DT>(ps, S, BS, wide, stream);
         }
@@ -2302,8 +2313,7 @@ int launch_partials(const DecodeParams& p, int S, int BS, hipStream_t stream, co
             DecodeParams ps = p;
             ps.G = 2 * p.G;                 // query heads of a pair of KV heads
             const int groups = d64_half ? 1 : p.H_KV / 16;
-            ps.balance_slots = staged_balance_slots(S, p.num_splits * groups, chunk_rows);
-            if (ps.balance_slots > 0) ps.balance_slots = ps.balance_slots / groups > 0 ? ps.balance_slots / groups : 1;
+            ps.balance_slots = staged_balance_slots(S, p.num_splits, groups, p.max_blocks, rows_per_page);
             const bool wide_rows = chunk_rows / rows_per_page > 64 || ps.balance_slots > 0 || (p.max_blocks > 64 && p.max_blocks <= 256);
             return launch_staged_d64<DT>(ps, S, rows_per_page, wide_rows, d64_half, stream);
         }
@@ -2311,7 +2321,7 @@ int launch_partials(const DecodeParams& p, int S, int BS, hipStream_t stream, co
     if (staged_linear_applies(D, p.H_KV, BS, var)) {     // (one partial per split: also for callers that bring their own partial buffers)
         const int rows_per_page = BS * p.H_KV / 8;
         DecodeParams ps = p;
-        ps.balance_slots = staged_balance_slots(S, p.num_splits, chunk_of(int64_t(p.max_blocks) * rows_per_page, p.num_splits));
+        ps.balance_slots = staged_balance_slots(S, p.num_splits, 1, p.max_blocks, rows_per_page);
         return launch_staged_linear<DT>(ps, S, rows_per_page, stream);
     }
     // pages a split can span: its tokens are ceil(max_ctx / splits) rounded up to a tile
@@ -2324,8 +2334,7 @@ int launch_partials(const DecodeParams& p, int S, int BS, hipStream_t stream, co
         DecodeParams ps = p;
         // every group of 8 heads is a slice of the grid with the same (sequence, split) pairs
         const int groups = p.H_KV / 8;
-        ps.balance_slots = staged_balance_slots(S, p.num_splits * groups, chunk);
-        if (ps.balance_slots > 0) ps.balance_slots = ps.balance_slots / groups > 0 ? ps.balance_slots / groups : 1;
+        ps.balance_slots = staged_balance_slots(S, p.num_splits, groups, p.max_blocks, BS);
         // a chosen chunk may span up to 256 pages: four page-id registers
         if (var.ring && p.new_key != nullptr) return FQ_ERR_LAUNCH;
         if (var.ring)
@@ -2853,8 +2862,7 @@ extern "C" int fq_prod_paged_decode(const void* q, const uint8_t* kv_cache, cons
     p.scale_log2e = sm_scale * kLog2e;
     // every group of 8 heads is a slice of the grid with the same (sequence, split) pairs
     const int groups = H_KV / 8;
-    p.balance_slots = staged_balance_slots(num_seqs, num_splits * groups, chunk_of(int64_t(max_blocks_per_seq) * block_size, num_splits));
-    if (p.balance_slots > 0) p.balance_slots = p.balance_slots / groups > 0 ? p.balance_slots / groups : 1;
+    p.balance_slots = staged_balance_slots(num_seqs, num_splits, groups, max_blocks_per_seq, block_size);
     p.heads_per_wg = 0;
     p.spin_limit = handoff_polls();
     p.cache_rw = nullptr; p.new_key = nullptr; p.new_value = nullptr; p.new_slots = nullptr; p.boundaries = nullptr;

@@ -42,33 +42,55 @@ struct DecodeParams {
 };
 
 
-// balance_chunks for 65 to 256 sequences, four a lane: eight candidates (to 1.9 times the smallest chunk; lane j holds the
-// j-th), the workgroups of two of them added up at a time.  Every workgroup pays for this, also one without work: a first form
-// with 16 candidates, each one's cost worked out in all lanes, took 3.4 us (80 sequences of 60 to 1200 tokens, 8 KV heads of 64:
-// 23.5 -> 26.9 us).  Where the smallest chunk makes one round, nothing is better and all stays as it was.
+// Sum of the lanes up to and including this one.
+__device__ __forceinline__ int wave_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);    // row_shr:1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);    // row_bcast:15 to rows 1 and 3, :31 to rows 2 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+    return v;
+}
+
+// x / d rounded up, both below 2^24 and the quotient below 2^18, rc about 1 / d (a division of integers takes four times the
+// instructions).
+__device__ __forceinline__ int quotient_up(int x, int d, float rc) {
+    const int q = int(float(x) * rc), r = x - q * d;           // q is off by one at most
+    return q + (r > 0 ? 1 : 0) + (r > d ? 1 : 0) - (r <= -d ? 1 : 0);
+}
+
+// balance_chunks for 65 to 256 sequences, four a lane: nine candidates (lane j holds the j-th; eight in steps of an eighth of the
+// smallest chunk, rounded up to 64 rows, and exactly twice the smallest), the workgroups of two of them added up at a time.
+// The cost of a candidate is that of its rounds of workgroups as long as the longest, or, where most are shorter, of a CU's share
+// of all rows and prologues and the longest workgroup on top (256 sequences of which one has 2048 tokens and the others at most
+// 340: 59 us, and 96 with the rounds alone, which saw 257 workgroups of 1024 rows against 256 of 2048).
+// Every workgroup pays for this, also one without work and one of a batch that nothing helps, so it is short: where the
+// smallest chunk makes one round, or is the best and leaves no pair without work, all stays as it was.  Twice the smallest
+// chunk is what a batch of equal lengths in an even number of rounds gains by, half the rounds with a prologue less.
 template <int TPR>
 __device__ __forceinline__ void balance_chunks_many(const DecodeParams& p, int lane, int NS, int cap, int max_tokens, int& chunk,
                                                     int& seq, int& split, int& L_known) {
-    constexpr int K = 4, CANDS = 8;
+    constexpr int K = 4, CANDS = 9;
     const int nseq = int(gridDim.x);
-    int l_real[K];
-    float rows[K];
+    int l_real[K], rows[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         const int at = K * lane + k;
         const int l = p.seq_lens[at < nseq ? at : nseq - 1];
         l_real[k] = at >= nseq || l < 0 ? 0 : (l > max_tokens ? max_tokens : l);
-        rows[k] = float((l_real[k] + TPR - 1) / TPR);
+        rows[k] = (l_real[k] + TPR - 1) / TPR;
     }
-    int cand = chunk + (lane & (CANDS - 1)) * (((chunk >> 3) + 63) & ~63);
+    int cand = lane >= CANDS - 1 ? 2 * chunk : chunk + lane * (((chunk >> 3) + 63) & ~63);
     cand = cand < cap ? cand : cap;
     cand = cand > chunk ? cand : chunk;
     const int rc_mine = int(__builtin_bit_cast(uint32_t, __builtin_amdgcn_rcpf(float(cand))));
+    auto rc_of = [&](int j) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(rc_mine, j)); };
     auto groups_of = [&](int j) {                              // (the host sees to it that 16 bits hold the sum)
-        const float rc = __builtin_bit_cast(float, __builtin_amdgcn_readlane(rc_mine, j));
+        const float rc = rc_of(j);
         float n = 0.0f;
 #pragma unroll
-        for (int k = 0; k < K; ++k) n += __builtin_ceilf(rows[k] * rc - 0.0009765625f);
+        for (int k = 0; k < K; ++k) n += __builtin_ceilf(float(rows[k]) * rc - 0.0009765625f);
         return uint32_t(n);
     };
     auto length_of = [&](int sq) {
@@ -80,42 +102,49 @@ __device__ __forceinline__ void balance_chunks_many(const DecodeParams& p, int l
         }
         return l;
     };
-    if (int(wave_sum(groups_of(0))) <= p.balance_slots) {
+    const uint32_t smallest = wave_sum(groups_of(0));
+    int best = 0;
+    if (int(smallest) > p.balance_slots) {
+        uint32_t mine = smallest, total = 0;
+        float longest = 0.0f;
+#pragma unroll
+        for (int j = 1; j < CANDS; j += 2) {
+            const uint32_t both = wave_sum(groups_of(j) | groups_of(j + 1) << 16);
+            mine = lane == j ? both & 0xffffu : (lane == j + 1 ? both >> 16 : mine);
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            total += uint32_t(rows[k]);
+            longest = __builtin_fmaxf(longest, float(rows[k]));
+        }
+        const float per_slot = __builtin_amdgcn_rcpf(float(p.balance_slots)), n = float(mine);
+        const float work = (float(wave_sum(total)) + 96.0f * n) * per_slot;
+        const float rounds = __builtin_ceilf(n * per_slot - 0.0009765625f);
+        const float largest = __builtin_fminf(float(cand), wave_max(longest)) + 96.0f;
+        const float cost = lane < CANDS ? __builtin_fminf(__builtin_fmaxf(rounds, 1.0f) * largest, work + largest) : __builtin_inff();
+        const uint64_t cheapest = __ballot(cost == -wave_max(-cost));
+        best = __ffsll(static_cast<unsigned long long>(cheapest)) - 1;
+    }
+    if (int(smallest) <= p.balance_slots || (best == 0 && int(smallest) == nseq * NS)) {
         L_known = length_of(seq);
         return;
     }
-    uint32_t mine = 0;
-#pragma unroll
-    for (int j = 0; j < CANDS; j += 2) {
-        const uint32_t both = wave_sum(groups_of(j) | groups_of(j + 1) << 16);
-        mine = lane == j ? both & 0xffffu : (lane == j + 1 ? both >> 16 : mine);
-    }
-    const float rounds = __builtin_ceilf(float(mine) * __builtin_amdgcn_rcpf(float(p.balance_slots)) - 0.0009765625f);
-    const float cost = lane < CANDS ? (rounds < 1.0f ? 1.0f : rounds) * float(cand + 96) : __builtin_inff();
-    const uint64_t cheapest = __ballot(cost == -wave_max(-cost));
-    chunk = __builtin_amdgcn_readlane(cand, __ffsll(static_cast<unsigned long long>(cheapest)) - 1);
+    chunk = __builtin_amdgcn_readlane(cand, best);
+    const float rc = rc_of(best);
     int n[K], live = 0, dead = 0;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        n[k] = ((l_real[k] + TPR - 1) / TPR + chunk - 1) / chunk;
+        n[k] = quotient_up(rows[k], chunk, rc);
         n[k] = n[k] < NS ? n[k] : NS;
         live += n[k];
         dead += K * lane + k < nseq ? NS - n[k] : 0;
     }
-    auto scan = [&](int v) {
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int t = __shfl_up(v, d, kWave);
-            v += lane >= d ? t : 0;
-        }
-        return v;
-    };
     // the w-th of the live pairs, else of the empty ones: the lane that holds it, then which of its sequences
-    const int live_incl = scan(live);
+    const int live_incl = wave_scan(live);
     const int total_live = __builtin_amdgcn_readlane(live_incl, 63);
     const int w = int(blockIdx.x) + int(gridDim.x) * int(blockIdx.y);
     const bool is_live = w < total_live;
-    const int incl = is_live ? live_incl : scan(dead), e = is_live ? w : w - total_live;
+    const int incl = is_live ? live_incl : wave_scan(dead), e = is_live ? w : w - total_live;
     int sl = __builtin_popcountll(__ballot(incl <= e));
     sl = sl < (nseq - 1) / K ? sl : (nseq - 1) / K;
     int rem = e - __builtin_amdgcn_readlane(incl - (is_live ? live : dead), sl);
@@ -134,7 +163,7 @@ __device__ __forceinline__ void balance_chunks_many(const DecodeParams& p, int l
     L_known = length_of(seq);
 }
 
-// Most sequences of a batch whose chunks follow from the actual lengths. 
+// Most sequences of a batch whose chunks follow from the actual lengths.
 constexpr int kBalanceSeqs = 256;
 
 // Ragged batches of long contexts (at most 64 sequences here, one lane each; more above).  With the chunk
