@@ -36,12 +36,14 @@ namespace fq {
 constexpr int kSplitMinTiles = 4;
 
 // Batches of more sequences than this are not ordered.  Every workgroup finds its own item, and the search for the longest
-// ones reads all lengths some fifteen times: 1 us up to 64 sequences, 40 us at 1024 (a workgroup's own time is 40 to 60).
+// ones reads all lengths about seven times (the first 64 once): 20 us at 1024 sequences, where a workgroup's own time is 30 to 60.
 // Beyond it a workgroup counts through the sequences once, or, where the grid has at most two places for every workgroup that
-// the batch can need, its place says which sequence it is.  32 query heads over 8 of 128, bf16, in us (grid order of all
-// sequences / ordered / not ordered): 256 sequences, sixteen of them prompts of up to 512 tokens, 1910 / 568 / 547, at one KV
-// head 175 / 98 / 122, 16 heads over 4 of 256 11,400 / 952 / 1014; 384 sequences 2804 / 904 / 751; 1024 single queries
-// 2060 / 2849 / 1630, 4096 8080 / 32,700 / 6400; 2048 prompts of 30 to 300 tokens 7409 / 16,800 / 4823.
+// the batch can need, its place says which sequence it is.  bf16, in us, ordered / not ordered, 32 query heads over 8 of 128, 8
+// over 1 of 128, 16 over 4 of 256: 256 sequences, sixteen of them prompts of 32 to 512 tokens, the others one query over 100 to
+// 2000, 433 / 437, 92 / 113, 587 / 736; 384 of them 709 / 657, 127 / 155, 917 / 1069; 512 988 / 882, 169 / 187, 1228 / 1366; 1024
+// 1854 / 1337, 283 / 236, 1859 / 1737.  256 single queries over 100 to 1000 257 / 246, 56 / 48, 340 / 409, 1024 1637 / 982,
+// 234 / 180, 1727 / 1542; 256 prompts of 30 to 300 tokens 687 / 590, 162 / 174, 817 / 865, 512 1686 / 1125, 383 / 327, 1693 / 1618.
+// In the order of the grid, all sequences with as many workgroups as the longest, 1024 single queries took 2060.
 constexpr int kOrderSeqs = 256;
 
 // One sequence as the kernel sees it.
@@ -145,7 +147,7 @@ FQ_HD int first_piece_with(const SeqShape& s, int T, int pieces, int G, bool cau
 // of one known length under a causal mask) is about one round of workgroups, the longest with twice the average work: two
 // pieces, if half of the longest workgroup outweighs that traffic and the second prologues too.  (Whether the shares are
 // uneven enough pieces_of decides; more workgroups than 4/3 of a round never are.)  8 heads x 6000 tokens of 256 coordinates,
-// one KV head, 188 workgroups: 538 us in one piece, 336 us in two; 16 heads x 3001 tokens on 4 KV heads 307 and 220 us (208 now).  Else only
+// one KV head, 188 workgroups: 538 us in one piece, 336 us in two; 16 heads x 3001 tokens on 4 KV heads 307 and 220 us (203 now).  Else only
 // sequences of one workgroup (single queries of a mixed batch) are.
 struct SplitPlan {
     int split_w, max_pieces;

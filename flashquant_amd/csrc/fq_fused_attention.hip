@@ -32,12 +32,12 @@
 // permutation on the coordinates, and the query operand is read to match.
 //
 // head_dim 256: tiles of 32 tokens (the accumulators of 32 rows, their query operand and the scores are 208 of a lane's
-// 256 registers, and 7 to 58 are spilled around the ends), the second product in groups of two coordinate blocks, the rotation
+// 256 registers, and 7 to 37 are spilled around the ends), the second product in groups of two coordinate blocks, the rotation
 // matrix in four rounds through LDS (it is 256 KB in two terms).  Per flop the tile loop costs what it costs at 128: 2.6 us for
 // 256 rows x 32 tokens, bound like it by the chain K reads - scores - weights - V reads - output.  The general kernel
 // (fq_attention_any_dim.hip), which served this dimension with 16 rows a wavefront, read twice the LDS bytes per row: 2 x 32 x
-// 700 tokens bf16 260 -> 110 us, 16 x 65 tokens 92 -> 51 us, 2 x 16 x 8192 tokens 4.11 -> 1.97 ms; in pieces 16 heads x 3001
-// tokens fp16 516 -> 208 us, one query over 3 x 3500 tokens 350 -> 57 us.
+// 700 tokens bf16 260 -> 110 us, 16 x 65 tokens 92 -> 51 us, 2 x 16 x 8192 tokens 4.11 -> 1.92 ms; in pieces 16 heads x 3001
+// tokens fp16 516 -> 203 us, one query over 3 x 3500 tokens 350 -> 57 us.
 //
 // The two head rotations run inside the kernel (prologue and epilogue) on the fp16 MFMA
 // with operands split into two fp16 terms, staged through the tile buffers.
@@ -459,8 +459,8 @@ __device__ __forceinline__ void finish_rows(const PrefillParams& p, RotationBloc
 }
 
 // Where a workgroup's work comes from and what becomes of its rows.  At 256 coordinates the end of a workgroup beside the
-// branch that leaves its rows to the combine costs 170 to 220 spilled registers, some of them inside the tile loop, either
-// one alone 8 to 58: 8 sequences of 120 queries over 1500 keys, 32 heads, 226 us with both compiled in, 170 with one.
+// branch that leaves its rows to the combine costs 157 to 195 spilled registers, some of them inside the tile loop, either
+// one alone 7 to 37: 8 sequences of 120 queries over 1500 keys, 32 heads, 226 us with both compiled in, 170 with one.
 enum Work {
     kGrid,            // one workgroup per grid position, rows finished in the kernel
     kOrdered,         // find_item, the same (paged)
@@ -510,7 +510,7 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     // chain (its work, the query rows, the rotation, the first tile); with the matrix fetched under the search, its operands
     // where the tiles will be, so that the tables are filled meanwhile, and wavefronts without a unit out of the
     // products, the first tile of one query over 4 x 2500 ring-buffer tokens begins after 6.5 us instead of 9.7 (24.3 -> 21.9 us
-    // in all), 16 heads x 3001 tokens of 256 coordinates 219 -> 208 us.
+    // in all), 16 heads x 3001 tokens of 256 coordinates 220 -> 208 us.
     SeqShape first{};
     if constexpr (kFind && PAGED) first = lane_shape(p, 0, lane);
     const float cent_k = p.centroids_k[lane & 15], cent_v = p.centroids_v[lane & 15];
@@ -1209,7 +1209,7 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillPar
 // The same for whole prompts in pieces, where the rotation is the work: a workgroup as the one that left the pieces, its
 // wavefronts gather their 32 rows in the accumulators and end as that kernel does (the kernel above fetches and splits the
 // matrix for every 16 rows).  When it was added, 16 heads x 3001 tokens of 256 coordinates, 188 workgroups in two pieces: 298 us
-// with the kernel above, 240 with this one (208 now); 8 heads x 5000 tokens of 128, 157 workgroups: 140 and 121; 16 heads x
+// with the kernel above, 240 with this one (203 now); 8 heads x 5000 tokens of 128, 157 workgroups: 140 and 121; 16 heads x
 // 2000 tokens of 64, 128 workgroups: 54.6 and 48.3 (45.8 now).  With 63 workgroups in four pieces the smaller workgroups above
 // are faster (128 and 148 us at 256 coordinates, 55 and 68 at 128): this one runs from half a round of workgroups on.  At 256
 // coordinates the rounds of the matrix share one area (64 KB, so that two workgroups fit a CU): with two of them 14 registers

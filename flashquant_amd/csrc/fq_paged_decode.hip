@@ -773,8 +773,9 @@ __global__ __launch_bounds__(512 + 64 * CW) void paged_decode_staged_kernel(cons
     const int tsel = (h / HPR) & (TPR - 1);
 
     // Every load that depends on nothing is asked for first, so that the memory
-    // latencies of the prologue overlap instead of adding up: the centroids, the
-    // rotation columns of this wavefront and the first 32 query heads.
+    // latencies of the prologue overlap instead of adding up: the centroids and, without copy
+    // wavefronts, the rotation columns of this wavefront (with them the lengths, page ids, query heads
+    // and new rows go before the columns, which are the last to be needed).
     // K table in the lower 128 bytes of every 256-byte table row (32 copies, one per bank),
     // V table in the upper 128 bytes
     const float cent_k_mine = p.centroids_k[lane & (PROD ? 7 : 15)];
