@@ -181,3 +181,21 @@ def test_captured_step_of_many_sequences_over_other_lengths(hq, hkv, splits, ctx
         step(cache_e, out_e)
         torch.cuda.synchronize()
         assert torch.equal(out_g, out_e) and torch.equal(cache_g, cache_e), kind
+
+
+@pytest.mark.parametrize("kind", ["alike", "ragged", "sparse"])
+def test_ring_kernel_with_many_sequences(kind):
+    """The ring kernel takes its chunks from the same search as the staged one."""
+    C, (n, hq, hkv, d, bs, splits, ctx) = load_native(), (130, 32, 8, 128, 16, 3, 2500)
+    c, _, r = (t.to(DEV) for t in book(d))
+    _, cache, table, q = _tq4_inputs(n, hq, hkv, d, bs, ctx, torch.bfloat16)
+    sl = torch.tensor(_lens(n, ctx, kind), dtype=torch.int32, device=DEV)
+    old = C.set_option("decode_ring", 1)
+    try:
+        got = K.split_k_paged_decode(q, cache, table, sl, c, c, r, hkv, d, bs, num_splits=splits, out=torch.full_like(q, 7.0))
+    finally:
+        C.set_option("decode_ring", old)
+    with torch.device(DEV):
+        want = O.split_k_paged_decode(q, cache, table, sl, c, c, r, hkv, d, bs)
+    assert _worst_row(got[sl > 0], want[sl > 0]) <= LIMIT[torch.bfloat16]
+    assert (got[sl == 0] == 0).all()
