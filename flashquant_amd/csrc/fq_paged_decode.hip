@@ -1278,7 +1278,8 @@ __global__ __launch_bounds__(512 + 64 * CW) void paged_decode_staged_kernel(cons
 #pragma unroll
                     for (int j = 0; j < KS; ++j) raw[j] = *reinterpret_cast<const uint4v*>(stage + kQStage + n * kNewStride + 64 * j + 16 * g);
                     // Later steps read what is stored here, also when this one's output is NaN: rows that may not be in `stage`
-                    // yet are fetched from where they came.
+                    // yet are fetched from where they came.  (The branch costs 0 to 0.2 us: 32 sequences of 18 to 72 tokens at
+                    // 64 coordinates 16.4 and 16.6 us, one of 777, 32 heads over 8 of 128, 17.6 either way.)
                     if (__builtin_expect(handoff_failed, 0)) {
 #pragma unroll
                         for (int j = 0; j < KS; ++j) raw[j] = *reinterpret_cast<const uint4v*>(new_row(n) + 32 * j + 8 * g);
