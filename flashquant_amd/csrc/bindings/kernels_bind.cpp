@@ -477,8 +477,8 @@ void tq4_compress_append(const at::Tensor& x, const at::Tensor& rot_T_even, cons
 
 // Room for the partial results of attention over split contexts; undefined where these sizes are never split.
 at::Tensor attention_workspace(const at::Tensor& q, int64_t seqs, int64_t max_q, int64_t max_kv, int64_t HQ, int64_t HKV, int64_t D,
-                               bool prompts) {
-    const size_t bytes = fq_attention_workspace_bytes(int(seqs), int(max_q), max_kv, int(HQ), int(HKV), int(D), prompts ? 1 : 0);
+                               int prompts) {
+    const size_t bytes = fq_attention_workspace_bytes(int(seqs), int(max_q), max_kv, int(HQ), int(HKV), int(D), prompts);
     return bytes == 0 ? at::Tensor() : at::empty({int64_t(bytes)}, q.options().dtype(at::kByte));
 }
 
@@ -527,7 +527,7 @@ at::Tensor fused_tq_attention(const at::Tensor& q, const at::Tensor& k_packed, c
     const at::Tensor ck = centroids_k.to(q.device()).contiguous(), cv = centroids_v.to(q.device()).contiguous();
     const RotationArg rot = rotation_arg(rotation, q.device(), D);
     at::Tensor result = at::empty_like(qc);
-    const at::Tensor ws = attention_workspace(q, B, NQ, NKV, HQ, HKV, D, is_causal);
+    const at::Tensor ws = attention_workspace(q, B, NQ, NKV, HQ, HKV, D, is_causal ? 1 : 2);
     const int st = fq_fused_tq_attention_split(
         qc.data_ptr(), kp.data_ptr<uint8_t>(), kn.data_ptr<float>(), vp.data_ptr<uint8_t>(), vn.data_ptr<float>(),
         ck.data_ptr<float>(), cv.data_ptr<float>(), rot.ptr, rot.col_major, result.data_ptr(),
@@ -579,7 +579,7 @@ at::Tensor paged_tq4_prefill(const at::Tensor& q, const at::Tensor& cu_seqlens_q
     } else {
         result = at::zeros_like(qc);
     }
-    const at::Tensor ws = attention_workspace(q, S, max_seqlen_q, bt.size(1) * block_size, HQ, num_kv_heads, head_dim, false);
+    const at::Tensor ws = attention_workspace(q, S, max_seqlen_q, bt.size(1) * block_size, HQ, num_kv_heads, head_dim, 0);
     const int st = fq_paged_tq4_prefill_split(
         qc.data_ptr(), cu.data_ptr<int32_t>(), kv_cache.data_ptr<uint8_t>(), bt.data_ptr<int32_t>(),
         sl.data_ptr<int32_t>(), ck.data_ptr<float>(), cv.data_ptr<float>(), rot.ptr, rot.col_major, result.data_ptr(),

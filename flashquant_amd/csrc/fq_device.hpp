@@ -386,4 +386,24 @@ __device__ __forceinline__ float4v rotate_block_f16x3(const half8 (&ahi)[D / 32]
     return acc_hi + acc_lo * (1.0f / 4096.0f);
 }
 
+// the power of two that brings a row's largest magnitude (over both lane halves) into [1, 2)
+__device__ __forceinline__ int row_exponent(float mx) {
+    mx = max_xor32(mx);
+    const int ex = int((float_to_bits(mx) >> 23) & 0xffu) - 127;
+    return (ex < -100 || ex > 100) ? 0 : ex;
+}
+__device__ __forceinline__ float pow2(int e) { return bits_to_float(uint32_t(127 + e) << 23); }
+
+// A pair of weights as fp16: towards zero in one instruction, at 256 coordinates to nearest.  Against 64 bits, fp16, 16 heads
+// x 3001 tokens: relative error 8.9e-4 on the general kernel that served this dimension, 9.1e-4 towards zero, 8.9e-4 to nearest.
+template <int D>
+__device__ __forceinline__ uint32_t pack_weights(float a, float b) {
+    if constexpr (D == 256) {
+        const half2v h = {_Float16(a), _Float16(b)};
+        return __builtin_bit_cast(uint32_t, h);
+    } else {
+        return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
+    }
+}
+
 }  // namespace fq

@@ -44,6 +44,7 @@
 #include "fq_common.hpp"
 #include "fq_device.hpp"
 #include "fq_attention_any_dim.hpp"
+#include "fq_attention_expanded.hpp"
 #include "fq_attention_schedule.hpp"
 
 namespace fq {
@@ -103,18 +104,6 @@ struct PrefillParams {
 __device__ __forceinline__ uint32_t scale_pair(uint32_t pair, half2v n2) {
     const half2v h = __builtin_bit_cast(half2v, pair) * n2;
     return __builtin_bit_cast(uint32_t, h);
-}
-
-// A pair of weights as fp16: towards zero in one instruction, at 256 coordinates to nearest.  Against 64 bits, fp16, 16 heads
-// x 3001 tokens: relative error 8.9e-4 on the general kernel that served this dimension, 9.1e-4 towards zero, 8.9e-4 to nearest.
-template <int D>
-__device__ __forceinline__ uint32_t pack_weights(float a, float b) {
-    if constexpr (D == 256) {
-        const half2v h = {_Float16(a), _Float16(b)};
-        return __builtin_bit_cast(uint32_t, h);
-    } else {
-        return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
-    }
 }
 
 template <bool PAGED>
@@ -360,14 +349,6 @@ struct RotationBlocks {
         }
     }
 };
-
-// the power of two that brings a row's largest magnitude (over both lane halves) into [1, 2)
-__device__ __forceinline__ int row_exponent(float mx) {
-    mx = max_xor32(mx);
-    const int ex = int((float_to_bits(mx) >> 23) & 0xffu) - 127;
-    return (ex < -100 || ex > 100) ? 0 : ex;
-}
-__device__ __forceinline__ float pow2(int e) { return bits_to_float(uint32_t(127 + e) << 23); }
 
 // The end of a workgroup: the rows in the accumulators normalised, rotated back (the first round of the matrix already lies
 // in LDS) and stored.  EARLY: with two areas the second round is asked for before the rows are converted, else after.
@@ -1373,7 +1354,10 @@ extern "C" size_t fq_attention_workspace_bytes(int num_seqs, int max_q_len, int6
                                                int prompts) {
     using namespace fq;
     if (num_seqs <= 0 || max_q_len <= 0 || max_kv_len <= 0 || H_KV <= 0 || H_Q <= 0 || H_Q % H_KV != 0) return 0;
-    return part_bytes(plan_of(num_seqs, max_q_len, max_kv_len, H_Q, H_KV, D, prompts != 0 && max_q_len > 1), num_seqs, H_KV, D);
+    const size_t split = part_bytes(plan_of(num_seqs, max_q_len, max_kv_len, H_Q, H_KV, D, prompts == 1 && max_q_len > 1), num_seqs, H_KV, D);
+    if (prompts == 0 || fq_host::force_any_dim_attention()) return split;
+    const size_t expanded = plan_expanded(int64_t(num_seqs) * H_KV, max_q_len, max_kv_len, H_Q / H_KV, D, prompts == 1).bytes;
+    return expanded > split ? expanded : split;
 }
 
 extern "C" int fq_fused_tq_attention_strided(const void* q, const uint8_t* k_packed, const float* k_norms,
@@ -1423,6 +1407,33 @@ extern "C" int fq_fused_tq_attention_split(const void* q, const uint8_t* k_packe
         a.causal = (is_causal && N_Q > 1) ? 1 : 0;
         a.scale_log2e = sm_scale * kLog2e;
         return launch_attention_any_dim(a, D, false, N_Q, B, dtype, stream);
+    }
+
+    const ExpandedPlan ep = plan_expanded(int64_t(B) * H_KV, N_Q, N_KV, H_Q / H_KV, D, is_causal && N_Q > 1);
+    if (ep.per_chunk > 0 && workspace != nullptr && workspace_bytes >= ep.bytes) {
+        if (!fq_host::aligned(workspace, 256)) return FQ_ERR_MISALIGNED;
+        uint8_t* ws = static_cast<uint8_t*>(workspace);
+        ExpandParams e{};
+        e.k_packed = k_packed; e.k_norms = k_norms; e.v_packed = v_packed; e.v_norms = v_norms;
+        e.centroids_k = centroids_k; e.centroids_v = centroids_v;
+        e.rotation = rotation; e.rot_col_major = rotation_col_major;
+        e.k_cap = k_capacity; e.v_cap = v_capacity;
+        e.keys = ep.keys; e.tiles = ep.tiles;
+        e.images = ws;
+        e.flags = reinterpret_cast<int*>(ws + ep.images);
+        e.exps = reinterpret_cast<int*>(ws + ep.images + ep.flags);
+        AttendParams a{};
+        a.q = static_cast<const uint16_t*>(q);
+        a.out = static_cast<uint16_t*>(out);
+        a.images = e.images; a.flags = e.flags; a.exps = e.exps;
+        a.H_Q = H_Q; a.H_KV = H_KV; a.G = H_Q / H_KV; a.N_Q = N_Q; a.N_KV = ep.keys;
+        a.causal = (is_causal && N_Q > 1) ? 1 : 0;
+        a.scale_log2e = sm_scale * kLog2e;
+        a.tiles = ep.tiles;
+        a.round_slots = fq_host::device_cu_count();
+        a.W = ((N_Q + 31) / 32 * a.G + 3) / 4;
+        a.out_wide = fq_host::aligned(out, 16);
+        return launch_attention_expanded(e, a, D, dtype, int64_t(B) * H_KV, ep.per_chunk, stream);
     }
 
     PrefillParams p;

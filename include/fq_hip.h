@@ -327,10 +327,14 @@ int fq_paged_tq4_prefill(const void* q, const int32_t* cu_seqlens_q, const uint8
  * different CUs, and a second launch combines their results (rounded as the unsplit result is; rows that are no numbers in
  * one piece are none in several).  The pieces follow from the whole batch, the longest context possible and the number of
  * CUs: the last bits of a row may differ with the batch that it is in.
- *   workspace        256-byte aligned, at least fq_attention_workspace_bytes bytes (0: these sizes are never split; at
- *                    most 65 MiB paged, 172 MiB for whole prompts); NULL: nothing is split
+ * Where many queries share their keys, fq_fused_tq_attention_split first writes keys and values, rotated back, as fp16
+ * matrix operands into the workspace and attends to these (no rounding of the rotated query, fewer of the keys and values).
+ *   workspace        256-byte aligned, at least fq_attention_workspace_bytes bytes (0: these sizes need none; at
+ *                    most 65 MiB paged, 172 MiB for prompts in pieces, 1.1 GiB for expanded keys and values); NULL:
+ *                    nothing is split or expanded.  With what suffices for pieces alone nothing is expanded.
  *   max_kv_len       the longest context possible: N_KV, or max_blocks_per_seq * block_size
- *   prompts          1: for fq_fused_tq_attention_split with is_causal (all sequences have these very lengths), else 0
+ *   prompts          for fq_fused_tq_attention_split 1 with is_causal, 2 without (all sequences have these very lengths);
+ *                    else 0
  *   total_q          cu_seqlens_q[num_seqs] where the caller knows it (sizes the grid), else 0
  */
 size_t fq_attention_workspace_bytes(int num_seqs, int max_q_len, int64_t max_kv_len, int H_Q, int H_KV, int D,

@@ -1,0 +1,141 @@
+"""Attention over expanded keys and values (many queries that share their keys): edges of the 32-row units, of the tiles and of the
+blocks of 32 tokens, numbers of heads and pairs that the workgroups and the XCDs do not divide, long norms, numbers that are none."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from flashquant_amd import kernels as K
+from oracle import tq_oracle as O
+from tests.gpu_util import attention_in_one_piece, attention_workspace_bytes, book
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _expanded(b, hkv, hq, nq, nkv, d, causal):
+    """Whether a call of these sizes asks for room for its keys and values as fp16 (in tiles of 64 tokens, 32 at 256)."""
+    tile = 32 if d == 256 else 64
+    keys = min(nq, nkv) if causal else nkv
+    return attention_workspace_bytes(b, nq, nkv, hq, hkv, d, 1 if causal else 2) >= b * hkv * -(-keys // tile) * tile * d * 4
+
+
+def _inputs(b, hq, hkv, nq, nkv, d, dtype, seed):
+    c, bnd, r = book(d)
+    g = torch.Generator().manual_seed(seed)
+    kv = []
+    for _ in range(2):
+        p, m = O.compress(torch.randn(b * hkv * nkv, 1, d, generator=g), r, bnd)
+        kv += [p.reshape(b, hkv, nkv, d // 2), m.reshape(b, hkv, nkv, 1)]
+    return torch.randn(b, hq, nq, d, generator=g).to(dtype), kv, c, r
+
+
+def _attend(q, kv, c, r, causal, dev=DEV):
+    return K.fused_tq_attention(q.to(dev), *[t.to(dev) for t in kv], c.to(dev), c.to(dev), r.to(dev), is_causal=causal)
+
+
+def _close(got, want, dtype):
+    """2-norms: bf16 rounds the rotated query (the oracle alone), the output there and here, 2^-9 of the norm each; fp16 the
+    same, and keys, values and weights are held in fp16 (2^-12, the weights towards zero 2^-11; centroids and result of a key or
+    value each): (3 + 2 + 2 + 4)^(1/2) * 2^-12.  Doubled."""
+    limit = 2 * (3 ** 0.5 * 2 ** -9 if dtype == torch.bfloat16 else 11 ** 0.5 * 2 ** -12)
+    got, want = got.cpu().double(), want.double()
+    rel = (got - want).norm() / want.norm()
+    assert rel <= limit, f"relative error {rel:.2e}, limit {limit:.2e}"
+    row = (got - want).norm(dim=-1) / want.norm(dim=-1)
+    assert row.max() <= 4 * limit, f"worst row {row.max():.2e}, limit {4 * limit:.2e}"
+
+
+# (batch, query heads, KV heads, queries, keys, causal): a last unit of one row and of 31, one more key than a tile and one fewer,
+# 1, 3 and 5 query heads a KV head (units of a workgroup at different positions), pairs that are and are not a multiple of 8, fewer
+# keys than queries and more, workgroups with wavefronts that have no unit, more workgroups than two a CU
+SIZES = [(1, 8, 8, 129, 129, True), (2, 5, 1, 191, 191, True), (1, 32, 8, 160, 160, True), (3, 6, 2, 193, 130, True), (1, 4, 1, 257, 300, True),
+         (1, 8, 2, 255, 255, False), (2, 8, 1, 131, 65, False), (1, 12, 4, 320, 33, False), (8, 16, 2, 300, 300, True), (5, 24, 8, 385, 385, True)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("b,hq,hkv,nq,nkv,causal", SIZES)
+def test_rows_at_the_edges(b, hq, hkv, nq, nkv, causal, d, dtype):
+    assert _expanded(b, hkv, hq, nq, nkv, d, causal)
+    q, kv, c, r = _inputs(b, hq, hkv, nq, nkv, d, dtype, 7 * nq + d)
+    want = O.fused_tq_attention(q, *kv, c, c, r, is_causal=causal)
+    got = _attend(q, kv, c, r, causal)
+    _close(got, want, dtype)
+    assert torch.equal(_attend(q, kv, c, r.t().contiguous().t(), causal), got)          # the matrix in the other layout
+    assert torch.equal(_attend(q, kv, c, r, causal), got)
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("at", [0, 31, 32, 63, 64, 140])
+def test_long_norms_beside_ordinary_ones(at, d):
+    """A key and a value whose rows would not fit fp16, in every place of a tile: the others keep their precision."""
+    b, hq, hkv, n = 1, 4, 1, 150
+    assert _expanded(b, hkv, hq, n, n, d, True)
+    q, kv, c, r = _inputs(b, hq, hkv, n, n, d, torch.float16, 31 + at)
+    kv[1][..., at, :] = 3e5
+    kv[3][..., at, :] = 2e5
+    q *= 1e-3
+    want = O.fused_tq_attention(q, *kv, c, c, r, is_causal=True).float()
+    got = _attend(q, kv, c, r, True).cpu().float()
+    # scores of up to 3e5 * 0.03 * 2^-12 (a key's and the oracle's rounded query's) / sqrt(d): their weights to about a tenth
+    ok = want.isfinite()
+    assert torch.equal(got.isfinite(), ok)
+    early = slice(0, at)
+    if at:
+        _close(got[:, :, early], want[:, :, early], torch.float16)
+    err = (got - want).where(ok, torch.zeros_like(want)).norm(dim=-1) / want.where(ok, torch.zeros_like(want)).norm(dim=-1)
+    assert err.median() < 0.1
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("side", [1, 3])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_numbers_that_are_none_stay_visible(value, side, d):
+    """Rows in front of such a key see nothing of it; the others are no numbers, as in the kernel that does not expand.  (A value's
+    tile is multiplied as a whole: rows of the same 32 tokens in front of it may show it.)"""
+    b, hq, hkv, n, at = 1, 8, 2, 400, 200
+    assert _expanded(b, hkv, hq, n, n, d, True)
+    q, kv, c, r = _inputs(b, hq, hkv, n, n, d, torch.bfloat16, 5)
+    kv[side][:, 0, at] = value
+    got = _attend(q, kv, c, r, True)
+    one = attention_in_one_piece(q.to(DEV), *[t.to(DEV) for t in kv], c.to(DEV), r.to(DEV), is_causal=True)
+    seen = at if side == 1 else at // 64 * 64
+    assert got[:, :4, :seen].isfinite().all() and got[:, 4:].isfinite().all()
+    assert not got[:, :4, at:].isfinite().any() and not one[:, :4, at:].isfinite().any()
+
+
+def test_under_capture():
+    b, hq, hkv, n, d = 2, 16, 4, 333, 128
+    q, kv, c, r = _inputs(b, hq, hkv, n, n, d, torch.bfloat16, 17)
+    dev = [t.to(DEV) for t in kv]
+    q, c, r = q.to(DEV), c.to(DEV), r.to(DEV)
+    K.fused_tq_attention(q, *dev, c, c, r, is_causal=True)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = K.fused_tq_attention(q, *dev, c, c, r, is_causal=True)
+    for k in range(4):
+        q.copy_(torch.randn(q.shape, generator=torch.Generator().manual_seed(63 + k)).to(q.dtype))
+        eager = K.fused_tq_attention(q, *dev, c, c, r, is_causal=True)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+
+
+def test_pairs_that_take_turns_in_the_workspace():
+    """More images than the workspace holds at a time: 72 KV heads of 16,448 tokens, 63 of which fit."""
+    b, h, n, d = 1, 72, 16448, 256
+    assert h * n * d * 4 > 2 ** 30 and 0.9 * 2 ** 30 < attention_workspace_bytes(b, n, n, h, h, d, 1) < 1.1 * 2 ** 30
+    c, _, r = (t.to(DEV) if isinstance(t, torch.Tensor) else t for t in book(d))
+    g = torch.Generator(device=DEV).manual_seed(3)
+    kv = []
+    for _ in range(2):
+        kv += [torch.randint(0, 256, (b, h, n, d // 2), dtype=torch.uint8, device=DEV, generator=g),
+               d ** 0.5 * (0.5 + torch.rand(b, h, n, 1, device=DEV, generator=g))]
+    q = torch.randn(b, h, n, d, device=DEV, generator=g).to(torch.bfloat16)
+    got = K.fused_tq_attention(q, *kv, c, c, r, is_causal=True)
+    want = attention_in_one_piece(q, *kv, c, r, is_causal=True)
+    # bf16: query and output rounded there, the output here
+    rel = ((got.float() - want.float()).flatten(2).norm(dim=2) / want.float().flatten(2).norm(dim=2)).max()
+    assert rel <= 2 * 3 ** 0.5 * 2 ** -9, f"{rel:.2e}"
