@@ -579,7 +579,8 @@ at::Tensor paged_tq4_prefill(const at::Tensor& q, const at::Tensor& cu_seqlens_q
     } else {
         result = at::zeros_like(qc);
     }
-    const at::Tensor ws = attention_workspace(q, S, max_seqlen_q, bt.size(1) * block_size, HQ, num_kv_heads, head_dim, 0);
+    const size_t need = fq_paged_prefill_workspace_bytes(int(S), int(max_seqlen_q), bt.size(1) * block_size, T, int(HQ), int(num_kv_heads), int(head_dim));
+    const at::Tensor ws = need == 0 ? at::Tensor() : at::empty({int64_t(need)}, q.options().dtype(at::kByte));
     const int st = fq_paged_tq4_prefill_split(
         qc.data_ptr(), cu.data_ptr<int32_t>(), kv_cache.data_ptr<uint8_t>(), bt.data_ptr<int32_t>(),
         sl.data_ptr<int32_t>(), ck.data_ptr<float>(), cv.data_ptr<float>(), rot.ptr, rot.col_major, result.data_ptr(),

@@ -5,8 +5,35 @@
 #include <cstddef>
 #include <cstdint>
 
+#if defined(__HIPCC__)
+#include <hip/hip_runtime.h>
+#ifndef FQ_HD
+#define FQ_HD __host__ __device__ __forceinline__
+#endif
+#elif !defined(FQ_HD)
+#define FQ_HD inline
+#endif
+
+namespace fq_host {
+int device_cu_count();
+}
+
 namespace fq {
 
+// One piece of a workgroup's work, written by the plan (fq_attention_expanded.hip): 128 rows over a part of their keys.
+struct WorkPiece {
+    int seq, q_first, NQ, NKV;
+    int x, pieces, tile_base, slot;     // x: workgroup of the sequence | piece << 20; slot: of its first piece
+};
+struct WorkPlan {
+    int* counts;                // pieces, workgroups in several pieces
+    WorkPiece* items;
+    WorkPiece* splits;
+    int max_items, max_slots;   // of a KV head: places, pieces of workgroups that have several
+    int cus, cu_slots;          // CUs, and workgroups that run at a time
+};
+
+// The keys: pairs of (batch, KV head) one behind the other, or sequences in the paged cache.
 struct ExpandParams {
     const uint8_t* k_packed;    // (pairs, cap, D/2), a pair being one (batch, KV head)
     const float* k_norms;
@@ -19,9 +46,18 @@ struct ExpandParams {
     int64_t k_cap, v_cap;
     int keys, tiles;            // keys of a pair, and the tiles they fill
     int pair0, pairs;           // the pairs of this launch
-    uint8_t* images;            // (pair, tile): TileCfg
-    int* flags;                 // (pair, tile, side, block of 32 tokens): whether it holds rows of long norms
+    uint8_t* images;            // (tile): TileCfg; tiles of a pair, or (tile, KV head) of a sequence, one behind the other
+    int* flags;                 // (tile, side, block of 32 tokens): whether it holds rows of long norms
     int* exps;                  // the same, by token: the binary orders by which a row is stored smaller
+    const int32_t* cu_seqlens_q;
+    const int32_t* seq_lens;
+    const int32_t* block_table;
+    const uint8_t* cache;
+    int max_blocks, num_blocks, bs_log2;
+    // the plan of the second launch, if it has one
+    bool planned;
+    int num_seqs, H_KV, G, N_Q, causal;
+    WorkPlan plan;
 };
 
 struct AttendParams {
@@ -36,6 +72,9 @@ struct AttendParams {
     int tiles, pair0, pairs, W;
     int round_slots;            // CUs
     bool out_wide;
+    bool paged;
+    WorkPlan plan;              // items == nullptr: the workgroups of all pairs, in one piece
+    float* part;                // slots of pieces
 };
 
 // Whether a call over contiguous keys runs on expanded ones, and the workspace that takes.  Expanding costs about 9 ns a tile of
@@ -48,32 +87,115 @@ struct AttendParams {
 //   * with few workgroups on the keys of very many pairs (4 x 32 heads of their own x 300 34 / 28, x 700 60 / 70);
 //   * with many keys for few queries, which it cuts into pieces (33 queries over 8000 keys, 32 heads over 8, 154 / 37).
 struct ExpandedPlan {
-    int keys = 0, tiles = 0;        // of a pair
+    int keys = 0, tiles = 0;        // of a pair; paged: tiles of all sequences at most
     int64_t per_chunk = 0;          // pairs whose images the workspace holds at a time; 0: not on this path
-    size_t images = 0, flags = 0, bytes = 0;
+    int max_items = 0, max_slots = 0, cus = 0, cu_slots = 0;      // WorkPlan; no items: no plan
+    size_t images = 0, flags = 0, exps = 0, plan = 0, bytes = 0;
 };
 constexpr int64_t kImageBytes = int64_t(1) << 30;      // images at a time: beyond it the pairs take turns
-inline ExpandedPlan plan_expanded(int64_t pairs, int64_t n_q, int64_t n_kv, int G, int D, bool causal) {
+inline size_t round_256(size_t n) { return (n + 255) / 256 * 256; }
+// The parts of the workspace, for `tiles` tiles in all.
+inline void lay_out(ExpandedPlan& e, int64_t tiles, int H_KV, int D) {
+    const int64_t tt = D == 256 ? 32 : 64;
+    e.images = size_t(tiles) * size_t(4 * tt * D);
+    e.flags = round_256(size_t(tiles) * (tt / 32) * 8);
+    e.exps = round_256(size_t(tiles) * 2 * tt * 4);
+    e.plan = e.max_items > 0 ? round_256(256 + (size_t(e.max_items) + e.max_slots / 2 + 1) * sizeof(WorkPiece)) : 0;
+    e.bytes = e.images + e.flags + e.exps + e.plan + size_t(e.max_slots) * H_KV * 4 * (32 * D + 64) * 4;
+}
+// What a batch takes with pieces of at most `piece` tiles (those of the kernel: 32 keys at 256 coordinates), in ns, for the choice
+// between them: the longest piece, slowed down while it shares its CU, or the share of a place; and what the rows of `split` pieces
+// cost in the combine, written and read.  Tiles as measured on an empty chip, and beside a second workgroup twice that; rows at 3.5
+// TB/s.  16 heads over 4 of 256 coordinates x 3001 tokens stay whole (144 us; in pieces of the share 151), 32 over 8 of 128 x 1500
+// too (46 and 53); 8 over 1 x 4000 run in pieces (82 whole, 71).
+constexpr int kPieceTiles = 4;                  // the shortest pieces, in tiles of 64 keys
+struct PieceCost {
+    int tile, rows;
+};
+FQ_HD PieceCost piece_cost(int D) { return D == 64 ? PieceCost{700, 19} : (D == 128 ? PieceCost{1100, 38} : PieceCost{1250, 76}); }
+FQ_HD int64_t batch_ns(int64_t piece, int64_t share, int64_t items, int64_t split, int cus, int D) {
+    const PieceCost c = piece_cost(D);
+    int64_t ns = c.tile * piece;
+    if (D != 256 && items > cus) ns += c.tile * (piece < share ? piece : share) * 6 / 10;
+    const int64_t all = D == 256 ? c.tile * share : c.tile * share * 19 / 10;
+    return (ns > all ? ns : all) + (split > 0 ? 7000 + split * c.rows : 0);
+}
+// The candidates: the longest workgroup's tiles in 1, 2, 3, 4, 6, 8, 12 and 16.
+constexpr int kPieceChoices = 8;
+FQ_HD int piece_choice(int i, int longest, int least) {
+    const int n = i < 4 ? i + 1 : (i & 1 ? 8 : 6) * (i < 6 ? 1 : 2), piece = (longest + n - 1) / n;
+    return piece > least ? piece : least;
+}
+// Room for the plan: the pieces of workgroups that have several are at most four times the workgroups that run at a time.
+inline void add_plan(ExpandedPlan& e, int64_t workgroups, int H_KV, int D, int cus, bool split) {
+    e.cus = cus;
+    e.cu_slots = (D == 256 ? 1 : 2) * cus;
+    e.max_slots = split ? 4 * cus / H_KV + 2 : 0;
+    e.max_items = int(workgroups) + e.max_slots;
+}
+inline ExpandedPlan plan_expanded(int64_t B, int H_KV, int64_t n_q, int64_t n_kv, int G, int D, bool causal) {
     ExpandedPlan e;
+    if (n_q <= (D == 64 ? 192 : 16)) return e;
+    const int64_t pairs = B * H_KV;
     const int64_t tt = D == 256 ? 32 : 64;
     const int64_t keys = causal && n_kv > n_q ? n_q : n_kv, tiles = (keys + tt - 1) / tt, per_pair = tiles * (4 * tt * D);
     if (per_pair > kImageBytes) return e;
     const int64_t W = ((n_q + 31) / 32 * G + 3) / 4, most = int64_t(1) << 23;      // workgroups of a pair, of a launch
     const int64_t blocks = (keys + 63) / 64;
-    if (n_q <= (D == 64 ? 128 : 16) || W > most) return e;
-    if (W < 5 && pairs * blocks > 256) return e;
+    if (W > most) return e;
+    if (W < 5 && pairs * blocks >= 128) return e;
     if (blocks > 4 * W + 4 || (!causal && blocks > 12 && pairs * W < 128)) return e;
     e.keys = int(keys);
     e.tiles = int(tiles);
     e.per_chunk = kImageBytes / per_pair < most / W ? kImageBytes / per_pair : most / W;
     if (e.per_chunk > pairs) e.per_chunk = pairs;
-    e.images = size_t(e.per_chunk * per_pair);
-    e.flags = (size_t(e.per_chunk * tiles) * (tt / 32) * 8 + 255) / 256 * 256;
-    e.bytes = e.images + e.flags + size_t(e.per_chunk * tiles * 2 * tt) * 4;
+    // In pieces where that is faster, the workgroups being few enough to be counted
+    const int cus = fq_host::device_cu_count();
+    if (e.per_chunk == pairs && B <= 256 && pairs * W <= 8 * cus && tiles > kPieceTiles) {
+        const int TS = D == 256 ? 5 : 6, units = int((n_q + 31) / 32 * G);
+        auto tiles_of = [&](int x) {
+            int64_t pos = 32 * ((4 * x + 3 < units - 1 ? 4 * x + 3 : units - 1) / G) + 31;
+            pos = pos < n_q - 1 ? pos : n_q - 1;
+            return causal && (pos >> TS) + 1 < tiles ? (pos >> TS) + 1 : tiles;
+        };
+        int64_t work = 0;
+        for (int x = 0; x < int(W); ++x) work += tiles_of(x);
+        const int64_t places = (D == 256 ? 1 : 2) * int64_t(cus), share = (pairs * work + places - 1) / places;
+        int64_t whole = 0, best = 0;
+        for (int i = 0; i < kPieceChoices; ++i) {
+            const int64_t piece = piece_choice(i, int(tiles_of(int(W) - 1)), kPieceTiles << (6 - TS));
+            int64_t items = 0, split = 0;
+            for (int x = 0; x < int(W); ++x) {
+                const int64_t k = (tiles_of(x) + piece - 1) / piece;
+                items += k;
+                split += k > 1 ? k : 0;
+            }
+            const int64_t ns = batch_ns(piece, share, pairs * items, pairs * split, cus, D);
+            if (i == 0) whole = best = ns;
+            best = ns < best ? ns : best;
+        }
+        if (20 * best < 19 * whole) add_plan(e, B * W, H_KV, D, cus, true);
+    }
+    lay_out(e, e.per_chunk * tiles, H_KV, D);
     return e;
 }
 
-int launch_attention_expanded(const ExpandParams& e, const AttendParams& a, int D, int dtype, int64_t pairs, int64_t per_chunk,
-                              void* stream);
+// The same for paged batches, of which the host knows the number of sequences, the tokens and the longest context possible.
+inline ExpandedPlan plan_expanded_paged(int64_t num_seqs, int64_t total_q, int64_t max_kv, int H_KV, int G, int D) {
+    ExpandedPlan e;
+    const int64_t tt = D == 256 ? 32 : 64, tiles = num_seqs * ((max_kv + tt - 1) / tt);
+    if (num_seqs > 256 || total_q <= 0 || tiles * H_KV * (4 * tt * D) > 0x7fffffff) return e;
+    if (10 * total_q * G < 3 * num_seqs * max_kv || (D == 64 && total_q < 256 * num_seqs)) return e;
+    const int64_t workgroups = (total_q / 32 + num_seqs) * G / 4 + num_seqs;
+    if (workgroups * H_KV > (int64_t(1) << 23) || workgroups >= (1 << 20)) return e;
+    e.tiles = int(tiles);
+    e.per_chunk = 1;
+    add_plan(e, workgroups, H_KV, D, fq_host::device_cu_count(), max_kv > 128 * kPieceTiles);
+    lay_out(e, tiles * H_KV, H_KV, D);
+    return e;
+}
+
+// `e` and `a` hold the operands; the rest is filled in from the plan.
+int launch_attention_expanded(ExpandParams e, AttendParams a, const ExpandedPlan& ep, int D, int dtype, void* workspace, void* stream);
 
 }  // namespace fq

@@ -406,4 +406,13 @@ __device__ __forceinline__ uint32_t pack_weights(float a, float b) {
     }
 }
 
+// The weight 2^(m - top) of a piece's row.  A piece without a visible key has m = -inf, a sum of 0 and rows of zeros; one whose
+// scores are all NaN has m = -inf and a sum of NaN, one with a score of +inf m = +inf: their weights multiply what they left,
+// also a weight of 0, so that a row which is no number in one piece is none in several.
+__device__ __forceinline__ float piece_weight(float m, float l, float top) {
+    return m == -__builtin_inff() && l == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(m - top);
+}
+// (0 only for rows that see no key: a sum that is NaN stays NaN)
+__device__ __forceinline__ float inverse_sum(float den) { return den == 0.0f ? 0.0f : 1.0f / den; }
+
 }  // namespace fq

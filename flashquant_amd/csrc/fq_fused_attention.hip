@@ -1055,15 +1055,6 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
     }
 }
 
-// The weight 2^(m - top) of a piece's row.  A piece without a visible key has m = -inf, a sum of 0 and rows of zeros; one whose
-// scores are all NaN has m = -inf and a sum of NaN, one with a score of +inf m = +inf: their weights multiply what they left,
-// also a weight of 0, so that a row which is no number in one piece is none in several.
-__device__ __forceinline__ float piece_weight(float m, float l, float top) {
-    return m == -__builtin_inff() && l == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(m - top);
-}
-// (0 only for rows that see no key: a sum that is NaN stays NaN)
-__device__ __forceinline__ float inverse_sum(float den) { return den == 0.0f ? 0.0f : 1.0f / den; }
-
 // Rows of the workgroups that ran in pieces: the pieces' rows weighted by 2^(m - max m), summed and normalised, rounded
 // as the kernel above rounds, rotated back.  A workgroup takes `rows` (4 or 16) rows of a unit, a wavefront a row at a
 // time; blockIdx.x numbers the (sequence, KV head, workgroup) triples that may have been split, blockIdx.y their row
@@ -1356,7 +1347,17 @@ extern "C" size_t fq_attention_workspace_bytes(int num_seqs, int max_q_len, int6
     if (num_seqs <= 0 || max_q_len <= 0 || max_kv_len <= 0 || H_KV <= 0 || H_Q <= 0 || H_Q % H_KV != 0) return 0;
     const size_t split = part_bytes(plan_of(num_seqs, max_q_len, max_kv_len, H_Q, H_KV, D, prompts == 1 && max_q_len > 1), num_seqs, H_KV, D);
     if (prompts == 0 || fq_host::force_any_dim_attention()) return split;
-    const size_t expanded = plan_expanded(int64_t(num_seqs) * H_KV, max_q_len, max_kv_len, H_Q / H_KV, D, prompts == 1).bytes;
+    const size_t expanded = plan_expanded(num_seqs, H_KV, max_q_len, max_kv_len, H_Q / H_KV, D, prompts == 1).bytes;
+    return expanded > split ? expanded : split;
+}
+
+extern "C" size_t fq_paged_prefill_workspace_bytes(int num_seqs, int max_q_len, int64_t max_kv_len, int64_t total_q, int H_Q, int H_KV,
+                                                   int D) {
+    using namespace fq;
+    const size_t split = fq_attention_workspace_bytes(num_seqs, max_q_len, max_kv_len, H_Q, H_KV, D, 0);
+    if (num_seqs <= 0 || max_q_len <= 0 || max_kv_len <= 0 || H_KV <= 0 || H_Q <= 0 || H_Q % H_KV != 0) return 0;
+    if (!fq_host::supported_dim(D) || fq_host::force_any_dim_attention()) return split;
+    const size_t expanded = plan_expanded_paged(num_seqs, total_q, max_kv_len, H_KV, H_Q / H_KV, D).bytes;
     return expanded > split ? expanded : split;
 }
 
@@ -1409,31 +1410,23 @@ extern "C" int fq_fused_tq_attention_split(const void* q, const uint8_t* k_packe
         return launch_attention_any_dim(a, D, false, N_Q, B, dtype, stream);
     }
 
-    const ExpandedPlan ep = plan_expanded(int64_t(B) * H_KV, N_Q, N_KV, H_Q / H_KV, D, is_causal && N_Q > 1);
+    const ExpandedPlan ep = plan_expanded(B, H_KV, N_Q, N_KV, H_Q / H_KV, D, is_causal && N_Q > 1);
     if (ep.per_chunk > 0 && workspace != nullptr && workspace_bytes >= ep.bytes) {
         if (!fq_host::aligned(workspace, 256)) return FQ_ERR_MISALIGNED;
-        uint8_t* ws = static_cast<uint8_t*>(workspace);
         ExpandParams e{};
         e.k_packed = k_packed; e.k_norms = k_norms; e.v_packed = v_packed; e.v_norms = v_norms;
         e.centroids_k = centroids_k; e.centroids_v = centroids_v;
         e.rotation = rotation; e.rot_col_major = rotation_col_major;
         e.k_cap = k_capacity; e.v_cap = v_capacity;
-        e.keys = ep.keys; e.tiles = ep.tiles;
-        e.images = ws;
-        e.flags = reinterpret_cast<int*>(ws + ep.images);
-        e.exps = reinterpret_cast<int*>(ws + ep.images + ep.flags);
+        e.num_seqs = B;
         AttendParams a{};
         a.q = static_cast<const uint16_t*>(q);
         a.out = static_cast<uint16_t*>(out);
-        a.images = e.images; a.flags = e.flags; a.exps = e.exps;
         a.H_Q = H_Q; a.H_KV = H_KV; a.G = H_Q / H_KV; a.N_Q = N_Q; a.N_KV = ep.keys;
         a.causal = (is_causal && N_Q > 1) ? 1 : 0;
         a.scale_log2e = sm_scale * kLog2e;
-        a.tiles = ep.tiles;
-        a.round_slots = fq_host::device_cu_count();
-        a.W = ((N_Q + 31) / 32 * a.G + 3) / 4;
         a.out_wide = fq_host::aligned(out, 16);
-        return launch_attention_expanded(e, a, D, dtype, int64_t(B) * H_KV, ep.per_chunk, stream);
+        return launch_attention_expanded(e, a, ep, D, dtype, workspace, stream);
     }
 
     PrefillParams p;
@@ -1508,6 +1501,27 @@ extern "C" int fq_paged_tq4_prefill_split(const void* q, const int32_t* cu_seqle
         !fq_host::aligned(out, 2))
         return FQ_ERR_MISALIGNED;
     if (num_seqs > 65535 || H_KV > 65535 || (D == 256 && H_Q > 65535)) return FQ_ERR_BAD_SHAPE;
+
+    const ExpandedPlan ep = plan_expanded_paged(num_seqs, total_q, int64_t(max_blocks_per_seq) * block_size, H_KV, H_Q / H_KV, D);
+    if (ep.per_chunk > 0 && workspace != nullptr && workspace_bytes >= ep.bytes && !fq_host::force_any_dim_attention()) {
+        if (!fq_host::aligned(workspace, 256)) return FQ_ERR_MISALIGNED;
+        ExpandParams e{};
+        e.centroids_k = centroids_k; e.centroids_v = centroids_v;
+        e.rotation = rotation; e.rot_col_major = rotation_col_major;
+        e.cu_seqlens_q = cu_seqlens_q; e.seq_lens = seq_lens; e.block_table = block_table; e.cache = kv_cache;
+        e.max_blocks = max_blocks_per_seq; e.num_blocks = int(num_blocks);
+        e.bs_log2 = block_size == 8 ? 3 : (block_size == 16 ? 4 : 5);
+        e.num_seqs = num_seqs;
+        AttendParams a{};
+        a.q = static_cast<const uint16_t*>(q);
+        a.out = static_cast<uint16_t*>(out);
+        a.H_Q = H_Q; a.H_KV = H_KV; a.G = H_Q / H_KV;
+        a.causal = is_causal ? 1 : 0;
+        a.scale_log2e = sm_scale * kLog2e;
+        a.out_wide = fq_host::aligned(out, 16);
+        a.paged = true;
+        return launch_attention_expanded(e, a, ep, D, dtype, workspace, stream);
+    }
 
     const int64_t wgs = workgroups_of(max_q_len, H_Q / H_KV);
     const SplitPlan sp = plan_of(num_seqs, max_q_len, int64_t(max_blocks_per_seq) * block_size, H_Q, H_KV, D, false);

@@ -339,6 +339,8 @@ int fq_paged_tq4_prefill(const void* q, const int32_t* cu_seqlens_q, const uint8
  */
 size_t fq_attention_workspace_bytes(int num_seqs, int max_q_len, int64_t max_kv_len, int H_Q, int H_KV, int D,
                                     int prompts);
+/* The same for fq_paged_tq4_prefill_split, which may expand keys and values where it knows the number of tokens. */
+size_t fq_paged_prefill_workspace_bytes(int num_seqs, int max_q_len, int64_t max_kv_len, int64_t total_q, int H_Q, int H_KV, int D);
 
 int fq_fused_tq_attention_split(const void* q, const uint8_t* k_packed, const float* k_norms,
                                 const uint8_t* v_packed, const float* v_norms,

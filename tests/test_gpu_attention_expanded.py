@@ -1,13 +1,16 @@
-"""Attention over expanded keys and values (many queries that share their keys): edges of the 32-row units, of the tiles and of the
-blocks of 32 tokens, numbers of heads and pairs that the workgroups and the XCDs do not divide, long norms, numbers that are none."""
+"""Attention over expanded keys and values (many queries that share their keys), contiguous and paged: edges of the 32-row units, of
+the tiles and of the blocks of 32 tokens, numbers of heads and pairs that the workgroups and the XCDs do not divide, long norms, numbers
+that are none, workgroups in pieces, every row of a mixed batch."""
 from __future__ import annotations
+
+import ctypes
 
 import pytest
 import torch
 
 from flashquant_amd import kernels as K
 from oracle import tq_oracle as O
-from tests.gpu_util import attention_in_one_piece, attention_workspace_bytes, book
+from tests.gpu_util import _entry, attention_in_one_piece, attention_workspace_bytes, book, build_paged_case
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -57,6 +60,8 @@ SIZES = [(1, 8, 8, 129, 129, True), (2, 5, 1, 191, 191, True), (1, 32, 8, 160, 1
 @pytest.mark.parametrize("d", [64, 128, 256])
 @pytest.mark.parametrize("b,hq,hkv,nq,nkv,causal", SIZES)
 def test_rows_at_the_edges(b, hq, hkv, nq, nkv, causal, d, dtype):
+    if d == 64:                                               # (fewer queries stay on the other kernel there)
+        nq, nkv = nq + 192, nkv + 128
     assert _expanded(b, hkv, hq, nq, nkv, d, causal)
     q, kv, c, r = _inputs(b, hq, hkv, nq, nkv, d, dtype, 7 * nq + d)
     want = O.fused_tq_attention(q, *kv, c, c, r, is_causal=causal)
@@ -70,7 +75,7 @@ def test_rows_at_the_edges(b, hq, hkv, nq, nkv, causal, d, dtype):
 @pytest.mark.parametrize("at", [0, 31, 32, 63, 64, 140])
 def test_long_norms_beside_ordinary_ones(at, d):
     """A key and a value whose rows would not fit fp16, in every place of a tile: the others keep their precision."""
-    b, hq, hkv, n = 1, 4, 1, 150
+    b, hq, hkv, n = 1, 4, 1, 210
     assert _expanded(b, hkv, hq, n, n, d, True)
     q, kv, c, r = _inputs(b, hq, hkv, n, n, d, torch.float16, 31 + at)
     kv[1][..., at, :] = 3e5
@@ -139,3 +144,108 @@ def test_pairs_that_take_turns_in_the_workspace():
     # bf16: query and output rounded there, the output here
     rel = ((got.float() - want.float()).flatten(2).norm(dim=2) / want.float().flatten(2).norm(dim=2)).max()
     assert rel <= 2 * 3 ** 0.5 * 2 ** -9, f"{rel:.2e}"
+
+
+# (batch, query heads, KV heads, queries, keys, dimension, causal): prompts whose longest workgroups run in pieces (the last tile of one
+# key, of all but one; rows that see nothing of a piece), and contexts that are long for their queries
+PIECES = [(1, 4, 1, 4033, 4033, 128, True), (1, 8, 1, 1535, 1535, 256, True), (2, 4, 1, 1601, 1601, 256, True), (1, 4, 1, 4033, 4033, 64, True)]
+
+
+def _planned(b, hkv, hq, nq, nkv, d, causal):
+    """Whether the workspace has room for the rows of pieces beside the images (4 rows of 32 and 64 numbers a slot)."""
+    tile = 32 if d == 256 else 64
+    tiles = b * hkv * -(-(min(nq, nkv) if causal else nkv) // tile)
+    return attention_workspace_bytes(b, nq, nkv, hq, hkv, d, 1 if causal else 2) - tiles * tile * (4 * d + 16) > 500 * 16 * (32 * d + 64)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,hq,hkv,nq,nkv,d,causal", PIECES)
+def test_prompts_in_pieces(b, hq, hkv, nq, nkv, d, causal, dtype):
+    assert _planned(b, hkv, hq, nq, nkv, d, causal)
+    q, kv, c, r = _inputs(b, hq, hkv, nq, nkv, d, dtype, nq + d)
+    kv[1][:, :, 37] *= 4e3                                    # a tile with a long norm in one piece
+    q *= 0.5
+    want = O.fused_tq_attention(q, *kv, c, c, r, is_causal=causal)
+    got = _attend(q, kv, c, r, causal)
+    err = (got.cpu().double() - want.double()).norm() / want.double().norm()
+    # (scores of that key reach 4e3 times the others': one weight is all or nothing there, and a rounded query moves it)
+    assert err <= 8 * 3 ** 0.5 * 2 ** -9
+    kv[1][:, :, 37] /= 4e3
+    _close(_attend(q, kv, c, r, causal), O.fused_tq_attention(q, *kv, c, c, r, is_causal=causal), dtype)
+
+
+def _paged_expanded(ql, kv_room, hq, hkv, d):
+    f = _entry("fq_paged_prefill_workspace_bytes", ctypes.c_size_t)
+    need = f(ctypes.c_int(len(ql)), ctypes.c_int(max(ql)), ctypes.c_int64(kv_room), ctypes.c_int64(sum(ql)), ctypes.c_int(hq),
+             ctypes.c_int(hkv), ctypes.c_int(d))
+    return need > attention_workspace_bytes(len(ql), max(ql), kv_room, hq, hkv, d)
+
+
+# (queries, keys): prompts, chunks with keys in front, single queries, idle sequences and ones without keys; key counts at and around
+# tiles; more sequences than a wavefront has lanes, and the most that the plan takes; long workgroups beside short ones
+BATCHES = [([600, 1, 64, 0, 129, 5], [600, 700, 500, 90, 129, 0]), ([257], [1025]), ([64, 63, 65, 300], [64, 63, 65, 300]),
+           ([260 + s % 5 for s in range(70)], [260 + s % 5 + 13 * (s % 7) for s in range(70)]), ([33 * (s % 17) for s in range(256)], [33 * (s % 17) + s % 3 for s in range(256)]),
+           ([2001, 1, 40, 1], [2001, 1900, 1500, 3])]
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(8, 2, 128), (5, 1, 128), (16, 2, 64), (8, 1, 256), (6, 2, 256)])
+@pytest.mark.parametrize("batch", range(len(BATCHES)))
+def test_every_row_of_a_paged_batch(batch, hq, hkv, d):
+    ql, kv = BATCHES[batch]
+    if d == 64:                                               # (shorter prompts stay on the other kernel there)
+        ql, kv = [4 * n for n in ql[:20]], kv[:20]
+        kv = [n + m // 4 * 3 if n else 0 for n, m in zip(kv, ql)]
+    if batch == 4 and d != 128:
+        pytest.skip("many sequences at one dimension")
+    bs, dtype = 16, torch.bfloat16
+    c, _, r = book(d)
+    _, cache, table, sl = build_paged_case(kv, hq, hkv, d=d, bs=bs, seed=141, dtype=dtype)
+    q = torch.randn(sum(ql), hq, d, generator=torch.Generator().manual_seed(142)).to(dtype)
+    cu = torch.tensor([0] + list(torch.tensor(ql).cumsum(0)), dtype=torch.int32)
+    assert _paged_expanded(ql, table.shape[1] * bs, hq, hkv, d)
+    room = torch.randint(-3, 1 << 20, table.shape, dtype=torch.int32, generator=torch.Generator().manual_seed(143))
+    pages = (torch.tensor(kv) + bs - 1) // bs
+    dirty = torch.where(torch.arange(table.shape[1])[None] < pages[:, None], table, room)      # ids past a sequence's pages
+    for causal in (True, False):
+        want = O.paged_prefill(q, cu, cache, table, sl, c, c, r, hkv, d, bs, causal=causal)
+        out = torch.full((q.numel() + 8,), 7.0, dtype=dtype, device=DEV)
+        got = out[1:1 + q.numel()].view_as(q)                                                  # not 16-byte aligned
+        K.paged_tq4_prefill(q.to(DEV), cu.to(DEV), max(ql), cache.to(DEV), dirty.to(DEV), sl.to(DEV), c.to(DEV), c.to(DEV), r.to(DEV),
+                            hkv, d, bs, causal=causal, out=got)
+        assert (out[:1] == 7).all() and (out[1 + q.numel():] == 7).all()
+        keyless = torch.cat([torch.full((n,), m == 0) for n, m in zip(ql, kv)])
+        assert (got.cpu()[keyless] == 0).all()
+        rel = (got.cpu().float() - want.float()).norm(dim=-1) / want.float().norm(dim=-1)
+        # query, result and output rounded to bf16 there, the output here; a worst row of some thousands
+        assert rel[~keyless].max() <= 4 * 2 ** -8 and rel[~keyless].square().mean().sqrt() <= 2 * 2 * 2 ** -9
+        assert torch.equal(K.paged_tq4_prefill(q.to(DEV), cu.to(DEV), max(ql), cache.to(DEV), table.to(DEV), sl.to(DEV), c.to(DEV), c.to(DEV),
+                                               r.to(DEV), hkv, d, bs, causal=causal), got)
+
+
+def test_paged_under_capture_with_other_lengths():
+    """One captured call: the plan follows from the lengths that each replay finds on the device."""
+    hq, hkv, d, bs, dtype = 16, 4, 128, 16, torch.bfloat16
+    kv, ql = [900, 700, 1200, 60], [300, 40, 600, 5]
+    c, _, r = book(d)
+    _, cache, table, sl = build_paged_case(kv, hq, hkv, d=d, bs=bs, seed=151, dtype=dtype)
+    assert _paged_expanded(ql, table.shape[1] * bs, hq, hkv, d)
+    q = torch.randn(sum(ql), hq, d, generator=torch.Generator().manual_seed(152)).to(dtype).to(DEV)
+    cu = torch.tensor([0] + list(torch.tensor(ql).cumsum(0)), dtype=torch.int32).to(DEV)
+    sl = sl.to(DEV)
+    out = torch.zeros_like(q)
+    args = (cu, max(ql), cache.to(DEV), table.to(DEV), sl, c.to(DEV), c.to(DEV), r.to(DEV), hkv, d, bs)
+    K.paged_tq4_prefill(q, *args, out=out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        K.paged_tq4_prefill(q, *args, out=out)
+    for lens in (kv, [300, 700, 600, 5], [900, 40, 1199, 60], [301, 41, 601, 6], kv):
+        sl.copy_(torch.tensor(lens, dtype=torch.int32))
+        eager = K.paged_tq4_prefill(q, *args)
+        out.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+        want = O.paged_prefill(q.cpu(), cu.cpu(), cache, table, sl.cpu(), c, c, r, hkv, d, bs)
+        rel = (out.cpu().float() - want.float()).norm(dim=-1) / want.float().norm(dim=-1)
+        assert rel.max() <= 4 * 2 ** -8
