@@ -162,11 +162,13 @@ constexpr int kRotRows = 16;
 
 // B operand values of one 16-column block.  TRANSPOSED: out = x @ R.T (B[k][n] = R[col+n][k],
 // contiguous in k); otherwise out = x @ R (B[k][n] = R[k][col+n], 16 lanes contiguous in n).
-template <int D, bool TRANSPOSED>
+// J: how many runs of 32 contraction indices (all, or those of a wavefront from k = k0 on).
+template <int D, bool TRANSPOSED, int J = D / 32>
 __device__ __forceinline__ void load_rotation_block(const float* __restrict__ R, int col, int n, int g,
-                                                    float (&b)[D / 32][8]) {
+                                                    float (&b)[J][8], int k0 = 0) {
+    R += TRANSPOSED ? k0 : k0 * D;
 #pragma unroll
-    for (int j = 0; j < D / 32; ++j) {
+    for (int j = 0; j < J; ++j) {
         if (TRANSPOSED) {
             const float4v* src = reinterpret_cast<const float4v*>(R + int64_t(col + n) * D + 32 * j + 8 * g);
             const float4v lo = src[0], hi = src[1];
@@ -182,12 +184,12 @@ __device__ __forceinline__ void load_rotation_block(const float* __restrict__ R,
 // Rotation matrix given either row-major (element (i, j) at i*D + j) or column-major
 // (at i + j*D, i.e. the transpose is the contiguous one, which is what a QR factor
 // moved to the GPU looks like).  `x_times_Rt` selects out = x @ R.T, else out = x @ R.
-template <int D>
+template <int D, int J = D / 32>
 __device__ __forceinline__ void load_rotation_any(const float* __restrict__ R, bool col_major, bool x_times_Rt,
-                                                  int col, int n, int g, float (&b)[D / 32][8]) {
+                                                  int col, int n, int g, float (&b)[J][8], int k0 = 0) {
     // x @ R.T on a column-major R reads the same addresses as x @ R on a row-major one
-    if (x_times_Rt != col_major) load_rotation_block<D, true>(R, col, n, g, b);
-    else load_rotation_block<D, false>(R, col, n, g, b);
+    if (x_times_Rt != col_major) load_rotation_block<D, true, J>(R, col, n, g, b, k0);
+    else load_rotation_block<D, false, J>(R, col, n, g, b, k0);
 }
 
 template <int D>

@@ -1839,24 +1839,28 @@ __global__ __launch_bounds__(256) void rotate_q_kernel(const uint16_t* __restric
 // rounded again (paged_decode.py:123).  rows = num_seqs * H_Q; a workgroup owns RW rows
 // (4, 8 or 16: the fewer, the more workgroups share the combine, the more often the matrix is
 // fetched): 256 / RW threads combine a row into LDS, then all rotate from there.
-// CS: the output columns of a row group are shared by CS workgroups (blockIdx.y), each combining the rows for
-// itself and fetching 1 / CS of the matrix: at head_dim 256 the matrix is 256 KB, and a workgroup that fetches all
-// of it holds 256 matrix values per lane.
-template <int D, int DT, int RW, int CS = 1>
+// The output columns of a row group are shared by several workgroups (blockIdx.y), each combining the rows for itself
+// and fetching its part of the matrix: CBW blocks of 16 columns a wavefront, or one for KS wavefronts, each
+// 1 / KS of the contraction, their sums added through LDS.  Bound by latency and, with few rows, by the part of the matrix that
+// one workgroup takes: 128 rows of 128 coordinates, 13 splits each, 4.9 us with the whole matrix in a workgroup (step of one sequence
+// of 777 tokens 17.6 us), 3.2 with a quarter (15.9).  Larger chunks of splits, the next one asked for while one is summed, or
+// the maxima read once for all threads of a row lost 0.4 to 1.4 us: there are few chunks, and the kernel's code comes from memory too.
+template <int D, int DT, int RW, int CBW, int KS>
 __global__ __launch_bounds__(256) void reduce_rotate_kernel(const float* __restrict__ part_acc,
                                                             const float* __restrict__ part_m,
                                                             const float* __restrict__ part_l,
                                                             const float* __restrict__ R, uint16_t* __restrict__ out,
                                                             int64_t rows, int NS, int col_major) {
-    static_assert((D / 64) % CS == 0, "whole rounds of column blocks per workgroup");
-    constexpr int CBW = D / 64 / CS;       // 16-column blocks per wavefront
-    const int cb0 = 4 * CBW * int(blockIdx.y);     // first column block of this workgroup
+    static_assert(KS == 1 || CBW == 1, "wavefronts that share a contraction have one column block");
+    static_assert((D / 32) % KS == 0 && (D / 16) % (4 * CBW / KS) == 0, "whole runs and whole workgroups");
+    constexpr int J = D / 32 / KS;         // runs of 32 contraction indices per wavefront
     constexpr int OSTRIDE = D + 8;         // 16-bit words per staged row (padded: conflict-free operand reads)
     constexpr int TPR = 256 / RW;          // threads that combine one row
     constexpr int CPT = D / TPR < 2 ? 2 : D / TPR;      // coordinates per thread and pass (2, 4 or 8)
     constexpr int ACTIVE = D / CPT < TPR ? D / CPT : TPR;   // threads of a row that have coordinates
     static_assert(CPT <= 8, "a thread stages at most eight coordinates of a row (head_dim 256: at most 8 rows a workgroup)");
     __shared__ __attribute__((aligned(16))) uint16_t os[RW * OSTRIDE];   // combined rows, query dtype
+    __shared__ float sums[KS == 1 ? 1 : 4][RW][16];                      // sums of the wavefronts that share a contraction
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n = lane & 15, g = lane >> 4;
     const int64_t row0 = int64_t(blockIdx.x) * RW;
@@ -1949,10 +1953,12 @@ __global__ __launch_bounds__(256) void reduce_rotate_kernel(const float* __restr
         }
     }
     // the matrix columns of this wavefront: asked for behind the partials, they arrive during the combine
-    float rbv[CBW][D / 32][8];
+    const int cb0 = 4 * CBW / KS * int(blockIdx.y) + wave / KS;
+    const int k0 = wave % KS * (D / KS);
+    float rbv[CBW][J][8];
     if (R != nullptr) {
 #pragma unroll
-        for (int i = 0; i < CBW; ++i) load_rotation_any<D>(R, col_major != 0, false, 16 * (cb0 + wave + 4 * i), n, g, rbv[i]);
+        for (int i = 0; i < CBW; ++i) load_rotation_any<D, J>(R, col_major != 0, false, 16 * (cb0 + (4 / KS) * i), n, g, rbv[i], k0);
     }
     {
         const bool live = row0 + r < rows && den > 0.0f;
@@ -1974,7 +1980,7 @@ __global__ __launch_bounds__(256) void reduce_rotate_kernel(const float* __restr
     }
     __syncthreads();
     if (R == nullptr) {
-        if (CS > 1 && blockIdx.y != 0) return;        // no rotation: one workgroup writes the combined rows
+        if (blockIdx.y != 0) return;        // no rotation: one workgroup writes the combined rows
         for (int c = threadIdx.x; c < RW * (D / 8); c += 256) {
             const int rr = c / (D / 8), q = c % (D / 8);
             const int64_t orow = row0 + rr;
@@ -1984,23 +1990,37 @@ __global__ __launch_bounds__(256) void reduce_rotate_kernel(const float* __restr
     }
     // ---- rotate back on the fp16 MFMA: the rows are exact in fp16 up to a power of two.  With fewer
     // than 16 rows the operand rows repeat (row n % RW) and only the first RW result rows are kept. ----
-    uint4v raw[D / 32];
+    uint4v raw[J];
 #pragma unroll
-    for (int j = 0; j < D / 32; ++j) raw[j] = *reinterpret_cast<const uint4v*>(&os[(n % RW) * OSTRIDE + 32 * j + 8 * g]);
-    half8 a[D / 32];
+    for (int j = 0; j < J; ++j) raw[j] = *reinterpret_cast<const uint4v*>(&os[(n % RW) * OSTRIDE + k0 + 32 * j + 8 * g]);
+    half8 a[J];
     float up;
-    rows_as_f16<D, DT>(raw, a, up);
+    rows_as_f16<32 * J, DT>(raw, a, up);
 #pragma unroll
     for (int i = 0; i < CBW; ++i) {
-        half8 rhi[D / 32], rlo[D / 32];
-        split_rotation_block<D>(rbv[i], rhi, rlo);
-        const float4v acc = rotate_block_f16<D>(a, rhi, rlo);
-        const int cb = cb0 + wave + 4 * i;
+        half8 rhi[J], rlo[J];
+        split_rotation_block<32 * J>(rbv[i], rhi, rlo);
+        const float4v acc = rotate_block_f16<32 * J>(a, rhi, rlo);
+        const int cb = cb0 + 4 / KS * i;
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const int rr = 4 * g + k;
             const int64_t orow = row0 + rr;
-            if (rr < RW && orow < rows) out[orow * D + 16 * cb + n] = store_elem<DT>(acc[k] * up);
+            if constexpr (KS == 1) {
+                if (rr < RW && orow < rows) out[orow * D + 16 * cb + n] = store_elem<DT>(acc[k] * up);
+            } else {
+                if (rr < RW) sums[wave][rr][n] = acc[k] * up;
+            }
+        }
+    }
+    if constexpr (KS > 1) {
+        __syncthreads();
+        for (int c = threadIdx.x; c < 4 / KS * RW * 16; c += 256) {
+            const int b = c / (RW * 16), rr = c / 16 % RW, col = c % 16;
+            float sum = sums[b * KS][rr][col];
+#pragma unroll
+            for (int k = 1; k < KS; ++k) sum += sums[b * KS + k][rr][col];
+            if (row0 + rr < rows) out[(row0 + rr) * D + 16 * (cb0 - wave / KS + b) + col] = store_elem<DT>(sum);
         }
     }
 }
@@ -2407,29 +2427,41 @@ int launch_reduce(const float* acc, const float* m, const float* l, const float*
     const int rw_opt = fq_host::option(FQ_OPT_REDUCE_ROWS);
     int rw = rows <= 4 * int64_t(cus) ? 4 : (rows <= 8 * int64_t(cus) ? 8 : 16);
     if (rw_opt == 4 || rw_opt == 8 || rw_opt == 16) rw = rw_opt;
-    // head_dim 256: four workgroups share the columns of a row group, 16 rows a group while that fills the chip
-    constexpr int kColumnSplit256 = 4;
-    if (D == 256) rw = (rw_opt == 4) ? 4 : 8;       // (a thread stages at most eight coordinates of a row; measured: 8 rows
-                                                    // x 4 column groups 79 us per step of 32 x 4096 tokens, 4 rows 81 us)
-    const dim3 grid(unsigned((rows + rw - 1) / rw), D == 256 ? kColumnSplit256 : 1), block(256);
+    if (D == 256) rw = rw_opt == 4 || (rw_opt == 0 && rows <= cus / 4) ? 4 : 8;    // a thread stages at most eight coordinates of a row
+    // Workgroups that share the columns of a row group: as many as there are idle CUs for.  A workgroup's part of
+    // the matrix is the longest thing it does (64 KB through one CU, and its split into fp16 terms, 2 us at 128 coordinates), so
+    // the steps of few rows gain: serving step, bf16, in us, with one workgroup a row group, two, and four of which two wavefronts share a
+    // contraction: 128 rows 17.7, 16.7, 16.0; 256 rows 20.7, 19.6, 19.0; 512 rows 21.7, 20.7, 20.7; 768 rows 25.4, 25.4, 25.3.
+    // 256 coordinates, four workgroups a row group, eight, sixteen: 128 rows 39.1, 38.1, 37.8, 256 rows 40.4, 39.4, 40.4, 512 rows
+    // 46.0, 46.0, 47.6; 64 rows 38.4, 37.2, 37.0, and 36.0 with sixteen for groups of four rows.  At 64 coordinates (16 KB)
+    // two workgroups gain 0 to 0.1 up to 384 rows and lose 0.3 at 768; at 128 eight gain 0.1 over four.
+    const int64_t groups = (rows + rw - 1) / rw;
+    auto fits = [&](int cs) { return groups * cs <= cus; };
     uint16_t* dst = reinterpret_cast<uint16_t*>(out);
-#define FQ_REDUCE(DD, RWV) \
-    hipLaunchKernelGGL((reduce_rotate_kernel<DD, DT, RWV, (DD == 256 ? kColumnSplit256 : 1)>), grid, block, 0, stream, acc, m, l, R, dst, rows, NS, col_major)
-#define FQ_REDUCE_D(DD)                       \
-    do {                                      \
-        if (rw == 4) FQ_REDUCE(DD, 4);        \
-        else if (rw == 8) FQ_REDUCE(DD, 8);   \
-        else FQ_REDUCE(DD, 16);               \
-    } while (0)
+#define FQ_REDUCE(DD, RWV, CBWV, KSV)                                                                                         \
+    hipLaunchKernelGGL((reduce_rotate_kernel<DD, DT, RWV, CBWV, KSV>), dim3(unsigned(groups), DD / 16 * KSV / (4 * CBWV)), \
+                       dim3(256), 0, stream, acc, m, l, R, dst, rows, NS, col_major)
     switch (D) {
-        case 64: FQ_REDUCE_D(64); break;
-        case 128: FQ_REDUCE_D(128); break;
+        case 64:
+            if (rw == 4) FQ_REDUCE(64, 4, 1, 1);
+            else if (rw == 8) FQ_REDUCE(64, 8, 1, 1);
+            else FQ_REDUCE(64, 16, 1, 1);
+            break;
+        case 128:
+            if (rw == 4 && fits(4)) FQ_REDUCE(128, 4, 1, 2);
+            else if (rw == 4 && fits(2)) FQ_REDUCE(128, 4, 1, 1);
+            else if (rw == 4) FQ_REDUCE(128, 4, 2, 1);
+            else if (rw == 8) FQ_REDUCE(128, 8, 2, 1);
+            else FQ_REDUCE(128, 16, 2, 1);
+            break;
         default:
-            if (rw == 4) FQ_REDUCE(256, 4);
-            else FQ_REDUCE(256, 8);
+            if (rw == 4 && fits(16)) FQ_REDUCE(256, 4, 1, 4);
+            else if (rw == 4) FQ_REDUCE(256, 4, 1, 1);
+            else if (fits(16)) FQ_REDUCE(256, 8, 1, 4);
+            else if (fits(8)) FQ_REDUCE(256, 8, 1, 2);
+            else FQ_REDUCE(256, 8, 1, 1);
             break;
     }
-#undef FQ_REDUCE_D
 #undef FQ_REDUCE
     return fq_host::check_launch();
 }

@@ -199,3 +199,33 @@ def test_ring_kernel_with_many_sequences(kind):
         want = O.split_k_paged_decode(q, cache, table, sl, c, c, r, hkv, d, bs)
     assert _worst_row(got[sl > 0], want[sl > 0]) <= LIMIT[torch.bfloat16]
     assert (got[sl == 0] == 0).all()
+
+
+# rows (sequences x query heads) on both sides of where 4, 2 and 1 workgroups (16, 8 and 4 at 256 coordinates) share the columns of
+# a group of rows, the last group not full; one split, one chunk of splits and several
+@pytest.mark.parametrize("splits", [2, 9, 21])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,hq,hkv,n", [(128, 8, 8, 1), (128, 7, 1, 3), (128, 32, 8, 8), (128, 24, 8, 11), (128, 8, 2, 64), (128, 24, 8, 22),
+                                        (256, 8, 8, 1), (256, 7, 1, 9), (256, 16, 4, 4), (256, 6, 2, 11), (256, 8, 1, 16), (256, 12, 4, 11),
+                                        (256, 16, 4, 16), (256, 16, 4, 17)])
+def test_workgroups_that_share_the_columns_of_a_row(d, hq, hkv, n, dtype, splits):
+    """Against the same merged rows rotated by other groupings of rows, columns and contraction: the rows are exact operands and
+    the matrix keeps 22 bits, so the float32 sums differ by their order alone, 2^-20 of the row's norm, and what is stored by one
+    rounding to the query type more."""
+    ctx, bs = 900, 16
+    c, _, r = (t.to(DEV) for t in book(d))
+    _, cache, table, q = _tq4_inputs(n, hq, hkv, d, bs, ctx, dtype)
+    sl = torch.tensor([0 if s == 5 else ctx - 37 * s % 800 for s in range(n)], dtype=torch.int32, device=DEV)
+    for rot in (r.contiguous(), r.t().contiguous().t()):                    # row-major and column-major
+        rest = (cache, table, sl, c, c, rot, hkv, d, bs)
+        got = K.split_k_paged_decode(q, *rest, num_splits=splits, out=torch.full_like(q, 7.0)).double()
+        for rows in ((16,) if d == 128 else (4, 8)):
+            C = load_native()
+            old = C.set_option("reduce_rows", rows)
+            try:
+                want = K.split_k_paged_decode(q, *rest, num_splits=splits).double()
+            finally:
+                C.set_option("reduce_rows", old)
+            near = 2.0 ** (-7 if dtype == torch.bfloat16 else -10) * want.abs() + 2.0 ** -20 * want.norm(dim=-1, keepdim=True)
+            assert ((got - want).abs() <= near).all(), rows
+        assert (got[sl == 0] == 0).all() and got[sl > 0].norm(dim=-1).min() > 0
