@@ -1056,14 +1056,21 @@ __global__ __launch_bounds__(512) void fused_tq_attention_kernel(const PrefillPa
 }
 
 // Rows of the workgroups that ran in pieces: the pieces' rows weighted by 2^(m - max m), summed and normalised, rounded
-// as the kernel above rounds, rotated back.  A workgroup takes `rows` (4 or 16) rows of a unit, a wavefront a row at a
-// time; blockIdx.x numbers the (sequence, KV head, workgroup) triples that may have been split, blockIdx.y their row
-// groups.  Bound by the launch and two round trips (partials and matrix are asked for together): 5.6 us.
-template <int D, int DT, bool PAGED>
-__global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillParams p, int rows) {
+// as the kernel above rounds, rotated back.  A workgroup takes `rows` (4 or 16) rows, of one unit or (one or two queries) a few of each
+// of 2^`units_log2` units, a wavefront a row at a time; blockIdx.x numbers the (sequence, KV head, workgroup) triples that may have
+// been split, blockIdx.y their row groups.  With KS > 1 the columns of a row group are shared by the workgroups of blockIdx.z,
+// each gathering the rows for itself, and a block of 16 columns by KS wavefronts, each 1 / KS of the contraction.
+// Bound by the launch, two round trips (partials and matrix are asked for together) and the part of the matrix that a
+// workgroup takes: 128 rows of 128 coordinates 5.2 us with a workgroup a row, 3.5 with four for four.
+template <int D, int DT, bool PAGED, int KS>
+__global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillParams p, int rows, int units_log2) {
     using Cfg = PrefillCfg<D>;
-    constexpr int NJ = D / 32, CBW = D / 64, CPL = D / 64;      // column blocks per wavefront, coordinates per lane
+    const int usplit = KS == 1 ? 0 : units_log2;
+    constexpr int CBW = KS == 1 ? D / 64 : 1, CPL = D / 64;     // column blocks per wavefront, coordinates per lane
+    constexpr int J = D / 32 / KS;                              // runs of 32 contraction indices per wavefront
+    static_assert(J * KS == D / 32, "whole runs");
     __shared__ __attribute__((aligned(16))) float os[16 * (D + 4)];
+    __shared__ float sums[KS == 1 ? 1 : 4][16][16];             // sums of the wavefronts that share a contraction
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n16 = lane & 15, g4 = lane >> 4;
     const int x = int(blockIdx.x) % p.split_w, pair = int(blockIdx.x) / p.split_w;
@@ -1071,25 +1078,33 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillPar
     const int pieces = PAGED ? p.left[blockIdx.x] : p.max_pieces;
     if (pieces == 0) return;
     const SeqShape sh = seq_shape<PAGED>(p, b);
-    const int groups = (int(gridDim.y) + 7) / 8, u = int(blockIdx.y) / groups, row0 = int(blockIdx.y) % groups * rows;
-    const int unit = 8 * x + u;
-    if (unit >= sh.units) return;
-    const int pos0 = 32 * (unit / p.G) + row0;
-    if (pos0 >= sh.NQ) return;
+    const int groups = int(gridDim.y) > (8 >> usplit) ? 2 : 1;
+    const int u0 = (int(blockIdx.y) / groups) << usplit, row0 = int(blockIdx.y) % groups * rows;
+    if (8 * x + u0 >= sh.units) return;
+    const int rsh = (rows == 16 ? 4 : 2) - usplit;              // 2^rsh rows of a unit
+    // units beside each other are heads of the same 32 positions (where there are several here, a head has only one)
+    const int block = (8 * x + u0) / p.G, head0 = 8 * x + u0 - block * p.G;
+    auto head_of = [&](int r) { return KS == 1 ? head0 : head0 + (r >> rsh); };
+    auto row_of = [&](int r) { return KS == 1 ? row0 + r : row0 + (r & ((1 << rsh) - 1)); };             // among the unit's 32
+    auto pos_of = [&](int r) { return 32 * block + row_of(r); };
+    auto live = [&](int r) { return (KS == 1 || (u0 + (r >> rsh) < 8 && head_of(r) < p.G)) && pos_of(r) < sh.NQ; };
+    if (!live(0)) return;
 
-    const float* src = p.part + (int64_t(blockIdx.x) * p.max_pieces) * Cfg::SLOT + u * (32 * D + 64);
-    constexpr bool kAhead = D <= 128;             // (256 coordinates: too many registers)
-    float rbv[kAhead ? CBW : 1][NJ][8];
+    const float* src = p.part + (int64_t(blockIdx.x) * p.max_pieces) * Cfg::SLOT;
+    constexpr bool kAhead = CBW * J <= 8;         // (256 coordinates in one workgroup: too many registers)
+    const int cb0 = KS == 1 ? wave : 4 / KS * int(blockIdx.z) + wave / KS, k0 = wave % KS * (D / KS);
+    float rbv[kAhead ? CBW : 1][J][8];
 #pragma unroll
     for (int i = 0; i < (kAhead ? CBW : 0); ++i)
-        load_rotation_any<D>(p.rotation, p.rot_col_major != 0, false, 16 * (wave + 4 * i), n16, g4, rbv[i]);
+        load_rotation_any<D, J>(p.rotation, p.rot_col_major != 0, false, 16 * (cb0 + 4 * i), n16, g4, rbv[i], k0);
     for (int r = wave; r < rows; r += 4) {
-        if (pos0 + r >= sh.NQ) {                                // no query: the pieces left no such row
+        if (!live(r)) {                                         // no query: the pieces left no such row
 #pragma unroll
             for (int e = 0; e < CPL; ++e) os[r * (D + 4) + CPL * lane + e] = 0.0f;
             continue;
         }
-        const float* head = src + 32 * D + row0 + r;
+        const float* unit_src = src + (KS == 1 ? u0 : u0 + (r >> rsh)) * (32 * D + 64);
+        const float* head = unit_src + 32 * D + row_of(r);
         const bool have = lane < pieces;                        // (at most 32 pieces)
         const float m = have ? head[int64_t(lane) * Cfg::SLOT] : -__builtin_inff();
         const float l = have ? head[int64_t(lane) * Cfg::SLOT + 32] : 0.0f;
@@ -1104,7 +1119,7 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillPar
 #pragma unroll
             for (int i = 0; i < 8; ++i) {                       // eight pieces in flight (past the end: the last one again)
                 const int k = k0 + i < pieces ? k0 + i : pieces - 1;
-                const float* row = src + int64_t(k) * Cfg::SLOT + (row0 + r) * D + CPL * lane;
+                const float* row = unit_src + int64_t(k) * Cfg::SLOT + row_of(r) * D + CPL * lane;
 #pragma unroll
                 for (int e = 0; e < CPL; ++e) at[i][e] = row[e];
             }
@@ -1124,27 +1139,27 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillPar
         }
     }
     __syncthreads();
-    float a[NJ][8];
+    float a[J][8];
 #pragma unroll
-    for (int j = 0; j < NJ; ++j)
+    for (int j = 0; j < J; ++j)
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const float4v v = *reinterpret_cast<const float4v*>(os + (n16 & (rows - 1)) * (D + 4) + 32 * j + 8 * g4 + 4 * h);
+            const float4v v = *reinterpret_cast<const float4v*>(os + (n16 & (rows - 1)) * (D + 4) + k0 + 32 * j + 8 * g4 + 4 * h);
 #pragma unroll
             for (int e = 0; e < 4; ++e) a[j][4 * h + e] = v[e];
         }
     // fp16 terms as in finish_rows, scaled row by row (the rows of a block may differ by any factor): lanes n16 + 16 g hold
     // row n16
     constexpr int kUp = PAGED ? 14 : 0;
-    half8 ahi[NJ], alo[NJ];
+    half8 ahi[J], alo[J];
     float mx = 0.0f;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j)
+    for (int j = 0; j < J; ++j)
 #pragma unroll
         for (int e = 0; e < 8; ++e) mx = __builtin_fmaxf(mx, __builtin_fabsf(a[j][e]));
     const int ex = row_exponent(max_xor16(mx)) - kUp;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j)
+    for (int j = 0; j < J; ++j)
 #pragma unroll
         for (int e = 0; e < 8; e += 2) {
             const float a0 = a[j][e] * pow2(-ex), a1 = a[j][e + 1] * pow2(-ex);
@@ -1160,20 +1175,32 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillPar
     float up[4];                       // of the result rows 4 g4 + k
 #pragma unroll
     for (int k = 0; k < 4; ++k) up[k] = pow2(__shfl(ex, 4 * g4 + k, kWave));
-    const int hq = hkv * p.G + unit % p.G;
-    uint16_t* out = PAGED ? p.out + (int64_t(p.cu_seqlens_q[b]) * p.H_Q + hq) * D : p.out + (int64_t(b) * p.H_Q + hq) * sh.NQ * D;
-    const int stride = PAGED ? p.H_Q * D : D;
+    const int stride = PAGED ? p.H_Q * D : D, head_stride = PAGED ? D : sh.NQ * D;
+    uint16_t* out = p.out + (PAGED ? int64_t(p.cu_seqlens_q[b]) : int64_t(b) * sh.NQ) * p.H_Q * D + int64_t(hkv * p.G) * head_stride;
+    auto store = [&](int r, int col, float v) {
+        out[int64_t(head_of(r)) * head_stride + int64_t(pos_of(r)) * stride + col] = store_elem<DT>(v);
+    };
 #pragma unroll
     for (int i = 0; i < CBW; ++i) {
-        half8 rhi[NJ], rlo[NJ];
-        if (!kAhead) load_rotation_any<D>(p.rotation, p.rot_col_major != 0, false, 16 * (wave + 4 * i), n16, g4, rbv[0]);
-        split_rotation_block<D>(rbv[kAhead ? i : 0], rhi, rlo);
-        const float4v acc = PAGED ? rotate_block_f16<D>(ahi, rhi, rlo) : rotate_block_f16x3<D>(ahi, alo, rhi, rlo);
+        half8 rhi[J], rlo[J];
+        if (!kAhead) load_rotation_any<D, J>(p.rotation, p.rot_col_major != 0, false, 16 * (cb0 + 4 * i), n16, g4, rbv[0], k0);
+        split_rotation_block<32 * J>(rbv[kAhead ? i : 0], rhi, rlo);
+        const float4v acc = PAGED ? rotate_block_f16<32 * J>(ahi, rhi, rlo) : rotate_block_f16x3<32 * J>(ahi, alo, rhi, rlo);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const int r = 4 * g4 + k;
-            if (r < rows && pos0 + r < sh.NQ)
-                out[int64_t(pos0 + r) * stride + 16 * (wave + 4 * i) + n16] = store_elem<DT>(acc[k] * up[k]);
+            if constexpr (KS > 1) sums[wave][r][n16] = acc[k] * up[k];
+            else if (r < rows && live(r)) store(r, 16 * (cb0 + 4 * i) + n16, acc[k] * up[k]);
+        }
+    }
+    if constexpr (KS > 1) {
+        __syncthreads();
+        for (int c = threadIdx.x; c < 4 / KS * 16 * rows; c += 256) {
+            const int col = c & 15, r = (c >> 4) & (rows - 1), cb = (c >> 4) / rows;
+            float sum = sums[cb * KS][r][col];
+#pragma unroll
+            for (int k = 1; k < KS; ++k) sum += sums[cb * KS + k][r][col];
+            if (live(r)) store(r, 16 * (4 / KS * int(blockIdx.z) + cb) + col, sum);
         }
     }
 }
@@ -1252,7 +1279,24 @@ int launch_prefill_as(const PrefillParams& p, dim3 grid, int max_q, hipStream_t 
         }
         const int rows = max_q <= 4 ? 4 : 16;
         const int groups = max_q <= 16 ? 1 : 2;             // 32 rows a unit at most
-        hipLaunchKernelGGL((attention_combine_kernel<D, DT, PAGED>), dim3(unsigned(slots), 8 * groups), dim3(256), 0, s, p, rows);
+        // Workgroups share the columns of the rows while CUs are idle, at 256 coordinates up to two workgroups a CU.  One query
+        // over ring buffers, 32 heads over 8 of 128, bf16, in us, without and with: 4 x 2500 tokens 21.8, 20.2; 1 x 16,000 27.9, 26.3;
+        // 16 x 700 (512 workgroups) 27.3, 27.4; 5 queries over 4 x 2500 (512) 23.0, 24.3.  16 heads over 4 of 256: 2 x 1000 42.1, 35.6;
+        // 8 x 1500 (512) 42.9, 38.7; 2 queries over 8 x 1000, 32 heads over 8 (2048), 43.8, 44.4.  At 64 coordinates, where
+        // the matrix is 16 KB, nothing helps: 15.1 and 15.3.
+        if constexpr (D >= 128) {
+            constexpr int KS = D == 256 ? 4 : 2, CS = D / 64 * KS;
+            const int usplit = max_q <= 1 ? 2 : (max_q == 2 ? 1 : 0);
+            const int units = p.G * ((max_q + 31) / 32) < 8 ? p.G * ((max_q + 31) / 32) : 8;
+            const int64_t live = slots * ((units + (1 << usplit) - 1) >> usplit) * groups * CS;
+            const bool shared = live <= (D == 256 ? 2 : 1) * int64_t(p.round_slots);
+            if (shared) {
+                hipLaunchKernelGGL((attention_combine_kernel<D, DT, PAGED, KS>), dim3(unsigned(slots), (8 >> usplit) * groups, CS), dim3(256),
+                                   0, s, p, rows, usplit);
+                return fq_host::check_launch();
+            }
+        }
+        hipLaunchKernelGGL((attention_combine_kernel<D, DT, PAGED, 1>), dim3(unsigned(slots), 8 * groups), dim3(256), 0, s, p, rows, 0);
         return fq_host::check_launch();
     }
     return st;

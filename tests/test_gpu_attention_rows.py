@@ -76,6 +76,21 @@ def test_attention_over_split_contexts(b, hq, hkv, nq, nkv, d, dtype):
     _close(got, want, dtype)
 
 
+# query heads that four do not divide, more than one workgroup of 8 units a KV head, a group of rows with one query and with two;
+# as many groups as still leave CUs for several workgroups each (b = 1, 2) and more (b = 40)
+@pytest.mark.parametrize("d", [128, 256])
+@pytest.mark.parametrize("b,hq,hkv,nq", [(1, 1, 1, 1), (2, 6, 2, 2), (1, 5, 1, 1), (2, 7, 1, 2), (1, 9, 1, 1), (1, 12, 1, 2), (2, 16, 1, 1), (1, 18, 2, 2),
+                                         (1, 6, 2, 3), (2, 5, 1, 6), (40, 5, 1, 1), (40, 3, 1, 2)])
+def test_heads_that_share_a_group_of_combined_rows(b, hq, hkv, nq, d):
+    kv, c, r = _packed(b, hkv, 640, d, 33)
+    q = torch.randn(b, hq, nq, d, generator=torch.Generator().manual_seed(34)).to(torch.bfloat16)
+    want = O.fused_tq_attention(q, *kv, c, c, r)
+    dev = [t.to(DEV) for t in (q, *kv, c, c, r)]
+    got = K.fused_tq_attention(*dev)
+    _close(got, want, torch.bfloat16)
+    assert torch.equal(K.fused_tq_attention(*dev[:-1], r.t().contiguous().to(DEV).t()), got)       # the matrix in the other layout
+
+
 @pytest.mark.parametrize("d", [64, 128])
 def test_attention_over_split_contexts_causal_and_huge_norms(d):
     """Causal rows that see nothing of a piece, and rows whose norms exceed fp16 in one piece only."""
