@@ -25,13 +25,14 @@ namespace fq {
 
 namespace {
 
-template <int D>
+// LONG: see launch_decompress_rotate
+template <int D, bool LONG>
 struct DecRotCfg {
     static constexpr int NK = D / 16;                  // MFMA k-steps
     static constexpr int CB = D / 32;                  // 32-coordinate output blocks
     static constexpr int WAVES = CB < 4 ? 4 : CB;
     static constexpr int THREADS = WAVES * kWave;
-    static constexpr int TT = D == 256 ? 32 : 64;      // rows per tile
+    static constexpr int TT = D == 256 && !LONG ? 32 : 64;     // rows per tile
     static constexpr int TB = TT / 32;                 // 32-row blocks per tile
     static constexpr int TB_STEP = WAVES / CB;         // row blocks handled in parallel
     static constexpr int UPR = D / 8;                  // packed dwords (8 coordinates) per row
@@ -65,13 +66,13 @@ struct DecRotSource {
     float inv_H;              // 1 / H
 };
 
-template <int D, int DT, bool CACHE>
-__global__ __launch_bounds__(DecRotCfg<D>::THREADS) void tq4_decompress_rotate_kernel(
+template <int D, int DT, bool CACHE, bool LONG>
+__global__ __launch_bounds__((DecRotCfg<D, LONG>::THREADS)) void tq4_decompress_rotate_kernel(
     const DecRotSource src, const float* __restrict__ centroids, const float* __restrict__ rotation, int col_major,
     uint16_t* __restrict__ out, uint16_t* __restrict__ out_v, int64_t M, int64_t num_tiles) {
-    using C = DecRotCfg<D>;
+    using C = DecRotCfg<D, LONG>;
     __shared__ __attribute__((aligned(16))) uint8_t xs[2][C::TT * C::STRIDE];   // dequantised rows, 16-bit
-    __shared__ __attribute__((aligned(16))) uint8_t os[C::TT * C::STRIDE];      // rotated rows, 16-bit
+    __shared__ __attribute__((aligned(16))) uint8_t os[LONG ? 2 : 1][C::TT * C::STRIDE];     // rotated rows, 16-bit
     __shared__ float lut[16];
 
     const int tid = threadIdx.x;
@@ -80,46 +81,6 @@ __global__ __launch_bounds__(DecRotCfg<D>::THREADS) void tq4_decompress_rotate_k
     const int cb = wave % C::CB, tb0 = wave / C::CB;
 
     if (tid < 16) lut[tid] = centroids[tid];
-
-    // ---- the matrix rows of this wavefront: A[j][k] = R[k][j], two 16-bit terms ---------------
-    constexpr bool kBf16 = DT == FQ_BF16;
-    half8 a_hi[kBf16 ? 1 : C::NK], a_lo[kBf16 ? 1 : C::NK];
-    bf16x8 a_t[kBf16 ? 2 : 1][kBf16 ? C::NK : 1];
-    {
-        const int j = 32 * cb + row_to_coord(n32);
-#pragma unroll
-        for (int ks = 0; ks < C::NK; ++ks) {
-            // a lane's eight elements of a k-step are contiguous in a column-major matrix (what a QR factor is);
-            // asked for one by one they were 64 requests of 64 lines each in front of the first tile
-            float rk[8];
-            const int k0 = 16 * ks + 8 * kg;
-            if (col_major) {
-                typedef float4v float4a __attribute__((aligned(4)));       // the matrix need not be aligned to 16 bytes
-                const float4v lo = *reinterpret_cast<const float4a*>(rotation + int64_t(j) * D + k0);
-                const float4v hi = *reinterpret_cast<const float4a*>(rotation + int64_t(j) * D + k0 + 4);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) { rk[e] = lo[e]; rk[4 + e] = hi[e]; }
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) rk[e] = rotation[int64_t(k0 + e) * D + j];
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float r = rk[e];
-                if constexpr (kBf16) {
-                    const uint16_t t0 = float_to_bf16(r);
-                    const uint16_t t1 = float_to_bf16(r - bf16_to_float(t0));
-                    a_t[0][ks][e] = __builtin_bit_cast(__bf16, t0);
-                    a_t[1][ks][e] = __builtin_bit_cast(__bf16, t1);
-                } else {
-                    const _Float16 hi = _Float16(r);
-                    a_hi[ks][e] = hi;
-                    a_lo[ks][e] = _Float16((r - float(hi)) * 4096.0f);
-                }
-            }
-        }
-    }
-    __syncthreads();
 
     // ---- staging: unit u of a tile = packed dword u % UPR of tile row u / UPR ------------------
     uint32_t word[C::UPT];
@@ -169,6 +130,51 @@ __global__ __launch_bounds__(DecRotCfg<D>::THREADS) void tq4_decompress_rotate_k
             nrm[i] = live ? norms[row] : 0.0f;
         }
     };
+    // the first tile's rows are asked for before the matrix, whose fetch and split they arrive behind (2 x 12,800 rows
+    // of 128 8.1 -> 7.7 us, 2 x 51,200 of 64 8.7 -> 8.3)
+    int64_t tile = blockIdx.x;
+    if (tile < num_tiles) issue_loads(tile);
+
+    // ---- the matrix rows of this wavefront: A[j][k] = R[k][j], two 16-bit terms ---------------
+    constexpr bool kBf16 = DT == FQ_BF16;
+    half8 a_hi[kBf16 ? 1 : C::NK], a_lo[kBf16 ? 1 : C::NK];
+    bf16x8 a_t[kBf16 ? 2 : 1][kBf16 ? C::NK : 1];
+    {
+        const int j = 32 * cb + row_to_coord(n32);
+#pragma unroll
+        for (int ks = 0; ks < C::NK; ++ks) {
+            // a lane's eight elements of a k-step are contiguous in a column-major matrix (what a QR factor is);
+            // asked for one by one they were 64 requests of 64 lines each in front of the first tile
+            float rk[8];
+            const int k0 = 16 * ks + 8 * kg;
+            if (col_major) {
+                typedef float4v float4a __attribute__((aligned(4)));       // the matrix need not be aligned to 16 bytes
+                const float4v lo = *reinterpret_cast<const float4a*>(rotation + int64_t(j) * D + k0);
+                const float4v hi = *reinterpret_cast<const float4a*>(rotation + int64_t(j) * D + k0 + 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { rk[e] = lo[e]; rk[4 + e] = hi[e]; }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) rk[e] = rotation[int64_t(k0 + e) * D + j];
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float r = rk[e];
+                if constexpr (kBf16) {
+                    const uint16_t t0 = float_to_bf16(r);
+                    const uint16_t t1 = float_to_bf16(r - bf16_to_float(t0));
+                    a_t[0][ks][e] = __builtin_bit_cast(__bf16, t0);
+                    a_t[1][ks][e] = __builtin_bit_cast(__bf16, t1);
+                } else {
+                    const _Float16 hi = _Float16(r);
+                    a_hi[ks][e] = hi;
+                    a_lo[ks][e] = _Float16((r - float(hi)) * 4096.0f);
+                }
+            }
+        }
+    }
+    __syncthreads();
+
     auto stage = [&](int buf) {
 #pragma unroll
         for (int i = 0; i < C::UPT; ++i) {
@@ -182,7 +188,7 @@ __global__ __launch_bounds__(DecRotCfg<D>::THREADS) void tq4_decompress_rotate_k
             *reinterpret_cast<uint4v*>(&xs[buf][(u / C::UPR) * C::STRIDE + (u % C::UPR) * 16]) = uint4v{h[0], h[1], h[2], h[3]};
         }
     };
-    auto store_tile = [&](int64_t any_tile) {
+    auto store_tile = [&](int64_t any_tile, const uint8_t* rows) {
         constexpr int OC = D / 8;            // 16-byte chunks per output row
         const bool is_v = CACHE && any_tile >= half_tiles;
         const int64_t tile = is_v ? any_tile - half_tiles : any_tile;
@@ -191,25 +197,15 @@ __global__ __launch_bounds__(DecRotCfg<D>::THREADS) void tq4_decompress_rotate_k
             const int r = c / OC, q = c % OC;
             const int64_t row = tile * C::TT + r;
             if (row < M) {
-                const uint4v v = *reinterpret_cast<const uint4v*>(&os[r * C::STRIDE + q * 16]);
+                const uint4v v = *reinterpret_cast<const uint4v*>(rows + r * C::STRIDE + q * 16);
                 __builtin_nontemporal_store(v, reinterpret_cast<uint4v*>(dst + row * D) + q);
             }
         }
     };
 
-    int64_t tile = blockIdx.x;
-    if (tile < num_tiles) {
-        issue_loads(tile);
-        stage(0);
-    }
-    __syncthreads();
-    for (int it = 0; tile < num_tiles; tile += gridDim.x, ++it) {
-        const int cur = it & 1;
-        const int64_t next = tile + gridDim.x;
-        if (next < num_tiles) issue_loads(next);
-
+    auto rotate_tile = [&](const uint8_t* xs_tile, uint8_t* os_tile) {
         for (int tb = tb0; tb < C::TB; tb += C::TB_STEP) {
-            const uint8_t* brow = &xs[cur][(32 * tb + n32) * C::STRIDE + kg * 16];
+            const uint8_t* brow = xs_tile + (32 * tb + n32) * C::STRIDE + kg * 16;
             float16v acc = {};
             float16v acc_lo = {};
             if constexpr (kBf16) {
@@ -238,29 +234,77 @@ __global__ __launch_bounds__(DecRotCfg<D>::THREADS) void tq4_decompress_rotate_k
                 }
                 w[i] = round_pair<DT>(v0, v1);
             }
-            uint8_t* dst = &os[(32 * tb + n32) * C::STRIDE + (32 * cb + 16 * kg) * 2];
+            uint8_t* dst = os_tile + (32 * tb + n32) * C::STRIDE + (32 * cb + 16 * kg) * 2;
             *reinterpret_cast<uint4v*>(dst) = uint4v{w[0], w[1], w[2], w[3]};
             *reinterpret_cast<uint4v*>(dst + 16) = uint4v{w[4], w[5], w[6], w[7]};
         }
+    };
+
+    if (tile < num_tiles) stage(0);
+    if constexpr (LONG) {
+        // one barrier a tile: behind it the tile's product, the staging of the next and the stores of the one before go side by
+        // side; one half of the wavefronts begins with the product, the other with the staging
+        const bool product_first = wave < C::WAVES / 2;
+        if (tile + gridDim.x < num_tiles) issue_loads(tile + gridDim.x);
+        __syncthreads();
+        for (int it = 0; tile < num_tiles; tile += gridDim.x, ++it) {
+            const int cur = it & 1;
+            const int64_t next = tile + gridDim.x;
+            auto stage_next = [&] {
+                if (next < num_tiles) stage(cur ^ 1);
+                if (next + gridDim.x < num_tiles) issue_loads(next + gridDim.x);
+            };
+            if (!product_first) stage_next();
+            rotate_tile(xs[cur], os[cur]);
+            if (product_first) stage_next();
+            if (it > 0) store_tile(tile - gridDim.x, os[cur ^ 1]);
+            __syncthreads();
+            if (next >= num_tiles) store_tile(tile, os[cur]);
+        }
+        return;
+    }
+    __syncthreads();
+    for (int it = 0; tile < num_tiles; tile += gridDim.x, ++it) {
+        const int cur = it & 1;
+        const int64_t next = tile + gridDim.x;
+        if (next < num_tiles) issue_loads(next);
+        rotate_tile(xs[cur], os[0]);
         __syncthreads();                       // the rotated rows of this tile are complete
-        store_tile(tile);
+        store_tile(tile, os[0]);
         if (next < num_tiles) stage(cur ^ 1);
         __syncthreads();                       // the next tile is staged; `os` is free again
     }
 }
 
+template <int D, int DT, bool CACHE, bool LONG>
+int launch_decompress_rotate_as(const DecRotSource& src, const float* centroids, const float* rotation, int col_major,
+                                void* out, void* out_v, int64_t M, int64_t cap, hipStream_t s) {
+    using C = DecRotCfg<D, LONG>;
+    const int64_t tiles = (M + C::TT - 1) / C::TT * (CACHE ? 2 : 1);
+    hipLaunchKernelGGL((tq4_decompress_rotate_kernel<D, DT, CACHE, LONG>), dim3(unsigned(tiles < cap ? tiles : cap)), dim3(C::THREADS), 0, s,
+                       src, centroids, rotation, col_major, static_cast<uint16_t*>(out), static_cast<uint16_t*>(out_v), M, tiles);
+    return fq_host::check_launch();
+}
+
 template <int D, int DT, bool CACHE>
 int launch_decompress_rotate(const DecRotSource& src, const float* centroids, const float* rotation, int col_major,
                              void* out, void* out_v, int64_t M, hipStream_t s) {
-    using C = DecRotCfg<D>;
-    const int64_t tiles = (M + C::TT - 1) / C::TT * (CACHE ? 2 : 1);
-    // workgroups per CU: three fit the LDS at head_dim <= 128; the fp16 route holds two
-    // accumulators per wavefront and runs faster with two
-    const int64_t cap = int64_t(fq_host::device_cu_count()) * ((D == 256 || DT == FQ_F16) ? 2 : 3);
-    const unsigned grid = unsigned(tiles < cap ? tiles : cap);
-    hipLaunchKernelGGL((tq4_decompress_rotate_kernel<D, DT, CACHE>), dim3(grid), dim3(C::THREADS), 0, s, src, centroids,
-                       rotation, col_major, static_cast<uint16_t*>(out), static_cast<uint16_t*>(out_v), M, tiles);
-    return fq_host::check_launch();
+    const int64_t cus = fq_host::device_cu_count();
+    // At head_dim 256 the matrix in two terms takes 128 registers, and one workgroup of eight wavefronts fills a CU; a second
+    // round of workgroups would fetch and split the 256 KB again, so there is one a CU: 2 x 38,400 rows of a cache in bf16
+    // 39.2 us with two, 30.2 with one.  Alone on its CU it hides nothing behind another one's work, so from two tiles of 32
+    // rows a CU on it is pipelined over tiles of 64 (LONG): 28.0 us; 2 x 192,000 rows 115 in the plain form, 111 pipelined over
+    // 32, 108 over 64 (bound by the product: 80 us at the power limit).  2 x 1920 rows 11.9, 12.1 and 13.0.
+    if constexpr (D == 256) {
+        return M * (CACHE ? 2 : 1) >= 64 * cus
+                   ? launch_decompress_rotate_as<D, DT, CACHE, true>(src, centroids, rotation, col_major, out, out_v, M, cus, s)
+                   : launch_decompress_rotate_as<D, DT, CACHE, false>(src, centroids, rotation, col_major, out, out_v, M, cus, s);
+    } else {
+        // workgroups per CU: three fit the LDS; the fp16 route holds two accumulators per wavefront and runs faster with two.
+        // (Pipelined, with the second area for rotated rows only two would fit: 2 x 192,128 rows of 128 in bf16 38.8 and 45.3 us.)
+        return launch_decompress_rotate_as<D, DT, CACHE, false>(src, centroids, rotation, col_major, out, out_v, M,
+                                                                cus * (DT == FQ_F16 ? 2 : 3), s);
+    }
 }
 
 template <bool CACHE>

@@ -51,6 +51,29 @@ def test_decompress_cache_equals_decompress_of_its_sections(pages, page, h, d):
     assert torch.equal(v.view(-1, h, d), K.tq4_decompress_rotated(vp, vn, layer.centroids, layer.rotation, torch.bfloat16))
 
 
+# rows of 256 coordinates: the fewest that run in the pipelined form (64 a CU), one more and one fewer, last tiles of 1, 63 and 64
+# rows, one tile and several a workgroup
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tiles,extra", [(1, -1), (1, 0), (1, 1), (2, -1), (3, 0), (3, 63), (4, 65)])
+def test_decompress_rotated_of_many_wide_rows(tiles, extra, dtype):
+    """The same bits as the same rows a few thousand at a time, which the other tests hold against a float32 product."""
+    layer = TQ4AttentionKernels(1, 256, 1.0 / 16, torch.device(DEV))
+    n = 64 * tiles * torch.cuda.get_device_properties(0).multi_processor_count + extra
+    g = torch.Generator(device=DEV).manual_seed(n)
+    packed = torch.randint(0, 256, (n, 1, 128), dtype=torch.uint8, generator=g, device=DEV)
+    norms = torch.rand(n, 1, 1, generator=g, device=DEV) * 30 + 0.01
+    for rotation in (layer.rotation.contiguous(), layer.rotation.t().contiguous().t()):
+        out = torch.full((n + 1, 1, 256), 7.0, dtype=dtype, device=DEV)
+        K.tq4_decompress_rotated(packed, norms, layer.centroids, rotation, dtype, out=out[:n])
+        want = torch.cat([K.tq4_decompress_rotated(packed[i:i + 4001], norms[i:i + 4001], layer.centroids, rotation, dtype)
+                          for i in range(0, n, 4001)])
+        assert torch.equal(out[:n], want) and (out[n] == 7).all()
+    # a cache row of one head: keys and values side by side
+    cache = torch.cat([packed.view(n, 128), norms.view(n, 1).view(torch.uint8).view(n, 4)] * 2, dim=1).view(n, 1, 264)
+    k, v = layer.decompress_cache(cache, dtype)
+    assert torch.equal(k.view_as(want), want) and torch.equal(v.view_as(want), want)
+
+
 def test_decompress_cache_of_no_pages_and_argument_errors():
     layer = TQ4AttentionKernels(8, 128, 1.0, torch.device(DEV))
     k, v = layer.decompress_cache(torch.empty(0, 16, 8 * 136, dtype=torch.uint8, device=DEV), torch.bfloat16)
