@@ -13,7 +13,7 @@
 // allows for and the number of CUs): within rounding, and the same for the same call.
 // Measured (MI355X, bf16, 32 query heads over 8 KV heads of 128): a batch of 12 with six prompts, three later chunks and
 // three single queries, 10,556 new tokens, 467 us in grid order and 385 us longest first; one query over 4 x 2500 tokens of a
-// ring buffer 67 us in one workgroup per KV head, 22 us in 8 pieces, over 1 x 16,384 tokens 31 us in 32 pieces (369 us
+// ring buffer 67 us in one workgroup per KV head, 22 us in 8 pieces (20 with the combine's columns shared), over 1 x 16,384 tokens 31 us in 32 pieces (369 us
 // before the kernel cut contexts).
 // Everything here is arithmetic on the lengths alone: the same in every workgroup and in the combine launch.
 #pragma once
@@ -147,7 +147,8 @@ FQ_HD int first_piece_with(const SeqShape& s, int T, int pieces, int G, bool cau
 // of one known length under a causal mask) is about one round of workgroups, the longest with twice the average work: two
 // pieces, if half of the longest workgroup outweighs that traffic and the second prologues too.  (Whether the shares are
 // uneven enough pieces_of decides; more workgroups than 4/3 of a round never are.)  8 heads x 6000 tokens of 256 coordinates,
-// one KV head, 188 workgroups: 538 us in one piece, 336 us in two; 16 heads x 3001 tokens on 4 KV heads 307 and 220 us (203 now).  Else only
+// one KV head, 188 workgroups: 538 us in one piece, 336 us in two; 16 heads x 3001 tokens on 4 KV heads 307 and 220 us (203 later; with room for their expanded keys
+// and values such prompts take another kernel: 136).  Else only
 // sequences of one workgroup (single queries of a mixed batch) are.
 struct SplitPlan {
     int split_w, max_pieces;

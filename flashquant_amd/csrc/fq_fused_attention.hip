@@ -1208,8 +1208,9 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const PrefillPar
 // The same for whole prompts in pieces, where the rotation is the work: a workgroup as the one that left the pieces, its
 // wavefronts gather their 32 rows in the accumulators and end as that kernel does (the kernel above fetches and splits the
 // matrix for every 16 rows).  When it was added, 16 heads x 3001 tokens of 256 coordinates, 188 workgroups in two pieces: 298 us
-// with the kernel above, 240 with this one (203 now); 8 heads x 5000 tokens of 128, 157 workgroups: 140 and 121; 16 heads x
-// 2000 tokens of 64, 128 workgroups: 54.6 and 48.3 (45.8 now).  With 63 workgroups in four pieces the smaller workgroups above
+// with the kernel above, 240 with this one (203 later; where the caller gives room for expanded
+// keys and values, 136 without either); 8 heads x 5000 tokens of 128, 157 workgroups: 140 and 121; 16 heads x
+// 2000 tokens of 64, 128 workgroups: 54.6 and 48.3 (45.8 later).  With 63 workgroups in four pieces the smaller workgroups above
 // are faster (128 and 148 us at 256 coordinates, 55 and 68 at 128): this one runs from half a round of workgroups on.  At 256
 // coordinates the rounds of the matrix share one area (64 KB, so that two workgroups fit a CU): with two of them 14 registers
 // were spilled and 16 heads x 3001 tokens took 209 us, 202 with one.

@@ -51,7 +51,8 @@ def paged_tq4_prefill(
     causal: bool = True,
     out: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
-    """Prefill (or chunked prefill) over the packed paged cache in one launch.
+    """Prefill (or chunked prefill) over the packed paged cache in one call (keys and values that many
+    queries share are expanded once, into a workspace).
 
     ``q`` (tokens, H_Q, D) holds the un-rotated queries of all sequences, the
     queries of sequence ``s`` at ``cu_seqlens_q[s]:cu_seqlens_q[s+1]``;

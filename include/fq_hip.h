@@ -308,7 +308,8 @@ int fq_fused_tq_attention_strided(const void* q, const uint8_t* k_packed, const 
  *   out           (total_q, H_Q, D) same dtype as q
  *   max_q_len     the largest query count of a sequence (sizes the grid)
  *   is_causal     query j of n in a sequence of L keys sees keys 0 .. L - n + j
- * The attention result is rounded to the query dtype before the rotation back,
+ * The attention result is rounded to the query dtype before the rotation back (not where
+ *   the keys and values are expanded: those are rotated back first, the result is rounded once),
  * as the attention library's output is in the reference.  A sequence with no
  * queries is skipped; with no keys its rows are zero.  D in {64, 128, 256} as for
  * fq_fused_tq_attention.
@@ -330,7 +331,7 @@ int fq_paged_tq4_prefill(const void* q, const int32_t* cu_seqlens_q, const uint8
  * Where many queries share their keys, fq_fused_tq_attention_split first writes keys and values, rotated back, as fp16
  * matrix operands into the workspace and attends to these (no rounding of the rotated query, fewer of the keys and values).
  *   workspace        256-byte aligned, at least fq_attention_workspace_bytes bytes (0: these sizes need none; at
- *                    most 65 MiB paged, 172 MiB for prompts in pieces, 1.1 GiB for expanded keys and values); NULL:
+ *                    most 65 MiB paged, 172 MiB for prompts in pieces, for expanded keys and values 1.1 GiB, 2.2 GiB paged); NULL:
  *                    nothing is split or expanded.  With what suffices for pieces alone nothing is expanded.
  *   max_kv_len       the longest context possible: N_KV, or max_blocks_per_seq * block_size
  *   prompts          for fq_fused_tq_attention_split 1 with is_causal, 2 without (all sequences have these very lengths);
