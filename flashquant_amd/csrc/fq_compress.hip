@@ -198,7 +198,11 @@ struct PagedDest {
 // 3: R = t0 + t1 + t2 exactly.  2: t0, t1 rounded to nearest, |R - t0 - t1| <= 2^-18 |R|: the rotated
 // coordinates move by about 2e-7 (standard deviation, unit rows of 128 coordinates), which puts about 6
 // indices in a million on the other side of a bucket boundary, for two thirds of the matrix instructions.
-template <int D, int DT, bool PAGED, int NT>
+// SHARED: the 32-coordinate blocks of a tile are shared by gridDim.y workgroups, each fetching and splitting its part of the
+// matrix; all stage the tile, the first one writes the norms.  The same products in the same order: the same bits.  A call of
+// few rows is the fetch of the matrix (256 KB through one CU at 256 coordinates), its split and the bucket table: rule at
+// launch_tiles.
+template <int D, int DT, bool PAGED, int NT, bool SHARED>
 __global__ __launch_bounds__(CompressCfg<D>::THREADS) void tq4_compress_kernel(
     const uint4v* __restrict__ x, const float* __restrict__ rot_T_even,
     const float* __restrict__ rot_T_odd, const float* __restrict__ boundaries,
@@ -328,8 +332,9 @@ __global__ __launch_bounds__(CompressCfg<D>::THREADS) void tq4_compress_kernel(
     half8 a_hi[kBf16 ? 1 : C::NK], a_lo[kBf16 ? 1 : C::NK];
     bf16x8 a_t[kBf16 ? NT : 1][kBf16 ? C::NK : 1];
     // the matrix rows are asked for, the bucket table is built while they arrive, then they are split
-    float rr[C::NK][8];
-    {
+    // (the other blocks' wavefronts of a shared tile stage rows and multiply by zero; nothing of theirs is stored)
+    float rr[C::NK][8] = {};
+    if (!SHARED || __builtin_amdgcn_readfirstlane(cb) * int(gridDim.y) / C::CB == int(blockIdx.y)) {
         const int j = 32 * cb + mfma_row_to_coord(n32);
         const float* src = (j & 1) ? rot_T_odd : rot_T_even;
         const int col = j >> 1;
@@ -441,7 +446,7 @@ __global__ __launch_bounds__(CompressCfg<D>::THREADS) void tq4_compress_kernel(
         if (chunk < C::PASSES) {
             const int r = chunk * C::ROWS_PER_PASS + row_in_pass;
             inv_s[buf][r] = up_mine * __builtin_amdgcn_rcpf(nrm + 1e-10f);
-            if (r < live) {
+            if (r < live && (!SHARED || blockIdx.y == 0)) {
                 if (PAGED) {
                     int head, is_v;
                     uint8_t* dst = paged_row(org, r, head, is_v);
@@ -461,8 +466,8 @@ __global__ __launch_bounds__(CompressCfg<D>::THREADS) void tq4_compress_kernel(
         const int live = rows_in(tile);
         const int64_t row0 = tile * C::TT;
         for (int c = tid; c < C::TT * OC; c += C::THREADS) {
-            const int r = c / OC, q = c % OC;
-            if (r < live) {
+            const int r = c / OC, q = c % OC;                   // chunk q: the coordinates of block q
+            if (r < live && (!SHARED || q * int(gridDim.y) / C::CB == int(blockIdx.y))) {
                 const uint2v lo = *reinterpret_cast<const uint2v*>(&ob[r * C::OUT_STRIDE + q * 16]);
                 const uint2v hi = *reinterpret_cast<const uint2v*>(&ob[r * C::OUT_STRIDE + q * 16 + 8]);
                 uint4v v = {lo.x, lo.y, hi.x, hi.y};
@@ -664,19 +669,35 @@ int bf16_terms() {
     return fq_host::option(FQ_OPT_COMPRESS_THREE_TERMS) != 0 ? 3 : 2;
 }
 
+// Workgroups share a tile while there are CUs for all of them.  bf16, in us, alone and shared: 128 coordinates, 1 tile 7.7 and 7.2, 32
+// tiles (by four) 8.0 and 6.9, 65 and 100 (by two) 8.0 and 7.75; 256 coordinates, 1 tile 14.5 and 9.8, 32 (by eight) 15.0 and
+// 9.4, 60 (by four) 15.0 and 10.7, 120 (by two) 15.0 and 11.9.  Two workgroups a CU lose: 60 tiles by eight 18.0, 100 of 128 by four 9.0.
+// Not at 64 coordinates, where the matrix is 16 KB: 6.7 us either way.
+template <int D, int DT, bool PAGED, class... Args>
+void launch_tiles(int64_t tiles, int num_cus, hipStream_t s, Args... args) {
+    using C = CompressCfg<D>;
+    const int64_t cap = int64_t(num_cus) * 2;
+    const unsigned grid = unsigned(tiles < cap ? tiles : cap);
+    const bool three = bf16_terms<D, DT>() == 3;
+    if constexpr (D >= 128) {
+        int share = C::CB;
+        while (share > 1 && tiles * share > num_cus) share /= 2;
+        if (share > 1) {
+            if (three) hipLaunchKernelGGL((tq4_compress_kernel<D, DT, PAGED, 3, true>), dim3(grid, share), dim3(C::THREADS), 0, s, args...);
+            else hipLaunchKernelGGL((tq4_compress_kernel<D, DT, PAGED, 2, true>), dim3(grid, share), dim3(C::THREADS), 0, s, args...);
+            return;
+        }
+    }
+    if (three) hipLaunchKernelGGL((tq4_compress_kernel<D, DT, PAGED, 3, false>), dim3(grid), dim3(C::THREADS), 0, s, args...);
+    else hipLaunchKernelGGL((tq4_compress_kernel<D, DT, PAGED, 2, false>), dim3(grid), dim3(C::THREADS), 0, s, args...);
+}
+
 template <int D, int DT>
 int launch_compress(const void* x, const float* re, const float* ro, const float* bnd, uint8_t* packed,
                     float* norms, int64_t M, int num_cus, hipStream_t s, const PagedDest& pd = PagedDest{}) {
     using C = CompressCfg<D>;
     const int64_t tiles = (M + C::TT - 1) / C::TT;
-    const int64_t cap = int64_t(num_cus) * 2;
-    const unsigned grid = unsigned(tiles < cap ? tiles : cap);
-    if (bf16_terms<D, DT>() == 3)
-        hipLaunchKernelGGL((tq4_compress_kernel<D, DT, false, 3>), dim3(grid), dim3(C::THREADS), 0, s,
-                           reinterpret_cast<const uint4v*>(x), re, ro, bnd, packed, norms, M, tiles, pd);
-    else
-        hipLaunchKernelGGL((tq4_compress_kernel<D, DT, false, 2>), dim3(grid), dim3(C::THREADS), 0, s,
-                           reinterpret_cast<const uint4v*>(x), re, ro, bnd, packed, norms, M, tiles, pd);
+    launch_tiles<D, DT, false>(tiles, num_cus, s, reinterpret_cast<const uint4v*>(x), re, ro, bnd, packed, norms, M, tiles, pd);
     return fq_host::check_launch();
 }
 
@@ -686,16 +707,8 @@ int launch_compress_store(const void* key, const float* re, const float* ro, con
     using C = CompressCfg<D>;
     const int64_t M = 2 * pd.rows_k;
     const int64_t tiles = (M + C::TT - 1) / C::TT;
-    const int64_t cap = int64_t(num_cus) * 2;
-    const unsigned grid = unsigned(tiles < cap ? tiles : cap);
-    if (bf16_terms<D, DT>() == 3)
-        hipLaunchKernelGGL((tq4_compress_kernel<D, DT, true, 3>), dim3(grid), dim3(C::THREADS), 0, s,
-                           reinterpret_cast<const uint4v*>(key), re, ro, bnd, static_cast<uint8_t*>(nullptr),
-                           static_cast<float*>(nullptr), M, tiles, pd);
-    else
-        hipLaunchKernelGGL((tq4_compress_kernel<D, DT, true, 2>), dim3(grid), dim3(C::THREADS), 0, s,
-                           reinterpret_cast<const uint4v*>(key), re, ro, bnd, static_cast<uint8_t*>(nullptr),
-                           static_cast<float*>(nullptr), M, tiles, pd);
+    launch_tiles<D, DT, true>(tiles, num_cus, s, reinterpret_cast<const uint4v*>(key), re, ro, bnd, static_cast<uint8_t*>(nullptr),
+                              static_cast<float*>(nullptr), M, tiles, pd);
     return fq_host::check_launch();
 }
 

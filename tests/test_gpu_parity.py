@@ -189,6 +189,23 @@ def test_compress_scales_and_adversarial_rows():
     assert torch.equal(packed.cpu(), want_p) and torch.equal(norms.cpu(), want_n)
 
 
+@pytest.mark.parametrize("three", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_compress_of_few_rows_is_compress_of_many(d, dtype, three, kernel_option):
+    """A tile of few rows is shared by several workgroups, each with its part of the coordinates: the same products in the same
+    order, so the same bits as in a call whose tiles are not, for rows around a tile and around the most tiles that 8, 4 and 2
+    workgroups share."""
+    kernel_option("compress_three_terms", three)
+    c, b, r = (t.to(DEV) for t in book(d))
+    tt, cus = 32 if d == 256 else 64, torch.cuda.get_device_properties(0).multi_processor_count
+    x = torch.randn(2 * cus * tt + 5, 1, d, generator=torch.Generator(device=DEV).manual_seed(d), device=DEV).to(dtype)
+    packed, norms = K.tq4_compress(x, r, b)
+    for n in (1, tt - 1, tt, tt + 1, *(cus // s * tt + e for s in (8, 4, 2, 1) for e in (-1, 0, 1))):
+        got_p, got_n = K.tq4_compress(x[:n], r, b)
+        assert torch.equal(got_p, packed[:n]) and torch.equal(got_n, norms[:n]), n
+
+
 @pytest.mark.parametrize("d", [64, 128, 256])
 def test_compress_bf16_two_and_three_matrix_terms(d, kernel_option):
     """bf16 rows are rotated against the matrix as two bf16 terms (default) or three (the float32
