@@ -180,12 +180,34 @@ inline ExpandedPlan plan_expanded(int64_t B, int H_KV, int64_t n_q, int64_t n_kv
     return e;
 }
 
-// The same for paged batches, of which the host knows the number of sequences, the tokens and the longest context possible.
-inline ExpandedPlan plan_expanded_paged(int64_t num_seqs, int64_t total_q, int64_t max_kv, int H_KV, int G, int D) {
+// The same for paged batches, of which the host knows the number of sequences, the tokens, the most of a sequence and the longest
+// context possible.  It stays on the other kernel too
+//   * with few queries under a wide block table (3 of its columns to 10 rows of a KV head);
+//   * at 128 coordinates where that kernel runs all sequences in one round of its workgroups (256 rows each) and the keys are many for it.
+//     Its round of up to 4 units of 32 rows a workgroup takes 15 us and more, of 5 to 8 units 23, several rounds 30.  Measured (bf16;
+//     sequences x tokens, query heads over KV heads; us here / there): up to 4 units, from 32 blocks of 64 keys on, 12 x 6, 16 over 16,
+//     17.4 / 15.3, 13 x 83, 16 over 16, 24.0 / 19.1, and below that 2 x 10, 8 over 8, 15.8 / 15.3; up to 8 units, from 384 blocks on (192
+//     where every sequence has only one), 12 x 214, 16 over 16, 36.3 / 28.7, 57 x 17, 32 over 4, 24.9 / 23.4, and below that 2 of 213 (up
+//     to 252), 4 over 4, 19.4 / 26.4; up to 12 units, from 640 blocks on, 8 x 380, 16 over 16, 35.4 / 32.5, 4 x 300, 32 over 32, 32.6 /
+//     31.3, and below that 16 x 300, 8 over 8, 31.9 / 31.2.
+// Of 18,000 batches of 1 to 256 sequences that the first line leaves 941 ran more than 3 % slower here (the worst 8 chunks of 93, 32 over
+// 32, 37.1 / 25.5); the others leave 29 of them and refuse 130 that would have run more than 3 % faster here.  What is left is mostly
+// chunks of 64 coordinates that two launches more do not pay for (2 % of those; 407 over 1551 tokens, 8 over 1, 32.3 / 26.9), which no line
+// on these sizes tells from ones that gain.
+inline bool one_round_is_faster(int64_t num_seqs, int64_t total_q, int64_t max_q, int64_t max_kv, int H_KV, int G, int D) {
+    const int64_t cus = fq_host::device_cu_count(), pairs = num_seqs * H_KV, units = (max_q + 31) / 32 * G, blocks = (max_kv + 63) / 64;
+    if (D != 128) return false;
+    if (units <= 8) return pairs <= cus && pairs * blocks >= (units <= 4 ? 32 : (blocks == 1 ? 192 : 384));
+    // workgroups of that kernel: a sequence has half a block of 32 queries and half a workgroup more than its tokens fill
+    const int64_t most = num_seqs * ((units + 7) / 8), about = ((total_q / 16 + num_seqs) * G / 8 + num_seqs) / 2;
+    return units <= 12 && (about < most ? about : most) * H_KV <= cus && pairs * blocks >= 640;
+}
+inline ExpandedPlan plan_expanded_paged(int64_t num_seqs, int64_t total_q, int64_t max_q, int64_t max_kv, int H_KV, int G, int D) {
     ExpandedPlan e;
     const int64_t tt = D == 256 ? 32 : 64, tiles = num_seqs * ((max_kv + tt - 1) / tt);
     if (num_seqs > 256 || total_q <= 0 || tiles * H_KV * (4 * tt * D) > 0x7fffffff) return e;
     if (10 * total_q * G < 3 * num_seqs * max_kv || (D == 64 && total_q < 256 * num_seqs)) return e;
+    if (one_round_is_faster(num_seqs, total_q, max_q, max_kv, H_KV, G, D)) return e;
     const int64_t workgroups = (total_q / 32 + num_seqs) * G / 4 + num_seqs;
     if (workgroups * H_KV > (int64_t(1) << 23) || workgroups >= (1 << 20)) return e;
     e.tiles = int(tiles);

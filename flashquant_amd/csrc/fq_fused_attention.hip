@@ -1402,7 +1402,7 @@ extern "C" size_t fq_paged_prefill_workspace_bytes(int num_seqs, int max_q_len, 
     const size_t split = fq_attention_workspace_bytes(num_seqs, max_q_len, max_kv_len, H_Q, H_KV, D, 0);
     if (num_seqs <= 0 || max_q_len <= 0 || max_kv_len <= 0 || H_KV <= 0 || H_Q <= 0 || H_Q % H_KV != 0) return 0;
     if (!fq_host::supported_dim(D) || fq_host::force_any_dim_attention()) return split;
-    const size_t expanded = plan_expanded_paged(num_seqs, total_q, max_kv_len, H_KV, H_Q / H_KV, D).bytes;
+    const size_t expanded = plan_expanded_paged(num_seqs, total_q, max_q_len, max_kv_len, H_KV, H_Q / H_KV, D).bytes;
     return expanded > split ? expanded : split;
 }
 
@@ -1547,7 +1547,7 @@ extern "C" int fq_paged_tq4_prefill_split(const void* q, const int32_t* cu_seqle
         return FQ_ERR_MISALIGNED;
     if (num_seqs > 65535 || H_KV > 65535 || (D == 256 && H_Q > 65535)) return FQ_ERR_BAD_SHAPE;
 
-    const ExpandedPlan ep = plan_expanded_paged(num_seqs, total_q, int64_t(max_blocks_per_seq) * block_size, H_KV, H_Q / H_KV, D);
+    const ExpandedPlan ep = plan_expanded_paged(num_seqs, total_q, max_q_len, int64_t(max_blocks_per_seq) * block_size, H_KV, H_Q / H_KV, D);
     if (ep.per_chunk > 0 && workspace != nullptr && workspace_bytes >= ep.bytes && !fq_host::force_any_dim_attention()) {
         if (!fq_host::aligned(workspace, 256)) return FQ_ERR_MISALIGNED;
         ExpandParams e{};

@@ -1,0 +1,44 @@
+"""Which attention calls run on keys and values expanded once (csrc/fq_attention_expanded.hpp), compiled for the host."""
+from __future__ import annotations
+
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "flashquant_amd", "csrc")
+
+SOURCE = r"""
+#include "fq_attention_expanded.hpp"
+namespace fq_host { int device_cu_count() { return 256; } }
+using namespace fq;
+extern "C" int paged(int64_t seqs, int64_t total_q, int64_t max_q, int64_t max_kv, int HQ, int HKV, int D) {
+    return plan_expanded_paged(seqs, total_q, max_q, max_kv, HKV, HQ / HKV, D).per_chunk > 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def plans(tmp_path_factory):
+    d = tmp_path_factory.mktemp("plans")
+    (d / "plans.cpp").write_text(SOURCE)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-shared", "-fPIC", f"-I{CSRC}", str(d / "plans.cpp"), "-o", str(d / "plans.so")], check=True)
+    return ctypes.CDLL(str(d / "plans.so"))
+
+
+# (sequences, tokens, most of a sequence, columns of the block table in tokens, query heads, KV heads, dimension), and whether expanding
+# is the faster way (measured): few rows of 128 coordinates on the keys of many pairs, several rounds of workgroups of the other kernel,
+# rows that fill its workgroups, the other dimensions
+PAGED = [((12, 12 * 214, 214, 224, 16, 16, 128), False), ((13, 13 * 83, 83, 96, 16, 16, 128), False), ((24, 24 * 150, 150, 160, 8, 8, 128), False), ((4, 4 * 300, 300, 304, 32, 32, 128), False),
+         ((16, 16 * 16, 16, 16, 32, 8, 128), False), ((57, 57 * 17, 17, 32, 32, 4, 128), False),
+         ((13, 980, 168, 288, 32, 16, 128), False),
+         ((8, 8, 1, 16, 64, 8, 128), True), ((2, 426, 252, 256, 4, 4, 128), True), ((24, 24 * 150, 150, 160, 32, 32, 128), True),
+         ((36, 141, 6, 16, 32, 8, 128), True), ((2, 20, 10, 16, 8, 8, 128), True),
+         ((12, 10558, 2048, 4816, 32, 8, 128), True), ((12, 12 * 214, 214, 224, 16, 16, 256), True), ((1, 8192, 8192, 8192, 32, 8, 64), True)]
+
+
+@pytest.mark.parametrize("sizes,expanded", PAGED)
+def test_paged_batches_run_where_they_are_faster(plans, sizes, expanded):
+    i64 = ctypes.c_int64
+    assert bool(plans.paged(*(i64(n) for n in sizes[:4]), *sizes[4:])) == expanded
