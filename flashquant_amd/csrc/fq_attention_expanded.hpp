@@ -84,7 +84,8 @@ struct AttendParams {
 // over 8 x 4000 1138 / 1489, 256 coordinates 1 x 16 over 4 x 65 18 / 49, 64 coordinates 4 x 16 over 4 x 1500 43 / 66.  It stays there
 //   * with 64 coordinates and few tokens, where the two launches cost what the one does (4 x 32 over 8 x 65 11.7 / 10.5, x 130 12.7
 //     / 12.1);
-//   * with few workgroups on the keys of very many pairs (4 x 32 heads of their own x 300 34 / 28, x 700 60 / 70);
+//   * with few workgroups on the keys of very many pairs (4 x 32 heads of their own x 300 34 / 28, x 700 60 / 70), at 128 coordinates and
+//     one workgroup a pair of as few as 56 (7 x 16 heads of their own x 20 15.6 / 14.3, 3 x 16 x 20 14.0 / 14.0);
 //   * with many keys for few queries, which it cuts into pieces (33 queries over 8000 keys, 32 heads over 8, 154 / 37).
 struct ExpandedPlan {
     int keys = 0, tiles = 0;        // of a pair; paged: tiles of all sequences at most
@@ -143,7 +144,7 @@ inline ExpandedPlan plan_expanded(int64_t B, int H_KV, int64_t n_q, int64_t n_kv
     const int64_t W = ((n_q + 31) / 32 * G + 3) / 4, most = int64_t(1) << 23;      // workgroups of a pair, of a launch
     const int64_t blocks = (keys + 63) / 64;
     if (W > most) return e;
-    if (W < 5 && pairs * blocks >= 128) return e;
+    if (W < 5 && pairs * blocks >= (D == 128 && (n_q + 31) / 32 * G <= 4 ? 56 : 128)) return e;
     if (blocks > 4 * W + 4 || (!causal && blocks > 12 && pairs * W < 128)) return e;
     e.keys = int(keys);
     e.tiles = int(tiles);

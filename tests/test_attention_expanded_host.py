@@ -16,6 +16,9 @@ using namespace fq;
 extern "C" int paged(int64_t seqs, int64_t total_q, int64_t max_q, int64_t max_kv, int HQ, int HKV, int D) {
     return plan_expanded_paged(seqs, total_q, max_q, max_kv, HKV, HQ / HKV, D).per_chunk > 0;
 }
+extern "C" int contiguous(int64_t batch, int HQ, int HKV, int64_t n_q, int64_t n_kv, int D, int causal) {
+    return plan_expanded(batch, HKV, n_q, n_kv, HQ / HKV, D, causal != 0).per_chunk > 0;
+}
 """
 
 
@@ -42,3 +45,16 @@ PAGED = [((12, 12 * 214, 214, 224, 16, 16, 128), False), ((13, 13 * 83, 83, 96, 
 def test_paged_batches_run_where_they_are_faster(plans, sizes, expanded):
     i64 = ctypes.c_int64
     assert bool(plans.paged(*(i64(n) for n in sizes[:4]), *sizes[4:])) == expanded
+
+
+# (batch, query heads, KV heads, queries, keys, dimension, causal)
+CONTIGUOUS = [((7, 16, 16, 20, 20, 128, 1), False), ((3, 32, 32, 28, 28, 128, 1), False), ((31, 4, 4, 17, 30, 128, 0), False), ((4, 32, 32, 300, 300, 128, 1), False),
+              ((4, 32, 8, 65, 65, 64, 1), False), ((1, 32, 8, 33, 8000, 128, 0), False),
+              ((3, 16, 16, 20, 20, 128, 1), True), ((4, 32, 32, 700, 700, 128, 1), True), ((1, 32, 8, 40, 40, 128, 1), True), ((7, 16, 16, 20, 20, 256, 1), True)]
+
+
+@pytest.mark.parametrize("sizes,expanded", CONTIGUOUS)
+def test_contiguous_calls_run_where_they_are_faster(plans, sizes, expanded):
+    b, hq, hkv, nq, nkv, d, causal = sizes
+    i64 = ctypes.c_int64
+    assert bool(plans.contiguous(i64(b), hq, hkv, i64(nq), i64(nkv), d, causal)) == expanded
