@@ -165,7 +165,7 @@ __device__ void make_plan(const ExpandParams& p, int* lds) {
         block_scan(n, all);
         block_scan(n_split, all_split);
         if (i > 0 && (all > p.plan.max_items || all_split > p.plan.max_slots)) break;
-        const int64_t ns = batch_ns(choice, share, int64_t(all) * p.H_KV, int64_t(all_split) * p.H_KV, p.plan.cus, D);
+        const int64_t ns = batch_ns(choice, share, int64_t(all) * p.H_KV, int64_t(all_split) * p.H_KV, p.plan.cus, D, !PAGED && !p.causal);
         if (i == 0 || 20 * ns < 19 * best) {
             best = ns;
             piece = choice;

@@ -19,6 +19,21 @@ extern "C" int paged(int64_t seqs, int64_t total_q, int64_t max_q, int64_t max_k
 extern "C" int contiguous(int64_t batch, int HQ, int HKV, int64_t n_q, int64_t n_kv, int D, int causal) {
     return plan_expanded(batch, HKV, n_q, n_kv, HQ / HKV, D, causal != 0).per_chunk > 0;
 }
+// pieces of a workgroup over keys without a mask at 256 coordinates, by the rule of the launch
+extern "C" int pieces(int workgroups, int tiles) {
+    const int64_t share = (int64_t(workgroups) * tiles + 255) / 256;
+    int best_k = 1;
+    int64_t best = 0;
+    for (int i = 0; i < kPieceChoices; ++i) {
+        const int64_t piece = piece_choice(i, tiles, 2 * kPieceTiles), k = (tiles + piece - 1) / piece;
+        const int64_t ns = batch_ns(piece, share, workgroups * k, k > 1 ? workgroups * k : 0, 256, 256, true);
+        if (i == 0 || 20 * ns < 19 * best) {
+            best = ns;
+            best_k = int(k);
+        }
+    }
+    return best_k;
+}
 """
 
 
@@ -58,3 +73,9 @@ def test_contiguous_calls_run_where_they_are_faster(plans, sizes, expanded):
     b, hq, hkv, nq, nkv, d, causal = sizes
     i64 = ctypes.c_int64
     assert bool(plans.contiguous(i64(b), hq, hkv, i64(nq), i64(nkv), d, causal)) == expanded
+
+
+# (workgroups, tiles of 32 keys, pieces): 166 workgroups in two pieces are two rounds of 256 CUs, as long as one whole, in three still two
+@pytest.mark.parametrize("workgroups,tiles,pieces", [(166, 383, 3), (150, 227, 3), (128, 200, 2), (250, 125, 1), (256, 300, 1), (20, 300, 12)])
+def test_pieces_of_one_length_fill_their_rounds(plans, workgroups, tiles, pieces):
+    assert plans.pieces(workgroups, tiles) == pieces
