@@ -1391,7 +1391,7 @@ extern "C" size_t fq_attention_workspace_bytes(int num_seqs, int max_q_len, int6
     using namespace fq;
     if (num_seqs <= 0 || max_q_len <= 0 || max_kv_len <= 0 || H_KV <= 0 || H_Q <= 0 || H_Q % H_KV != 0) return 0;
     const size_t split = part_bytes(plan_of(num_seqs, max_q_len, max_kv_len, H_Q, H_KV, D, prompts == 1 && max_q_len > 1), num_seqs, H_KV, D);
-    if (prompts == 0 || fq_host::force_any_dim_attention()) return split;
+    if (prompts == 0 || !fq_host::supported_dim(D) || fq_host::force_any_dim_attention()) return split;
     const size_t expanded = plan_expanded(num_seqs, H_KV, max_q_len, max_kv_len, H_Q / H_KV, D, prompts == 1).bytes;
     return expanded > split ? expanded : split;
 }

@@ -319,3 +319,7 @@ def test_attention_workspace_errors(lib):
         assert call_paged(8192 + 128, need) == FQ_ALIGN
     # sizes that are never split, or that no call can have
     assert size(1, 1, 300, 32, 8, 128, 0) == 0 and size(0, 1, 9000, 32, 8, 128, 0) == 0 and size(1, 1, 9000, 30, 8, 128, 0) == 0
+    # a dimension that no kernel has: no room for expanded keys, which the operator would allocate before the call raises
+    for d in (32, 96, 512):
+        for prompts in (1, 2):
+            assert size(4, 8192, 8192, 32, 8, d, prompts) == size(4, 8192, 8192, 32, 8, d, 0) < size(4, 8192, 8192, 32, 8, 128, prompts)
