@@ -475,11 +475,17 @@ void tq4_compress_append(const at::Tensor& x, const at::Tensor& rot_T_even, cons
     fqbind::raise_on_error(st, "tq4_compress_append");
 }
 
-// Room for the partial results of attention over split contexts; undefined where these sizes are never split.
-at::Tensor attention_workspace(const at::Tensor& q, int64_t seqs, int64_t max_q, int64_t max_kv, int64_t HQ, int64_t HKV, int64_t D,
-                               int prompts) {
-    const size_t bytes = fq_attention_workspace_bytes(int(seqs), int(max_q), max_kv, int(HQ), int(HKV), int(D), prompts);
-    return bytes == 0 ? at::Tensor() : at::empty({int64_t(bytes)}, q.options().dtype(at::kByte));
+// Scratch of an attention call: `bytes`, or where the device has no such room what the kernel that expands nothing takes
+// (`pieces`); undefined where it needs none.
+at::Tensor attention_workspace(const at::Tensor& q, size_t bytes, size_t pieces) {
+    const auto options = q.options().dtype(at::kByte);
+    if (bytes > pieces) {
+        try {
+            return at::empty({int64_t(bytes)}, options);
+        } catch (const c10::OutOfMemoryError&) {
+        }
+    }
+    return pieces == 0 ? at::Tensor() : at::empty({int64_t(pieces)}, options);
 }
 
 at::Tensor fused_tq_attention(const at::Tensor& q, const at::Tensor& k_packed, const at::Tensor& k_norms,
@@ -527,7 +533,10 @@ at::Tensor fused_tq_attention(const at::Tensor& q, const at::Tensor& k_packed, c
     const at::Tensor ck = centroids_k.to(q.device()).contiguous(), cv = centroids_v.to(q.device()).contiguous();
     const RotationArg rot = rotation_arg(rotation, q.device(), D);
     at::Tensor result = at::empty_like(qc);
-    const at::Tensor ws = attention_workspace(q, B, NQ, NKV, HQ, HKV, D, is_causal ? 1 : 2);
+    const int prompts = is_causal ? 1 : 2;
+    const at::Tensor ws = attention_workspace(
+        q, fq_attention_workspace_bytes(int(B), int(NQ), NKV, int(HQ), int(HKV), int(D), prompts),
+        fq_attention_pieces_workspace_bytes(int(B), int(NQ), NKV, int(HQ), int(HKV), int(D), prompts));
     const int st = fq_fused_tq_attention_split(
         qc.data_ptr(), kp.data_ptr<uint8_t>(), kn.data_ptr<float>(), vp.data_ptr<uint8_t>(), vn.data_ptr<float>(),
         ck.data_ptr<float>(), cv.data_ptr<float>(), rot.ptr, rot.col_major, result.data_ptr(),
@@ -579,8 +588,10 @@ at::Tensor paged_tq4_prefill(const at::Tensor& q, const at::Tensor& cu_seqlens_q
     } else {
         result = at::zeros_like(qc);
     }
-    const size_t need = fq_paged_prefill_workspace_bytes(int(S), int(max_seqlen_q), bt.size(1) * block_size, T, int(HQ), int(num_kv_heads), int(head_dim));
-    const at::Tensor ws = need == 0 ? at::Tensor() : at::empty({int64_t(need)}, q.options().dtype(at::kByte));
+    const int64_t room = bt.size(1) * block_size;
+    const at::Tensor ws = attention_workspace(
+        q, fq_paged_prefill_workspace_bytes(int(S), int(max_seqlen_q), room, T, int(HQ), int(num_kv_heads), int(head_dim)),
+        fq_attention_pieces_workspace_bytes(int(S), int(max_seqlen_q), room, int(HQ), int(num_kv_heads), int(head_dim), 0));
     const int st = fq_paged_tq4_prefill_split(
         qc.data_ptr(), cu.data_ptr<int32_t>(), kv_cache.data_ptr<uint8_t>(), bt.data_ptr<int32_t>(),
         sl.data_ptr<int32_t>(), ck.data_ptr<float>(), cv.data_ptr<float>(), rot.ptr, rot.col_major, result.data_ptr(),

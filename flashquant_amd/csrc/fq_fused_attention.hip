@@ -1386,11 +1386,18 @@ extern "C" int fq_fused_tq_attention(const void* q, const uint8_t* k_packed, con
                                          is_causal, dtype, stream);
 }
 
+extern "C" size_t fq_attention_pieces_workspace_bytes(int num_seqs, int max_q_len, int64_t max_kv_len, int H_Q, int H_KV, int D,
+                                                      int prompts) {
+    using namespace fq;
+    if (num_seqs <= 0 || max_q_len <= 0 || max_kv_len <= 0 || H_KV <= 0 || H_Q <= 0 || H_Q % H_KV != 0) return 0;
+    return part_bytes(plan_of(num_seqs, max_q_len, max_kv_len, H_Q, H_KV, D, prompts == 1 && max_q_len > 1), num_seqs, H_KV, D);
+}
+
 extern "C" size_t fq_attention_workspace_bytes(int num_seqs, int max_q_len, int64_t max_kv_len, int H_Q, int H_KV, int D,
                                                int prompts) {
     using namespace fq;
+    const size_t split = fq_attention_pieces_workspace_bytes(num_seqs, max_q_len, max_kv_len, H_Q, H_KV, D, prompts);
     if (num_seqs <= 0 || max_q_len <= 0 || max_kv_len <= 0 || H_KV <= 0 || H_Q <= 0 || H_Q % H_KV != 0) return 0;
-    const size_t split = part_bytes(plan_of(num_seqs, max_q_len, max_kv_len, H_Q, H_KV, D, prompts == 1 && max_q_len > 1), num_seqs, H_KV, D);
     if (prompts == 0 || !fq_host::supported_dim(D) || fq_host::force_any_dim_attention()) return split;
     const size_t expanded = plan_expanded(num_seqs, H_KV, max_q_len, max_kv_len, H_Q / H_KV, D, prompts == 1).bytes;
     return expanded > split ? expanded : split;
@@ -1399,7 +1406,7 @@ extern "C" size_t fq_attention_workspace_bytes(int num_seqs, int max_q_len, int6
 extern "C" size_t fq_paged_prefill_workspace_bytes(int num_seqs, int max_q_len, int64_t max_kv_len, int64_t total_q, int H_Q, int H_KV,
                                                    int D) {
     using namespace fq;
-    const size_t split = fq_attention_workspace_bytes(num_seqs, max_q_len, max_kv_len, H_Q, H_KV, D, 0);
+    const size_t split = fq_attention_pieces_workspace_bytes(num_seqs, max_q_len, max_kv_len, H_Q, H_KV, D, 0);
     if (num_seqs <= 0 || max_q_len <= 0 || max_kv_len <= 0 || H_KV <= 0 || H_Q <= 0 || H_Q % H_KV != 0) return 0;
     if (!fq_host::supported_dim(D) || fq_host::force_any_dim_attention()) return split;
     const size_t expanded = plan_expanded_paged(num_seqs, total_q, max_q_len, max_kv_len, H_KV, H_Q / H_KV, D).bytes;

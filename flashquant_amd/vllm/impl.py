@@ -106,8 +106,11 @@ def _make_impl_class() -> type:
         Where the reference decompresses the whole cache and hands it to a FlashAttention library
         (src/flashquant/vllm/impl.py:395-512), a batch of single-token queries runs the split-K paged
         decode and everything else the paged prefill, both reading the packed pages.  Their scratch
-        memory (split partials; of the prefill at most 65 MiB) comes from torch's caching
-        allocator, so either can be captured in a graph."""
+        memory comes from torch's caching allocator, so either can be captured in a graph: split
+        partials (of the prefill at most 65 MiB) and, where many queries share their keys, these as
+        fp16, which the prefill sizes from the columns of the block table (about 7 times the bytes of
+        the queries and 0.2 GiB, at most 2.2 GiB).  The profiling run launches nothing and does not
+        see it.  Where it cannot be had, the prefill reads the packed pages instead."""
 
         def __init__(self, *args, **kwargs) -> None:
             super().__init__(*args, **kwargs)

@@ -331,8 +331,9 @@ int fq_paged_tq4_prefill(const void* q, const int32_t* cu_seqlens_q, const uint8
  * Where many queries share their keys, fq_fused_tq_attention_split first writes keys and values, rotated back, as fp16
  * matrix operands into the workspace and attends to these (no rounding of the rotated query, fewer of the keys and values).
  *   workspace        256-byte aligned, at least fq_attention_workspace_bytes bytes (0: these sizes need none; at
- *                    most 65 MiB paged, 172 MiB for prompts in pieces, for expanded keys and values 1.1 GiB, 2.2 GiB paged); NULL:
- *                    nothing is split or expanded.  With what suffices for pieces alone nothing is expanded.
+ *                    most 65 MiB paged, 172 MiB for prompts in pieces, for expanded keys and values 1.1 GiB, 2.2 GiB paged);
+ *                    NULL: nothing is split or expanded.  With what suffices for pieces alone
+ *                    (fq_attention_pieces_workspace_bytes) nothing is expanded.
  *   max_kv_len       the longest context possible: N_KV, or max_blocks_per_seq * block_size
  *   prompts          for fq_fused_tq_attention_split 1 with is_causal, 2 without (all sequences have these very lengths);
  *                    else 0
@@ -340,7 +341,10 @@ int fq_paged_tq4_prefill(const void* q, const int32_t* cu_seqlens_q, const uint8
  */
 size_t fq_attention_workspace_bytes(int num_seqs, int max_q_len, int64_t max_kv_len, int H_Q, int H_KV, int D,
                                     int prompts);
-/* The same for fq_paged_tq4_prefill_split, which may expand keys and values where it knows the number of tokens. */
+/* What suffices for pieces alone, for a caller who has no more (prompts 0 for fq_paged_tq4_prefill_split): at most 172 MiB. */
+size_t fq_attention_pieces_workspace_bytes(int num_seqs, int max_q_len, int64_t max_kv_len, int H_Q, int H_KV, int D,
+                                           int prompts);
+/* fq_attention_workspace_bytes for fq_paged_tq4_prefill_split, which may expand keys and values where it knows the number of tokens. */
 size_t fq_paged_prefill_workspace_bytes(int num_seqs, int max_q_len, int64_t max_kv_len, int64_t total_q, int H_Q, int H_KV, int D);
 
 int fq_fused_tq_attention_split(const void* q, const uint8_t* k_packed, const float* k_norms,

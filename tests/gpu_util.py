@@ -98,6 +98,35 @@ def attention_in_one_piece(q, kp, kn, vp, vn, c, r, is_causal=False):
     return out
 
 
+def _pieces_room(seqs, max_q, max_kv, hq, hkv, d, prompts, dev):
+    """A workspace that suffices for contexts in pieces and for nothing else, and its bytes."""
+    n = int(_entry("fq_attention_pieces_workspace_bytes", ctypes.c_size_t)(*_args(seqs, max_q, (max_kv,), hq, hkv, d, prompts)))
+    return torch.empty(n, dtype=torch.uint8, device=dev) if n else None, ctypes.c_size_t(n)
+
+
+def attention_on_packed_rows(q, kp, kn, vp, vn, c, r, is_causal=False):
+    """fq_fused_tq_attention_split with room for contexts in pieces alone: keys and values are not expanded first."""
+    b, hq, nq, d = q.shape
+    hkv, nkv = kp.shape[1:3]
+    out, r = torch.empty_like(q), r.contiguous()
+    ws, n = _pieces_room(b, nq, nkv, hq, hkv, d, 1 if is_causal else 2, q.device)
+    st = _entry("fq_fused_tq_attention_split")(*_args(q, kp, kn, vp, vn, c, c, r, 0, out, b, hq, hkv, nq, nkv, (nkv,), (nkv,), d, d ** -0.5,
+                                                      int(is_causal), _dtype(q), ws), n, _stream())
+    assert st == 0, st
+    return out
+
+
+def prefill_on_packed_rows(q, cu, max_q, cache, table, sl, c, r, hkv, d, bs, causal=True):
+    """fq_paged_tq4_prefill_split with room for contexts in pieces alone."""
+    out, r = torch.zeros_like(q), r.contiguous()
+    ws, n = _pieces_room(table.shape[0], max_q, table.shape[1] * bs, q.shape[1], hkv, d, 0, q.device)
+    st = _entry("fq_paged_tq4_prefill_split")(*_args(q, cu, cache, table, sl, c, c, r, 0, out, table.shape[0], max_q, q.shape[1], hkv, d, bs,
+                                                     table.shape[1], (cache.shape[0],), d ** -0.5, int(causal), _dtype(q), (q.shape[0],), ws), n,
+                                              _stream())
+    assert st == 0, st
+    return out
+
+
 def prefill_in_one_piece(q, cu, max_q, cache, table, sl, c, r, hkv, d, bs, causal=True):
     """fq_paged_tq4_prefill: the paged entry without a workspace."""
     out, r = torch.zeros_like(q), r.contiguous()

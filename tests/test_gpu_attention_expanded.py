@@ -10,7 +10,8 @@ import torch
 
 from flashquant_amd import kernels as K
 from oracle import tq_oracle as O
-from tests.gpu_util import _entry, attention_in_one_piece, attention_workspace_bytes, book, build_paged_case
+from tests.gpu_util import (_entry, attention_in_one_piece, attention_on_packed_rows, attention_workspace_bytes, book, build_paged_case,
+                            prefill_on_packed_rows)
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -249,3 +250,66 @@ def test_paged_under_capture_with_other_lengths():
         want = O.paged_prefill(q.cpu(), cu.cpu(), cache, table, sl.cpu(), c, c, r, hkv, d, bs)
         rel = (out.cpu().float() - want.float()).norm(dim=-1) / want.float().norm(dim=-1)
         assert rel.max() <= 4 * 2 ** -8
+
+
+class _LittleMemory:
+    """At most `spare` bytes more than what torch's allocator holds now (and nothing larger in what it holds)."""
+
+    def __init__(self, spare):
+        self.spare = spare
+
+    def __enter__(self):
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        total = torch.cuda.get_device_properties(0).total_memory
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + self.spare) / total)
+
+    def __exit__(self, *exc):
+        torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+def _random_rows(b, h, n, d, g):
+    return [t for _ in range(2) for t in (torch.randint(0, 256, (b, h, n, d // 2), dtype=torch.uint8, device=DEV, generator=g),
+                                          d ** 0.5 * (0.5 + torch.rand(b, h, n, 1, device=DEV, generator=g)))]
+
+
+@pytest.mark.parametrize("causal", [True, False])
+def test_without_room_for_expanded_keys(causal):
+    """A call whose expanded keys (96 MiB) do not fit the memory that is left runs on the packed ones."""
+    b, h, n, d = 1, 32, 6144, 128
+    assert _expanded(b, h, h, n, n, d, causal)
+    c, _, r = (t.to(DEV) for t in book(d))
+    g = torch.Generator(device=DEV).manual_seed(7)
+    kv = _random_rows(b, h, n, d, g)
+    q = torch.randn(b, h, n, d, device=DEV, generator=g, dtype=torch.bfloat16)
+    want = attention_on_packed_rows(q, *kv, c, r, is_causal=causal).cpu()
+    with _LittleMemory(90 << 20):                              # (the result takes 48 MiB, rows of pieces 33)
+        got = K.fused_tq_attention(q, *kv, c, c, r, is_causal=causal)
+    assert torch.equal(got.cpu(), want)
+    roomy = K.fused_tq_attention(q, *kv, c, c, r, is_causal=causal).cpu()
+    assert not torch.equal(roomy, want)
+    rel = (roomy.float() - want.float()).norm() / want.float().norm()
+    assert rel <= 2 * 3 ** 0.5 * 2 ** -9                       # bf16: query and output rounded there, the output here
+
+
+def test_paged_without_room_for_expanded_keys():
+    ql, kv, hq, hkv, d, bs = [2000, 1500, 1], [2000, 1900, 700], 16, 16, 128, 16
+    c, _, r = (t.to(DEV) for t in book(d))
+    g = torch.Generator(device=DEV).manual_seed(8)
+    pages = 3 * 125
+    assert _paged_expanded(ql, 125 * bs, hq, hkv, d)
+    cache = torch.randint(0, 256, (pages, bs, hkv * (d + 8)), dtype=torch.uint8, device=DEV, generator=g)
+    norms = cache.view(-1, hkv * (d + 8)).view(torch.float32)
+    norms[:, hkv * 16:hkv * 17] = d ** 0.5 * (0.5 + torch.rand(pages * bs, hkv, device=DEV, generator=g))
+    norms[:, hkv * 33:] = d ** 0.5 * (0.5 + torch.rand(pages * bs, hkv, device=DEV, generator=g))
+    table = torch.randperm(pages, device=DEV, generator=g).to(torch.int32).view(3, 125)
+    q = torch.randn(sum(ql), hq, d, device=DEV, generator=g, dtype=torch.bfloat16)
+    cu = torch.tensor([0] + list(torch.tensor(ql).cumsum(0)), dtype=torch.int32, device=DEV)
+    args = (cu, max(ql), cache, table, torch.tensor(kv, dtype=torch.int32, device=DEV), c)
+    want = prefill_on_packed_rows(q, *args, r, hkv, d, bs).cpu()
+    torch.cuda.empty_cache()
+    out = torch.empty_like(q)
+    with _LittleMemory(40 << 20):
+        K.paged_tq4_prefill(q, *args, c, r, hkv, d, bs, out=out)
+    assert torch.equal(out.cpu(), want)
+    assert not torch.equal(K.paged_tq4_prefill(q, *args, c, r, hkv, d, bs).cpu(), want)
