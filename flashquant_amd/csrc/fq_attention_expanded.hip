@@ -88,6 +88,7 @@ __device__ void make_plan(const ExpandParams& p, int* lds) {
     int* wfirst = lds;                          // first workgroup of a sequence, [num_seqs]: all
     int* tfirst = lds + 260;                    // first tile
     int* sums = lds + 520;                      // of the wavefronts
+    int64_t* parts = reinterpret_cast<int64_t*>(lds + 560);
     int* hist = lds + 640;                      // pieces by (class, thread)
     auto block_scan = [&](int v, int& total) {  // sum over the threads up to this one, and over all
         const int incl = wave_scan(v, lane);
@@ -102,6 +103,16 @@ __device__ void make_plan(const ExpandParams& p, int* lds) {
         }
         return before + incl;
     };
+    auto block_sum = [&](int64_t v) {
+#pragma unroll
+        for (int d = 1; d < kWave; d <<= 1) v += __shfl_xor(v, d, kWave);
+        __syncthreads();
+        if (lane == 0) parts[wave] = v;
+        __syncthreads();
+        int64_t total = 0;
+        for (int i = 0; i < 8; ++i) total += parts[i];
+        return total;
+    };
     auto tiles_of = [&](const Seq& q, int x) {  // that the workgroup's last row sees
         const int all = (q.NKV + (1 << TS) - 1) >> TS, units = ((q.NQ + 31) >> 5) * p.G;
         if (!p.causal) return all;
@@ -111,17 +122,18 @@ __device__ void make_plan(const ExpandParams& p, int* lds) {
         const int t = ((q.qoff + pos) >> TS) + 1;
         return t < all ? t : all;
     };
-    int W = 0, tiles = 0, work = 0, most = 0;
+    int W = 0, tiles = 0, most = 0;
+    int64_t work = 0;
     if (tid < p.num_seqs) {
         const Seq q = seq_of<PAGED>(p, tid);
         W = (((q.NQ + 31) >> 5) * p.G + 3) >> 2;
         tiles = q.tiles(TS);
         most = W > 0 ? tiles_of(q, W - 1) : 0;
-        work = W > 0 ? int((int64_t(W) * (tiles_of(q, 0) + most) + 1) / 2) : 0;
+        work = W > 0 ? work_of(W, tiles_of(q, 0), most) : 0;
     }
-    int groups, all_tiles, all_work;
+    int groups, all_tiles;
     const int wincl = block_scan(W, groups), tincl = block_scan(tiles, all_tiles);
-    block_scan(work, all_work);
+    const int64_t all_work = block_sum(work);
     if (tid < p.num_seqs) {
         wfirst[tid] = wincl - W;
         tfirst[tid] = tincl - tiles;
@@ -150,7 +162,7 @@ __device__ void make_plan(const ExpandParams& p, int* lds) {
             f(s, q, end - 1 - i, tiles_of(q, end - 1 - i));
         }
     };
-    const int64_t share = (int64_t(all_work) * p.H_KV + p.plan.cu_slots - 1) / p.plan.cu_slots;
+    const int64_t share = share_of_work(all_work, p.H_KV, p.plan.cu_slots);
     auto pieces_of = [&](int t, int piece) { return t <= piece ? 1 : (t + piece - 1) / piece; };
     int piece = longest;
     int64_t best = 0;

@@ -124,6 +124,10 @@ FQ_HD int64_t batch_ns(int64_t piece, int64_t share, int64_t items, int64_t spli
     if (alike && D == 256) all = c.tile * piece * ((items + cus - 1) / cus);
     return (ns > all ? ns : all) + (split > 0 ? 7000 + split * c.rows : 0);
 }
+// Tiles of `workgroups` workgroups, the first of which has `first` and the last `last` (2^38 where a batch is as large as it may be).
+FQ_HD int64_t work_of(int64_t workgroups, int first, int last) { return (workgroups * (int64_t(first) + last) + 1) / 2; }
+// The share of one of `places` of all KV heads' tiles.
+FQ_HD int64_t share_of_work(int64_t work, int H_KV, int places) { return (work * H_KV + places - 1) / places; }
 // The candidates: the longest workgroup's tiles in 1, 2, 3, 4, 6, 8, 12 and 16.
 constexpr int kPieceChoices = 8;
 FQ_HD int piece_choice(int i, int longest, int least) {

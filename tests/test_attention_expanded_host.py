@@ -34,6 +34,9 @@ extern "C" int pieces(int workgroups, int tiles) {
     }
     return best_k;
 }
+extern "C" int64_t share(int64_t workgroups, int first, int last, int H_KV, int places) {
+    return share_of_work(work_of(workgroups, first, last), H_KV, places);
+}
 """
 
 
@@ -79,3 +82,11 @@ def test_contiguous_calls_run_where_they_are_faster(plans, sizes, expanded):
 @pytest.mark.parametrize("workgroups,tiles,pieces", [(166, 383, 3), (150, 227, 3), (128, 200, 2), (250, 125, 1), (256, 300, 1), (20, 300, 12)])
 def test_pieces_of_one_length_fill_their_rounds(plans, workgroups, tiles, pieces):
     assert plans.pieces(workgroups, tiles) == pieces
+
+
+def test_the_share_of_large_batches(plans):
+    """Workgroups times tiles go beyond 32 bits: 3 * 10^5 queries over 8 * 10^6 keys on one KV head, 16 query heads."""
+    f = plans.share
+    f.restype, f.argtypes = ctypes.c_int64, [ctypes.c_int64] + [ctypes.c_int] * 4
+    for w, first, last, hkv in ((37500, 120000, 125000, 1), (1 << 20, 1, 1 << 18, 1), (1 << 20, 1 << 18, 1 << 18, 8), (3, 1, 4, 5)):
+        assert f(w, first, last, hkv, 512) == (((w * (first + last) + 1) // 2) * hkv + 511) // 512
