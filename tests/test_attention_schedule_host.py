@@ -153,8 +153,14 @@ def test_every_piece_is_handed_out_once(program):
 
 
 CONTIGUOUS = r"""
+#include "fq_attention_expanded.hpp"
 #include "fq_attention_schedule.hpp"
+namespace fq_host { int device_cu_count() { return 256; } }
 using namespace fq;
+// whether the operator, with room for all that it asks for, runs such a call on expanded keys instead
+extern "C" int expanded(int B, int HQ, int HKV, int NQ, int NKV, int D, int is_causal) {
+    return plan_expanded(B, HKV, NQ, NKV, HQ / HKV, D, is_causal && NQ > 1).per_chunk > 0;
+}
 // pieces of a call over contiguous keys on 256 CUs, as its entry works them out; + 100: whole prompts' combine launch
 extern "C" int pieces(int B, int HQ, int HKV, int NQ, int NKV, int D, int is_causal) {
     const int G = HQ / HKV, max_w = ((NQ + 31) / 32 * G + 7) / 8;
@@ -172,22 +178,25 @@ extern "C" int pieces(int B, int HQ, int HKV, int NQ, int NKV, int D, int is_cau
 
 
 @pytest.fixture(scope="module")
-def pieces(tmp_path_factory):
+def library(tmp_path_factory):
     d = tmp_path_factory.mktemp("pieces")
     (d / "pieces.cpp").write_text(CONTIGUOUS)
     subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", f"-I{CSRC}", str(d / "pieces.cpp"), "-o", str(d / "pieces.so")], check=True)
-    return ctypes.CDLL(str(d / "pieces.so")).pieces
+    return ctypes.CDLL(str(d / "pieces.so"))
 
 
-def test_the_gpu_tests_reach_what_they_name(pieces):
-    """The cases of the tests on contexts in pieces run in pieces, and through the combine launch that they are there for."""
+def test_the_gpu_tests_reach_what_they_name(library):
+    """The cases of the tests on contexts in pieces run in pieces, and through the combine launch that they are there for: as the
+    operator runs them, or (causal prompts, which have room for expanded keys there) with room for pieces alone."""
+    pieces, expanded = library.pieces, library.expanded
     assert all(pieces(*c, 0) > 1 for c in rows.SPLIT) and all(pieces(*c, 0) == 1 for c in rows.NOT_SPLIT)
+    assert not any(expanded(*c, 0) for c in rows.SPLIT + rows.NOT_SPLIT)
     for shortest in ((1, 8, 2, 1, 449, 128), (1, 4, 1, 3, 705, 64), (1, 8, 1, 2, 449, 256)):
         assert shortest in rows.SPLIT and pieces(*shortest[:4], shortest[4] - 1, shortest[5], 0) == 1
     for d in (64, 128, 256):
         for c in rows.IN_PIECES:
-            assert (pieces(*c, d, 0) > 100) == (c[3] == 390) and pieces(*c, d, 0) > 1, (c, d)
+            assert (pieces(*c, d, 0) > 100) == (c[3] == 390) and pieces(*c, d, 0) > 1 and not expanded(*c, d, 0), (c, d)
         for c in rows.WHOLE_PROMPTS:
-            assert pieces(*c[:5], d, int(c[5])) > 100, (c, d)
-        assert pieces(1, 8, 1, 4201, 4201, d, 1) > 100
-    assert {pieces(*c[:5], 256, int(c[5])) > 1 for c in rows.WIDE} == {True, False}
+            assert pieces(*c[:5], d, int(c[5])) > 100 and bool(expanded(*c[:5], d, int(c[5]))) == c[5], (c, d)
+        assert pieces(1, 8, 1, 4201, 4201, d, 1) > 100 and expanded(1, 8, 1, 4201, 4201, d, 1)
+    assert {pieces(*c[:5], 256, int(c[5])) > 1 for c in rows.WIDE if not expanded(*c[:5], 256, int(c[5]))} == {True, False}

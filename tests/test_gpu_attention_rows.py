@@ -7,7 +7,8 @@ import torch
 
 from flashquant_amd import kernels as K
 from oracle import tq_oracle as O
-from tests.gpu_util import attention_in_one_piece, attention_workspace_bytes, book, build_paged_case, prefill_in_one_piece
+from tests.gpu_util import (attention_in_one_piece, attention_on_packed_rows, attention_workspace_bytes, book, build_paged_case,
+                            prefill_in_one_piece, prefill_on_packed_rows)
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -102,6 +103,9 @@ def test_attention_over_split_contexts_causal_and_huge_norms(d):
         want = O.fused_tq_attention(q[:, :, :n], *kv, c, c, r, is_causal=n > 40)
         got = K.fused_tq_attention(q[:, :, :n].contiguous().to(DEV), *[t.to(DEV) for t in kv], c.to(DEV), c.to(DEV), r.to(DEV), is_causal=n > 40)
         _close(got, want, torch.bfloat16)
+        # the prompt of 2400 runs on expanded keys: here in pieces on the packed ones
+        _close(attention_on_packed_rows(q[:, :, :n].contiguous().to(DEV), *[t.to(DEV) for t in kv], c.to(DEV), r.to(DEV), is_causal=n > 40), want,
+               torch.bfloat16)
 
 
 # (queries, keys) per sequence: a mixed batch with long single queries, chunks of one and of several workgroups on long
@@ -193,6 +197,8 @@ def test_prompts_in_pieces(b, hq, hkv, nq, nkv, causal, d):
     want = O.fused_tq_attention(q, *kv, c, c, r, is_causal=causal)
     got = K.fused_tq_attention(q.to(DEV), *[t.to(DEV) for t in kv], c.to(DEV), c.to(DEV), r.to(DEV), is_causal=causal)
     _close(got, want, torch.float16)
+    # (with room for its expanded keys the causal prompt takes no part of this kernel)
+    _close(attention_on_packed_rows(q.to(DEV), *[t.to(DEV) for t in kv], c.to(DEV), r.to(DEV), is_causal=causal), want, torch.float16)
 
 
 @pytest.mark.parametrize("d", [64, 128, 256])
@@ -203,9 +209,10 @@ def test_paged_prompts_in_pieces(d):
     q = torch.randn(sum(ql), hq, d, generator=torch.Generator().manual_seed(92)).to(torch.bfloat16)
     cu = torch.tensor([0] + list(torch.tensor(ql).cumsum(0)), dtype=torch.int32)
     want = O.paged_prefill(q, cu, cache, table, sl, c, c, r, hkv, d, bs, causal=True)
-    got = K.paged_tq4_prefill(q.to(DEV), cu.to(DEV), max(ql), cache.to(DEV), table.to(DEV), sl.to(DEV), c.to(DEV), c.to(DEV),
-                              r.to(DEV), hkv, d, bs)
+    args = (q.to(DEV), cu.to(DEV), max(ql), cache.to(DEV), table.to(DEV), sl.to(DEV), c.to(DEV))
+    got = K.paged_tq4_prefill(*args, c.to(DEV), r.to(DEV), hkv, d, bs)
     _close(got, want, torch.bfloat16)
+    _close(prefill_on_packed_rows(*args, r.to(DEV), hkv, d, bs), want, torch.bfloat16)
 
 
 # (batch, query heads, KV heads, queries, keys): rows for the combine launch by 4 and by 16 rows, and enough workgroups for
@@ -287,20 +294,23 @@ def test_nan_and_inf_stay_visible_in_pieces_paged(ql, kv, hq, hkv, kind, d):
     cu = torch.tensor([0] + list(torch.tensor(ql).cumsum(0)), dtype=torch.int32).to(DEV)
     cache, table, sl, c, r = (t.to(DEV) for t in (cache, table, sl, c, r))
     args = (cu, max(ql), cache, table, sl, c)
-    clean = K.paged_tq4_prefill(q, *args, c, r, hkv, d, bs, causal=False)
+    def prefill():                                                  # as the operator runs it, and in pieces on the packed rows
+        return (K.paged_tq4_prefill(q, *args, c, r, hkv, d, bs, causal=False), prefill_on_packed_rows(q, *args, r, hkv, d, bs, causal=False))
+
+    cleans = prefill()
     pos = torch.arange(kv[0])
     slots = table[0].long().cpu()[pos // bs] * bs + pos % bs
     norms = cache.view(-1, hkv * (d + 8)).view(torch.float32)
     kn, vn = norms[slots, hkv * d // 8], norms[slots, hkv * (d + 4) // 4]
     _poison(kind, kn, vn, q[1, 0])
     norms[slots, hkv * d // 8], norms[slots, hkv * (d + 4) // 4] = kn, vn
-    got = K.paged_tq4_prefill(q, *args, c, r, hkv, d, bs, causal=False)
     want = prefill_in_one_piece(q, *args, r, hkv, d, bs, causal=False)
     first = lambda t: t[:ql[0]].transpose(0, 1)                     # noqa: E731  (heads, rows of the first sequence, D)
-    if "far" in kind:
-        clean[:ql[0], :hq // hkv] = got[:ql[0], :hq // hkv]
-    _check_poisoned(first(got), first(want), first(clean), POISON[kind], 1, hq // hkv)
-    assert torch.equal(got[ql[0]:], clean[ql[0]:])
+    for got, clean in zip(prefill(), cleans):
+        if "far" in kind:
+            clean[:ql[0], :hq // hkv] = got[:ql[0], :hq // hkv]
+        _check_poisoned(first(got), first(want), first(clean), POISON[kind], 1, hq // hkv)
+        assert torch.equal(got[ql[0]:], clean[ql[0]:])
 
 
 @pytest.mark.parametrize("d", [64, 128, 256])
@@ -312,9 +322,9 @@ def test_nan_stays_where_it_is_seen_in_causal_prompts(d):
     kv[1][..., key, :] = float("nan")
     q = torch.randn(1, 8, n, d, generator=torch.Generator().manual_seed(100)).to(torch.bfloat16).to(DEV)
     kv, c, r = [t.to(DEV) for t in kv], c.to(DEV), r.to(DEV)
-    got = K.fused_tq_attention(q, *kv, c, c, r, is_causal=True)
-    assert got[:, :, :key].isfinite().all() and not got[:, :, key:].isfinite().any()
-    assert torch.equal(got.isfinite(), attention_in_one_piece(q, *kv, c, r, is_causal=True).isfinite())
+    for got in (K.fused_tq_attention(q, *kv, c, c, r, is_causal=True), attention_on_packed_rows(q, *kv, c, r, is_causal=True)):
+        assert got[:, :, :key].isfinite().all() and not got[:, :, key:].isfinite().any()
+        assert torch.equal(got.isfinite(), attention_in_one_piece(q, *kv, c, r, is_causal=True).isfinite())
 
 
 def _rows_close(got, want, limit, what=""):
@@ -383,15 +393,14 @@ def test_coordinates_of_very_different_size_in_one_row(nq, n, d, dtype):
     O.store_rows(cache, torch.arange(n), same, ones, same, ones)
     q = (torch.randn(nq, hq, d, generator=g) * 1e-3).to(dtype).to(DEV)
     eye = torch.eye(d, device=DEV)
-    got = K.paged_tq4_prefill(q, torch.tensor([0, nq], dtype=torch.int32, device=DEV), nq, cache.to(DEV),
-                              torch.arange(pages, dtype=torch.int32, device=DEV)[None],
-                              torch.tensor([n], dtype=torch.int32, device=DEV), c.to(DEV), c.to(DEV), eye, hkv, d, bs,
-                              causal=False).cpu().double()
+    args = (q, torch.tensor([0, nq], dtype=torch.int32, device=DEV), nq, cache.to(DEV), torch.arange(pages, dtype=torch.int32, device=DEV)[None],
+            torch.tensor([n], dtype=torch.int32, device=DEV), c.to(DEV))
     value = c[O.nibble_unpack(token).long()].double().repeat_interleave(hq // hkv, 0)      # (heads, D)
     # held as fp16 (2^-11), the weights' sum as theirs (2^-11), rounded to the query dtype once: nothing more for one key
     limit = 2 * 2 ** -11 + (2 ** -8 if dtype == torch.bfloat16 else 2 ** -11)
-    err = ((got - value) / value).abs().max()
-    assert err <= limit, f"{err:.2e}, limit {limit:.2e}"
+    for got in (K.paged_tq4_prefill(*args, c.to(DEV), eye, hkv, d, bs, causal=False), prefill_on_packed_rows(*args, eye, hkv, d, bs, causal=False)):
+        err = ((got.cpu().double() - value) / value).abs().max()
+        assert err <= limit, f"{err:.2e}, limit {limit:.2e}"
 
 
 # more sequences than are ordered: single queries (the grid has a place for every sequence), the same with one long prompt
@@ -437,12 +446,12 @@ def test_paged_prefill_under_a_wide_table(batch, hq, hkv, d):
     want = O.paged_prefill(q, cu, cache, table, sl, c, c, r, hkv, d, bs)
     wide = torch.randint(-3, 1 << 20, (len(ql), 256), dtype=torch.int32, generator=torch.Generator().manual_seed(123))
     wide[:, :table.shape[1]] = table
-    got = torch.full_like(q, 7.0).to(DEV)
-    K.paged_tq4_prefill(q.to(DEV), cu.to(DEV), max(ql), cache.to(DEV), wide.to(DEV), sl.to(DEV), c.to(DEV), c.to(DEV), r.to(DEV),
-                        hkv, d, bs, out=got)
+    args = (q.to(DEV), cu.to(DEV), max(ql), cache.to(DEV), wide.to(DEV), sl.to(DEV), c.to(DEV))
+    out = K.paged_tq4_prefill(*args, c.to(DEV), r.to(DEV), hkv, d, bs, out=torch.full_like(q, 7.0).to(DEV))
     keyless = torch.cat([torch.full((n,), m == 0) for n, m in zip(ql, kv)])
-    assert (got.cpu()[keyless] == 0).all()
-    _rows_close(got.cpu()[~keyless], want[~keyless], 4 * 2 ** -8)
+    for got in (out, prefill_on_packed_rows(*args, r.to(DEV), hkv, d, bs)):
+        assert (got.cpu()[keyless] == 0).all()
+        _rows_close(got.cpu()[~keyless], want[~keyless], 4 * 2 ** -8)
 
 
 def test_paged_attention_under_capture_with_other_lengths():
