@@ -107,8 +107,8 @@ inline void lay_out(ExpandedPlan& e, int64_t tiles, int H_KV, int D) {
 // What a batch takes with pieces of at most `piece` tiles (those of the kernel: 32 keys at 256 coordinates), in ns, for the choice
 // between them: the longest piece, slowed down while it shares its CU, or the share of a place; and what the rows of `split` pieces
 // cost in the combine, written and read.  Tiles as measured on an empty chip, and beside a second workgroup twice that; rows at 3.5
-// TB/s.  16 heads over 4 of 256 coordinates x 3001 tokens stay whole (144 us; in pieces of the share 151), 32 over 8 of 128 x 1500
-// too (46 and 53); 8 over 1 x 4000 run in pieces (82 whole, 71).
+// TB/s.  16 heads over 4 of 256 coordinates x 3001 tokens stay whole (144 us, 136 to 150 by card; in pieces of the share 151 beside the 144), 32
+// over 8 of 128 x 1500 too (46 and 53); 8 over 1 x 4000 run in pieces (82 whole, 71).
 constexpr int kPieceTiles = 4;                  // the shortest pieces, in tiles of 64 keys
 struct PieceCost {
     int tile, rows;
