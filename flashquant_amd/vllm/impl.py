@@ -110,7 +110,8 @@ def _make_impl_class() -> type:
         partials (of the prefill at most 65 MiB) and, where many queries share their keys, these as
         fp16, which the prefill sizes from the columns of the block table (about 7 times the bytes of
         the queries and 0.2 GiB, at most 2.2 GiB).  The profiling run launches nothing and does not
-        see it.  Where it cannot be had, the prefill reads the packed pages instead."""
+        see it; a captured graph keeps its own.  Where it cannot be had, the prefill reads the packed
+        pages instead, each call after an attempt."""
 
         def __init__(self, *args, **kwargs) -> None:
             super().__init__(*args, **kwargs)

@@ -116,9 +116,9 @@ def attention_on_packed_rows(q, kp, kn, vp, vn, c, r, is_causal=False):
     return out
 
 
-def prefill_on_packed_rows(q, cu, max_q, cache, table, sl, c, r, hkv, d, bs, causal=True):
+def prefill_on_packed_rows(q, cu, max_q, cache, table, sl, c, r, hkv, d, bs, causal=True, out=None):
     """fq_paged_tq4_prefill_split with room for contexts in pieces alone."""
-    out, r = torch.zeros_like(q), r.contiguous()
+    out, r = torch.zeros_like(q) if out is None else out, r.contiguous()
     ws, n = _pieces_room(table.shape[0], max_q, table.shape[1] * bs, q.shape[1], hkv, d, 0, q.device)
     st = _entry("fq_paged_tq4_prefill_split")(*_args(q, cu, cache, table, sl, c, c, r, 0, out, table.shape[0], max_q, q.shape[1], hkv, d, bs,
                                                      table.shape[1], (cache.shape[0],), d ** -0.5, int(causal), _dtype(q), (q.shape[0],), ws), n,

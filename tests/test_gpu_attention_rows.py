@@ -26,12 +26,18 @@ def test_paged_prefill_output_at_any_alignment(hq, hkv, d, dtype):
     cu = torch.tensor([0] + list(torch.tensor(ql).cumsum(0)), dtype=torch.int32).to(DEV)
     args = (cu, max(ql), cache.to(DEV), table.to(DEV), sl.to(DEV), c.to(DEV), c.to(DEV))
     want = K.paged_tq4_prefill(q, *args, r.to(DEV), hkv, d, bs)
+    packed = prefill_on_packed_rows(q, *args[:-1], r.to(DEV), hkv, d, bs)                  # (keys and values not expanded)
     for shift in (1, 4):
-        room = torch.full((q.numel() + 16,), 7.0, dtype=dtype, device=DEV)
-        K.paged_tq4_prefill(q, *args, r.to(DEV), hkv, d, bs, out=room[shift:shift + q.numel()].view_as(q))
-        torch.cuda.synchronize()
-        assert torch.equal(room[shift:shift + q.numel()].view_as(q), want)
-        assert (room[:shift] == 7).all() and (room[shift + q.numel():] == 7).all()
+        for same in (want, packed):
+            room = torch.full((q.numel() + 16,), 7.0, dtype=dtype, device=DEV)
+            out = room[shift:shift + q.numel()].view_as(q)
+            if same is want:
+                K.paged_tq4_prefill(q, *args, r.to(DEV), hkv, d, bs, out=out)
+            else:
+                prefill_on_packed_rows(q, *args[:-1], r.to(DEV), hkv, d, bs, out=out)
+            torch.cuda.synchronize()
+            assert torch.equal(out, same)
+            assert (room[:shift] == 7).all() and (room[shift + q.numel():] == 7).all()
     other = K.paged_tq4_prefill(q, *args, r.t().contiguous().to(DEV).t(), hkv, d, bs)      # the matrix in the other layout
     assert torch.equal(other, want)
 
@@ -131,10 +137,13 @@ def test_paged_prefill_order_and_split(batch, hq, hkv, d):
         out = torch.full_like(q, 7.0).to(DEV)
         K.paged_tq4_prefill(q.to(DEV), cu.to(DEV), max(ql), cache.to(DEV), table.to(DEV), sl.to(DEV), c.to(DEV), c.to(DEV),
                             r.to(DEV), hkv, d, bs, causal=causal, out=out)
-        _close(out, want, dtype)
-        for s, n in enumerate(kv):
-            if n == 0:
-                assert (out[int(cu[s]):int(cu[s + 1])] == 0).all()
+        packed = prefill_on_packed_rows(q.to(DEV), cu.to(DEV), max(ql), cache.to(DEV), table.to(DEV), sl.to(DEV), c.to(DEV), r.to(DEV), hkv, d,
+                                        bs, causal=causal, out=torch.full_like(q, 7.0).to(DEV))
+        for got in (out, packed):
+            _close(got, want, dtype)
+            for s, n in enumerate(kv):
+                if n == 0:
+                    assert (got[int(cu[s]):int(cu[s + 1])] == 0).all()
 
 
 def test_split_attention_under_capture():
@@ -176,6 +185,7 @@ def test_head_dim_256_rows(b, hq, hkv, nq, nkv, causal, dtype):
     _close(room, want, dtype)
     other = K.fused_tq_attention(*dev[:-1], r.t().contiguous().to(DEV).t(), is_causal=causal)      # the matrix in the other layout
     assert torch.equal(other, room)
+    _close(attention_on_packed_rows(*dev[:5], *dev[6:], is_causal=causal), want, dtype)
 
 
 @pytest.mark.parametrize("hq,hkv", [(8, 2), (5, 1)])
@@ -497,6 +507,7 @@ def test_every_row_once_at_the_edges_of_the_search(batch, hq, hkv, d):
     q = torch.randn(sum(ql), hq, d, generator=torch.Generator().manual_seed(92)).to(dtype)
     cu = torch.tensor([0] + list(torch.tensor(ql).cumsum(0)), dtype=torch.int32)
     want = O.paged_prefill(q, cu, cache, table, sl, c, c, r, hkv, d, bs)
-    got = K.paged_tq4_prefill(q.to(DEV), cu.to(DEV), max(ql), cache.to(DEV), table.to(DEV), sl.to(DEV), c.to(DEV), c.to(DEV),
-                              r.to(DEV), hkv, d, bs, out=torch.full_like(q, 7.0).to(DEV))
+    args = (q.to(DEV), cu.to(DEV), max(ql), cache.to(DEV), table.to(DEV), sl.to(DEV), c.to(DEV))
+    got = K.paged_tq4_prefill(*args, c.to(DEV), r.to(DEV), hkv, d, bs, out=torch.full_like(q, 7.0).to(DEV))
     _close(got, want, dtype)
+    _close(prefill_on_packed_rows(*args, r.to(DEV), hkv, d, bs, out=torch.full_like(q, 7.0).to(DEV)), want, dtype)
