@@ -37,6 +37,32 @@ extern "C" int pieces(int workgroups, int tiles) {
 extern "C" int64_t share(int64_t workgroups, int first, int last, int H_KV, int places) {
     return share_of_work(work_of(workgroups, first, last), H_KV, places);
 }
+// against workgroups and their tiles counted one by one; how many differ
+extern "C" int counted(int n_q, int n_kv, int G, int D, int causal) {
+    const int TS = D == 256 ? 5 : 6, units = (n_q + 31) / 32 * G, W = (units + 3) / 4, keys = causal && n_kv > n_q ? n_q : n_kv;
+    const int tiles = (keys + (1 << TS) - 1) >> TS;
+    const ContiguousWork work{W, tiles, (1 << TS) / 32 * G, causal != 0};
+    auto tiles_of = [&](int x) {
+        int pos = 32 * ((4 * x + 3 < units - 1 ? 4 * x + 3 : units - 1) / G) + 31;
+        pos = pos < n_q - 1 ? pos : n_q - 1;
+        return causal && (pos >> TS) + 1 < tiles ? (pos >> TS) + 1 : tiles;
+    };
+    int64_t all = 0;
+    int wrong = tiles_of(W - 1) != tiles;
+    for (int x = 0; x < W; ++x) all += tiles_of(x);
+    wrong += all != work.all();
+    for (int i = 0; i < kPieceChoices; ++i) {
+        const int piece = piece_choice(i, tiles, kPieceTiles << (6 - TS));
+        int64_t items = 0, split = 0;
+        for (int x = 0; x < W; ++x) {
+            const int k = (tiles_of(x) + piece - 1) / piece;
+            items += k;
+            split += k > 1 ? k : 0;
+        }
+        wrong += items != work.items(piece) || split != work.split(piece);
+    }
+    return wrong;
+}
 """
 
 
@@ -90,3 +116,12 @@ def test_the_share_of_large_batches(plans):
     f.restype, f.argtypes = ctypes.c_int64, [ctypes.c_int64] + [ctypes.c_int] * 4
     for w, first, last, hkv in ((37500, 120000, 125000, 1), (1 << 20, 1, 1 << 18, 1), (1 << 20, 1 << 18, 1 << 18, 8), (3, 1, 4, 5)):
         assert f(w, first, last, hkv, 512) == (((w * (first + last) + 1) // 2) * hkv + 511) // 512
+
+
+def test_workgroups_and_pieces_are_counted_right(plans):
+    sizes = [(nq, nkv) for nq in (17, 31, 32, 33, 64, 65, 100, 128, 129, 1000, 3001, 4096, 5003) for nkv in (1, 31, 33, 64, 65, 129, nq - 1, nq, nq + 1, 2 * nq + 7)]
+    for nq, nkv in sizes:
+        for g in (1, 2, 3, 4, 5, 8, 12, 32):
+            for d in (64, 128, 256):
+                for causal in (0, 1):
+                    assert plans.counted(nq, nkv, g, d, causal) == 0, (nq, nkv, g, d, causal)
